@@ -14,12 +14,14 @@
 // k-steps when at most 16 / AG rows are in use (the spare lanes carry the other
 // steps' data and a row rotation hands it over).
 //
+// Up to 8 rows the products with an epilogue mostly run the kernel of gemm_rows.hip instead.
 // With 32,768 weight rows or more and up to 16 rows of A (the output head) a second kernel runs, in which
 // waves own whole weight tiles (gemm_wide_kernel below).
 //
 // 16x16x32 layout (lane l): A[i = l%16][k = 8(l/16)..+7], B[k = 8(l/16)..+7][j = l%16],
 // D[i = 4(l/16) + e][j = l%16], e = 0..3.
 #include "common.h"
+#include "gemm_rows.h"
 #include "infinicore_infer_variants.h"
 #include <utility>
 
@@ -45,44 +47,7 @@ __device__ __forceinline__ void load8(const uint16_t* __restrict__ p, int valid,
     }
 }
 
-// What the fused projection + rotary + cache-write epilogue needs beside the product.
-struct RopeEpilogue {
-    const int* positions;      // [M]
-    const int* slots;          // [M] token slot in the cache (page * page_size + offset), < 0: no write
-    const float* cos_t;        // [max_pos, dh/2]
-    const float* sin_t;
-    void* kcache;              // [pages, nkvh, page_size, dh]
-    void* vcache;
-    int nh, nkvh, dh, page_size;
-    int rr;                    // weight rows per tile that are used: 16, 8 or 4 (few heads: smaller tiles make more blocks)
-};
-
-// A norm split over two products (M <= 16).  The product BEFORE the norm (EPI == 3) owns the
-// residual add: h = x + rscale * (its result), written back to x; it stores y = h * g (g: the
-// norm's weight) instead of its result, and per column block the sums of h^2 of every row.  The
-// product AFTER the norm takes y as its operand and multiplies row m of its result by
-// rsqrt(sum over the column blocks / width + eps): the norm's row factor commutes with the product.
-constexpr int kMaxSumParts = 256;
 constexpr int kOwnKFrom = 8192;          // from this K on the waves of the few-row product own contiguous runs of k-steps
-struct NormFuse {
-    const float* ss_in;        // [n_parts_in, 16] sums of squares per column block and row; nullptr: rows are normed already
-    int n_parts_in;            // <= kMaxSumParts
-    float inv_width, eps;
-    float* x;                  // EPI == 3: float32 residual stream [M, N], row stride ldx, updated in place
-    int ldx;
-    const float* g;            // [N]
-    float rscale;
-    float* ss_out;             // [gridDim.x, 16]
-    int act;                   // plain store only: 0 none, else the product (rounded to its type first, as when stored) goes
-                               // through an activation: 1 relu(z)^2, 2 gelu_tanh(z), 3 silu(z)
-    float glu_limit, glu_slope; // the gated epilogue: limit > 0: the unit with bounded branches instead of up * silu(gate)
-};
-
-__device__ __forceinline__ float gemm_act(float z, int act) {
-    if (act == 1) { const float r = fmaxf(z, 0.f); return r * r; }
-    if (act == 2) return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
-    return z / (1.0f + expf(-z));
-}
 
 // lane i of a row of 16 lanes takes the value of lane (i + S) % 16 (a DPP row rotation, no LDS)
 template <int S> __device__ __forceinline__ v4s row_from_above(v4s v) {
@@ -922,6 +887,7 @@ static int gemm_nt_impl(const void* A, int a_dtype, const void* W, int w_dtype, 
         // 16 waves a block throughout; up to 4 rows 4 k-steps in flight, above that 2 (from a sweep over the O and
         // down projections of the 1B..8B shapes with one block per compute unit)
         const int blocks = ic_gemm_nt_residual_parts(N);
+        if (t_variant.lines && gemm_rows_launch(3, A, W, C, M, N, K, lda, ldw, ldc, alpha, RopeEpilogue{}, nf, blocks, stream)) return ic_launch_status();
         // rows of 16 KB and more: a wave owns one stretch of every row (8B shape's down projection: 36 -> 30 us)
         // up to 8 (4) rows one load of the token operand serves 2 (4) k-steps
 #define IC_RES(UN, OWN, AG) launch_gemm<bf16, 1, 1, 16, UN, 3, OWN, AG>(A, W, C, M, N, K, lda, ldw, ldc, alpha, aligned, nf, stream, blocks)
@@ -933,6 +899,8 @@ static int gemm_nt_impl(const void* A, int a_dtype, const void* W, int w_dtype, 
         return ic_launch_status();
     }
     if (c_mode == 1) {
+        if (t_variant.lines && c_dtype == IC_BF16 && gemm_rows_launch(1, A, W, C, M, N, K, lda, ldw, ldc, 1.0f, RopeEpilogue{}, nf, 0, stream))
+            return ic_launch_status();
         const int tiles = (N / 2 + 15) / 16, cus = compute_units();
         // Between one and two 16-column tiles per compute unit the second round of blocks would be part-filled:
         // then every block takes ceil(columns / units) columns (two tiles, the second one partial) and one round does it.
@@ -989,6 +957,8 @@ IC_EXPORT int ic_gemm_qkv_rope(const void* A, const void* W, void* C, int M, int
     const int N = (nh + 2 * nkvh) * dh;
     NormFuse nf{};
     if (!norm_fuse_args(row_factor, nullptr, M, N, K, IC_BF16, 0, nf)) return IC_ERR_ARG;
+    if (!t_variant.rope_tile_rows && dh % 16 == 0 && gemm_rows_launch(2, A, W, C, M, N, K, lda, ldw, ldc, 1.0f, rope, nf, 0, stream))
+        return ic_launch_status();
     const int blocks = pairs16 * (16 / rr);
     dim3 grid(blocks, 1);
 #define IC_ROPE(WPB, UN, AL)                                                                             \
