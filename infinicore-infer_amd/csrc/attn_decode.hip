@@ -284,8 +284,8 @@ attn_decode_reduce_kernel(const float* __restrict__ part_acc, const float* __res
 // Grouped queries on the matrix cores (bfloat16): the query heads that share a kv head are the
 // columns of one 16-wide tile, so keys and values are read once for the whole group.
 //
-// Same grid and partial-result layout as above.  A wave owns tiles of 32 keys of the block's
-// share (tile i -> wave i % 4).  S^T = K Q^T with v_mfma_f32_16x16x32_bf16, keys as rows: the K
+// Same grid and partial-result layout as above, 4 or 8 waves.  A wave owns tiles of 32 keys of the block's
+// share (tile i -> wave i % waves).  S^T = K Q^T with v_mfma_f32_16x16x32_bf16, keys as rows: the K
 // operand comes straight from memory in operand layout (lane l: key l%16, dims 8(l/16)..+7 of a
 // 32-dim chunk).  A lane then holds 4+4 keys of ONE head (l%16), so the running softmax needs two
 // cross-lane steps.  O^T = V^T P^T: P^T is already the B operand (slot (l/16, e) stands for key
@@ -304,8 +304,8 @@ union GqFrag {
     gq_bf16x8 v;
 };
 
-template <int DH, bool STAGED>
-__global__ void __launch_bounds__(kDecThreads)
+template <int DH, bool STAGED, int WV>
+__global__ void __launch_bounds__(64 * WV)
 attn_decode_gqa_kernel(const uint16_t* __restrict__ q, int q_stride,
                        const uint16_t* __restrict__ kcache, const uint16_t* __restrict__ vcache,
                        const int* __restrict__ block_tables, int bt_stride,
@@ -318,8 +318,8 @@ attn_decode_gqa_kernel(const uint16_t* __restrict__ q, int q_stride,
     constexpr int ND = DH / 16;                    // 16-dim chunks of the output
     constexpr int VS = DH + 8;                     // LDS row stride of a V tile (elements)
     constexpr int NV = kGqaKeys * (DH / 8) / 64;   // 16-byte V loads per lane and tile
-    __shared__ __attribute__((aligned(16))) uint16_t Vs[kDecWaves][kGqaKeys * VS];
-    __shared__ float sm_ml[kDecWaves][16][2];
+    __shared__ __attribute__((aligned(16))) uint16_t Vs[WV][kGqaKeys * VS];
+    __shared__ float sm_ml[WV][16][2];
     __shared__ int pages[kDecMaxPages];
     static_assert(sizeof(uint16_t) * kGqaKeys * VS >= sizeof(float) * 16 * DH, "merge buffer fits in the V tiles");
     float* sm_o = reinterpret_cast<float*>(&Vs[0][0]);       // [waves][16 heads][DH] after the key loop
@@ -347,7 +347,7 @@ attn_decode_gqa_kernel(const uint16_t* __restrict__ q, int q_stride,
     const int page_lo = lo / page_size;
     const int n_pages = (hi > lo) ? (hi - 1) / page_size - page_lo + 1 : 0;
     if (STAGED)
-        for (int i = threadIdx.x; i < n_pages; i += kDecThreads) pages[i] = bt[page_lo + i];
+        for (int i = threadIdx.x; i < n_pages; i += 64 * WV) pages[i] = bt[page_lo + i];
     __syncthreads();
     auto row_of = [&](int key) -> size_t {
         const int lp = key / page_size;
@@ -356,7 +356,7 @@ attn_decode_gqa_kernel(const uint16_t* __restrict__ q, int q_stride,
     };
 
     const int n_tiles = (hi > lo) ? (hi - lo + kGqaKeys - 1) / kGqaKeys : 0;
-    const int rounds = (n_tiles + kDecWaves - 1) / kDecWaves;
+    const int rounds = (n_tiles + WV - 1) / WV;
 
     for (int h0 = 0; h0 < g; h0 += 16) {
         // Q^T operand: head lr of this chunk, dims 32c + 8 lg .. +7
@@ -411,7 +411,7 @@ attn_decode_gqa_kernel(const uint16_t* __restrict__ q, int q_stride,
         // moving LDS accesses across it).
         fetch(wave);
         for (int r = 0; r < rounds; ++r) {
-            const int tile = r * kDecWaves + wave;
+            const int tile = r * WV + wave;
             if (tile >= n_tiles) break;             // uniform in the wave
             const int kt = lo + tile * kGqaKeys;
             __builtin_amdgcn_wave_barrier();
@@ -435,7 +435,7 @@ attn_decode_gqa_kernel(const uint16_t* __restrict__ q, int q_stride,
                 for (int c = 0; c < NC; ++c)
                     sacc[s2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kreg[s2][c].v, qf[c].v, sacc[s2], 0, 0, 0);
             }
-            fetch(tile + kDecWaves);                // the next tile's loads fly during the rest of this one
+            fetch(tile + WV);                // the next tile's loads fly during the rest of this one
             float sv[8];
             float mloc = -INFINITY;
 #pragma unroll
@@ -486,14 +486,14 @@ attn_decode_gqa_kernel(const uint16_t* __restrict__ q, int q_stride,
             for (int e = 0; e < 4; ++e) sm_o[(wave * 16 + lr) * DH + 16 * c + 4 * lg + e] = oacc[c][e];
         if (lg == 0) { sm_ml[wave][lr][0] = m; sm_ml[wave][lr][1] = l; }
         __syncthreads();
-        for (int idx = threadIdx.x; idx < 16 * DH; idx += kDecThreads) {
+        for (int idx = threadIdx.x; idx < 16 * DH; idx += 64 * WV) {
             const int j = idx / DH, d = idx - j * DH;
             if (h0 + j >= g) continue;
             float mm = -INFINITY;
-            for (int w = 0; w < kDecWaves; ++w) mm = fmaxf(mm, sm_ml[w][j][0]);
+            for (int w = 0; w < WV; ++w) mm = fmaxf(mm, sm_ml[w][j][0]);
             float a = 0.f, ll = 0.f;
             if (mm != -INFINITY) {
-                for (int w = 0; w < kDecWaves; ++w) {
+                for (int w = 0; w < WV; ++w) {
                     const float cw = __builtin_amdgcn_exp2f(sm_ml[w][j][0] - mm);
                     a += sm_o[(w * 16 + j) * DH + d] * cw;
                     ll += sm_ml[w][j][1] * cw;
@@ -529,8 +529,17 @@ static int launch_decode(const void* q, int q_stride, void* out, int out_stride,
                        (const TQ*)vcache, block_tables, bt_stride, tok_list, token_req, positions, part_acc, \
                        part_ml, nh, nkvh, page_size, scale, window, nsplit, (TQ*)direct, out_stride)
     if (ic_attn_decode_on_matrix_cores(sizeof(T) == 2 ? IC_BF16 : IC_F32, nh, nkvh)) {
-        if (staged) IC_DEC_LAUNCH((attn_decode_gqa_kernel<DH, true>), uint16_t);
-        else IC_DEC_LAUNCH((attn_decode_gqa_kernel<DH, false>), uint16_t);
+        // Eight waves where a block's share of the keys is long for four and the blocks are too few to fill the units anyway: one
+        // split of few (row, kv head) pairs (24:8 heads of 64, 258 keys: 1 row 6.4 -> 5.6 us, 8 rows 7.0 -> 6.5; 512 keys 8.2 -> 7.2;
+        // with 320 pairs 19.9 -> 22.0), and many splits of heads of 128 (32:2 heads, 4 rows, 16,385 keys in 32 splits: 24.3 -> 22.1;
+        // in 16 splits of 2,000 keys 11.3 -> 11.8).
+        const bool eight = DH == 64 ? nsplit == 1 && n_tok * nkvh <= 128 : nsplit >= 24;
+        if (eight) {
+            block = dim3(512);
+            if (staged) IC_DEC_LAUNCH((attn_decode_gqa_kernel<DH, true, 8>), uint16_t);
+            else IC_DEC_LAUNCH((attn_decode_gqa_kernel<DH, false, 8>), uint16_t);
+        } else if (staged) IC_DEC_LAUNCH((attn_decode_gqa_kernel<DH, true, 4>), uint16_t);
+        else IC_DEC_LAUNCH((attn_decode_gqa_kernel<DH, false, 4>), uint16_t);
     } else if (nh == nkvh) {
         if (staged) IC_DEC_LAUNCH((attn_decode_split_kernel<T, DH, 1, true>), T);
         else IC_DEC_LAUNCH((attn_decode_split_kernel<T, DH, 1, false>), T);

@@ -446,7 +446,7 @@ IC_EXPORT int ic_decoder_forward(IcDecoder* decoder, const IcStepBatch* batch, v
 
 // ---- the key split of single-token rows --------------------------------------------------------------------------
 // One split writes the result itself; more cost a second kernel (about 5 us), so short contexts are never split: up to
-// 1,024 keys with one query head per kv head (a wave walks keys with vector instructions), up to 256 with grouped query
+// 1,024 keys with one query head per kv head (a wave walks keys with vector instructions), up to 256 or 512 with grouped query
 // heads on the matrix cores (its blocks walk 128 keys a round).  Beyond that, one head per kv head: few (row, kv head)
 // pairs want about 1.75 blocks per compute unit but at least 384 keys a block; a middling number of pairs already draws
 // the full bandwidth unsplit up to 2,048 keys; many pairs want about 3.4 blocks per unit.  Grouped heads: a wave has a
@@ -462,8 +462,9 @@ IC_EXPORT int ic_attn_decode_splits(int n_decode_rows, int n_heads, int n_kv_hea
         // The grouped-query kernel: the same kind of model as below with constants of its own (fitted to 215 shapes of
         // 24:8 and 16:4 heads of 64, 32:2 and 32:8 of 128, 1..64 rows, 600..16,500 keys: 1.1 % from the best count on
         // average, worst 9 %; "128 / head size blocks a unit", which it replaces, 1.9 % and 32 %).  Up to 256 keys it
-        // does not split.
-        if (keys <= 256) return 1;
+        // does not split; with heads of 64 and few pairs, which eight waves of one block then walk, up to 512 (1 row of 24:8 heads over
+        // 258 keys: 8 splits 7.3 us, one split 5.6; over 512: 7.3 and 7.2; 8 rows over 258 keys: 7.8 and 6.5).
+        if (keys <= 256 || (keys <= 512 && head_dim == 64 && base <= 128)) return 1;
         const double stream_us = (double)base * keys * std::max(1, head_dim) * 2.0 * std::max(1, elem_bytes) / (6.42e6 * cu / 256.0);
         const double group = (double)std::max(1, n_heads) / std::max(1, n_kv_heads);
         int best = 1;
