@@ -16,9 +16,10 @@
 // O^T = V^T P^T accumulator r of S^T is the B operand as it stands: it holds key 8 (r / 4) + r % 4 in the
 // lower half of the wave and the key four further on in the upper half.
 //
-// Simple on purpose (the 32-bit path is for checking): one wave group, no cut walks, a tile is loaded
-// when it is needed (the float32 matrix instructions take 16 times as long as the bfloat16 ones, so the
-// loop is bound by them, not by the loads).
+// The float32 matrix instructions take 16 times as long as the bfloat16 ones, so what counts is that every SIMD has some: with
+// few tiles (a portion of 512 tokens of 24 heads makes 96) a block of four waves takes only 64 or 32 of a tile's rows and its waves
+// share the keys between them, KG key groups of 32 keys a step, merged through LDS at the end.  The next step's keys and
+// values are on their way in registers while this one's are used.
 //
 // Cache layout of one layer: K and V planes [num_pages, n_kv_heads, page_size, head_dim].
 #include "common.h"
@@ -27,10 +28,10 @@ typedef float f32_v16 __attribute__((ext_vector_type(16)));
 
 constexpr int kF32Threads = 256;
 constexpr int kF32Rows = 128;     // query rows per block (must equal the bfloat16 kernel's tile height: one tile list serves both)
-constexpr int kF32Keys = 64;      // keys per step
 
-template <int DH>
-__global__ void __launch_bounds__(kF32Threads, 2)
+// KG key groups: 1 (a step of 64 keys, every wave all of them), 2 (64 keys, 32 a group) or 4 (128 keys, 32 a group).
+template <int DH, int KG>
+__global__ void __launch_bounds__(kF32Threads, (KG == 4 || DH == 128) ? 1 : 2)
 attn_prefill_f32_kernel(const float* __restrict__ q, int q_stride, float* __restrict__ out, int out_stride,
                         const float* __restrict__ kcache, const float* __restrict__ vcache,
                         const int* __restrict__ block_tables, int bt_stride, const int4* __restrict__ tiles,
@@ -39,17 +40,27 @@ attn_prefill_f32_kernel(const float* __restrict__ q, int q_stride, float* __rest
     constexpr int ND = DH / 32;           // 32-row tiles of O^T
     constexpr int KS = DH + 4;            // row stride of the K tile (floats): 16-byte reads of 16 consecutive rows cover all banks
     constexpr int VS = DH + 8;            // row stride of the V tile: rows four apart (the wave's two halves) fall into different banks
-    constexpr int NL = kF32Keys * (DH / 4) / kF32Threads;     // 16-byte loads per thread and plane
-    __shared__ __attribute__((aligned(16))) float Ks[kF32Keys * KS];
-    __shared__ __attribute__((aligned(16))) float Vs[kF32Keys * VS];
+    constexpr int KEYS = KG == 4 ? 128 : 64;                  // keys per step
+    constexpr int GK = KG == 1 ? 64 : 32;                     // of them, a group's
+    constexpr int NT = GK / 32;                               // 32-key tiles of a group
+    constexpr int RW = 4 / KG;                                // waves that own rows, 32 each
+    constexpr int NL = KEYS * (DH / 4) / kF32Threads;         // 16-byte loads per thread and plane
+    constexpr int MF = 2 + ND * 16;                           // floats a lane hands over at the end
+    static_assert(KG == 1 || KEYS * (KS + VS) >= (4 - RW) * 64 * MF, "the merge buffer fits in the tiles");
+    __shared__ __attribute__((aligned(16))) float tile_mem[KEYS * (KS + VS)];
+    float* const Ks = tile_mem;
+    float* const Vs = tile_mem + KEYS * KS;
 
-    const int slot = (int)blockIdx.x;                   // tile-major: all heads of the longest tile first
+    const int slot = (int)blockIdx.x / KG, sub = (int)blockIdx.x % KG;      // tile-major: all heads of the longest tile first
     const int h = slot % nh;
     const int4 tile = tiles[slot / nh];
-    const int req = tile.x, row0 = tile.y, n_rows = tile.z, pos0 = tile.w;
+    const int skip = 32 * RW * sub;                           // rows of the tile before this block's
+    const int req = tile.x, row0 = tile.y + skip, pos0 = tile.w + skip;
+    const int n_rows = tile.z - skip < 32 * RW ? tile.z - skip : 32 * RW;
+    if (n_rows <= 0) return;                                  // (the whole block)
     const int kvh = h / (nh / nkvh);
     const int* bt = block_tables + (size_t)req * bt_stride;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) % RW, grp = (tid >> 6) / RW;
     const int lq = lane & 31, half = lane >> 5;
     const int page_size = 1 << page_shift, page_mask = page_size - 1;
 
@@ -62,7 +73,7 @@ attn_prefill_f32_kernel(const float* __restrict__ q, int q_stride, float* __rest
     const int last_key = pos0 + n_rows - 1;
     int first_key = 0;
     if (window > 0 && pos0 - window + 1 > 0) first_key = pos0 - window + 1;
-    const int kb_begin = (first_key / kF32Keys) * kF32Keys;
+    const int kb_begin = (first_key / KEYS) * KEYS;
 
     // Q operands: Q[query lq][HALF * half + c], scores in units of log 2 (the softmax scale folded in)
     float qf[HALF];
@@ -87,34 +98,48 @@ attn_prefill_f32_kernel(const float* __restrict__ q, int q_stride, float* __rest
     const float* vbase = vcache + (size_t)kvh * head_stride;
     const size_t page_stride = (size_t)nkvh * head_stride;
 
-    for (int kb = kb_begin; kb <= last_key; kb += kF32Keys) {
-        __syncthreads();                                // the previous step's readers are done
-        // the step's 64 keys and values into LDS as rows (keys outside the tile's range as zeros: they are masked)
+    // a step's keys and values (those outside the tile's range as zeros: they are masked)
+    float4 kr[NL], vr[NL];
+    auto fetch = [&](int kb) {
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
             const int idx = tid + i * kF32Threads;
             const int key = idx / (DH / 4), quad = idx - key * (DH / 4);
             const int ka = kb + key;
-            float4 kv = make_float4(0.f, 0.f, 0.f, 0.f), vv = kv;
+            kr[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+            vr[i] = kr[i];
             if (ka <= last_key && ka >= first_key) {
                 const size_t off = (size_t)bt[ka >> page_shift] * page_stride + (size_t)(ka & page_mask) * DH + quad * 4;
-                kv = *reinterpret_cast<const float4*>(kbase + off);
-                vv = *reinterpret_cast<const float4*>(vbase + off);
+                kr[i] = *reinterpret_cast<const float4*>(kbase + off);
+                vr[i] = *reinterpret_cast<const float4*>(vbase + off);
             }
-            *reinterpret_cast<float4*>(&Ks[key * KS + quad * 4]) = kv;
-            *reinterpret_cast<float4*>(&Vs[key * VS + quad * 4]) = vv;
+        }
+    };
+    fetch(kb_begin);
+    for (int kb = kb_begin; kb <= last_key; kb += KEYS) {
+        __syncthreads();                                // the previous step's readers are done
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            const int idx = tid + i * kF32Threads;
+            const int key = idx / (DH / 4), quad = idx - key * (DH / 4);
+            *reinterpret_cast<float4*>(&Ks[key * KS + quad * 4]) = kr[i];
+            *reinterpret_cast<float4*>(&Vs[key * VS + quad * 4]) = vr[i];
         }
         __syncthreads();
-        if (!wave_ok || kb > wave_last) continue;       // nothing this wave may see
-        if (window > 0 && kb + kF32Keys - 1 < wave_first - window + 1) continue;
+        if (kb + KEYS <= last_key) fetch(kb + KEYS);    // in flight while this step is used
+        const int kt = kb + GK * grp;                   // this group's keys
+        if (!wave_ok || kt > wave_last) continue;       // nothing this wave may see
+        if (window > 0 && kt + GK - 1 < wave_first - window + 1) continue;
+        const float* const Kg = Ks + GK * grp * KS;
+        const float* const Vg = Vs + GK * grp * VS;
 
-        // ---- S^T = K Q^T : two tiles of 32 keys ----------------------------------------------------------
-        f32_v16 sacc[2];
+        // ---- S^T = K Q^T : tiles of 32 keys ----------------------------------------------------------
+        f32_v16 sacc[NT];
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
+        for (int tt = 0; tt < NT; ++tt) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) sacc[tt][r] = 0.f;
-            const float* kp = &Ks[(32 * tt + lq) * KS + HALF * half];
+            const float* kp = &Kg[(32 * tt + lq) * KS + HALF * half];
 #pragma unroll
             for (int c = 0; c < HALF; c += 4) {
                 const float4 kx = *reinterpret_cast<const float4*>(kp + c);
@@ -125,18 +150,18 @@ attn_prefill_f32_kernel(const float* __restrict__ q, int q_stride, float* __rest
             }
         }
         // ---- mask (only steps that touch the diagonal, the window's edge, or keys before the window) --------
-        const bool need_mask = (kb + kF32Keys - 1 > wave_first) || (window > 0);
+        const bool need_mask = (kt + GK - 1 > wave_first) || (window > 0);
         if (need_mask) {
-            // key kb + 4 half + e of this lane's accumulator (e a constant per accumulator) is seen when e <= lim
-            const int lim = qpos - kb - 4 * half;
+            // key kt + 4 half + e of this lane's accumulator (e a constant per accumulator) is seen when e <= lim
+            const int lim = qpos - kt - 4 * half;
 #pragma unroll
-            for (int tt = 0; tt < 2; ++tt)
+            for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
                     if (32 * tt + 8 * (r >> 2) + (r & 3) > lim) sacc[tt][r] = -INFINITY;
             if (window > 0) {
 #pragma unroll
-                for (int tt = 0; tt < 2; ++tt)
+                for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
                     for (int r = 0; r < 16; ++r)
                         if (32 * tt + 8 * (r >> 2) + (r & 3) <= lim - window) sacc[tt][r] = -INFINITY;
@@ -145,7 +170,7 @@ attn_prefill_f32_kernel(const float* __restrict__ q, int q_stride, float* __rest
         // ---- running softmax, base 2 -------------------------------------------------------------------
         float mloc = sacc[0][0];
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
+        for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
             for (int r = 0; r < 16; ++r) mloc = fmaxf(mloc, sacc[tt][r]);
         mloc = fmaxf(mloc, __shfl_xor(mloc, 32, kWave));
@@ -154,7 +179,7 @@ attn_prefill_f32_kernel(const float* __restrict__ q, int q_stride, float* __rest
         const float corr = exp2f(m - m_use);            // 0 on the first step (m = -inf)
         float rs = 0.f;
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
+        for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const float p = exp2f(sacc[tt][r] - m_use);
@@ -171,16 +196,45 @@ attn_prefill_f32_kernel(const float* __restrict__ q, int q_stride, float* __rest
 
         // ---- O^T += V^T P^T : accumulator r of S^T is the B operand as it stands -------------------------------
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
+        for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const float* vp = &Vs[(32 * tt + 8 * (r >> 2) + 4 * half + (r & 3)) * VS + lq];
+                const float* vp = &Vg[(32 * tt + 8 * (r >> 2) + 4 * half + (r & 3)) * VS + lq];
 #pragma unroll
                 for (int dt = 0; dt < ND; ++dt)
                     oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vp[32 * dt], sacc[tt][r], oacc[dt], 0, 0, 0);
             }
     }
 
+    // ---- the key groups' states meet in group 0 (same lane, same rows) ---------------------------------------
+    if constexpr (KG > 1) {
+        __syncthreads();                                // the last step's readers are done
+        float* const mine = tile_mem + (size_t)((grp > 0 ? grp - 1 : 0) * RW + wave) * 64 * MF + lane;
+        if (grp > 0) {
+            mine[0] = m;
+            mine[64] = l;
+#pragma unroll
+            for (int i = 0; i < ND; ++i)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) mine[(2 + 16 * i + r) * 64] = oacc[i][r];
+        }
+        __syncthreads();
+        if (grp > 0) return;
+#pragma unroll
+        for (int g = 0; g < KG - 1; ++g) {
+            const float* const other = tile_mem + (size_t)(g * RW + wave) * 64 * MF + lane;
+            const float m1 = other[0], l1 = other[64];
+            const float m_new = fmaxf(m, m1);
+            const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
+            const float c0 = exp2f(m - m_use), c1 = exp2f(m1 - m_use);
+            l = l * c0 + l1 * c1;
+            m = m_new;
+#pragma unroll
+            for (int i = 0; i < ND; ++i)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) oacc[i][r] = oacc[i][r] * c0 + other[(2 + 16 * i + r) * 64] * c1;
+        }
+    }
     if (!row_ok) return;
     const float inv = 1.0f / l;
     float* op = out + (size_t)(row0 + my_row) * out_stride + (size_t)h * DH;
@@ -202,13 +256,20 @@ int ic_attn_prefill_f32_launch(const void* q, int q_stride, void* out, int out_s
         ((uintptr_t)vcache & 15) || ((uintptr_t)tiles & 15))
         return IC_ERR_ARG;
     const float sl2 = scale * 1.4426950408889634f;
-    dim3 grid((unsigned)nh * (unsigned)n_tiles), block(kF32Threads);
-#define IC_F32_LAUNCH(DD)                                                                                            \
-    hipLaunchKernelGGL((attn_prefill_f32_kernel<DD>), grid, block, 0, stream, (const float*)q, q_stride, (float*)out, \
-                       out_stride, (const float*)kcache, (const float*)vcache, block_tables, bt_stride,              \
+    // Key groups from the number of (tile, head) pairs; one / two / four groups, us (24:8, 36:36 heads of 64; 32:2 of 128): 96 pairs (509
+    // tokens after 130; the kernel without groups and loads ahead took 70) 58 / 38 / 35; 144 (512 tokens) 47 / 35 / 33; 192 (window of
+    // 300) 45 / 39 / 53; 288 (1,024 tokens) 100 / 78 / 88; 576 (2,048) 248 / 230 / 280; of 128: 96 (300 after 1,000) 215 / 138 / 162;
+    // 128 (512) 86 / 58 / 54; 384 (1,500) 268 / 295 / 356.
+    const long long pairs = (long long)nh * n_tiles;
+    const int kg = dh == 64 ? (pairs <= 160 ? 4 : pairs <= 700 ? 2 : 1) : (pairs <= 256 ? 2 : 1);
+    if (pairs * kg > 0x7fffffffLL) return IC_ERR_ARG;
+    dim3 grid((unsigned)nh * (unsigned)n_tiles * (unsigned)kg), block(kF32Threads);
+#define IC_F32_LAUNCH(DD, GG)                                                                                            \
+    hipLaunchKernelGGL((attn_prefill_f32_kernel<DD, GG>), grid, block, 0, stream, (const float*)q, q_stride, (float*)out, \
+                       out_stride, (const float*)kcache, (const float*)vcache, block_tables, bt_stride,                  \
                        (const int4*)tiles, n_tiles, nh, nkvh, page_shift, sl2, window)
-    if (dh == 64) IC_F32_LAUNCH(64);
-    else if (dh == 128) IC_F32_LAUNCH(128);
+    if (dh == 64) { if (kg == 1) IC_F32_LAUNCH(64, 1); else if (kg == 2) IC_F32_LAUNCH(64, 2); else IC_F32_LAUNCH(64, 4); }
+    else if (dh == 128) { if (kg == 1) IC_F32_LAUNCH(128, 1); else IC_F32_LAUNCH(128, 2); }
     else return IC_ERR_UNSUPPORTED;
 #undef IC_F32_LAUNCH
     return ic_launch_status();
