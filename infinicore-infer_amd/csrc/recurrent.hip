@@ -331,6 +331,174 @@ static int ssm_launch(int ni, dim3 grid, size_t lds, hipStream_t stream, const v
     return IC_OK;
 }
 
+constexpr int kSsmBatch = 4;           // tokens staged at a time, one a wave
+
+// The swap of lane halves of a and b and the sum of the two: lanes with bit D clear get a[i] + a[i + D], the others b[i - D] + b[i].
+template <int D> __device__ __forceinline__ float swap_halves(float a, float b) {
+    const auto r = D == 32 ? __builtin_amdgcn_permlane32_swap((unsigned)__float_as_int(a), (unsigned)__float_as_int(b), false, false)
+                           : __builtin_amdgcn_permlane16_swap((unsigned)__float_as_int(a), (unsigned)__float_as_int(b), false, false);
+    return __int_as_float((int)r[0]) + __int_as_float((int)r[1]);
+}
+
+// The same recurrence for the chunks of prompt portions (modes 1 and 2).  In the kernel above a thread owns one column, so every
+// token's B and C go through its wave's LDS port whole (32 + 32 values for 32 rows: the LDS, not the arithmetic, is what it waits
+// for), and every token costs two barriers.  Here a thread owns 4 columns x RT rows (2 RT + 4 values a token for 4 RT state entries),
+// tokens come TB at a time, the next ones' inputs in registers meanwhile, and what the thread rows of a wave add up to is
+// halved and summed with lane swaps.  All three passes of a portion, the kernel above / this one, us: 128 heads of 128 x 64, 3,304
+// tokens in chunks of 69: 1,574 / 748 (of them the chunks' states 87; multiply-adds alone 470 at 39 T a second); linear attention,
+// 2,048 tokens in chunks of 64, 32 heads of 128 x 128: 506 / 284, 36 heads of 64 x 64: 177 / 129; 500 tokens of 48 heads in chunks of 32:
+// 133 / 73.
+// Takes N = RT * 1,024 / P, P / 4 a power of two from 8 to 64.
+template <typename T, int RT, int mode>
+__global__ void __launch_bounds__(256)
+ssm_tile_kernel(const void* __restrict__ xbc, int x_stride, int x_f32, int in_act, const T* __restrict__ dt_raw, int dt_stride,
+                const float* __restrict__ dt_bias, const float* __restrict__ neg_a, const float* __restrict__ Dw,
+                int heads, int P, int G, float* __restrict__ y, const int* __restrict__ req_start, int chunk_len,
+                int max_chunks, float* __restrict__ scr_s, float* __restrict__ scr_a) {
+    constexpr int TB = kSsmBatch;
+    extern __shared__ __align__(16) float lds[];
+    const int h = blockIdx.x, r = blockIdx.y, ck = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int begin = req_start[r] + ck * chunk_len, end = min(req_start[r + 1], begin + chunk_len);
+    if (begin >= end) return;
+    const int cgs = P >> 2, N = RT * 256 / cgs, W = 2 * N + P;              // column groups; rows of the state; inputs of a token
+    const int cg = tid & (cgs - 1), n0 = RT * (tid / cgs), inner = heads * P, g = h / (heads / G);
+    float* const in = lds;                                                  // [TB][B (N), C (N), x (P)]
+    float* const step = in + TB * W;                                        // [TB][dt, decay]
+    float* const part = step + 2 * TB;                                      // [TB][4 waves][P]
+    float* const sc = scr_s + (((size_t)r * max_chunks + ck) * heads + h) * N * P + (size_t)n0 * P + 4 * cg;
+    float s[RT][4];
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+        const float4 v = mode == 2 ? *reinterpret_cast<const float4*>(sc + i * P) : make_float4(0.f, 0.f, 0.f, 0.f);
+        s[i][0] = v.x; s[i][1] = v.y; s[i][2] = v.z; s[i][3] = v.w;
+    }
+    const float db = dt_bias ? dt_bias[h] : 0.f, na = neg_a[h], dw = Dw ? Dw[h] : 0.f;
+    const int off_b = inner + g * N, off_c = inner + G * N + g * N, off_x = h * P;
+    // a wave brings the inputs of one of the batch's tokens, in registers until the batch before is done (tokens beyond the chunk
+    // repeat its last one and are not used)
+    constexpr int kMost = 512 / 64;                                         // W <= 512
+    int col[kMost];
+#pragma unroll
+    for (int k = 0; k < kMost; ++k) {
+        const int c = lane + 64 * k;
+        col[k] = c < N ? off_b + c : c < 2 * N ? off_c + (c - N) : off_x + (c - 2 * N);
+    }
+    float pre[kMost], dt_pre = 0.f;
+    auto fetch = [&](int t) {
+        const int row = min(t + wave, end - 1);
+        const float* const xf = reinterpret_cast<const float*>(xbc) + (size_t)row * x_stride;
+        const T* const xt = reinterpret_cast<const T*>(xbc) + (size_t)row * x_stride;
+#pragma unroll
+        for (int k = 0; k < kMost; ++k)
+            if (lane + 64 * k < W) pre[k] = x_f32 ? xf[col[k]] : to_f32(xt[col[k]]);
+        if (dt_raw) dt_pre = to_f32(dt_raw[(size_t)row * dt_stride + h]);
+    };
+    auto stash = [&]() {
+#pragma unroll
+        for (int k = 0; k < kMost; ++k)
+            if (lane + 64 * k < W) in[wave * W + lane + 64 * k] = in_act ? silu_f(pre[k]) : pre[k];
+        if (lane == 0) {
+            const float dt = dt_raw ? softplus_f(dt_pre + db) : 1.f;        // no step sizes: a fixed decay per head, steps of one
+            step[2 * wave] = dt;
+            step[2 * wave + 1] = dt_raw ? expf(na * dt) : na;
+        }
+    };
+    float a_total = 1.f;
+    fetch(begin);
+    for (int t0 = begin; t0 < end; t0 += TB) {
+        stash();
+        __syncthreads();
+        if (t0 + TB < end) fetch(t0 + TB);
+        const int cnt = min(TB, end - t0);
+        for (int u = 0; u < cnt; ++u) {
+            const float* const row = in + u * W;
+            const float dt = step[2 * u], da = step[2 * u + 1];
+            a_total *= da;
+            const float4 x4 = *reinterpret_cast<const float4*>(row + 2 * N + 4 * cg);
+            const float dx[4] = {dt * x4.x, dt * x4.y, dt * x4.z, dt * x4.w};
+            float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < RT; i += 4) {
+                const float4 b4 = *reinterpret_cast<const float4*>(row + n0 + i);
+                const float b[4] = {b4.x, b4.y, b4.z, b4.w};
+                if (mode == 1) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) s[i + j][c] = da * s[i + j][c] + b[j] * dx[c];
+                } else {
+                    const float4 c4 = *reinterpret_cast<const float4*>(row + N + n0 + i);
+                    const float cc[4] = {c4.x, c4.y, c4.z, c4.w};
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) {
+                            s[i + j][c] = da * s[i + j][c] + b[j] * dx[c];
+                            acc[c] += s[i + j][c] * cc[j];
+                        }
+                }
+            }
+            if (mode == 2) {
+                // sums over the wave's thread rows (lanes cgs, 2 cgs, .. apart): a swap of lane halves between two registers and
+                // an add leave each half with one register's sum, so the halvings of 32 and 16 lanes also share out the 4 columns
+                float* const out = part + (u * 4 + wave) * P;
+                const float lo = swap_halves<32>(acc[0], acc[1]), hi = swap_halves<32>(acc[2], acc[3]);      // columns 0 | 1 and 2 | 3
+                if (cgs <= 16) {
+                    float v = swap_halves<16>(lo, hi);                      // rows of 16 lanes: columns 0, 2, 1, 3
+                    if (cgs <= 8) v = dpp_add<0x128>(v);                    // lane i + lane i ^ 8
+                    const int q = lane >> 4;
+                    if ((lane & 15) < cgs) out[4 * (lane & (cgs - 1)) + ((q & 1) << 1) + (q >> 1)] = v;
+                } else if (cgs == 32) {
+                    out[4 * (lane & 31) + (lane >> 5)] = lo;
+                    out[4 * (lane & 31) + 2 + (lane >> 5)] = hi;
+                } else *reinterpret_cast<float4*>(out + 4 * lane) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+            }
+        }
+        __syncthreads();
+        if (mode == 2) {
+            if (wave < cnt)
+                for (int c = lane; c < P; c += 64) {
+                    float v = dw * in[wave * W + 2 * N + c];
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) v += part[(wave * 4 + w) * P + c];
+                    y[(size_t)(t0 + wave) * inner + h * P + c] = v;
+                }
+            __syncthreads();                                                // the inputs have been read (x above)
+        }
+    }
+    if (mode == 2) return;
+#pragma unroll
+    for (int i = 0; i < RT; ++i) *reinterpret_cast<float4*>(sc + i * P) = make_float4(s[i][0], s[i][1], s[i][2], s[i][3]);
+    if (tid == 0) scr_a[((size_t)r * max_chunks + ck) * heads + h] = a_total;
+}
+
+// Rows of the state a thread owns when the kernel above takes these sizes, else 0.
+static int ssm_tile_rows(int P, int N) {
+    if (P != 32 && P != 64 && P != 128 && P != 256) return 0;
+    const int rt = N * P / 1024;
+    return rt * 1024 == N * P && (rt == 4 || rt == 8 || rt == 16) && 2 * N + P <= 512 ? rt : 0;
+}
+static size_t ssm_tile_lds(int P, int N) { return (size_t)kSsmBatch * (2 * N + P + 2 + 4 * P) * sizeof(float); }
+
+template <typename T>
+static int ssm_tile_launch(dim3 grid, hipStream_t stream, const void* xbc, int x_stride, int x_f32, int in_act, const void* dt_raw, int dt_stride,
+                           const float* dt_bias, const float* neg_a, const float* Dw, int heads, int P, int N, int G, float* y,
+                           const int* req_start, int mode, int chunk_len, int max_chunks, float* scr_s, float* scr_a) {
+#define IC_SSM_TILE_MODE(RT, MODE)                                                                                                \
+    hipLaunchKernelGGL((ssm_tile_kernel<T, RT, MODE>), grid, dim3(256), ssm_tile_lds(P, N), stream, xbc, x_stride, x_f32, in_act,  \
+                       (const T*)dt_raw, dt_stride, dt_bias, neg_a, Dw, heads, P, G, y, req_start, chunk_len, max_chunks, scr_s, scr_a)
+#define IC_SSM_TILE(RT) do { if (mode == 1) IC_SSM_TILE_MODE(RT, 1); else IC_SSM_TILE_MODE(RT, 2); } while (0)
+    switch (ssm_tile_rows(P, N)) {
+    case 4: IC_SSM_TILE(4); break;
+    case 8: IC_SSM_TILE(8); break;
+    case 16: IC_SSM_TILE(16); break;
+    default: return IC_ERR_TOO_LARGE;
+    }
+#undef IC_SSM_TILE
+#undef IC_SSM_TILE_MODE
+    return IC_OK;
+}
+
 IC_EXPORT int ic_ssm_scan(const void* xbc, int x_stride, int x_dtype, int in_act, const void* dt_raw, int dt_stride, int dtype, const float* dt_bias,
                           const float* neg_a, const float* Dw, int heads, int P, int N, int G, float* y, float* state,
                           long long state_stride, const int* req_start, const int* state_slots, int R, int chunk_len,
@@ -354,7 +522,13 @@ IC_EXPORT int ic_ssm_scan(const void* xbc, int x_stride, int x_dtype, int in_act
         }
         dim3 grid(heads, R, chunked ? max_chunks : 1);
         int st;
-        if (dtype == IC_F32)
+        if (mode != 0 && ssm_tile_rows(P, N) && (dtype == IC_F32 || dtype == IC_BF16) && !((uintptr_t)scr_s & 15)) {
+            st = dtype == IC_F32
+                     ? ssm_tile_launch<float>(grid, stream, xbc, x_stride, x_f32, in_act, dt_raw, dt_stride, dt_bias, neg_a, Dw, heads, P, N, G, y,
+                                              req_start, mode, chunk_len, max_chunks, scr_s, scr_a)
+                     : ssm_tile_launch<bf16>(grid, stream, xbc, x_stride, x_f32, in_act, dt_raw, dt_stride, dt_bias, neg_a, Dw, heads, P, N, G, y,
+                                             req_start, mode, chunk_len, max_chunks, scr_s, scr_a);
+        } else if (dtype == IC_F32)
             st = ssm_launch<float>(ni, grid, lds, stream, xbc, x_stride, x_f32, in_act, dt_raw, dt_stride, dt_bias, neg_a, Dw, heads, P, N, G, y, state,
                                    state_stride, req_start, state_slots, mode, chunk_len, max_chunks, scr_s, scr_a);
         else if (dtype == IC_BF16)
