@@ -279,11 +279,20 @@ attn_span_prefill_kernel(const uint16_t* __restrict__ q, int q_stride, uint16_t*
         for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
             for (int r = 0; r < 16; ++r) mloc = fmaxf(mloc, sacc[tt][r]);
-        mloc = fmaxf(mloc, __shfl_xor(mloc, 32, kWave));
-        const float m_new = fmaxf(m, mloc);
-        const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-        const float mc = m_use * scale_log2e;
-        const float corr = (m == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m * scale_log2e - mc);
+        mloc = swap_max32(mloc);
+        // The running maximum follows the scores only when some row's grew by more than kMaxSlack powers of two: p then reaches 2^kMaxSlack
+        // instead of 1, which costs no precision, and after the first tiles the accumulators are hardly ever rescaled.
+        if (__builtin_amdgcn_ballot_w64((mloc - m) * scale_log2e > kMaxSlack)) {
+            const float m_new = fmaxf(m, mloc);
+            const float corr = (m == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m - m_new) * scale_log2e);
+            l *= corr;
+            m = m_new;
+#pragma unroll
+            for (int i = 0; i < ND; ++i)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) oacc[i][r] *= corr;
+        }
+        const float mc = (m == -INFINITY) ? 0.f : m * scale_log2e;
         float rs = 0.f;
 #pragma unroll
         for (int tt = 0; tt < 2; ++tt)
@@ -293,13 +302,7 @@ attn_span_prefill_kernel(const uint16_t* __restrict__ q, int q_stride, uint16_t*
                 sacc[tt][r] = p;
                 rs += p;
             }
-        rs += __shfl_xor(rs, 32, kWave);
-        l = l * corr + rs;
-        m = m_new;
-#pragma unroll
-        for (int i = 0; i < ND; ++i)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) oacc[i][r] *= corr;
+        l += swap_add<32>(rs);
 
         // ---- O^T += V^T P^T : four chunks of 16 keys ------------------------------------------
 #pragma unroll
