@@ -58,7 +58,7 @@ attn_decode_split_kernel(const T* __restrict__ q, int q_stride,
                          const int* __restrict__ tok_list, const int* __restrict__ token_req,
                          const int* __restrict__ positions,
                          float* __restrict__ part_acc, float* __restrict__ part_ml,
-                         int nh, int nkvh, int page_size, float scale, int window, int nsplit,
+                         int nh, int nkvh, int page_size, float scale, int window, int nsplit, unsigned page_rcp,
                          T* __restrict__ final_out, int out_stride) {
     constexpr int VEC = Vec16<T>::N;
     constexpr int LPK = DH / VEC;                 // lanes per key
@@ -94,15 +94,18 @@ attn_decode_split_kernel(const T* __restrict__ q, int q_stride,
     // STAGED is a compile-time choice (the host knows the block table's width): a run-time choice
     // between the two arrays would make every lookup a flat load, whose wait also waits for the
     // key and value loads in flight.
-    const int page_lo = lo / page_size;
-    const int n_pages = (hi > lo) ? (hi - 1) / page_size - page_lo + 1 : 0;
+    // A request whose ids are staged has at most kDecMaxPages pages, so key / page_size is one multiplication by
+    // page_rcp = ceil(2^32 / page_size) instead of some 20 instructions.
+    auto page_of = [&](int key) { return STAGED ? (int)__umulhi((unsigned)key, page_rcp) : key / page_size; };
+    const int page_lo = page_of(lo);
+    const int n_pages = (hi > lo) ? page_of(hi - 1) - page_lo + 1 : 0;
     if (STAGED)
         for (int i = threadIdx.x; i < n_pages; i += kDecThreads) pages[i] = bt[page_lo + i];
     __syncthreads();
 
     // element offset of a key's row piece in a plane
     auto row_of = [&](int key) -> size_t {
-        const int lp = key / page_size;
+        const int lp = page_of(key);
         const int pg = STAGED ? pages[lp - page_lo] : bt[lp];
         return (size_t)pg * page_stride + (size_t)(key - lp * page_size) * DH;
     };
@@ -286,12 +289,17 @@ attn_decode_reduce_kernel(const float* __restrict__ part_acc, const float* __res
 //
 // Same grid and partial-result layout as above, 4 or 8 waves.  A wave owns tiles of 32 keys of the block's
 // share (tile i -> wave i % waves).  S^T = K Q^T with v_mfma_f32_16x16x32_bf16, keys as rows: the K
-// operand comes straight from memory in operand layout (lane l: key l%16, dims 8(l/16)..+7 of a
-// 32-dim chunk).  A lane then holds 4+4 keys of ONE head (l%16), so the running softmax needs two
+// operand is read from LDS in operand layout (lane l: key l%16, dims 8(l/16)..+7 of a 32-dim chunk).  A lane then holds 4+4 keys of ONE head (l%16), so the running softmax needs two
 // cross-lane steps.  O^T = V^T P^T: P^T is already the B operand (slot (l/16, e) stands for key
-// 4(l/16) + e of the first 16 keys for e < 4, of the second 16 for e >= 4); V goes through LDS
+// 4(l/16) + e of the first 16 keys for e < 4, of the second 16 for e >= 4); V goes through LDS too
 // (written as rows, read as columns with ds_read_b64_tr_b16).  16x16x32 layout: A[i = l%16][k = 8(l/16)..+7],
 // B[k = 8(l/16)..+7][j = l%16], D[i = 4(l/16) + e][j = l%16].
+//
+// What bounds a block is the chain of one tile's steps in a wave, not memory (two tiles in flight gain nothing): scalar loop
+// control, accumulators in plain vector registers (two waves a SIMD asked for), one multiplication for a key's page, lane groups
+// that meet by register swaps, a sum that meets only at the end and a maximum that may lag took a tile from 1.25 to
+// 0.85 us.  24:8 heads of 64: 40 rows of 100..2,048 keys 25.1 -> 20.2 us, one row of 258 keys 6.7 -> 5.7; 32:2 heads of 128: 4 rows
+// of 16,385 keys 24.0 -> 21.2, 60 rows of 100..8,000 keys 49.9 -> 43.
 typedef __bf16 gq_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float gq_v4f __attribute__((ext_vector_type(4)));
 typedef float gq_v8f __attribute__((ext_vector_type(8)));
@@ -305,14 +313,14 @@ union GqFrag {
 };
 
 template <int DH, bool STAGED, int WV>
-__global__ void __launch_bounds__(64 * WV)
+__global__ void __launch_bounds__(64 * WV, 2)
 attn_decode_gqa_kernel(const uint16_t* __restrict__ q, int q_stride,
                        const uint16_t* __restrict__ kcache, const uint16_t* __restrict__ vcache,
                        const int* __restrict__ block_tables, int bt_stride,
                        const int* __restrict__ tok_list, const int* __restrict__ token_req,
                        const int* __restrict__ positions,
                        float* __restrict__ part_acc, float* __restrict__ part_ml,
-                       int nh, int nkvh, int page_size, float scale, int window, int nsplit,
+                       int nh, int nkvh, int page_size, float scale, int window, int nsplit, unsigned page_rcp,
                        uint16_t* __restrict__ final_out, int out_stride) {
     constexpr int NC = DH / 32;                    // 32-dim chunks of the score product
     constexpr int ND = DH / 16;                    // 16-dim chunks of the output
@@ -336,7 +344,7 @@ attn_decode_gqa_kernel(const uint16_t* __restrict__ q, int q_stride,
     int hi = lo + per;
     if (hi > pos + 1) hi = pos + 1;
 
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const float scale2 = scale * 1.4426950408889634f;   // scores and running maxima in units of log 2: exp2 is one instruction
     const int lr = lane & 15, lg = lane >> 4;      // row / column of a tile, and the lane group
     const size_t head_stride = (size_t)page_size * DH;
@@ -344,19 +352,19 @@ attn_decode_gqa_kernel(const uint16_t* __restrict__ q, int q_stride,
     const uint16_t* kbase = kcache + (size_t)kvh * head_stride;
     const uint16_t* vbase = vcache + (size_t)kvh * head_stride;
 
-    const int page_lo = lo / page_size;
-    const int n_pages = (hi > lo) ? (hi - 1) / page_size - page_lo + 1 : 0;
+    auto page_of = [&](int key) { return STAGED ? (int)__umulhi((unsigned)key, page_rcp) : key / page_size; };
+    const int page_lo = page_of(lo);
+    const int n_pages = (hi > lo) ? page_of(hi - 1) - page_lo + 1 : 0;
     if (STAGED)
         for (int i = threadIdx.x; i < n_pages; i += 64 * WV) pages[i] = bt[page_lo + i];
     __syncthreads();
     auto row_of = [&](int key) -> size_t {
-        const int lp = key / page_size;
+        const int lp = page_of(key);
         const int pg = STAGED ? pages[lp - page_lo] : bt[lp];
         return (size_t)pg * page_stride + (size_t)(key - lp * page_size) * DH;
     };
 
     const int n_tiles = (hi > lo) ? (hi - lo + kGqaKeys - 1) / kGqaKeys : 0;
-    const int rounds = (n_tiles + WV - 1) / WV;
 
     for (int h0 = 0; h0 < g; h0 += 16) {
         // Q^T operand: head lr of this chunk, dims 32c + 8 lg .. +7
@@ -379,41 +387,31 @@ attn_decode_gqa_kernel(const uint16_t* __restrict__ q, int q_stride,
         // covers whole cache lines) with loads the caches do not keep.  The keys then pass through the wave's LDS tile
         // into operand layout (key 16 s2 + lr, dims 32 c + 8 lg .. +7) before the values take the tile over: loaded
         // straight in operand layout a wave's load covered 64 bytes of each of 16 rows, half a line.
-        GqFrag kreg[2][NC];
         uint4 kraw[NV], vreg[NV];
+        constexpr int KPI = 512 / DH;              // keys a wave's load covers
+        const int key0 = lane / (DH / 8), oct = lane % (DH / 8);
+        // No condition around a load: keys beyond the share read its last key.
         auto fetch = [&](int tile) {
-            const int kt = lo + tile * kGqaKeys;
+            const int kt = lo + tile * kGqaKeys + key0;
 #pragma unroll
             for (int i = 0; i < NV; ++i) {
-                const int idx = lane + 64 * i;
-                const int vkey = idx / (DH / 8), oct = idx - vkey * (DH / 8);
-                const int key = kt + vkey;
-                kraw[i] = make_uint4(0, 0, 0, 0);
-                vreg[i] = make_uint4(0, 0, 0, 0);
-                if (tile < n_tiles && key < hi) {
-                    const size_t at = row_of(key) + oct * 8;
-                    kraw[i] = load_stream16(kbase + at);
-                    vreg[i] = load_stream16(vbase + at);
-                }
+                const size_t at = row_of(min(kt + KPI * i, hi - 1)) + oct * 8;
+                kraw[i] = load_stream16(kbase + at);
+                vreg[i] = load_stream16(vbase + at);
             }
         };
+        uint16_t* const mine = &Vs[wave][key0 * VS + oct * 8];
         auto stash = [&](const uint4* regs) {
 #pragma unroll
-            for (int i = 0; i < NV; ++i) {
-                const int idx = lane + 64 * i;
-                const int vkey = idx / (DH / 8), oct = idx - vkey * (DH / 8);
-                *reinterpret_cast<uint4*>(&Vs[wave][vkey * VS + oct * 8]) = regs[i];
-            }
+            for (int i = 0; i < NV; ++i) *reinterpret_cast<uint4*>(mine + KPI * i * VS) = regs[i];
         };
-
-        // A wave writes and reads only its own V tile in LDS, and LDS serves a wave's instructions
-        // in order, so no block barrier is needed in this loop (wave_barrier keeps the compiler from
-        // moving LDS accesses across it).
-        fetch(wave);
-        for (int r = 0; r < rounds; ++r) {
-            const int tile = r * WV + wave;
-            if (tile >= n_tiles) break;             // uniform in the wave
+        // A wave writes and reads only its own tile in LDS, and LDS serves a wave's instructions in order, so no
+        // block barrier is needed in this loop (wave_barrier keeps the compiler from moving LDS accesses across it).
+        if (wave < n_tiles) fetch(wave);
+        for (int tile = wave; tile < n_tiles; tile += WV) {
             const int kt = lo + tile * kGqaKeys;
+            const bool last = kt + kGqaKeys > hi;
+            GqFrag kreg[2][NC];
             __builtin_amdgcn_wave_barrier();
             stash(kraw);
             __builtin_amdgcn_wave_barrier();
@@ -422,9 +420,15 @@ attn_decode_gqa_kernel(const uint16_t* __restrict__ q, int q_stride,
 #pragma unroll
                 for (int c = 0; c < NC; ++c)
                     kreg[s2][c].u = *reinterpret_cast<const uint4*>(&Vs[wave][(16 * s2 + lr) * VS + 32 * c + 8 * lg]);
+            if (last) {                             // stand-ins for keys beyond the share: weight 0, but 0 * infinity is NaN
+#pragma unroll
+                for (int i = 0; i < NV; ++i)
+                    if (kt + key0 + KPI * i >= hi) vreg[i] = make_uint4(0, 0, 0, 0);
+            }
             __builtin_amdgcn_wave_barrier();
             stash(vreg);
             __builtin_amdgcn_wave_barrier();
+            if (tile + WV < n_tiles) fetch(tile + WV);      // the next tile's loads fly during the rest of this one
 
             // ---- S^T = K Q^T, two subtiles of 16 keys ----------------------------------
             gq_v4f sacc[2];
@@ -435,30 +439,30 @@ attn_decode_gqa_kernel(const uint16_t* __restrict__ q, int q_stride,
                 for (int c = 0; c < NC; ++c)
                     sacc[s2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kreg[s2][c].v, qf[c].v, sacc[s2], 0, 0, 0);
             }
-            fetch(tile + WV);                // the next tile's loads fly during the rest of this one
-            float sv[8];
-            float mloc = -INFINITY;
+            float sv[8], mloc = -INFINITY;
 #pragma unroll
-            for (int s2 = 0; s2 < 2; ++s2)
+            for (int e = 0; e < 8; ++e) sv[e] = sacc[e >> 2][e & 3] * scale2;       // in units of log 2
+            if (last) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int key = kt + 16 * s2 + 4 * lg + e;
-                    const float x = (key < hi) ? sacc[s2][e] * scale2 : -INFINITY;     // in units of log 2
-                    sv[4 * s2 + e] = x;
-                    mloc = fmaxf(mloc, x);
-                }
-            mloc = fmaxf(mloc, __shfl_xor(mloc, 16, kWave));
-            mloc = fmaxf(mloc, __shfl_xor(mloc, 32, kWave));
-            const float m_new = fmaxf(m, mloc);     // finite: every tile has at least one key
-            const float corr = __builtin_amdgcn_exp2f(m - m_new);
-            float rs = 0.f;
+                for (int e = 0; e < 8; ++e)
+                    if (kt + 16 * (e >> 2) + 4 * lg + (e & 3) >= hi) sv[e] = -INFINITY;
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) mloc = fmaxf(mloc, sv[e]);
+            mloc = swap_max<16>(swap_max<32>(mloc));
+            if (__builtin_amdgcn_ballot_w64(mloc - m > kMaxSlack)) {     // (finite: every tile has at least one key)
+                const float m_new = fmaxf(m, mloc);
+                const float corr = __builtin_amdgcn_exp2f(m - m_new);
+                l *= corr;
+                m = m_new;
+#pragma unroll
+                for (int c = 0; c < ND; ++c) oacc[c] *= corr;
+            }
             gq_v8f pf;
+            float rs = 0.f;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) { const float p = __builtin_amdgcn_exp2f(sv[e] - m_new); pf[e] = p; rs += p; }
-            rs += __shfl_xor(rs, 16, kWave);
-            rs += __shfl_xor(rs, 32, kWave);
-            l = l * corr + rs;
-            m = m_new;
+            for (int e = 0; e < 8; ++e) { const float p = __builtin_amdgcn_exp2f(sv[e] - m); pf[e] = p; rs += p; }
+            l += rs;                                // of this lane's keys; the lane groups meet after the loop
             const gq_bf16x8 pb = __builtin_convertvector(pf, gq_bf16x8);
 
             // ---- O^T += V^T P^T ----------------------------------------------------------------
@@ -468,15 +472,13 @@ attn_decode_gqa_kernel(const uint16_t* __restrict__ q, int q_stride,
             const uint16_t* vrow = &Vs[wave][(4 * lg + (lr >> 2)) * VS + 4 * (lr & 3)];
 #pragma unroll
             for (int c = 0; c < ND; ++c) {
-                GqFrag a;
-                const gq_v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gq_v4s __attribute__((address_space(3)))*)(vrow + 16 * c));
-                const gq_v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gq_v4s __attribute__((address_space(3)))*)(vrow + 16 * VS + 16 * c));
-#pragma unroll
-                for (int e = 0; e < 4; ++e) { a.h[e] = (uint16_t)lo[e]; a.h[4 + e] = (uint16_t)hi[e]; }
-                oacc[c] *= corr;
-                oacc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, pb, oacc[c], 0, 0, 0);
+                const gq_v4s lo4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gq_v4s __attribute__((address_space(3)))*)(vrow + 16 * c));
+                const gq_v4s hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gq_v4s __attribute__((address_space(3)))*)(vrow + 16 * VS + 16 * c));
+                const auto both = __builtin_shufflevector(lo4, hi4, 0, 1, 2, 3, 4, 5, 6, 7);
+                oacc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gq_bf16x8, both), pb, oacc[c], 0, 0, 0);
             }
         }
+        l = swap_add<16>(swap_add<32>(l));
 
         // ---- merge the four waves; O^T[d = 16c + 4 lg + e][head lr] ---------------------------
         __syncthreads();
@@ -522,23 +524,29 @@ static int launch_decode(const void* q, int q_stride, void* out, int out_stride,
                          int n_tok, int nh, int nkvh, int page_size, float scale, int window, int nsplit,
                          hipStream_t stream) {
     dim3 grid(nsplit, nkvh, n_tok), block(kDecThreads);
-    const bool staged = bt_stride <= kDecMaxPages;      // a block never needs more page ids than a request has
+    // A block never needs more page ids than a request has.  The multiplication that stands for a division by the page size is exact
+    // for keys below 2^32 / page_size, which kDecMaxPages pages of fewer than 2,048 keys stay below.
+    const bool staged = bt_stride <= kDecMaxPages && page_size >= 2 && page_size < 2048;
+    const unsigned page_rcp = (unsigned)(((1ull << 32) + page_size - 1) / page_size);
     void* direct = (nsplit == 1) ? out : nullptr;       // one split writes the result itself
 #define IC_DEC_LAUNCH(KERNEL, TQ)                                                                           \
     hipLaunchKernelGGL(KERNEL, grid, block, 0, stream, (const TQ*)q, q_stride, (const TQ*)kcache,           \
                        (const TQ*)vcache, block_tables, bt_stride, tok_list, token_req, positions, part_acc, \
-                       part_ml, nh, nkvh, page_size, scale, window, nsplit, (TQ*)direct, out_stride)
+                       part_ml, nh, nkvh, page_size, scale, window, nsplit, page_rcp, (TQ*)direct, out_stride)
     if (ic_attn_decode_on_matrix_cores(sizeof(T) == 2 ? IC_BF16 : IC_F32, nh, nkvh)) {
-        // Eight waves where a block's share of the keys is long for four and the blocks are too few to fill the units anyway: one
-        // split of few (row, kv head) pairs (24:8 heads of 64, 258 keys: 1 row 6.4 -> 5.6 us, 8 rows 7.0 -> 6.5; 512 keys 8.2 -> 7.2;
-        // with 320 pairs 19.9 -> 22.0), and many splits of heads of 128 (32:2 heads, 4 rows, 16,385 keys in 32 splits: 24.3 -> 22.1;
-        // in 16 splits of 2,000 keys 11.3 -> 11.8).
-        const bool eight = DH == 64 ? nsplit == 1 && n_tok * nkvh <= 128 : nsplit >= 24;
-        if (eight) {
-            block = dim3(512);
-            if (staged) IC_DEC_LAUNCH((attn_decode_gqa_kernel<DH, true, 8>), uint16_t);
-            else IC_DEC_LAUNCH((attn_decode_gqa_kernel<DH, false, 8>), uint16_t);
-        } else if (staged) IC_DEC_LAUNCH((attn_decode_gqa_kernel<DH, true, 4>), uint16_t);
+        // Eight waves where one split's share is long for four and the blocks are too few to fill the units anyway (24:8 heads of 64,
+        // one split: 258 keys 6.1 -> 5.8 us, 16 rows of up to 2,000 keys 18.6 -> 14.1; with 320 pairs of 1,000 keys 19.2 -> 21.1).
+        // Heads of 128 and shares of several splits gain nothing by them (32:2 heads, 16,385 keys in 32 splits: 21.6 and 21.3).
+        const bool eight = DH == 64 && nsplit == 1 && n_tok * nkvh <= 128;
+        if constexpr (DH == 64) {
+            if (eight) {
+                block = dim3(512);
+                if (staged) IC_DEC_LAUNCH((attn_decode_gqa_kernel<DH, true, 8>), uint16_t);
+                else IC_DEC_LAUNCH((attn_decode_gqa_kernel<DH, false, 8>), uint16_t);
+            }
+        }
+        if (eight) { /* launched */ }
+        else if (staged) IC_DEC_LAUNCH((attn_decode_gqa_kernel<DH, true, 4>), uint16_t);
         else IC_DEC_LAUNCH((attn_decode_gqa_kernel<DH, false, 4>), uint16_t);
     } else if (nh == nkvh) {
         if (staged) IC_DEC_LAUNCH((attn_decode_split_kernel<T, DH, 1, true>), T);

@@ -280,7 +280,7 @@ attn_prefill_mfma_kernel(const uint16_t* __restrict__ q, int q_stride, uint16_t*
         for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
             for (int r = 0; r < 16; ++r) mloc = fmaxf(mloc, sacc[tt][r]);
-        mloc = swap_max32(mloc);
+        mloc = swap_max<32>(mloc);
         // The running maximum follows the scores only when some row's grew by more than kMaxSlack powers of two: p then reaches 2^kMaxSlack
         // instead of 1, which costs no precision, and after the first tiles the accumulators are hardly ever rescaled.  The vector
         // instructions of the softmax bound this loop, not the products: without the rescaling, and with the halves' exchange in

@@ -88,10 +88,10 @@ template <int D> __device__ __forceinline__ float swap_add(float v) {
     const auto r = D == 32 ? __builtin_amdgcn_permlane32_swap(b, b, false, false) : __builtin_amdgcn_permlane16_swap(b, b, false, false);
     return __int_as_float((int)r[0]) + __int_as_float((int)r[1]);
 }
-// The larger of the two halves' values in every lane: max(v[i], v[i ^ 32]).
-__device__ __forceinline__ float swap_max32(float v) {
+// The larger of v[i] and v[i ^ D], D = 32 or 16, likewise.
+template <int D> __device__ __forceinline__ float swap_max(float v) {
     const unsigned b = (unsigned)__float_as_int(v);
-    const auto r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    const auto r = D == 32 ? __builtin_amdgcn_permlane32_swap(b, b, false, false) : __builtin_amdgcn_permlane16_swap(b, b, false, false);
     return fmaxf(__int_as_float((int)r[0]), __int_as_float((int)r[1]));
 }
 // Powers of two by which a running softmax's maximum may lag behind the scores before its accumulators are rescaled.

@@ -15,3 +15,12 @@ def test_grouped_queries_with_four_and_eight_waves(nh, nkvh, dh, rows, n_split, 
     lens = [((0, 31, 32, 255, 256, 257, 511, 1031)[i % 8] + i // 8, 1) for i in range(rows)]
     got, want = _attention_case(torch.bfloat16, nh, nkvh, dh, 64, lens, window, 51, "decode", n_split=n_split)
     _close(got, want, torch.bfloat16, factor=3)
+
+
+@pytest.mark.parametrize("page", [1, 2, 3, 48, 2047, 2048])          # a key's page by a multiplication, where ids are staged and exact
+@pytest.mark.parametrize("dtype,nh,nkvh,dh", [(torch.bfloat16, 6, 2, 64), (torch.bfloat16, 3, 3, 64), (torch.bfloat16, 4, 2, 128),
+                                              (torch.float32, 6, 2, 64)])
+def test_page_sizes(page, dtype, nh, nkvh, dh):
+    lens = [(n, 1) for n in (0, page - 1, page, 46, 95, 96, 500, min(1031, 1000 * page))]
+    got, want = _attention_case(dtype, nh, nkvh, dh, page, lens, None, 52, "decode", n_split=3)
+    _close(got, want, dtype, factor=3)

@@ -1,4 +1,4 @@
-"""Prompt attention where scores climb along the keys: the running maximum may lag by up to eight powers of two before the accumulators are
+"""Attention where scores climb along the keys: the running maximum may lag by up to eight powers of two before the accumulators are
 rescaled, and rows of one wave climb, fall and stay level at once."""
 import math
 
@@ -22,7 +22,7 @@ def _inputs(dh, climb):
     return q.bfloat16(), k.bfloat16(), v.bfloat16()
 
 
-@pytest.mark.parametrize("kernel", ["prefill", "span"])
+@pytest.mark.parametrize("kernel", ["prefill", "span", "decode"])
 @pytest.mark.parametrize("dh", [64, 128])
 @pytest.mark.parametrize("climb", [1.0, 7.75, 8.0, 8.25, 40.0])
 def test_climbing_scores(kernel, dh, climb):
@@ -35,7 +35,11 @@ def test_climbing_scores(kernel, dh, climb):
     out = torch.full_like(qd, float("nan"))
     rows = ops.attention_prefill_tile_rows()
     tiles = torch.tensor([[0, o, min(rows, n - o), PAST + o] for o in range(0, n, rows)], dtype=torch.int32).cuda()
-    if kernel == "prefill":
+    if kernel == "decode":
+        part = [torch.empty(n * 2 * 3 * m, device="cuda") for m in (dh, 2)]
+        rows = torch.arange(PAST, KEYS, dtype=torch.int32).cuda()
+        ops.attention_decode(qd, out, kc, vc, bt, None, n, torch.zeros_like(rows), rows, *part, 2, 1, dh, 64, scale, 0, 3)
+    elif kernel == "prefill":
         ops.attention_prefill(qd, out, kc, vc, bt, tiles, len(tiles), 2, 1, dh, 64, scale, 0, 1)
     else:
         ops.attention_span_prefill(qd, out, None, kc, vc, bt, tiles, len(tiles), 2, 1, dh, dh, 64, scale, 0, 0, None, 0.0)
