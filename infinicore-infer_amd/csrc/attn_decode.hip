@@ -576,6 +576,36 @@ IC_EXPORT int ic_attn_decode_supported(int dtype, int dh) {
     return (dtype == IC_F32 || dtype == IC_BF16) && (dh == 64 || dh == 128);
 }
 
+// order[r] = the row whose position is the r-th largest (of equal ones the first): where more blocks are launched than the chip holds
+// at once, the longest walks over the keys must not be the last to start.  One block; n rows at most kOrderRows.
+constexpr int kOrderRows = 1024;
+__global__ void __launch_bounds__(kOrderRows)
+attn_decode_order_kernel(const int* __restrict__ positions, int* __restrict__ order, int n) {
+    __shared__ int pos[kOrderRows];
+    const int i = threadIdx.x;
+    const int mine = i < n ? positions[i] : 0;
+    pos[i] = mine;
+    __syncthreads();
+    if (i >= n) return;
+    int rank = 0;
+    for (int j = 0; j < n; ++j) rank += (pos[j] > mine || (pos[j] == mine && j < i)) ? 1 : 0;
+    order[rank] = i;
+}
+
+// Whether a step of n_rows single tokens, all its rows, is worth the kernel above (2 us a step): 64 rows of 36 heads of 64 over 300..2,100
+// keys 94.8 -> 89.1 us a layer, 40 rows of 24:8 heads over 100..2,048 22.2 -> 20.2, 24 rows of 36 heads over 100..1,500 27.4 -> 25.7.  Several
+// splits balance the walks already (16 rows of 36 heads in 4 splits 26.7 and 28.2), and up to one block a unit all start at once.
+IC_EXPORT int ic_attn_decode_wants_order(int n_rows, int nkvh, int nsplit, int compute_units) {
+    return nsplit == 1 && n_rows > 1 && n_rows <= kOrderRows && (long long)n_rows * nkvh > (compute_units > 0 ? compute_units : 256);
+}
+
+IC_EXPORT int ic_attn_decode_order(const int* positions, int* order, int n_rows, hipStream_t stream) {
+    if (n_rows <= 0) return IC_OK;
+    if (n_rows > kOrderRows || !positions || !order) return IC_ERR_ARG;
+    hipLaunchKernelGGL(attn_decode_order_kernel, dim3(1), dim3((n_rows + 63) / 64 * 64), 0, stream, positions, order, n_rows);
+    return ic_launch_status();
+}
+
 // part_acc: float32 [n_tok, nh, nsplit, dh]; part_ml: float32 [n_tok, nh, nsplit, 2].
 // tok_list: rows of q/out that are decoded (nullptr: rows 0..n_tok-1).
 IC_EXPORT int ic_attn_decode(const void* q, int q_stride, void* out, int out_stride, int dtype,

@@ -31,7 +31,7 @@ inline int dtype_size(int dtype) { return dtype == IC_BF16 ? 2 : 4; }
 struct Workspace {
     // byte offsets into the caller's workspace
     size_t residual, normed, qkv, attn_out, mixer_out, ffn_out, mixer_tail, mixer_sumsq, ffn_tail, ffn_sumsq, gate_up, act,
-        part_acc, part_ml, head_in, tail_parts, tile_parts, total;
+        part_acc, part_ml, decode_order, head_in, tail_parts, tile_parts, total;
 };
 
 // Rows whose norm is half done: values = x * w, sums of squares per column block; the row factor
@@ -155,6 +155,7 @@ struct IcDecoder {
             }
         w.part_acc = take(acc * 4);
         w.part_ml = take(ml * 4);
+        w.decode_order = take(b.decode_rows_identity ? (size_t)b.n_decode_rows * 4 : 0);
         w.head_in = take((size_t)b.n_want * d * ds);
         size_t slices = 0;           // the O and down products as slices over K, where that pays
         for (const IcLayer& l : layers)
@@ -217,6 +218,9 @@ struct IcDecoder {
 
         st = ic_embed(b.tokens, meta.embed_table, dt, x, T, d, meta.embed_scale, stream);
         if (st) return fail(st, "the embedding gather", -1);
+
+        const int* decode_rows = b.decode_rows_identity ? nullptr : b.decode_rows;
+        bool ordered = !b.decode_rows_identity;      // a list of the caller's has the longest rows first
 
         // what the residual stream still owes when a layer starts
         enum { NONE, BRANCH, DEFERRED, NORMED } owed = NONE;      // NORMED: the add and the whole norm are done, `normed` holds the rows
@@ -287,8 +291,14 @@ struct IcDecoder {
             } else {
                 if (use_dec) {
                     const int n_split = splits_for(b, A);
+                    if (!ordered && ic_attn_decode_wants_order(n_dec, A.n_kv_heads, n_split, meta.compute_units)) {
+                        decode_rows = (int*)(base + ws.decode_order);
+                        st = ic_attn_decode_order(b.positions, (int*)(base + ws.decode_order), n_dec, stream);
+                        if (st) return fail(st, "the order of the single tokens", i);
+                        ordered = true;
+                    }
                     st = ic_attn_decode(qkv, width, attn_out, ow, dt, e.k_cache, e.v_cache, tables, bts,
-                                        b.decode_rows_identity ? nullptr : b.decode_rows, b.token_req, b.positions,
+                                        decode_rows, b.token_req, b.positions,
                                         (float*)(base + ws.part_acc), (float*)(base + ws.part_ml), n_dec, A.n_heads, A.n_kv_heads,
                                         A.head_dim, ps, A.softmax_scale, A.window, n_split, stream);
                     if (st) return fail(st, "attention of single tokens", i);

@@ -99,6 +99,7 @@ _SIGNATURES = {
     "ic_rope_kv_write": [_P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
     "ic_attn_generic": [_P, _I, _P, _I, _I, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _F, _I, _P],
     "ic_attn_decode_supported": [_I, _I],
+    "ic_attn_decode_order": [_P, _P, _I, _P],
     "ic_attn_decode": [_P, _I, _P, _I, _I, _P, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I, _I, _P],
     "ic_attn_prefill_supported": [_I, _I, _I],
     "ic_attn_prefill_tile_rows": [],
