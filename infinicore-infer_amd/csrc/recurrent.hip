@@ -50,24 +50,113 @@ causal_conv_kernel(const T* __restrict__ xin, int xin_stride, const float* __res
     if (out_copy) out_copy[(size_t)t * copy_stride + c] = from_f32<T>(acc);
 }
 
+// The same for four taps and long steps: a thread takes four channels through a run of kConvRun tokens, so an input is read once (and
+// the three before the run), in 8 or 16 bytes a lane, and the request's lists are scalar loads.  Memory bounds it (3,304 tokens of 10,240
+// bfloat16 channels 183 -> 43 us, 4.7 TB/s; of 4,096 with the copy 81 -> 25); the kernel above, one (channel, token) a thread, is
+// bound by its dependent 2-byte reads.  The sums are taken in the same order.
+constexpr int kConvRun = 8;
+template <typename T> struct Conv4 { T v[4]; };
+template <typename T>
+__global__ void __launch_bounds__(256)
+causal_conv4_kernel(const T* __restrict__ xin, int xin_stride, const float* __restrict__ in_bias,
+                    const float* __restrict__ w, const float* __restrict__ b, int C,
+                    float* __restrict__ out, T* __restrict__ out_copy, int copy_stride, int act,
+                    const float* __restrict__ state, long long state_stride,
+                    const int* __restrict__ token_req, const int* __restrict__ req_start,
+                    const int* __restrict__ state_slots, int n_tok) {
+    typedef Conv4<T> __attribute__((aligned(4 * sizeof(T)))) row4;
+    const int c = (blockIdx.x * 256 + threadIdx.x) * 4, t0 = blockIdx.y * kConvRun;
+    if (c >= C) return;
+    float wt[4][4], ib[4], bb[4], h[3][4];                   // h: the three inputs before the token, oldest first
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float4 v = *reinterpret_cast<const float4*>(w + (size_t)(c + i) * 4);
+        wt[i][0] = v.x; wt[i][1] = v.y; wt[i][2] = v.z; wt[i][3] = v.w;
+        ib[i] = in_bias ? in_bias[c + i] : 0.f;
+        bb[i] = b ? b[c + i] : 0.f;
+    }
+    Conv4<T> raw[kConvRun];
+#pragma unroll
+    for (int j = 0; j < kConvRun; ++j) raw[j] = *reinterpret_cast<const row4*>(xin + (size_t)min(t0 + j, n_tok - 1) * xin_stride + c);
+    // inputs t - 3 .. t - 1: rows of the same request, before its first one the state
+    auto history = [&](int t, int r) {
+        const int start = req_start[r];
+        const float* st = state + (long long)state_slots[r] * state_stride;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int src = t - 3 + k;
+            if (src >= start) {
+                const Conv4<T> x = *reinterpret_cast<const row4*>(xin + (size_t)src * xin_stride + c);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) h[k][i] = to_f32(x.v[i]) + ib[i];
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) h[k][i] = st[(size_t)(3 - (start - src)) * C + c + i];
+            }
+        }
+    };
+    int r = token_req[t0];
+    history(t0, r);
+#pragma unroll
+    for (int j = 0; j < kConvRun; ++j) {
+        const int t = t0 + j;
+        if (t >= n_tok) return;
+        if (token_req[t] != r) { r = token_req[t]; history(t, r); }
+        float y[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float x = to_f32(raw[j].v[i]) + ib[i];
+            float acc = bb[i];
+            acc += wt[i][0] * h[0][i];
+            acc += wt[i][1] * h[1][i];
+            acc += wt[i][2] * h[2][i];
+            acc += wt[i][3] * x;
+            h[0][i] = h[1][i]; h[1][i] = h[2][i]; h[2][i] = x;
+            y[i] = act == 1 ? silu_f(acc) : acc;
+        }
+        *reinterpret_cast<float4*>(out + (size_t)t * C + c) = make_float4(y[0], y[1], y[2], y[3]);
+        if (out_copy) {
+            Conv4<T> o;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o.v[i] = from_f32<T>(y[i]);
+            *reinterpret_cast<row4*>(out_copy + (size_t)t * copy_stride + c) = o;
+        }
+    }
+}
+
+template <typename T>
+static void launch_conv(const void* xin, int xin_stride, const float* in_bias, const float* w, const float* b, int taps, int C, float* out,
+                        void* out_copy, int copy_stride, int act, const float* state, long long state_stride, const int* token_req,
+                        const int* req_start, const int* state_slots, int n_tok, hipStream_t stream) {
+    auto aligned = [](const void* p, size_t n) { return ((uintptr_t)p & (n - 1)) == 0; };
+    // A million results make it worth a thread's longer chain: 128 tokens of 10,240 channels 11.1 -> 9.8 us, 256 of 4,096 9.9 and 9.8, 1,012
+    // of 1,536 12.8 -> 10.3; but 40 of 10,240 6.5 and 8.9, 256 of 1,536 6.6 and 9.1.
+    if (taps == 4 && (long long)n_tok * C >= (1 << 20) && C % 4 == 0 && xin_stride % 4 == 0 && (!out_copy || copy_stride % 4 == 0) && aligned(xin, 4 * sizeof(T)) &&
+        aligned(out_copy, 4 * sizeof(T)) && aligned(w, 16) && aligned(out, 16)) {
+        hipLaunchKernelGGL(causal_conv4_kernel<T>, dim3((C + 1023) / 1024, (n_tok + kConvRun - 1) / kConvRun), dim3(256), 0, stream, (const T*)xin,
+                           xin_stride, in_bias, w, b, C, out, (T*)out_copy, copy_stride, act, state, state_stride, token_req, req_start, state_slots, n_tok);
+        return;
+    }
+    hipLaunchKernelGGL(causal_conv_kernel<T>, dim3((C + 255) / 256, n_tok), dim3(256), 0, stream, (const T*)xin, xin_stride, in_bias, w, b, taps, C,
+                       out, (T*)out_copy, copy_stride, act, state, state_stride, token_req, req_start, state_slots);
+}
+
 IC_EXPORT int ic_causal_conv(const void* xin, int xin_stride, int dtype, const float* in_bias, const float* w,
                              const float* b, int taps, int C, float* out, void* out_copy, int copy_stride, int act,
                              float* state, long long state_stride, const int* token_req, const int* req_start,
                              const int* state_slots, int T, int R, hipStream_t stream) {
     if (T <= 0) return IC_OK;
     if (taps < 1 || taps > kConvMaxTaps || C <= 0 || R <= 0 || !state || !req_start || !state_slots) return IC_ERR_ARG;
-    dim3 grid((C + 255) / 256, T), sgrid((C + 255) / 256, R), block(256);
+    dim3 sgrid((C + 255) / 256, R), block(256);
     if (dtype == IC_F32) {
-        hipLaunchKernelGGL(causal_conv_kernel<float>, grid, block, 0, stream, (const float*)xin, xin_stride, in_bias, w, b,
-                           taps, C, out, (float*)out_copy, copy_stride, act, state, state_stride, token_req, req_start,
-                           state_slots);
+        launch_conv<float>(xin, xin_stride, in_bias, w, b, taps, C, out, out_copy, copy_stride, act, state, state_stride, token_req, req_start, state_slots,
+                           T, stream);
         if (taps > 1)
             hipLaunchKernelGGL(conv_state_kernel<float>, sgrid, block, 0, stream, (const float*)xin, xin_stride, in_bias,
                                taps, C, state, state_stride, req_start, state_slots);
     } else if (dtype == IC_BF16) {
-        hipLaunchKernelGGL(causal_conv_kernel<bf16>, grid, block, 0, stream, (const bf16*)xin, xin_stride, in_bias, w, b,
-                           taps, C, out, (bf16*)out_copy, copy_stride, act, state, state_stride, token_req, req_start,
-                           state_slots);
+        launch_conv<bf16>(xin, xin_stride, in_bias, w, b, taps, C, out, out_copy, copy_stride, act, state, state_stride, token_req, req_start, state_slots,
+                          T, stream);
         if (taps > 1)
             hipLaunchKernelGGL(conv_state_kernel<bf16>, sgrid, block, 0, stream, (const bf16*)xin, xin_stride, in_bias,
                                taps, C, state, state_stride, req_start, state_slots);
