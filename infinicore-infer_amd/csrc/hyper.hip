@@ -126,24 +126,8 @@ hc_step_kernel(float* __restrict__ x, int n_tokens, int d, const TY* __restrict_
     }
     float ss = 0.f;
     const int width = (d % 4 == 0) ? 4 : 1;          // four columns per thread and round where rows allow 16-byte accesses
-#pragma unroll 2
-    for (int j0 = width * threadIdx.x; j0 < d; j0 += width * blockDim.x) {
-        float xs[S][4], yv[4] = {0.f, 0.f, 0.f, 0.f};
-        if (width == 4) {
-#pragma unroll
-            for (int s = 0; s < S; ++s) {
-                const float4 v = load4(x + ((size_t)s * n_tokens + t) * d + j0);
-                xs[s][0] = v.x; xs[s][1] = v.y; xs[s][2] = v.z; xs[s][3] = v.w;
-            }
-            if (y) {
-                const float4 v = load4(y + (size_t)t * d + j0);
-                yv[0] = v.x; yv[1] = v.y; yv[2] = v.z; yv[3] = v.w;
-            }
-        } else {
-#pragma unroll
-            for (int s = 0; s < S; ++s) xs[s][0] = x[((size_t)s * n_tokens + t) * d + j0];
-            if (y) yv[0] = to_f32(y[(size_t)t * d + j0]);
-        }
+    // the write and the read of `width` columns from j0 on
+    auto columns = [&](int j0, float (*xs)[4], const float* yv) {
         if (y) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -177,20 +161,60 @@ hc_step_kernel(float* __restrict__ x, int n_tokens, int d, const TY* __restrict_
                 ss += u * u;
             }
         }
+    };
+    // RR rounds' loads are sent before the first of their stores: with few tokens the kernel's time is its chain of loads (4 tokens of 2
+    // streams of 4,096 columns 6.0 -> 5.2 us), and the compiler cannot move a load of x above a store to it.
+    constexpr int RR = S <= 2 ? 4 : S <= 4 ? 2 : 1, AHEAD = S <= 4 ? 4 : 1;
+    float4 wv[AHEAD];                                // the norm's weights of the first rounds, loaded before the sum they wait for
+    if (width == 4) {
+        if (norm_w && in_w)
+#pragma unroll
+            for (int i = 0; i < AHEAD; ++i)
+                if (4 * (threadIdx.x + 256 * i) < d) wv[i] = load4(norm_w + 4 * (threadIdx.x + 256 * i));
+        for (int base = 4 * threadIdx.x; base < d; base += 1024 * RR) {
+            float xs[RR][S][4], yv[RR][4];
+#pragma unroll
+            for (int i = 0; i < RR; ++i) {
+                const int j0 = base + 1024 * i;
+                if (j0 >= d) break;
+#pragma unroll
+                for (int s = 0; s < S; ++s) {
+                    const float4 v = load4(x + ((size_t)s * n_tokens + t) * d + j0);
+                    xs[i][s][0] = v.x; xs[i][s][1] = v.y; xs[i][s][2] = v.z; xs[i][s][3] = v.w;
+                }
+                if (y) {
+                    const float4 v = load4(y + (size_t)t * d + j0);
+                    yv[i][0] = v.x; yv[i][1] = v.y; yv[i][2] = v.z; yv[i][3] = v.w;
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < RR; ++i) {
+                if (base + 1024 * i >= d) break;
+                columns(base + 1024 * i, xs[i], yv[i]);
+            }
+        }
+    } else {
+        for (int j0 = threadIdx.x; j0 < d; j0 += 256) {
+            float xs[S][4], yv[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < S; ++s) xs[s][0] = x[((size_t)s * n_tokens + t) * d + j0];
+            if (y) yv[0] = to_f32(y[(size_t)t * d + j0]);
+            columns(j0, xs, yv);
+        }
     }
     if (!in_w) return;
     float r = 1.f;
     if (norm_w) r = 1.0f / sqrtf(block_sum(ss, red) / (float)d + eps);
     if (width == 4) {
-#pragma unroll 2
-        for (int j0 = 4 * threadIdx.x; j0 < d; j0 += 4 * blockDim.x) {     // a thread reads back what it wrote itself
+        auto put = [&](int j0, const float4& w) {                          // a thread reads back what it wrote itself
             float4 u = *reinterpret_cast<const float4*>(u_row + j0);
-            if (norm_w) {
-                const float4 w = load4(norm_w + j0);
-                u = float4{u.x * r * w.x, u.y * r * w.y, u.z * r * w.z, u.w * r * w.w};
-            }
+            if (norm_w) u = float4{u.x * r * w.x, u.y * r * w.y, u.z * r * w.z, u.w * r * w.w};
             store4(h + (size_t)t * d + j0, u);
-        }
+        };
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i)
+            if (4 * (threadIdx.x + 256 * i) < d) put(4 * (threadIdx.x + 256 * i), wv[i]);
+        for (int j0 = 4 * (threadIdx.x + 256 * AHEAD); j0 < d; j0 += 1024) put(j0, norm_w ? load4(norm_w + j0) : float4{1.f, 1.f, 1.f, 1.f});
     } else {
         for (int j = threadIdx.x; j < d; j += blockDim.x) {
             const float u = u_row[j];
