@@ -297,7 +297,7 @@ attn_decode_reduce_kernel(const float* __restrict__ part_acc, const float* __res
 //
 // What bounds a block is the chain of one tile's steps in a wave, not memory (two tiles in flight gain nothing): scalar loop
 // control, accumulators in plain vector registers (two waves a SIMD asked for), one multiplication for a key's page, lane groups
-// that meet by register swaps, a sum that meets only at the end and a maximum that may lag took a tile from 1.25 to
+// that meet by register swaps, a sum that meets only at the end and no rescaling where no maximum grew took a tile from 1.25 to
 // 0.85 us.  24:8 heads of 64: 40 rows of 100..2,048 keys 25.1 -> 20.2 us, one row of 258 keys 6.7 -> 5.7; 32:2 heads of 128: 4 rows
 // of 16,385 keys 24.0 -> 21.2, 60 rows of 100..8,000 keys 49.9 -> 43.
 typedef __bf16 gq_bf16x8 __attribute__((ext_vector_type(8)));
@@ -450,7 +450,7 @@ attn_decode_gqa_kernel(const uint16_t* __restrict__ q, int q_stride,
 #pragma unroll
             for (int e = 0; e < 8; ++e) mloc = fmaxf(mloc, sv[e]);
             mloc = swap_max<16>(swap_max<32>(mloc));
-            if (__builtin_amdgcn_ballot_w64(mloc - m > kMaxSlack)) {     // (finite: every tile has at least one key)
+            if (__builtin_amdgcn_ballot_w64(mloc > m)) {     // rescaled only where a maximum grew; a row's largest weight stays exactly 1
                 const float m_new = fmaxf(m, mloc);
                 const float corr = __builtin_amdgcn_exp2f(m - m_new);
                 l *= corr;

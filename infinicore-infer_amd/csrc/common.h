@@ -94,8 +94,6 @@ template <int D> __device__ __forceinline__ float swap_max(float v) {
     const auto r = D == 32 ? __builtin_amdgcn_permlane32_swap(b, b, false, false) : __builtin_amdgcn_permlane16_swap(b, b, false, false);
     return fmaxf(__int_as_float((int)r[0]), __int_as_float((int)r[1]));
 }
-// Powers of two by which a running softmax's maximum may lag behind the scores before its accumulators are rescaled.
-constexpr float kMaxSlack = 8.0f;
 template <int LPK> __device__ __forceinline__ float group_sum(float d) {
     if (LPK >= 64) d = swap_add<32>(d);
     if (LPK >= 32) d = swap_add<16>(d);

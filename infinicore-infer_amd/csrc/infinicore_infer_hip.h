@@ -51,7 +51,7 @@ int ic_attn_decode_on_matrix_cores(int dtype, int n_heads, int n_kv_heads);
 int ic_attn_decode_wants_order(int n_rows, int nkvh, int nsplit, int compute_units);
 int ic_attn_decode_order(const int* positions, int* order, int n_rows, hipStream_t stream);
 int ic_attn_decode(const void* q, int q_stride, void* out, int out_stride, int dtype, const void* kcache, const void* vcache, const int* block_tables, int bt_stride, const int* tok_list, const int* token_req, const int* positions, float* part_acc, float* part_ml, int n_tok, int nh, int nkvh, int dh, int page_size, float scale, int window, int nsplit, hipStream_t stream);
-// Matrix-core kernels for prompt portions (bfloat16; and true float32 with float32 matrix instructions, one wave group, walks never cut).
+// Matrix-core kernels for prompt portions (bfloat16; and true float32 with float32 matrix instructions, walks never cut).
 // tiles: int32 [n_tiles, 4] = (request row, first token row, rows <= tile_rows, first position).
 int ic_attn_prefill_supported(int dtype, int dh, int page_size);
 int ic_attn_prefill_tile_rows();

@@ -1,5 +1,5 @@
-"""Attention where scores climb along the keys: the running maximum may lag by up to eight powers of two before the accumulators are
-rescaled, and rows of one wave climb, fall and stay level at once."""
+"""Attention where scores climb along the keys: the accumulators are rescaled only in steps where some row's maximum grew, and rows of
+one wave climb, fall and stay level at once."""
 import math
 
 import pytest
