@@ -4,8 +4,8 @@
 // What runs for a layer depends on the step alone, never on the model: up to 16 rows in bfloat16 take the
 // few-row products with their epilogues (rotary and cache write after QKV; residual add, the next norm's
 // weight and sums of squares after O and down; SwiGLU after gate/up), the norm between two products being
-// split over them; more rows, or float32, take the library's products and the norm, rotary and activation
-// kernels.  Single-token rows go to the split-key attention kernel, prompt portions to the tiled one, what
+// split over them; more rows take the products in tiles (gate/up with SwiGLU in its epilogue) or the library's, as
+// ic_product chooses, float32 the library's, and the norm, rotary and activation kernels.  Single-token rows go to the split-key attention kernel, prompt portions to the tiled one, what
 // neither takes to the general one.
 #include "common.h"
 #include "infinicore_infer_engine.h"
@@ -64,6 +64,11 @@ IC_EXPORT int ic_rule_gate_up_fused(int dtype, int rows, int K, int lda, int ldw
     if (dtype != IC_BF16) return 0;
     if (rows <= kFewRows) return 1;
     return !row_factors_owed && rows <= ic_gemm_nt_epilogue_rows(1, K, lda, ldw);
+}
+
+IC_EXPORT int ic_rule_gate_up_tiles(int dtype, const void* A, const void* W, const void* C, int rows, int N, int K, int lda, int ldw, int ldc) {
+    const bool aligned = !(((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) & 15);
+    return dtype == IC_BF16 && aligned && ic_gemm_tiles_supported(rows, N, K, lda, ldw, ldc, 1) && ic_gemm_tiles_pays(rows, N, K, 1);
 }
 
 IC_EXPORT int ic_rule_tail(int dtype, int rows, int N, int K, int lda, int ldw) {
@@ -174,7 +179,7 @@ struct IcDecoder {
         w.total = o;
         return w;
     }
-    // out[M, N] = alpha * a w^T: the few-row product, or the library's.
+    // out[M, N] = alpha * a w^T: the few-row product, or what ic_product takes.
     int linear(const void* a, int lda, const void* w, void* out, int out_dtype, int M, int N, int K, float alpha,
                const Deferred* rows, void* lib_ws, long long lib_ws_bytes, hipStream_t stream) const {
         if (ic_rule_own_product(meta.dtype, meta.dtype, out_dtype, M)) {
@@ -184,7 +189,7 @@ struct IcDecoder {
                               nullptr, stream);
         }
         if (rows) return IC_ERR_ARG;      // half-normed rows exist only where the few-row product runs
-        return ic_matmul(a, meta.dtype, w, out, out_dtype, M, N, K, lda, K, N, alpha, lib_ws, lib_ws_bytes, stream);
+        return ic_product(a, meta.dtype, w, out, out_dtype, M, N, K, lda, K, N, alpha, lib_ws, lib_ws_bytes, stream);
     }
 
     // 17..64 rows (and 13..16 long ones) into the residual stream: x += alpha * (a w^T), out = rmsnorm(x) * weight, through the sliced
@@ -347,6 +352,9 @@ struct IcDecoder {
                 st = ic_gemm_nt(g, IC_BF16, L.ffn.w_gate_up, IC_BF16, act, IC_BF16, T, 2 * di, d, d, d, di, 1.0f, 1, g_def ? &gf : nullptr,
                                 nullptr, stream);
                 if (st) return fail(st, "the gate/up product with SwiGLU", i);
+            } else if (ic_rule_gate_up_tiles(dt, g, L.ffn.w_gate_up, act, T, 2 * di, d, d, d, di)) {
+                st = ic_gemm_tiles(g, L.ffn.w_gate_up, act, T, 2 * di, d, d, d, di, 1, stream);
+                if (st) return fail(st, "the gate/up product with SwiGLU, in tiles", i);
             } else {
                 st = linear(g, d, L.ffn.w_gate_up, base + ws.gate_up, dt, T, 2 * di, d, 1.0f, nullptr, lib_ws, lib_ws_bytes, stream);
                 if (st) return fail(st, "the gate/up product", i);

@@ -1,0 +1,438 @@
+// C[M, N] = A[M, K] * W[N, K]^T for many rows M (prompts and mixed steps): bfloat16 operands on the matrix cores, float32
+// accumulation, the result's next operation in the epilogue.
+//
+// A block of WM x WN x WK waves owns a tile of BM rows of A by BN rows of W.  Both operands go from memory straight into LDS
+// (global_load_lds_dwordx4, 1 KB an instruction and wave), STAGES stages of 64 k deep: rows of 128 bytes without padding, the
+// 16-byte chunk c of row r at position c ^ (r / 2 % 8), which each lane arranges by what it fetches, so that the operand reads of
+// 16 rows cover the 64 banks once.  A wave holds TM x TN results (TM = BM / WM, TN = BN / WN) in registers and walks every WK-th
+// k-step of 32; with WK > 1 the waves of a tile meet in LDS at the end.
+//
+// The walk over K: the operands of a k-step are read from LDS while the previous step is multiplied.  Before the last step of a
+// stage is multiplied a wave waits for its own loads of the next stage and for its reads of this one, then all waves meet: after
+// that barrier the next stage is whole and this one is free, and the loads of the stage STAGES further on go into it.  So loads
+// have STAGES - 1 stages of products to arrive, and there is one barrier a stage.  The loads are written as inline assembly: the
+// compiler, which cannot see which LDS bytes such a load writes, otherwise waits for all of them before every operand read.  They
+// have no register results, so nothing but LDS is written while they are in flight.
+//
+// What bounds it.  Few tiles (up to one a compute unit): a stage's products at the matrix cores' rate plus its barrier and what the loads hold up the
+// products: 256 x 256 0.96 us a stage (0.87 with products alone), 192 x 192 0.58 (0.49), 128 x 128 0.30 (0.23), and about 4 us for launch, first
+// loads and the way out.  128 x 128 tiles take all of a unit's 64 bytes a cycle from L2 for their loads, 256 x 256 half of it, hence the large
+// tiles where there are rows and columns enough.  The whole chip busy for long: its power, the clock gives way (256 x 256: 1.38..1.5 us a stage).
+// Waves of 64 x 64 results and more need four waves of up to 512 registers a block: eight waves of half the size read 1.5 times as much from LDS
+// (256 x 256: 1.07 us a stage).  v_mfma_f32_32x32x16_bf16 instead of 16x16x32 is no faster (0.96 and 0.97).
+//
+// 16x16x32 layout (lane l): A[i = l%16][k = 8(l/16)..+7], B[k = 8(l/16)..+7][j = l%16], D[i = 4(l/16) + e][j = l%16], e = 0..3;
+// i are weight rows here and j token rows, so a lane holds four neighbouring columns of one row of C.
+#include "common.h"
+#include "infinicore_infer_variants.h"
+#include <type_traits>
+#include <utility>
+
+namespace {
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef __bf16 v8b __attribute__((ext_vector_type(8)));
+
+struct TilesArgs {
+    const uint16_t* A;
+    const uint16_t* W;
+    uint16_t* C;
+    int M, N, K, lda, ldw, ldc;   // N: rows of W
+    int tiles_m, tiles_n;         // the grid: tiles_m * tiles_n blocks
+    int group_m;                  // row tiles that are walked together
+};
+
+enum { EPI_BF16 = 0, EPI_SWIGLU = 1 };
+
+// 16 bytes a lane from base + off (bytes; base the same for the wave) to LDS at lds + plus + 16 * lane.
+template <int PLUS> __device__ __forceinline__ void load_to_lds(unsigned lds, unsigned off, const char* base) {
+    asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base), "i"(PLUS) : "memory", "scc");
+}
+// waits until at most N of this wave's loads are on their way and all its LDS reads are done
+template <int N> __device__ __forceinline__ void wait_loads() {
+    static_assert(N >= 0 && N < 64, "vmcnt has six bits");
+    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (0 << 8));
+}
+constexpr int min_of(int a, int b) { return a < b ? a : b; }
+// f(0), f(1), .. f(N - 1), each with its number as a type
+template <typename F, int... Is> __device__ __forceinline__ void each_of(F&& f, std::integer_sequence<int, Is...>) {
+    (f(std::integral_constant<int, Is>{}), ...);
+}
+template <int N, typename F> __device__ __forceinline__ void each(F&& f) { each_of(f, std::make_integer_sequence<int, N>{}); }
+
+// acc += w a, the accumulator in the registers' second half (an operand that is read and written by one instruction: where a wave holds more
+// than 128 of them the compiler's own product copies them from product to product)
+__device__ __forceinline__ void product(v4f& acc, const v8b& w, const v8b& a) {
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(w), "v"(a));
+}
+
+template <int BM_, int BN_, int WM_, int WN_, int WK_, int STAGES_> struct Tile {
+    static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, WK = WK_, STAGES = STAGES_;
+    static constexpr int WAVES = WM * WN * WK, TM = BM / WM, TN = BN / WN, MT = TM / 16, NT = TN / 16;
+    static constexpr int STEPS = 2 / WK;                           // k-steps of a stage that a wave multiplies
+    static constexpr int STAGE_BYTES = (BM + BN) * 128;
+    static constexpr int LOADS_A = BM / 8 / WAVES, LOADS = LOADS_A + BN / 8 / WAVES;    // of 1 KB, a wave and stage
+    static constexpr int SUM_BYTES = BM * BN * 4 * (WK - 1);
+    static constexpr int LDS_BYTES = STAGES * STAGE_BYTES > SUM_BYTES ? STAGES * STAGE_BYTES : SUM_BYTES;
+    static constexpr int REGISTERS = TM * TN / 64 + (MT + NT) * 8 + LOADS + 24;
+    static constexpr int BLOCKS_PER_CU = (LDS_BYTES <= 80 * 1024 && REGISTERS <= 256 && WAVES == 4) ? 2 : 1;
+    static constexpr int MIN_WAVES = WAVES * BLOCKS_PER_CU / 4;    // a SIMD's
+    static_assert(BM % (16 * WM) == 0 && BN % (16 * WN) == 0, "whole matrix tiles");
+    static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "every wave loads as much");
+    static_assert(STEPS == 1 || STEPS == 2, "a stage is two k-steps");
+    static_assert(MT % WK == 0 && LDS_BYTES <= 160 * 1024 && LOADS * (STAGES - 1) < 64 && MIN_WAVES >= 1, "limits");
+};
+
+template <typename T, int EPI>
+__global__ void __launch_bounds__(T::WAVES * 64, T::MIN_WAVES) gemm_tiles_kernel(TilesArgs a) {
+    constexpr int BM = T::BM, BN = T::BN, WN = T::WN, WK = T::WK, STAGES = T::STAGES, WAVES = T::WAVES;
+    constexpr int TM = T::TM, TN = T::TN, MT = T::MT, NT = T::NT, STEPS = T::STEPS, LOADS = T::LOADS, LOADS_A = T::LOADS_A;
+    static_assert(EPI != EPI_SWIGLU || NT % 2 == 0, "a wave holds gate and up columns alike");
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[T::LDS_BYTES];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, kq = lane >> 4;
+    const int wk = wave % WK, wn = wave / WK % WN, wm = wave / (WK * WN);
+
+    // Which tile: blocks go to the 8 XCDs in turn, so block b is the (b / 8)-th of XCD b % 8, and every XCD takes one run of tiles
+    // (its L2 then holds few rows of W and A); a run goes down group_m row tiles, then to the next columns.
+    const int total = a.tiles_m * a.tiles_n;
+    const int xcd = blockIdx.x & 7, nth = blockIdx.x >> 3;
+    const int t = xcd * (total >> 3) + min(xcd, total & 7) + nth;
+    const int group = t / (a.group_m * a.tiles_n), first_m = group * a.group_m;
+    const int gm = min(a.group_m, a.tiles_m - first_m), in_group = t - group * a.group_m * a.tiles_n;
+    const int bn = in_group / gm, bm = first_m + in_group - bn * gm;
+    const int m0 = bm * BM;
+    const int NO = EPI == EPI_SWIGLU ? a.N / 2 : a.N;              // columns of C
+    constexpr int BNO = EPI == EPI_SWIGLU ? BN / 2 : BN;
+    const int n0 = bn * BNO;
+
+    const int n_stages = a.K / 64;
+
+    // What this lane fetches: byte offsets from the tile's first row of A, or from W (rows beyond the matrix repeat the last one)
+    const char* base_a = (const char*)(a.A + (size_t)m0 * a.lda);
+    const char* base_w = (const char*)(a.W + (EPI == EPI_SWIGLU ? (size_t)0 : (size_t)n0 * a.ldw));
+    unsigned off[LOADS];
+    each<LOADS>([&](auto at) {
+        constexpr int I = decltype(at)::value;
+        const int row = 8 * (wave + WAVES * (I < LOADS_A ? I : I - LOADS_A)) + (lane >> 3);
+        const unsigned chunk = 16 * ((lane & 7) ^ ((row >> 1) & 7));
+        if constexpr (I < LOADS_A) {
+            off[I] = (unsigned)min(row, a.M - 1 - m0) * (unsigned)(a.lda * 2) + chunk;
+        } else if constexpr (EPI == EPI_SWIGLU) {                  // a wave's TN columns: TN / 2 of gate, then the same of up
+            const int x = row % TN, col = min(n0 + row / TN * (TN / 2) + x % (TN / 2), NO - 1);
+            off[I] = (unsigned)(col + (x >= TN / 2 ? NO : 0)) * (unsigned)(a.ldw * 2) + chunk;
+        } else {
+            off[I] = (unsigned)min(row, a.N - 1 - n0) * (unsigned)(a.ldw * 2) + chunk;
+        }
+    });
+    // this wave's I-th load of a stage: at_a, at_w are the stage's bases, into the buffer at LDS address `into` (of this wave's first chunk)
+    const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds + wave * 1024;
+    auto fetch = [&](auto at, const char* at_a, const char* at_w, unsigned into) {
+        constexpr int I = decltype(at)::value;
+        if constexpr (I < LOADS_A) load_to_lds<I * WAVES * 1024>(into, off[I], at_a);
+        else load_to_lds<BM * 128 + (I - LOADS_A) * WAVES * 1024>(into, off[I], at_w);
+    };
+
+    v4f acc[NT][MT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = v4f{0.f, 0.f, 0.f, 0.f};
+    asm volatile("s_nop 7");
+
+    // operand registers of two k-steps: one is multiplied while the other is read
+    v8b fa[2][MT], fw[2][NT];
+    const unsigned char* const pa = lds + (wm * TM + r) * 128;
+    const unsigned char* const pw = lds + (BM + wn * TN + r) * 128;
+    const int sw = (r >> 1) & 7;
+    // byte of a row where step `step` (of the wave's STEPS in a stage) has this lane's eight k
+    auto place = [&](int step) { return 16 * ((4 * (step * WK + wk) + kq) ^ sw); };
+
+    // The loads of stage s + STAGES go into the buffer of stage s from that stage's barrier on: with more than two stages SPREAD of them in each
+    // k-step up to the next barrier, so that they do not queue up behind one another (a 1 KB load takes the unit 16 cycles, and a wave that
+    // waits to issue one issues no products: 192 x 192 tiles 0.72 -> 0.58 us a stage); with two the last ones would have to arrive too soon.
+    constexpr int SPREAD = STAGES > 2 ? (LOADS + STEPS - 1) / STEPS : LOADS;
+    // the first stages, the last of them without what the first stage's steps load
+    each<STAGES>([&](auto sc) {
+        constexpr int S = decltype(sc)::value;
+        const int from = 128 * min(S, n_stages - 1);
+        each<S + 1 < STAGES ? LOADS : SPREAD>([&](auto i) { fetch(i, base_a + from, base_w + from, lds0 + S * T::STAGE_BYTES); });
+    });
+    wait_loads<LOADS * (STAGES - 2) + SPREAD>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) fw[0][nt] = *reinterpret_cast<const v8b*>(pw + place(0) + nt * 2048);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) fa[0][mt] = *reinterpret_cast<const v8b*>(pa + place(0) + mt * 2048);
+
+    // One k-step: the registers CUR are multiplied while the others are read (step `step` of the stage in `buf`) and this wave's loads
+    // FROM .. TO - 1 of the stage at at_a, at_w go out.  The reads are dealt over the first three quarters of the products, the loads over all of
+    // them: left to itself the scheduler moves them all to the end, where the next step waits for them.
+    auto step_of = [&](auto curc, auto fromc, auto toc, int buf, int step, const char* at_a, const char* at_w, unsigned into) {
+        constexpr int CUR = decltype(curc)::value, P = MT * NT, R = NT + MT, L0 = decltype(fromc)::value, L = decltype(toc)::value - L0;
+        const unsigned char* const qa = pa + buf * T::STAGE_BYTES + place(step);
+        const unsigned char* const qw = pw + buf * T::STAGE_BYTES + place(step);
+        each<P>([&](auto at) {
+            constexpr int I = decltype(at)::value;
+            constexpr int R0 = I == 0 ? 0 : min_of(R, 4 * (I - 1) * R / (3 * P) + 1), R1 = min_of(R, 4 * I * R / (3 * P) + 1);
+            constexpr int F0 = I == 0 || L == 0 ? 0 : min_of(L, (I - 1) * L / P + 1), F1 = L == 0 ? 0 : min_of(L, I * L / P + 1);
+            each<R1 - R0>([&](auto k) {
+                constexpr int O = R0 + decltype(k)::value;
+                if constexpr (O < NT) fw[CUR ^ 1][O] = *reinterpret_cast<const v8b*>(qw + O * 2048);
+                else fa[CUR ^ 1][O - NT] = *reinterpret_cast<const v8b*>(qa + (O - NT) * 2048);
+            });
+            each<F1 - F0>([&](auto k) { fetch(std::integral_constant<int, L0 + F0 + decltype(k)::value>{}, at_a, at_w, into); });
+            if constexpr (R1 > R0 || F1 > F0) __builtin_amdgcn_sched_barrier(0);
+            product(acc[I / MT][I % MT], fw[CUR][I / MT], fa[CUR][I % MT]);
+        });
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // where they come from: beyond the last stage that one is loaded again (and read by nobody)
+    const char *ahead_a = base_a + 128 * min(STAGES - 1, n_stages - 1), *ahead_w = base_w + 128 * min(STAGES - 1, n_stages - 1);
+    auto whole_stage = [&](int s, int buf, auto cur0) {            // cur0: which operand registers hold its first step
+        const int next = buf + 1 == STAGES ? 0 : buf + 1, before = buf == 0 ? STAGES - 1 : buf - 1;
+        each<STEPS>([&](auto pc) {
+            constexpr int P = decltype(pc)::value;
+            using Cur = std::integral_constant<int, (decltype(cur0)::value + P) & 1>;
+            if constexpr (P + 1 < STEPS) {
+                step_of(Cur{}, std::integral_constant<int, SPREAD>{}, std::integral_constant<int, LOADS>{}, buf, P + 1, ahead_a, ahead_w,
+                        lds0 + before * T::STAGE_BYTES);
+            } else {
+                wait_loads<LOADS * (STAGES - 2)>();                // under way: stages s + 1 .. s + STAGES - 1
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+                const int on = s + STAGES < n_stages ? 128 : 0;
+                ahead_a += on;
+                ahead_w += on;
+                step_of(Cur{}, std::integral_constant<int, 0>{}, std::integral_constant<int, SPREAD>{}, next, 0, ahead_a, ahead_w,
+                        lds0 + buf * T::STAGE_BYTES);
+            }
+        });
+        return next;
+    };
+    int s = 0, buf = 0;
+    if constexpr (STEPS == 1) {                                    // two stages a round, so that the operand registers are named by constants
+        for (; s + 1 < n_stages; s += 2) {
+            buf = whole_stage(s, buf, std::integral_constant<int, 0>{});
+            buf = whole_stage(s + 1, buf, std::integral_constant<int, 1>{});
+        }
+        if (s < n_stages) whole_stage(s, buf, std::integral_constant<int, 0>{});
+    } else {
+        for (; s < n_stages; ++s) buf = whole_stage(s, buf, std::integral_constant<int, 0>{});
+    }
+    wait_loads<0>();
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop 15\n\ts_nop 15");                          // the last products are done before other instructions read their results
+    __builtin_amdgcn_sched_barrier(0);
+    __syncthreads();                                               // LDS is free
+
+    constexpr int SH = MT / WK;                                    // row tiles of C this wave writes: SH from the wk-th run on
+    if constexpr (WK > 1) {
+        // the WK waves of the same results add up, each its own run of rows
+        float* const red = reinterpret_cast<float*>(lds) + (size_t)(wm * WN + wn) * (WK * (WK - 1) * SH * NT * 256);
+        auto cell = [&](int whose, int src, int j, int nt) {
+            return reinterpret_cast<v4f*>(red + ((((whose * (WK - 1) + src) * SH + j) * NT + nt) * 64 + lane) * 4);
+        };
+#pragma unroll
+        for (int o = 0; o < WK; ++o)                               // o: whose run
+            if (o != wk) {
+#pragma unroll
+                for (int j = 0; j < SH; ++j)
+#pragma unroll
+                    for (int nt = 0; nt < NT; ++nt) *cell(o, wk < o ? wk : wk - 1, j, nt) = acc[nt][o * SH + j];
+            }
+        __syncthreads();
+#pragma unroll
+        for (int o = 1; o < WK; ++o)
+            if (o == wk) {
+#pragma unroll
+                for (int j = 0; j < SH; ++j)
+#pragma unroll
+                    for (int nt = 0; nt < NT; ++nt) acc[nt][j] = acc[nt][o * SH + j];
+            }
+#pragma unroll
+        for (int src = 0; src < WK - 1; ++src)
+#pragma unroll
+            for (int j = 0; j < SH; ++j)
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) acc[nt][j] += *cell(wk, src, j, nt);
+        __syncthreads();
+    }
+    constexpr int ONT = EPI == EPI_SWIGLU ? NT / 2 : NT;           // column tiles of C
+    const int c0 = n0 + wn * (ONT * 16);
+    const int row0 = m0 + wm * TM + wk * (16 * SH);
+
+    // 16 rows at a time through LDS of the wave's own, so that whole lines are stored
+    constexpr int ROW = ONT * 32 + 16, PER_ROW = ONT * 2;          // bytes of a row in LDS; 16-byte chunks of a row
+    unsigned char* const mine = lds + wave * (16 * ROW);
+    static_assert(WAVES * 16 * ROW <= T::LDS_BYTES, "room for the rows");
+#pragma unroll
+    for (int j = 0; j < SH; ++j) {
+#pragma unroll
+        for (int nt = 0; nt < ONT; ++nt) {
+            uint16_t b[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float v = acc[nt][j][e];
+                if constexpr (EPI == EPI_SWIGLU) v = silu_mul_fast(v, acc[nt + ONT][j][e]);
+                b[e] = __builtin_bit_cast(uint16_t, __float2bfloat16(v));
+            }
+            *reinterpret_cast<uint2*>(mine + r * ROW + 32 * nt + 8 * kq) =
+                uint2{(unsigned)b[0] | ((unsigned)b[1] << 16), (unsigned)b[2] | ((unsigned)b[3] << 16)};
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < (16 * PER_ROW + 63) / 64; ++i) {
+            const int q = lane + 64 * i, lr = q / PER_ROW, ch = q - lr * PER_ROW;
+            const int m = row0 + 16 * j + lr, n = c0 + 8 * ch;
+            if ((16 * PER_ROW % 64 == 0 || q < 16 * PER_ROW) && m < a.M && n < NO)
+                *reinterpret_cast<uint4*>(a.C + (size_t)m * a.ldc + n) = *reinterpret_cast<const uint4*>(mine + lr * ROW + 16 * ch);
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+template <typename T, int EPI> int launch(TilesArgs a, hipStream_t stream) {
+    a.tiles_m = (a.M + T::BM - 1) / T::BM;
+    a.tiles_n = EPI == EPI_SWIGLU ? (a.N / 2 + T::BN / 2 - 1) / (T::BN / 2) : (a.N + T::BN - 1) / T::BN;
+    const int groups = (a.tiles_m + 7) / 8;
+    a.group_m = (a.tiles_m + groups - 1) / groups;
+    const long long blocks = (long long)a.tiles_m * a.tiles_n;
+    if (blocks > (1LL << 30)) return IC_ERR_ARG;
+    hipLaunchKernelGGL((gemm_tiles_kernel<T, EPI>), dim3((unsigned)blocks), dim3(T::WAVES * 64), 0, stream, a);
+    return ic_launch_status();
+}
+
+// The tiles, smallest first, and what one costs in microseconds: FIXED + rounds * (ROUND + stages * STAGE * (1 + FULL * x)), where x is the part of
+// the 256 compute units that have a block and a round is one block a unit (two of 64 x 64, which then share it: 1.7 times the stage).  Fitted to 5,900
+// timed products (17 pairs of N in 512..32,768 and K in 512..16,384, 33..16,384 rows, weights out of memory); the tile with the least cost loses 1.1 % to
+// the best of 20 tiles on average and 7 % at the 95th percentile.  Of those 20 these 12 are kept: the others were never needed for more than 0.1 %.
+#define IC_TILES(X) \
+    /* number, FIXED, STAGE, FULL, ROUND, tile: BM, BN, WM, WN, WK, STAGES */ \
+    X(0, 2.75, 0.191, 0.33, 0.00, 64, 64, 2, 1, 2, 4) \
+    X(1, 2.31, 0.306, 0.24, 0.79, 64, 128, 2, 2, 1, 6) \
+    X(2, 1.97, 0.325, 0.32, 1.54, 96, 128, 2, 2, 1, 5) \
+    X(3, 2.10, 0.377, 0.37, 1.72, 128, 128, 2, 2, 1, 5) \
+    X(4, 2.60, 0.463, 0.42, 1.36, 192, 128, 2, 2, 1, 3) \
+    X(5, 2.75, 0.514, 0.32, 1.19, 128, 192, 2, 2, 1, 4) \
+    X(6, 2.56, 0.571, 0.30, 1.81, 160, 192, 2, 2, 1, 3) \
+    X(7, 2.31, 0.570, 0.38, 2.54, 256, 128, 2, 2, 1, 3) \
+    X(8, 2.36, 0.653, 0.27, 1.85, 128, 256, 2, 2, 1, 3) \
+    X(9, 2.76, 0.700, 0.31, 2.54, 160, 256, 2, 2, 1, 3) \
+    X(10, 4.21, 0.952, 0.27, 0.00, 256, 192, 2, 2, 1, 2) \
+    X(11, 6.10, 1.077, 0.33, 0.00, 256, 256, 2, 2, 1, 2)
+
+constexpr int kTiles = 12;
+constexpr double kUnits = 256.0;
+
+struct TileCost { int bm, bn, blocks_per_unit; double fixed, stage, full, round; };
+constexpr TileCost kCosts[kTiles] = {
+#define X(I, FIXED, STAGE, FULL, ROUND, ...) {Tile<__VA_ARGS__>::BM, Tile<__VA_ARGS__>::BN, Tile<__VA_ARGS__>::BLOCKS_PER_CU, FIXED, STAGE, FULL, ROUND},
+    IC_TILES(X)
+#undef X
+};
+
+double cost_of(const TileCost& t, int M, int N, int K, int mode) {
+    const long long tm = (M + t.bm - 1) / t.bm, tn = mode == EPI_SWIGLU ? (N / 2 + t.bn / 2 - 1) / (t.bn / 2) : (N + t.bn - 1) / t.bn;
+    const double tiles = (double)(tm * tn), x = tiles / kUnits, stages = K / 64;
+    double rounds = 1.0, busy = x < 1.0 ? x : 1.0, shared = 1.0;
+    if (x > 1.0) {
+        rounds = __builtin_ceil(x / t.blocks_per_unit);
+        if (t.blocks_per_unit > 1) shared = 1.7;
+    }
+    const double walk = t.fixed + rounds * (t.round + stages * t.stage * (1.0 + t.full * busy) * shared);
+    // the weights come from memory once, and about half of them again for every further row tile (blocks of one column of tiles seldom run abreast)
+    const double read = 3.0 + 2.0 * N * K * (1.0 + 0.5 * (tm < 4 ? tm - 1 : 3)) / 7e6;
+    return walk > read ? walk : read;
+}
+
+int best_tile(int M, int N, int K, int mode, double* cost) {
+    int best = 0;
+    for (int i = 0; i < kTiles; ++i) {
+        const double c = cost_of(kCosts[i], M, N, K, mode);
+        if (i == 0 || c < *cost) { *cost = c; best = i; }
+    }
+    return best;
+}
+
+template <int EPI> int by_number(int tile, const TilesArgs& a, hipStream_t stream) {
+    switch (tile) {
+#define X(I, FIXED, STAGE, FULL, ROUND, ...) case I: return launch<Tile<__VA_ARGS__>, EPI>(a, stream);
+        IC_TILES(X)
+#undef X
+    }
+    return IC_ERR_ARG;
+}
+
+bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+
+// Whole stages of K, 16-byte pieces of every row, byte offsets within 32 bits.
+bool takes(int M, int N, int K, int lda, int ldw, int ldc, int mode) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % 64 || lda < K || ldw < K || lda % 8 || ldw % 8) return false;
+    const int cols = mode == EPI_SWIGLU ? N / 2 : N;
+    if (N % (mode == EPI_SWIGLU ? 16 : 8) || ldc < cols || ldc % 8) return false;
+    if ((long long)lda * 2 * 256 >= (1LL << 31) || (long long)ldw * 2 * (mode == EPI_SWIGLU ? N : 256) >= (1LL << 32)) return false;
+    return (long long)((M + 63) / 64) * ((N + 63) / 64) < (1LL << 29);
+}
+
+int run(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, int mode, int tile, hipStream_t stream) {
+    TilesArgs a{(const uint16_t*)A, (const uint16_t*)W, (uint16_t*)C, M, N, K, lda, ldw, ldc, 0, 0, 0};
+    return mode == EPI_SWIGLU ? by_number<EPI_SWIGLU>(tile, a, stream) : by_number<EPI_BF16>(tile, a, stream);
+}
+
+}  // namespace
+
+IC_EXPORT int ic_gemm_tiles_supported(int M, int N, int K, int lda, int ldw, int ldc, int mode) {
+    return (mode == EPI_BF16 || mode == EPI_SWIGLU) && takes(M, N, K, lda, ldw, ldc, mode);
+}
+
+// Whether the library would be faster.  Two kinds of product where it is, fitted to the same sweep (own against library, the choice loses 2.2 % to the
+// faster of the two on average; the own kernel everywhere: 6.3 %):
+//   full rounds of 256 x 256 tiles, where nothing is left to choose and its kernel spends less on a stage (8,192 x 4,096 x 14,336: 601 us against 691;
+//   4,096 x 4,096 x 4,096: 90 against 93);
+//   long rows and few tiles, which it splits over K (256 x 1,024 x 8,192: 20 us against 32): the own kernel's walk over K is compared with what a
+//   product split over the whole chip takes.
+// Elsewhere the own kernel is faster (1,045 x 2,560 x 1,536: 17.0 -> 12.2 us; 871 x 1,536 x 1,536: 12.5 -> 10.0; 2,048 x 2,304 x 2,304: 28 -> 22.6).
+// With the gated unit in the epilogue it is compared with the library's product and the unit's own kernel, and is always faster from 33 rows on
+// (1,045 x 7,680 x 1,536: 42.0 -> 28.0; 2,048 x 11,520 x 2,304: 131 -> 97; 16,384 x 32,768 x 4,096: 3,135 -> 2,942).
+IC_EXPORT int ic_gemm_tiles_pays(int M, int N, int K, int mode) {
+    if (M <= 32) return 0;
+    const double t = (double)((M + 255) / 256) * ((N + 255) / 256), fill = t / (kUnits * __builtin_ceil(t / kUnits));
+    if (mode == EPI_SWIGLU) return K <= 8192 || fill < 0.93;
+    if (t >= 200.0 && fill >= 0.93) return 0;
+    double cost = 0.0;
+    best_tile(M, N, K, mode, &cost);
+    const double products = 2.0 * M * N * K / 0.6e9, read = 2.0 * N * K / 5e6;
+    return cost <= 1.4 * (6.0 + (products > read ? products : read));
+}
+
+IC_EXPORT int ic_gemm_tiles_plan(int M, int N, int K, int mode) {
+    double cost = 0.0;
+    return M > 0 && N > 0 && K > 0 ? best_tile(M, N, K, mode, &cost) : -1;
+}
+
+IC_EXPORT int ic_gemm_tiles(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, int mode, hipStream_t stream) {
+    if (M <= 0) return IC_OK;
+    if (!A || !W || !C || !ic_gemm_tiles_supported(M, N, K, lda, ldw, ldc, mode) || !aligned16(A) || !aligned16(W) || !aligned16(C)) return IC_ERR_ARG;
+    double cost = 0.0;
+    return run(A, W, C, M, N, K, lda, ldw, ldc, mode, best_tile(M, N, K, mode, &cost), stream);
+}
+
+IC_EXPORT int ic_gemm_tiles_cfg(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, int mode, int tile,
+                                hipStream_t stream) {
+    if (M <= 0) return IC_OK;
+    if (!A || !W || !C || tile < 0 || tile >= kTiles || !ic_gemm_tiles_supported(M, N, K, lda, ldw, ldc, mode) || !aligned16(A) || !aligned16(W) ||
+        !aligned16(C)) return IC_ERR_ARG;
+    return run(A, W, C, M, N, K, lda, ldw, ldc, mode, tile, stream);
+}
+
+// The product by the kernel that is faster for it: this file's or the library's.
+IC_EXPORT int ic_product(const void* A, int a_dtype, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldw, int ldc, float alpha,
+                         void* workspace, long long workspace_bytes, hipStream_t stream) {
+    if (a_dtype == IC_BF16 && c_dtype == IC_BF16 && alpha == 1.0f && A && W && C && ic_gemm_tiles_supported(M, N, K, lda, ldw, ldc, EPI_BF16) &&
+        aligned16(A) && aligned16(W) && aligned16(C) && ic_gemm_tiles_pays(M, N, K, EPI_BF16))
+        return ic_gemm_tiles(A, W, C, M, N, K, lda, ldw, ldc, EPI_BF16, stream);
+    return ic_matmul(A, a_dtype, W, C, c_dtype, M, N, K, lda, ldw, ldc, alpha, workspace, workspace_bytes, stream);
+}

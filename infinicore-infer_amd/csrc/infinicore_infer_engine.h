@@ -171,6 +171,8 @@ int ic_rule_own_product(int a_dtype, int w_dtype, int c_dtype, int rows);
 int ic_rule_qkv_fused(int dtype, int rows, int K, int lda, int ldw, int head_dim, int rot_dim, int kv_heads_written, int row_factors_owed);
 // 1: the gate/up projection runs with SwiGLU in its epilogue (ic_gemm_nt, c_mode 1); 0: product, then ic_swiglu.
 int ic_rule_gate_up_fused(int dtype, int rows, int K, int lda, int ldw, int row_factors_owed);
+// More rows: 1: the gate/up projection with SwiGLU in its epilogue in tiles (ic_gemm_tiles, mode 1).  N: rows of W; ldc: the row stride of its result.
+int ic_rule_gate_up_tiles(int dtype, const void* A, const void* W, const void* C, int rows, int N, int K, int lda, int ldw, int ldc);
 // How a projection into the residual stream (O, down: N = hidden) that a norm follows runs: IC_TAIL_*.
 int ic_rule_tail(int dtype, int rows, int N, int K, int lda, int ldw);
 // Which attention kernels a step with n_decode_rows single-token rows and n_tiles prompt tiles takes: IC_ATTN_GENERAL, or bits.

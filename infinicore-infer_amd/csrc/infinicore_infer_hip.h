@@ -148,6 +148,16 @@ int ic_gemm_splitk(const void* A, const void* W, float* P, int M, int N, int K, 
 // P [S, M, d]: x += alpha * (the product, rounded to bfloat16) + s0 y0 + s1 y1 (bfloat16 [M, d], nullable); out = rmsnorm(x) * w.
 int ic_splitk_add_rmsnorm(const float* P, int n_slices, int M, float* x, float alpha, const float* w, void* out, int d, float eps, const void* y0, float s0, const void* y1, float s1, hipStream_t stream);
 
+// ---- gemm_tiles.hip -----------------------------------------------------------------------------------
+// Products of many rows in tiles on the matrix cores: bfloat16 operands and result, float32 accumulation.  mode 0: C[M, N] = A[M, K] W[N, K]^T.
+// mode 1: W = [gate; up], C[M, N/2] = up * silu(gate), computed from the float32 products.  K a multiple of 64, strides and columns of C multiples
+// of 8, operands 16-byte aligned.  ic_gemm_tiles_pays: whether it is the faster way (else the library's product, and for mode 1 ic_swiglu).
+int ic_gemm_tiles_supported(int M, int N, int K, int lda, int ldw, int ldc, int mode);
+int ic_gemm_tiles_pays(int M, int N, int K, int mode);
+int ic_gemm_tiles(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, int mode, hipStream_t stream);
+// C[M, N] = alpha * A[M, K] W[N, K]^T for many rows by the faster of ic_gemm_tiles and ic_matmul; arguments and results as ic_matmul.
+int ic_product(const void* A, int a_dtype, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldw, int ldc, float alpha, void* workspace, long long workspace_bytes, hipStream_t stream);
+
 // ---- matmul_library.hip ------------------------------------------------------------------------------
 // The library (hipBLASLt) matrix product for many rows: C[M, N] = alpha * A[M, K] W[N, K]^T, bfloat16 operands with a
 // bfloat16 or float32 result, or all float32 (true float32).  Descriptors and the algorithm are kept per shape.

@@ -185,6 +185,12 @@ _SIGNATURES = {
     "ic_gemm_rows_plan": [_I, _I, _I, _I, _I, _I, _c.POINTER(_I)],
     "ic_gemm_nt_cfg": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I, _I, _I, _P],
     "ic_attn_decode_splits": [_I, _I, _I, _I, _I, _I, _I, _I, _I],
+    "ic_gemm_tiles_supported": [_I, _I, _I, _I, _I, _I, _I],
+    "ic_gemm_tiles_pays": [_I, _I, _I, _I],
+    "ic_gemm_tiles_plan": [_I, _I, _I, _I],
+    "ic_gemm_tiles": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
+    "ic_gemm_tiles_cfg": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P],
+    "ic_product": [_P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _P, _LL, _P],
     "ic_gemm_splitk_supported": [_I, _I, _I, _I, _I],
     "ic_gemm_splitk_slices": [_I, _I],
     "ic_gemm_splitk": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
@@ -195,6 +201,7 @@ _SIGNATURES = {
     "ic_rule_own_product": [_I, _I, _I, _I],
     "ic_rule_qkv_fused": [_I, _I, _I, _I, _I, _I, _I, _I, _I],
     "ic_rule_gate_up_fused": [_I, _I, _I, _I, _I, _I],
+    "ic_rule_gate_up_tiles": [_I, _P, _P, _P, _I, _I, _I, _I, _I, _I],
     "ic_rule_tail": [_I, _I, _I, _I, _I, _I],
     "ic_rule_attention": [_I, _I, _I, _I, _I],
     "ic_rule_context_bucket": [_I],

@@ -401,6 +401,14 @@ def rule_gate_up_fused(dtype, rows: int, a, w, row_factors_owed: bool) -> bool:
                                                                      int(w.stride(0)), int(bool(row_factors_owed))))
 
 
+def rule_gate_up_tiles(a, w, out) -> bool:
+    """True when the gate/up projection of the many rows a with w runs with SwiGLU in its epilogue, in tiles (gemm_tiles)."""
+    code = _code_or_none(a.dtype)
+    return code is not None and a.dtype == w.dtype == out.dtype and a.stride(1) == w.stride(1) == out.stride(1) == 1 and \
+        bool(get_lib().ic_rule_gate_up_tiles(code, a.data_ptr(), w.data_ptr(), out.data_ptr(), a.shape[0], w.shape[0], a.shape[1],
+                                             a.stride(0), w.stride(0), out.stride(0)))
+
+
 def rule_tail(dtype, a, w) -> int:
     """How the projection a w^T into the residual stream, followed by a norm, runs: TAIL_PLAIN, TAIL_SPLIT_NORM or TAIL_SLICES."""
     code = _code_or_none(dtype)
@@ -562,21 +570,62 @@ def _matmul_args(a, w, out, what):
 def matmul_library(a, w, out, alpha: float = 1.0):
     """out[M, N] = alpha * a[M, K] @ w[N, K]^T through the library (hipBLASLt), any number of rows.
     bfloat16 operands with a bfloat16 or float32 result, or all float32."""
-    M, N, K, ca, cc, sa, sw, so = _matmul_args(a, w, out, "matmul_library")
+    return _matmul(get_lib().ic_matmul, a, w, out, alpha, "matmul_library")
+
+
+def product(a, w, out, alpha: float = 1.0):
+    """matmul_library, or the package's own product in tiles (gemm_tiles) where that is the faster one."""
+    return _matmul(get_lib().ic_product, a, w, out, alpha, "product")
+
+
+def _matmul(entry, a, w, out, alpha, what):
+    M, N, K, ca, cc, sa, sw, so = _matmul_args(a, w, out, what)
     stream = _stream()
     ws = _matmul_workspace.get((a.device, stream))
     if ws is None:
         ws = _workspace(a.device)
-    st = get_lib().ic_matmul(a.data_ptr(), ca, w.data_ptr(), out.data_ptr(), cc, M, N, K, sa, sw, so, alpha,
-                        ws.data_ptr(), MATMUL_WORKSPACE_BYTES, stream)
+    st = entry(a.data_ptr(), ca, w.data_ptr(), out.data_ptr(), cc, M, N, K, sa, sw, so, alpha,
+               ws.data_ptr(), MATMUL_WORKSPACE_BYTES, stream)
     if st == 0:
         return out
     if st == -4:
-        raise NoLibraryAlgorithm("matmul_library: no algorithm for %d x %d x %d" % (M, N, K))
+        raise NoLibraryAlgorithm("%s: no algorithm for %d x %d x %d" % (what, M, N, K))
     if st == -3:
-        raise KernelError("matmul_library: the library refused the product %d x %d x %d" % (M, N, K))
-    check(st, "matmul_library")
+        raise KernelError("%s: the library refused the product %d x %d x %d" % (what, M, N, K))
+    check(st, what)
     return out
+
+
+def _gemm_tiles_args(a, w, out, swiglu_output):
+    _dev(a, w, out)
+    M, K = a.shape
+    N = w.shape[0]
+    _need(w.shape[1] == K and tuple(out.shape) == (M, N // 2 if swiglu_output else N), "gemm_tiles: shape mismatch")
+    _need(a.stride(1) == 1 and w.stride(1) == 1 and out.stride(1) == 1, "gemm_tiles: inner strides must be 1")
+    _need(a.dtype == w.dtype == out.dtype == torch.bfloat16, "gemm_tiles: bfloat16 only")
+    return [a.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K, a.stride(0), w.stride(0), out.stride(0), int(swiglu_output)]
+
+
+def gemm_tiles(a, w, out, swiglu_output: bool = False, tile=None):
+    """out[M, N] = a[M, K] @ w[N, K]^T for many rows, bfloat16, float32 accumulation; swiglu_output: w = [gate rows; up rows] and
+    out[M, N/2] = up * silu(gate) of the products before any rounding.  K a multiple of 64; row strides and out's columns multiples of 8;
+    16-byte aligned.  tile (tests): the number of the tile, otherwise chosen from M, N and K."""
+    args = _gemm_tiles_args(a, w, out, swiglu_output)
+    if tile is None:
+        check(get_lib().ic_gemm_tiles(*args, _stream()), "gemm_tiles")
+    else:
+        check(get_lib().ic_gemm_tiles_cfg(*args, int(tile), _stream()), "gemm_tiles")
+    return out
+
+
+def gemm_tiles_plan(m: int, n: int, k: int, swiglu_output: bool = False) -> int:
+    """The number of the tile that gemm_tiles chooses."""
+    return int(get_lib().ic_gemm_tiles_plan(int(m), int(n), int(k), int(swiglu_output)))
+
+
+def gemm_tiles_pays(m: int, n: int, k: int, swiglu_output: bool = False) -> bool:
+    """True when gemm_tiles beats the library's product (with swiglu_output: that and the activation kernel)."""
+    return bool(get_lib().ic_gemm_tiles_pays(int(m), int(n), int(k), int(swiglu_output)))
 
 
 def matmul_library_tune(a, w, out, reps: int = 5, flush=None) -> int:

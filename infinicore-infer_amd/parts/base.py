@@ -25,7 +25,7 @@ class Runtime:
     dtype: torch.dtype                 # compute dtype of activations and cache: bfloat16 or float32
     device: object                     # torch device of weights and buffers
     attention_impl: str = "auto"       # "auto": tiled kernels where they apply; "generic": the general kernel only
-    gemm_impl: str = "auto"            # "auto": own kernel for few rows; "library": always the library GEMM
+    gemm_impl: str = "auto"            # "auto": own kernels where they are faster; "library": always the library GEMM
 
 
 @dataclass(frozen=True)

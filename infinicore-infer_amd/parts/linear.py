@@ -1,9 +1,10 @@
 """y = x W^T for weights stored [out, in] (the checkpoint's layout; the
 reference views them transposed, src/models/jiuge/jiuge_weight.hpp:51-54).
 
-The matrix product itself is a library routine for many rows, as in the
-reference (inference_context.cpp:59-79 calls the library's Gemm), and the
-package's own matrix-core kernel for few rows (decoding, the output head).
+The matrix product itself is the package's own matrix-core kernel for few rows
+(decoding, the output head) and for most many-row products, and a library
+routine for the rest (the reference calls the library's Gemm for every product,
+inference_context.cpp:59-79).
 float32 operands always go to the library with reduced-precision matrix modes
 switched off.
 """
@@ -28,10 +29,9 @@ TUNE_MIN_SIDE = 256
 _tuned = set()
 
 
-def _library(x, w, out, alpha: float = 1.0):
-    """out = alpha * x w^T through the library, as the reference does for every product
-    (inference_context.cpp:59-79): hipBLASLt called directly, torch's routine if it has no
-    algorithm for the shape."""
+def _library(x, w, out, alpha: float = 1.0, impl: str = "auto"):
+    """out = alpha * x w^T of many rows: the product in tiles where the kernel library finds it the faster one (impl "auto"),
+    otherwise hipBLASLt called directly; torch's routine if that has no algorithm for the shape."""
     if TUNE_LIBRARY and min(w.shape[0], w.shape[1]) >= TUNE_MIN_SIDE:
         key = (x.dtype, out.dtype, x.shape[0], w.shape[0], w.shape[1], x.stride(0), w.stride(0), out.stride(0))
         if key not in _tuned:
@@ -41,7 +41,7 @@ def _library(x, w, out, alpha: float = 1.0):
             except ops.KernelError:
                 pass
     try:
-        return ops.matmul_library(x, w, out, alpha)
+        return (ops.product if impl == "auto" else ops.matmul_library)(x, w, out, alpha)
     except ops.NoLibraryAlgorithm:
         if out.dtype == x.dtype:
             torch.mm(x, w.t(), out=out)
@@ -73,14 +73,14 @@ def linear(x, w, out, impl: str = "auto", alpha: float = 1.0, ws=None):
         x32 = x if x.dtype == torch.float32 else scratch("linear_x32", tuple(x.shape)).copy_(x)
         w32 = w if w.dtype == torch.float32 else w.to(torch.float32)
         if out.dtype == torch.float32:
-            return _library(x32, w32, out, alpha)
+            return _library(x32, w32, out, alpha, impl)
         tmp = scratch("linear_out32", tuple(out.shape))
-        _library(x32, w32, tmp, alpha)
+        _library(x32, w32, tmp, alpha, impl)
         out.copy_(tmp)
         return out
     if own_kernel_applies(x.shape[0], x.dtype, w.dtype, out.dtype, impl):
         return ops.gemm_nt(x, w, out, alpha=alpha)
-    return _library(x, w, out, alpha)
+    return _library(x, w, out, alpha, impl)
 
 
 def linear_tail(x, w, tail, ws, name: str, impl: str = "auto"):

@@ -82,6 +82,8 @@ class SwiGLU(FeedForward):
                 ops.gemm_nt(h.values, self.w_gate_up, act, swiglu_output=True, row_factor=h.row_factor(), glu_clamped=unit)
             else:
                 ops.gemm_nt(h, self.w_gate_up, act, swiglu_output=True, glu_clamped=unit)
+        elif rt.gemm_impl == "auto" and self.variant == "silu" and not owed and ops.rule_gate_up_tiles(rows, self.w_gate_up, act):
+            ops.gemm_tiles(rows, self.w_gate_up, act, swiglu_output=True)      # many rows: likewise, in tiles
         else:
             gate_up = ctx.ws.buffer("gate_up", (T, 2 * self.intermediate_size), rt.dtype)
             linear(h, self.w_gate_up, gate_up, rt.gemm_impl, ws=ctx.ws)

@@ -1,0 +1,120 @@
+"""The product of many rows in tiles: every tile at its edges, plain and with SwiGLU, and the choice between it and the library."""
+import pytest
+import torch
+
+from infinicore_infer_amd.kernels import ops
+
+BF16 = torch.bfloat16
+TILES = ((64, 64), (64, 128), (96, 128), (128, 128), (192, 128), (128, 192), (160, 192), (256, 128), (128, 256), (160, 256), (256, 192), (256, 256))
+
+
+def _operands(M, N, K, seed, pad=0):
+    g = torch.Generator().manual_seed(seed)
+    a = torch.randn(M, K + pad, generator=g).to(BF16)[:, :K]
+    w = (torch.randn(N, K + pad, generator=g) * K ** -0.5).to(BF16)[:, :K]
+    return a, w
+
+
+def _strided(t, pad):
+    d = torch.empty(t.shape[0], t.shape[1] + pad, dtype=t.dtype, device="cuda")[:, :t.shape[1]]
+    return d.copy_(t)
+
+
+def _check(a, w, got, swiglu):
+    """Element by element: the result's rounding to bfloat16 (2^-8 of it) and float32 sums of K products in any order (each partial sum
+    rounds by 2^-24 of at most the sum of the products' magnitudes; K of them, of which the roundings of random sign leave far less than 2^-6)."""
+    a, w = a.double(), w.double()
+    ref, mag = a @ w.t(), (a.abs() @ w.abs().t()) * a.shape[1] * 2.0 ** -24
+    if swiglu:
+        n = ref.shape[1] // 2
+        g, u, mg, mu = ref[:, :n], ref[:, n:], mag[:, :n], mag[:, n:]
+        s = torch.nn.functional.silu(g)
+        # |silu'| <= 1.1; exp2 and reciprocal of the hardware: an ulp each
+        ref, mag = u * s, 1.1 * mg * (u.abs() + mu) + mu * s.abs() + 2.0 ** -21 * (u * s).abs()
+    assert torch.isfinite(got).all()
+    err = (got.double().cpu() - ref).abs() - ref.abs() * 2.0 ** -8 - mag
+    assert err.max() <= 0, "off by %.3g beyond the bound" % err.max()
+
+
+def test_tile_rule_cpu():
+    """Every choice names a tile; what the kernel cannot take is refused; up to 32 rows other kernels run."""
+    from infinicore_infer_amd.kernels.lib import get_lib
+    lib = get_lib()
+    for m in (1, 33, 64, 65, 871, 4096, 100000):
+        for n in (8, 64, 2304, 32768):
+            for k in (64, 1536, 16384):
+                for mode in (0, 1):
+                    assert 0 <= lib.ic_gemm_tiles_plan(m, n, k, mode) < len(TILES)
+                    assert not (m <= 32 and lib.ic_gemm_tiles_pays(m, n, k, mode))
+    sup = lib.ic_gemm_tiles_supported
+    assert sup(100, 64, 128, 128, 128, 64, 0) and sup(100, 64, 128, 136, 144, 72, 0) and sup(100, 64, 128, 128, 128, 32, 1)
+    assert not sup(100, 64, 96, 96, 96, 64, 0)               # K in whole stages
+    assert not sup(100, 68, 128, 128, 128, 72, 0)            # columns in 16-byte pieces
+    assert not sup(100, 64, 128, 132, 128, 64, 0) and not sup(100, 64, 128, 128, 132, 64, 0) and not sup(100, 64, 128, 128, 128, 68, 0)
+    assert not sup(100, 72, 128, 128, 128, 40, 1)            # gate and up in 16-byte pieces each
+    assert not sup(100, 64, 128, 120, 128, 64, 0) and not sup(100, 64, 128, 128, 128, 56, 0) and not sup(0, 64, 128, 128, 128, 64, 0)
+    assert not sup(100, 1 << 16, 1 << 15, 1 << 15, 1 << 15, 1 << 15, 1)     # gate and up rows more than 32 bits of bytes apart
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", range(len(TILES)))
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_tiles_at_their_edges(tile, swiglu):
+    bm, bn = TILES[tile]
+    # one row; one tile exactly and one row and column piece more and less; several tiles; one stage of K, fewer and more stages than are loaded ahead
+    for M, N, K, pad in ((1, 16, 64, 0), (bm, bn, 128, 0), (bm + 1, bn + 16, 192, 8), (bm - 1, 2 * bn - 16, 320, 0), (2 * bm + 3, 3 * bn + 48, 448, 64)):
+        a, w = _operands(M, N, K, 7 * tile + M)
+        cols = N // 2 if swiglu else N
+        out = torch.full((M + 1, cols + pad), 3.0, dtype=BF16, device="cuda")
+        ops.gemm_tiles(_strided(a, pad), _strided(w, pad), out[:M, :cols], swiglu_output=swiglu, tile=tile)
+        _check(a, w, out[:M, :cols], swiglu)
+        assert (out[M] == 3.0).all() and (out[:, cols:] == 3.0).all()       # nothing beside the result is written
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(33, 7680, 1536), (65, 512, 512), (129, 1536, 3840), (871, 2560, 1536), (1045, 1536, 1536), (2049, 2304, 2304)])
+def test_chosen_tiles_and_their_replays(M, N, K):
+    """The tile that the rule names, recorded and replayed with other rows in between."""
+    a, w = _operands(M, N, K, M)
+    ad, wd, out = a.cuda(), w.cuda(), torch.empty(M, N, dtype=BF16, device="cuda")
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        ops.product(ad, wd, out)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            ops.gemm_tiles(ad, wd, out)
+    torch.cuda.current_stream().wait_stream(side)
+    for _ in range(3):
+        a = a.roll(1, 0)
+        ad.copy_(a)
+        graph.replay()
+        torch.cuda.synchronize()
+        _check(a, w, out, False)
+
+
+@pytest.mark.gpu
+def test_infinities_and_nan_stay_where_they_are():
+    a, w = _operands(200, 256, 256, 1)
+    a[3, 5], a[70, 255], a[199, 0] = float("inf"), float("nan"), -float("inf")
+    for tile in range(len(TILES)):
+        out = torch.empty(200, 256, dtype=BF16, device="cuda")
+        ops.gemm_tiles(a.cuda(), w.cuda(), out, tile=tile)
+        bad = ~torch.isfinite(out).all(1).cpu()
+        assert bad.nonzero().view(-1).tolist() == [3, 70, 199]
+        keep = ~bad
+        _check(a[keep], w, out.cpu()[keep], False)
+
+
+@pytest.mark.gpu
+def test_refused_operands_go_to_the_library():
+    """What the tiles do not take is an error there and the library's in ops.product."""
+    for M, N, K, at in ((100, 200, 96, 0), (100, 250, 128, 0), (100, 200, 128, 1)):
+        a, w = _operands(M, N, K, 3)
+        room = torch.empty(M * K + 8, dtype=BF16, device="cuda")
+        ad = room[at:at + M * K].view(M, K).copy_(a)            # at 1: not 16-byte aligned
+        out = torch.empty(M, N, dtype=BF16, device="cuda")
+        with pytest.raises(ops.KernelError):
+            ops.gemm_tiles(ad, w.cuda(), out)
+        ops.product(ad, w.cuda(), out)
+        _check(a, w, out, False)
