@@ -18,7 +18,7 @@
 // products: 256 x 256 0.96 us a stage (0.87 with products alone), 192 x 192 0.58 (0.49), 128 x 128 0.30 (0.23), and about 4 us for launch, first
 // loads and the way out.  128 x 128 tiles take all of a unit's 64 bytes a cycle from L2 for their loads, 256 x 256 half of it, hence the large
 // tiles where there are rows and columns enough.  The whole chip busy for long: its power, the clock gives way (256 x 256: 1.38..1.5 us a stage).
-// Waves of 64 x 64 results and more need four waves of up to 512 registers a block: eight waves of half the size read 1.5 times as much from LDS
+// Large tiles take four waves of up to 512 registers a block: eight waves of half the size read 1.5 times as much from LDS
 // (256 x 256: 1.07 us a stage).  v_mfma_f32_32x32x16_bf16 instead of 16x16x32 is no faster (0.96 and 0.97).
 //
 // 16x16x32 layout (lane l): A[i = l%16][k = 8(l/16)..+7], B[k = 8(l/16)..+7][j = l%16], D[i = 4(l/16) + e][j = l%16], e = 0..3;
@@ -60,10 +60,14 @@ template <typename F, int... Is> __device__ __forceinline__ void each_of(F&& f, 
 }
 template <int N, typename F> __device__ __forceinline__ void each(F&& f) { each_of(f, std::make_integer_sequence<int, N>{}); }
 
-// acc += w a, the accumulator in the registers' second half (an operand that is read and written by one instruction: where a wave holds more
-// than 128 of them the compiler's own product copies them from product to product)
-__device__ __forceinline__ void product(v4f& acc, const v8b& w, const v8b& a) {
-    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(w), "v"(a));
+// acc += w a.  OWN: with 256 accumulators a lane, all of the second half of its 512 registers, the compiler's own product copies them from product to
+// product (192 copies a stage); written as assembly, with an operand that is read and written, it does not.  The compiler does not know such a
+// product for one and adds no wait before an instruction that reads its result: LAST, on the last product of a stage, waits here (11 wait states
+// after eight passes), so that whatever follows the stage may read any accumulator.
+template <bool OWN, bool LAST> __device__ __forceinline__ void product(v4f& acc, const v8b& w, const v8b& a) {
+    if constexpr (!OWN) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, a, acc, 0, 0, 0);
+    else if constexpr (LAST) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\ts_nop 15" : "+a"(acc) : "v"(w), "v"(a));
+    else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(w), "v"(a));
 }
 
 template <int BM_, int BN_, int WM_, int WN_, int WK_, int STAGES_> struct Tile {
@@ -74,20 +78,20 @@ template <int BM_, int BN_, int WM_, int WN_, int WK_, int STAGES_> struct Tile 
     static constexpr int LOADS_A = BM / 8 / WAVES, LOADS = LOADS_A + BN / 8 / WAVES;    // of 1 KB, a wave and stage
     static constexpr int SUM_BYTES = BM * BN * 4 * (WK - 1);
     static constexpr int LDS_BYTES = STAGES * STAGE_BYTES > SUM_BYTES ? STAGES * STAGE_BYTES : SUM_BYTES;
-    static constexpr int REGISTERS = TM * TN / 64 + (MT + NT) * 8 + LOADS + 24;
-    static constexpr int BLOCKS_PER_CU = (LDS_BYTES <= 80 * 1024 && REGISTERS <= 256 && WAVES == 4) ? 2 : 1;
-    static constexpr int MIN_WAVES = WAVES * BLOCKS_PER_CU / 4;    // a SIMD's
+    static constexpr bool takes(int mode) { return mode == EPI_BF16 || NT % 2 == 0; }
+    static constexpr bool OWN_PRODUCT = TM * TN / 64 > 192;        // accumulators a lane
+    static constexpr int BLOCKS_PER_CU = LDS_BYTES <= 80 * 1024 ? 2 : 1;
     static_assert(BM % (16 * WM) == 0 && BN % (16 * WN) == 0, "whole matrix tiles");
     static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "every wave loads as much");
     static_assert(STEPS == 1 || STEPS == 2, "a stage is two k-steps");
-    static_assert(MT % WK == 0 && LDS_BYTES <= 160 * 1024 && LOADS * (STAGES - 1) < 64 && MIN_WAVES >= 1, "limits");
+    static_assert((WAVES == 4) && MT % WK == 0 && LDS_BYTES <= 160 * 1024 && LOADS * (STAGES - 1) < 64, "limits");
 };
 
 template <typename T, int EPI>
-__global__ void __launch_bounds__(T::WAVES * 64, T::MIN_WAVES) gemm_tiles_kernel(TilesArgs a) {
+__global__ void __launch_bounds__(T::WAVES * 64, T::BLOCKS_PER_CU) gemm_tiles_kernel(TilesArgs a) {
     constexpr int BM = T::BM, BN = T::BN, WN = T::WN, WK = T::WK, STAGES = T::STAGES, WAVES = T::WAVES;
     constexpr int TM = T::TM, TN = T::TN, MT = T::MT, NT = T::NT, STEPS = T::STEPS, LOADS = T::LOADS, LOADS_A = T::LOADS_A;
-    static_assert(EPI != EPI_SWIGLU || NT % 2 == 0, "a wave holds gate and up columns alike");
+    static_assert(T::takes(EPI), "a wave holds gate and up columns alike");
     __shared__ __attribute__((aligned(1024))) unsigned char lds[T::LDS_BYTES];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, kq = lane >> 4;
@@ -138,7 +142,7 @@ __global__ void __launch_bounds__(T::WAVES * 64, T::MIN_WAVES) gemm_tiles_kernel
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = v4f{0.f, 0.f, 0.f, 0.f};
-    asm volatile("s_nop 7");
+    if constexpr (T::OWN_PRODUCT) asm volatile("s_nop 7");         // (and none between these writes and the first products)
 
     // operand registers of two k-steps: one is multiplied while the other is read
     v8b fa[2][MT], fw[2][NT];
@@ -184,7 +188,7 @@ __global__ void __launch_bounds__(T::WAVES * 64, T::MIN_WAVES) gemm_tiles_kernel
             });
             each<F1 - F0>([&](auto k) { fetch(std::integral_constant<int, L0 + F0 + decltype(k)::value>{}, at_a, at_w, into); });
             if constexpr (R1 > R0 || F1 > F0) __builtin_amdgcn_sched_barrier(0);
-            product(acc[I / MT][I % MT], fw[CUR][I / MT], fa[CUR][I % MT]);
+            product<T::OWN_PRODUCT, I + 1 == P>(acc[I / MT][I % MT], fw[CUR][I / MT], fa[CUR][I % MT]);
         });
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -223,9 +227,6 @@ __global__ void __launch_bounds__(T::WAVES * 64, T::MIN_WAVES) gemm_tiles_kernel
         for (; s < n_stages; ++s) buf = whole_stage(s, buf, std::integral_constant<int, 0>{});
     }
     wait_loads<0>();
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_nop 15\n\ts_nop 15");                          // the last products are done before other instructions read their results
-    __builtin_amdgcn_sched_barrier(0);
     __syncthreads();                                               // LDS is free
 
     constexpr int SH = MT / WK;                                    // row tiles of C this wave writes: SH from the wk-th run on
@@ -301,35 +302,44 @@ template <typename T, int EPI> int launch(TilesArgs a, hipStream_t stream) {
     a.group_m = (a.tiles_m + groups - 1) / groups;
     const long long blocks = (long long)a.tiles_m * a.tiles_n;
     if (blocks > (1LL << 30)) return IC_ERR_ARG;
-    hipLaunchKernelGGL((gemm_tiles_kernel<T, EPI>), dim3((unsigned)blocks), dim3(T::WAVES * 64), 0, stream, a);
-    return ic_launch_status();
+    if constexpr (T::takes(EPI)) {
+        hipLaunchKernelGGL((gemm_tiles_kernel<T, EPI>), dim3((unsigned)blocks), dim3(T::WAVES * 64), 0, stream, a);
+        return ic_launch_status();
+    }
+    return IC_ERR_ARG;
 }
 
 // The tiles, smallest first, and what one costs in microseconds: FIXED + rounds * (ROUND + stages * STAGE * (1 + FULL * x)), where x is the part of
-// the 256 compute units that have a block and a round is one block a unit (two of 64 x 64, which then share it: 1.7 times the stage).  Fitted to 5,900
-// timed products (17 pairs of N in 512..32,768 and K in 512..16,384, 33..16,384 rows, weights out of memory); the tile with the least cost loses 1.1 % to
-// the best of 20 tiles on average and 7 % at the 95th percentile.  Of those 20 these 12 are kept: the others were never needed for more than 0.1 %.
+// the 256 compute units that have a block and a round is one block a unit (two of 64 x 32 and 64 x 64, which then share it: 1.7 times the stage).
+// Fitted to 6,900 timed products (17 pairs of N in 512..32,768 and K in 512..16,384, 33..16,384 rows, weights out of memory); the tile with the least
+// cost loses 0.7 % to the best one on average and 5 % at the 95th percentile.  64 x 32 is for few rows of narrow matrices, where only many small tiles
+// reach all units (64 x 6,912 x 2,304: 15.0 us with 64 x 64, 11.8), 64 x 96 and 128 x 64 likewise (200 x 4,608 x 4,096: 25.4 -> 21.3).  Tried and not
+// kept: 192 x 256, 96 x 192, 96 x 256, 64 x 192; two lines of 64 k a stage; more stages of the small tiles (no faster: what bounds them is the rate at
+// which one unit takes bytes).
 #define IC_TILES(X) \
     /* number, FIXED, STAGE, FULL, ROUND, tile: BM, BN, WM, WN, WK, STAGES */ \
-    X(0, 2.75, 0.191, 0.33, 0.00, 64, 64, 2, 1, 2, 4) \
-    X(1, 2.31, 0.306, 0.24, 0.79, 64, 128, 2, 2, 1, 6) \
-    X(2, 1.97, 0.325, 0.32, 1.54, 96, 128, 2, 2, 1, 5) \
-    X(3, 2.10, 0.377, 0.37, 1.72, 128, 128, 2, 2, 1, 5) \
-    X(4, 2.60, 0.463, 0.42, 1.36, 192, 128, 2, 2, 1, 3) \
-    X(5, 2.75, 0.514, 0.32, 1.19, 128, 192, 2, 2, 1, 4) \
-    X(6, 2.56, 0.571, 0.30, 1.81, 160, 192, 2, 2, 1, 3) \
-    X(7, 2.31, 0.570, 0.38, 2.54, 256, 128, 2, 2, 1, 3) \
-    X(8, 2.36, 0.653, 0.27, 1.85, 128, 256, 2, 2, 1, 3) \
-    X(9, 2.76, 0.700, 0.31, 2.54, 160, 256, 2, 2, 1, 3) \
-    X(10, 4.21, 0.952, 0.27, 0.00, 256, 192, 2, 2, 1, 2) \
-    X(11, 6.10, 1.077, 0.33, 0.00, 256, 256, 2, 2, 1, 2)
+    X(0, 2.76, 0.112, 0.65, 0.00, 64, 32, 2, 1, 2, 6) \
+    X(1, 2.60, 0.198, 0.29, 0.00, 64, 64, 2, 1, 2, 4) \
+    X(2, 2.07, 0.252, 0.20, 0.89, 64, 96, 2, 2, 1, 7) \
+    X(3, 2.67, 0.256, 0.41, 0.43, 128, 64, 2, 2, 1, 6) \
+    X(4, 2.51, 0.315, 0.21, 0.50, 64, 128, 2, 2, 1, 6) \
+    X(5, 2.35, 0.332, 0.29, 1.04, 96, 128, 2, 2, 1, 5) \
+    X(6, 2.69, 0.385, 0.34, 0.98, 128, 128, 2, 2, 1, 5) \
+    X(7, 3.04, 0.467, 0.39, 0.89, 192, 128, 2, 2, 1, 3) \
+    X(8, 3.43, 0.525, 0.28, 0.47, 128, 192, 2, 2, 1, 4) \
+    X(9, 3.41, 0.574, 0.28, 0.96, 160, 192, 2, 2, 1, 3) \
+    X(10, 2.90, 0.575, 0.35, 1.89, 256, 128, 2, 2, 1, 3) \
+    X(11, 3.39, 0.662, 0.25, 0.83, 128, 256, 2, 2, 1, 3) \
+    X(12, 3.69, 0.708, 0.29, 1.53, 160, 256, 2, 2, 1, 3) \
+    X(13, 4.33, 0.956, 0.24, 0.00, 256, 192, 2, 2, 1, 2) \
+    X(14, 6.27, 1.084, 0.30, 0.00, 256, 256, 2, 2, 1, 2)
 
-constexpr int kTiles = 12;
+constexpr int kTiles = 15;
 constexpr double kUnits = 256.0;
 
-struct TileCost { int bm, bn, blocks_per_unit; double fixed, stage, full, round; };
+struct TileCost { int bm, bn, blocks_per_unit; bool pairs; double fixed, stage, full, round; };
 constexpr TileCost kCosts[kTiles] = {
-#define X(I, FIXED, STAGE, FULL, ROUND, ...) {Tile<__VA_ARGS__>::BM, Tile<__VA_ARGS__>::BN, Tile<__VA_ARGS__>::BLOCKS_PER_CU, FIXED, STAGE, FULL, ROUND},
+#define X(I, FIXED, STAGE, FULL, ROUND, ...) {Tile<__VA_ARGS__>::BM, Tile<__VA_ARGS__>::BN, Tile<__VA_ARGS__>::BLOCKS_PER_CU, Tile<__VA_ARGS__>::takes(EPI_SWIGLU), FIXED, STAGE, FULL, ROUND},
     IC_TILES(X)
 #undef X
 };
@@ -343,14 +353,16 @@ double cost_of(const TileCost& t, int M, int N, int K, int mode) {
         if (t.blocks_per_unit > 1) shared = 1.7;
     }
     const double walk = t.fixed + rounds * (t.round + stages * t.stage * (1.0 + t.full * busy) * shared);
-    // the weights come from memory once, and about half of them again for every further row tile (blocks of one column of tiles seldom run abreast)
-    const double read = 3.0 + 2.0 * N * K * (1.0 + 0.5 * (tm < 4 ? tm - 1 : 3)) / 7e6;
+    // the weights come from memory once, and about half of them again for every further row tile (blocks of one column of tiles seldom run abreast);
+    // narrow tiles of pairs read them in pieces of 32 rows and less, which memory serves more slowly (64 x 32,768 x 4,096: 83 us against 63)
+    const double read = 3.0 + 2.0 * N * K * (1.0 + 0.5 * (tm < 4 ? tm - 1 : 3)) * (mode != EPI_BF16 && t.bn <= 64 ? 1.35 : 1.0) / 7e6;
     return walk > read ? walk : read;
 }
 
 int best_tile(int M, int N, int K, int mode, double* cost) {
     int best = 0;
     for (int i = 0; i < kTiles; ++i) {
+        if (mode != EPI_BF16 && !kCosts[i].pairs) continue;
         const double c = cost_of(kCosts[i], M, N, K, mode);
         if (i == 0 || c < *cost) { *cost = c; best = i; }
     }
@@ -388,24 +400,24 @@ IC_EXPORT int ic_gemm_tiles_supported(int M, int N, int K, int lda, int ldw, int
     return (mode == EPI_BF16 || mode == EPI_SWIGLU) && takes(M, N, K, lda, ldw, ldc, mode);
 }
 
-// Whether the library would be faster.  Two kinds of product where it is, fitted to the same sweep (own against library, the choice loses 2.2 % to the
-// faster of the two on average; the own kernel everywhere: 6.3 %):
+// Whether the library would be faster.  Two kinds of product where it is, fitted to the same sweep (own against library, the choice loses 1.0 % to the
+// faster of the two on average; the own kernel everywhere: 2.1 %, the library everywhere: 16 %):
 //   full rounds of 256 x 256 tiles, where nothing is left to choose and its kernel spends less on a stage (8,192 x 4,096 x 14,336: 601 us against 691;
 //   4,096 x 4,096 x 4,096: 90 against 93);
-//   long rows and few tiles, which it splits over K (256 x 1,024 x 8,192: 20 us against 32): the own kernel's walk over K is compared with what a
+//   long rows and few tiles, which it splits over K (256 x 1,024 x 8,192: 20 us against 25): the own kernel's walk over K is compared with what a
 //   product split over the whole chip takes.
 // Elsewhere the own kernel is faster (1,045 x 2,560 x 1,536: 17.0 -> 12.2 us; 871 x 1,536 x 1,536: 12.5 -> 10.0; 2,048 x 2,304 x 2,304: 28 -> 22.6).
-// With the gated unit in the epilogue it is compared with the library's product and the unit's own kernel, and is always faster from 33 rows on
+// With the gated unit in the epilogue it is compared with the library's product and the unit's own kernel, and is faster from 33 rows on
 // (1,045 x 7,680 x 1,536: 42.0 -> 28.0; 2,048 x 11,520 x 2,304: 131 -> 97; 16,384 x 32,768 x 4,096: 3,135 -> 2,942).
 IC_EXPORT int ic_gemm_tiles_pays(int M, int N, int K, int mode) {
     if (M <= 32) return 0;
     const double t = (double)((M + 255) / 256) * ((N + 255) / 256), fill = t / (kUnits * __builtin_ceil(t / kUnits));
     if (mode == EPI_SWIGLU) return K <= 8192 || fill < 0.93;
-    if (t >= 200.0 && fill >= 0.93) return 0;
+    if (t >= 200.0 && fill >= 0.97) return 0;
     double cost = 0.0;
     best_tile(M, N, K, mode, &cost);
-    const double products = 2.0 * M * N * K / 0.6e9, read = 2.0 * N * K / 5e6;
-    return cost <= 1.4 * (6.0 + (products > read ? products : read));
+    const double products = 2.0 * M * N * K / 0.6e9, read = 2.0 * N * K / 4e6;
+    return cost <= 1.6 * (6.0 + (products > read ? products : read));
 }
 
 IC_EXPORT int ic_gemm_tiles_plan(int M, int N, int K, int mode) {

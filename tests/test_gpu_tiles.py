@@ -5,7 +5,8 @@ import torch
 from infinicore_infer_amd.kernels import ops
 
 BF16 = torch.bfloat16
-TILES = ((64, 64), (64, 128), (96, 128), (128, 128), (192, 128), (128, 192), (160, 192), (256, 128), (128, 256), (160, 256), (256, 192), (256, 256))
+TILES = ((64, 32), (64, 64), (64, 96), (128, 64), (64, 128), (96, 128), (128, 128), (192, 128), (128, 192), (160, 192), (256, 128), (128, 256), (160, 256),
+         (256, 192), (256, 256))
 
 
 def _operands(M, N, K, seed, pad=0):
@@ -61,6 +62,8 @@ def test_tile_rule_cpu():
 @pytest.mark.parametrize("swiglu", [False, True])
 def test_tiles_at_their_edges(tile, swiglu):
     bm, bn = TILES[tile]
+    if swiglu and bn == 96:
+        pytest.skip("three column tiles a wave: no pairs of gate and up")
     # one row; one tile exactly and one row and column piece more and less; several tiles; one stage of K, fewer and more stages than are loaded ahead
     for M, N, K, pad in ((1, 16, 64, 0), (bm, bn, 128, 0), (bm + 1, bn + 16, 192, 8), (bm - 1, 2 * bn - 16, 320, 0), (2 * bm + 3, 3 * bn + 48, 448, 64)):
         a, w = _operands(M, N, K, 7 * tile + M)
