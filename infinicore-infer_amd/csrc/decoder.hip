@@ -4,8 +4,8 @@
 // What runs for a layer depends on the step alone, never on the model: up to 16 rows in bfloat16 take the
 // few-row products with their epilogues (rotary and cache write after QKV; residual add, the next norm's
 // weight and sums of squares after O and down; SwiGLU after gate/up), the norm between two products being
-// split over them; more rows take the products in tiles (gate/up with SwiGLU in its epilogue) or the library's, as
-// ic_product chooses, float32 the library's, and the norm, rotary and activation kernels.  Single-token rows go to the split-key attention kernel, prompt portions to the tiled one, what
+// split over them; more rows take the products in tiles (QKV with rotary and cache write, gate/up with SwiGLU in
+// the epilogue) or the library's, as ic_product chooses, float32 the library's, and the norm, rotary and activation kernels.  Single-token rows go to the split-key attention kernel, prompt portions to the tiled one, what
 // neither takes to the general one.
 #include "common.h"
 #include "infinicore_infer_engine.h"
@@ -58,6 +58,14 @@ IC_EXPORT int ic_rule_qkv_fused(int dtype, int rows, int K, int lda, int ldw, in
     if (dtype != IC_BF16 || kv_heads_written <= 0 || rot_dim != head_dim || !ic_gemm_qkv_rope_supported(IC_BF16, head_dim)) return 0;
     if (rows <= kFewRows) return 1;
     return !row_factors_owed && rows <= ic_gemm_nt_epilogue_rows(2, K, lda, ldw);
+}
+
+IC_EXPORT int ic_rule_qkv_tiles(int dtype, const void* A, const void* W, const void* C, int rows, int K, int lda, int ldw, int ldc, const float* cos_t,
+                                const float* sin_t, const void* kcache, const void* vcache, int nh, int kv_heads_written, int head_dim, int rot_dim,
+                                int page_size) {
+    return dtype == IC_BF16 && kv_heads_written > 0 && rot_dim == head_dim &&
+           ic_gemm_tiles_rope_supported(A, W, C, rows, K, lda, ldw, ldc, cos_t, sin_t, kcache, vcache, nh, kv_heads_written, head_dim, page_size) &&
+           ic_gemm_tiles_pays(rows, (nh + 2 * kv_heads_written) * head_dim, K, 2);
 }
 
 IC_EXPORT int ic_rule_gate_up_fused(int dtype, int rows, int K, int lda, int ldw, int row_factors_owed) {
@@ -271,6 +279,11 @@ struct IcDecoder {
                 st = ic_gemm_qkv_rope(h, A.w_qkv, qkv, T, d, d, d, width, b.positions, slots, A.cos, A.sin, e.k_cache, e.v_cache,
                                       A.n_heads, nkv, A.head_dim, ps, h_def ? &rf : nullptr, stream);
                 if (st) return fail(st, "the QKV product with rotary and cache write", i);
+            } else if (!h_def && ic_rule_qkv_tiles(dt, h, A.w_qkv, qkv, T, d, d, d, width, A.cos, A.sin, e.k_cache, e.v_cache, A.n_heads, nkv,
+                                                   A.head_dim, A.rot_dim, ps)) {
+                st = ic_gemm_tiles_rope(h, A.w_qkv, qkv, T, d, d, d, width, b.positions, slots, A.cos, A.sin, e.k_cache, e.v_cache, A.n_heads, nkv,
+                                        A.head_dim, ps, stream);
+                if (st) return fail(st, "the QKV product with rotary and cache write, in tiles", i);
             } else {
                 st = linear(h, d, A.w_qkv, qkv, dt, T, width, d, 1.0f, h_def, lib_ws, lib_ws_bytes, stream);
                 if (st) return fail(st, "the QKV product", i);

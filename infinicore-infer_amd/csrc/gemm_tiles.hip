@@ -40,9 +40,19 @@ struct TilesArgs {
     int M, N, K, lda, ldw, ldc;   // N: rows of W
     int tiles_m, tiles_n;         // the grid: tiles_m * tiles_n blocks
     int group_m;                  // row tiles that are walked together
+    // EPI_ROPE: W = [q heads; k heads; v heads], rows of 2 half = 2 << half_log
+    const int* positions;
+    const int* slots;
+    const float* cos_t;           // [positions, half]
+    const float* sin_t;
+    uint16_t* kcache;             // [pages, kv heads, page size, 2 half]
+    uint16_t* vcache;
+    int nh, nkvh, half_log, page_size;
 };
 
-enum { EPI_BF16 = 0, EPI_SWIGLU = 1 };
+// What follows the product.  SWIGLU and ROPE are about pairs of columns (gate and up of one column; a head's entries j and j + half): C counts in
+// pairs, and a wave's TN weight rows are the first members of TN / 2 neighbouring pairs, then their second ones, so that a lane has both.
+enum { EPI_BF16 = 0, EPI_SWIGLU = 1, EPI_ROPE = 2 };
 
 // 16 bytes a lane from base + off (bytes; base the same for the wave) to LDS at lds + plus + 16 * lane.
 template <int PLUS> __device__ __forceinline__ void load_to_lds(unsigned lds, unsigned off, const char* base) {
@@ -61,9 +71,10 @@ template <typename F, int... Is> __device__ __forceinline__ void each_of(F&& f, 
 template <int N, typename F> __device__ __forceinline__ void each(F&& f) { each_of(f, std::make_integer_sequence<int, N>{}); }
 
 // acc += w a.  OWN: with 256 accumulators a lane, all of the second half of its 512 registers, the compiler's own product copies them from product to
-// product (192 copies a stage); written as assembly, with an operand that is read and written, it does not.  The compiler does not know such a
-// product for one and adds no wait before an instruction that reads its result: LAST, on the last product of a stage, waits here (11 wait states
-// after eight passes), so that whatever follows the stage may read any accumulator.
+// product (192 copies a stage; with ROPE's way out, which needs more registers, in all tiles of 32 accumulators and more); written as assembly, with
+// an operand that is read and written, it does not.  The compiler does not know such a product for one and adds no wait before an instruction that
+// reads its result: LAST, on the last product of a stage, waits here (11 wait states after eight passes), so that whatever follows the stage may read
+// any accumulator.
 template <bool OWN, bool LAST> __device__ __forceinline__ void product(v4f& acc, const v8b& w, const v8b& a) {
     if constexpr (!OWN) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, a, acc, 0, 0, 0);
     else if constexpr (LAST) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\ts_nop 15" : "+a"(acc) : "v"(w), "v"(a));
@@ -78,8 +89,9 @@ template <int BM_, int BN_, int WM_, int WN_, int WK_, int STAGES_> struct Tile 
     static constexpr int LOADS_A = BM / 8 / WAVES, LOADS = LOADS_A + BN / 8 / WAVES;    // of 1 KB, a wave and stage
     static constexpr int SUM_BYTES = BM * BN * 4 * (WK - 1);
     static constexpr int LDS_BYTES = STAGES * STAGE_BYTES > SUM_BYTES ? STAGES * STAGE_BYTES : SUM_BYTES;
-    static constexpr bool takes(int mode) { return mode == EPI_BF16 || NT % 2 == 0; }
-    static constexpr bool OWN_PRODUCT = TM * TN / 64 > 192;        // accumulators a lane
+    // (with ROPE 256 accumulators a lane leave too few registers for the way out: 2,048 x 6,912 x 2,304 71 us, product and rotary's own kernel 67)
+    static constexpr bool takes(int epi) { return epi == EPI_BF16 || (NT % 2 == 0 && !(epi == EPI_ROPE && TM * TN / 64 > 192)); }
+    static constexpr bool own_product(int epi) { return TM * TN / 64 > 192 || (epi == EPI_ROPE && STEPS > 1); }
     static constexpr int BLOCKS_PER_CU = LDS_BYTES <= 80 * 1024 ? 2 : 1;
     static_assert(BM % (16 * WM) == 0 && BN % (16 * WN) == 0, "whole matrix tiles");
     static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "every wave loads as much");
@@ -91,7 +103,7 @@ template <typename T, int EPI>
 __global__ void __launch_bounds__(T::WAVES * 64, T::BLOCKS_PER_CU) gemm_tiles_kernel(TilesArgs a) {
     constexpr int BM = T::BM, BN = T::BN, WN = T::WN, WK = T::WK, STAGES = T::STAGES, WAVES = T::WAVES;
     constexpr int TM = T::TM, TN = T::TN, MT = T::MT, NT = T::NT, STEPS = T::STEPS, LOADS = T::LOADS, LOADS_A = T::LOADS_A;
-    static_assert(T::takes(EPI), "a wave holds gate and up columns alike");
+    static_assert(T::takes(EPI), "a wave holds both of a pair");
     __shared__ __attribute__((aligned(1024))) unsigned char lds[T::LDS_BYTES];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, kq = lane >> 4;
@@ -106,15 +118,16 @@ __global__ void __launch_bounds__(T::WAVES * 64, T::BLOCKS_PER_CU) gemm_tiles_ke
     const int gm = min(a.group_m, a.tiles_m - first_m), in_group = t - group * a.group_m * a.tiles_n;
     const int bn = in_group / gm, bm = first_m + in_group - bn * gm;
     const int m0 = bm * BM;
-    const int NO = EPI == EPI_SWIGLU ? a.N / 2 : a.N;              // columns of C
-    constexpr int BNO = EPI == EPI_SWIGLU ? BN / 2 : BN;
+    constexpr bool PAIRS = EPI != EPI_BF16;
+    const int NO = PAIRS ? a.N / 2 : a.N;                          // columns of C, or pairs
+    constexpr int BNO = PAIRS ? BN / 2 : BN;
     const int n0 = bn * BNO;
 
     const int n_stages = a.K / 64;
 
     // What this lane fetches: byte offsets from the tile's first row of A, or from W (rows beyond the matrix repeat the last one)
     const char* base_a = (const char*)(a.A + (size_t)m0 * a.lda);
-    const char* base_w = (const char*)(a.W + (EPI == EPI_SWIGLU ? (size_t)0 : (size_t)n0 * a.ldw));
+    const char* base_w = (const char*)(a.W + (PAIRS ? (size_t)0 : (size_t)n0 * a.ldw));
     unsigned off[LOADS];
     each<LOADS>([&](auto at) {
         constexpr int I = decltype(at)::value;
@@ -122,9 +135,11 @@ __global__ void __launch_bounds__(T::WAVES * 64, T::BLOCKS_PER_CU) gemm_tiles_ke
         const unsigned chunk = 16 * ((lane & 7) ^ ((row >> 1) & 7));
         if constexpr (I < LOADS_A) {
             off[I] = (unsigned)min(row, a.M - 1 - m0) * (unsigned)(a.lda * 2) + chunk;
-        } else if constexpr (EPI == EPI_SWIGLU) {                  // a wave's TN columns: TN / 2 of gate, then the same of up
-            const int x = row % TN, col = min(n0 + row / TN * (TN / 2) + x % (TN / 2), NO - 1);
-            off[I] = (unsigned)(col + (x >= TN / 2 ? NO : 0)) * (unsigned)(a.ldw * 2) + chunk;
+        } else if constexpr (PAIRS) {
+            const int x = row % TN, pair = min(n0 + row / TN * (TN / 2) + x % (TN / 2), NO - 1);
+            const int first = EPI == EPI_ROPE ? pair + ((pair >> a.half_log) << a.half_log) : pair;
+            const int apart = EPI == EPI_ROPE ? 1 << a.half_log : NO;
+            off[I] = (unsigned)(first + (x >= TN / 2 ? apart : 0)) * (unsigned)(a.ldw * 2) + chunk;
         } else {
             off[I] = (unsigned)min(row, a.N - 1 - n0) * (unsigned)(a.ldw * 2) + chunk;
         }
@@ -137,12 +152,25 @@ __global__ void __launch_bounds__(T::WAVES * 64, T::BLOCKS_PER_CU) gemm_tiles_ke
         else load_to_lds<BM * 128 + (I - LOADS_A) * WAVES * 1024>(into, off[I], at_w);
     };
 
+    constexpr int SH = MT / WK;                                    // row tiles of C this wave writes: SH from the wk-th run on
+    const int row0 = m0 + wm * TM + wk * (16 * SH);
+    // ROPE: positions and cache slots of this lane's rows, asked for now and used last
+    int pos[SH], slot[SH];
+    if constexpr (EPI == EPI_ROPE) {
+#pragma unroll
+        for (int j = 0; j < SH; ++j) {
+            const int row = min(row0 + 16 * j + r, a.M - 1);
+            pos[j] = a.positions[row];
+            slot[j] = a.slots[row];
+        }
+    }
+
     v4f acc[NT][MT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = v4f{0.f, 0.f, 0.f, 0.f};
-    if constexpr (T::OWN_PRODUCT) asm volatile("s_nop 7");         // (and none between these writes and the first products)
+    if constexpr (T::own_product(EPI)) asm volatile("s_nop 7");         // (and none between these writes and the first products)
 
     // operand registers of two k-steps: one is multiplied while the other is read
     v8b fa[2][MT], fw[2][NT];
@@ -188,7 +216,7 @@ __global__ void __launch_bounds__(T::WAVES * 64, T::BLOCKS_PER_CU) gemm_tiles_ke
             });
             each<F1 - F0>([&](auto k) { fetch(std::integral_constant<int, L0 + F0 + decltype(k)::value>{}, at_a, at_w, into); });
             if constexpr (R1 > R0 || F1 > F0) __builtin_amdgcn_sched_barrier(0);
-            product<T::OWN_PRODUCT, I + 1 == P>(acc[I / MT][I % MT], fw[CUR][I / MT], fa[CUR][I % MT]);
+            product<T::own_product(EPI), I + 1 == P>(acc[I / MT][I % MT], fw[CUR][I / MT], fa[CUR][I % MT]);
         });
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -229,7 +257,6 @@ __global__ void __launch_bounds__(T::WAVES * 64, T::BLOCKS_PER_CU) gemm_tiles_ke
     wait_loads<0>();
     __syncthreads();                                               // LDS is free
 
-    constexpr int SH = MT / WK;                                    // row tiles of C this wave writes: SH from the wk-th run on
     if constexpr (WK > 1) {
         // the WK waves of the same results add up, each its own run of rows
         float* const red = reinterpret_cast<float*>(lds) + (size_t)(wm * WN + wn) * (WK * (WK - 1) * SH * NT * 256);
@@ -261,35 +288,87 @@ __global__ void __launch_bounds__(T::WAVES * 64, T::BLOCKS_PER_CU) gemm_tiles_ke
                 for (int nt = 0; nt < NT; ++nt) acc[nt][j] += *cell(wk, src, j, nt);
         __syncthreads();
     }
-    constexpr int ONT = EPI == EPI_SWIGLU ? NT / 2 : NT;           // column tiles of C
+    constexpr int ONT = PAIRS ? NT / 2 : NT;                       // column tiles of C, or of pairs
     const int c0 = n0 + wn * (ONT * 16);
-    const int row0 = m0 + wm * TM + wk * (16 * SH);
 
     // 16 rows at a time through LDS of the wave's own, so that whole lines are stored
-    constexpr int ROW = ONT * 32 + 16, PER_ROW = ONT * 2;          // bytes of a row in LDS; 16-byte chunks of a row
-    unsigned char* const mine = lds + wave * (16 * ROW);
-    static_assert(WAVES * 16 * ROW <= T::LDS_BYTES, "room for the rows");
+    constexpr int PARTS = EPI == EPI_ROPE ? 2 : 1;                 // of a row: a pair's first members, then its second ones
+    constexpr int ROW = PARTS * ONT * 32 + 16, PER_ROW = PARTS * ONT * 2;      // bytes of a row in LDS; 16-byte chunks of a row
+    constexpr int CELLS = EPI == EPI_ROPE ? SH * 128 : 0;
+    unsigned char* const mine = lds + wave * (16 * ROW + CELLS);
+    long long* const cell_of = reinterpret_cast<long long*>(mine + 16 * ROW);  // where a row's kv head 0 lies in the cache, -1: nowhere
+    static_assert(WAVES * (16 * ROW + CELLS) <= T::LDS_BYTES, "room for the rows");
+    if constexpr (EPI == EPI_ROPE)
+        if (kq == 0) {
+#pragma unroll
+            for (int j = 0; j < SH; ++j) {
+                const int pg = slot[j] >= 0 ? slot[j] / a.page_size : 0, at = slot[j] - pg * a.page_size;
+                cell_of[16 * j + r] = slot[j] >= 0 ? (((long long)pg * a.nkvh * a.page_size + at) << (a.half_log + 1)) : -1;
+            }
+        }
+    auto put = [&](int at, const float* v) {
+        uint16_t b[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) b[e] = __builtin_bit_cast(uint16_t, __float2bfloat16(v[e]));
+        *reinterpret_cast<uint2*>(mine + r * ROW + at + 8 * kq) = uint2{(unsigned)b[0] | ((unsigned)b[1] << 16), (unsigned)b[2] | ((unsigned)b[3] << 16)};
+    };
+    // the rotation of 16 rows is fetched while the 16 before are stored
+    v4f cs[ONT], sn[ONT];
+    auto fetch_rotation = [&](int j) {
+#pragma unroll
+        for (int nt = 0; nt < ONT; ++nt) {
+            const size_t at = ((size_t)pos[j] << a.half_log) + ((c0 + 16 * nt) & ((1 << a.half_log) - 1)) + 4 * kq;
+            cs[nt] = *reinterpret_cast<const v4f*>(a.cos_t + at);
+            sn[nt] = *reinterpret_cast<const v4f*>(a.sin_t + at);
+        }
+    };
+    if constexpr (EPI == EPI_ROPE) fetch_rotation(0);
 #pragma unroll
     for (int j = 0; j < SH; ++j) {
 #pragma unroll
         for (int nt = 0; nt < ONT; ++nt) {
-            uint16_t b[4];
+            float v[4], u[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                float v = acc[nt][j][e];
-                if constexpr (EPI == EPI_SWIGLU) v = silu_mul_fast(v, acc[nt + ONT][j][e]);
-                b[e] = __builtin_bit_cast(uint16_t, __float2bfloat16(v));
+                v[e] = acc[nt][j][e];
+                if constexpr (PAIRS) u[e] = acc[nt + ONT][j][e];
+                if constexpr (EPI == EPI_SWIGLU) v[e] = silu_mul_fast(v[e], u[e]);
             }
-            *reinterpret_cast<uint2*>(mine + r * ROW + 32 * nt + 8 * kq) =
-                uint2{(unsigned)b[0] | ((unsigned)b[1] << 16), (unsigned)b[2] | ((unsigned)b[3] << 16)};
+            if constexpr (EPI == EPI_ROPE) {
+                if (((c0 + 16 * nt) >> a.half_log) < a.nh + a.nkvh) {          // 16 pairs lie in one head
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float x = v[e], y = u[e];
+                        v[e] = x * cs[nt][e] - y * sn[nt][e];
+                        u[e] = x * sn[nt][e] + y * cs[nt][e];
+                    }
+                }
+                put(32 * (nt + ONT), u);
+            }
+            put(32 * nt, v);
         }
+        if constexpr (EPI == EPI_ROPE)
+            if (j + 1 < SH) fetch_rotation(j + 1);
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int i = 0; i < (16 * PER_ROW + 63) / 64; ++i) {
             const int q = lane + 64 * i, lr = q / PER_ROW, ch = q - lr * PER_ROW;
-            const int m = row0 + 16 * j + lr, n = c0 + 8 * ch;
-            if ((16 * PER_ROW % 64 == 0 || q < 16 * PER_ROW) && m < a.M && n < NO)
-                *reinterpret_cast<uint4*>(a.C + (size_t)m * a.ldc + n) = *reinterpret_cast<const uint4*>(mine + lr * ROW + 16 * ch);
+            const int m = row0 + 16 * j + lr, n = c0 + 8 * (ch % (2 * ONT));
+            if ((16 * PER_ROW % 64 != 0 && q >= 16 * PER_ROW) || m >= a.M || n >= NO) continue;
+            const uint4 w = *reinterpret_cast<const uint4*>(mine + lr * ROW + 16 * ch);
+            if constexpr (EPI == EPI_ROPE) {
+                const int head = n >> a.half_log, col = (n & ((1 << a.half_log) - 1)) + (ch < 2 * ONT ? 0 : 1 << a.half_log);
+                uint16_t* to = a.C + (size_t)m * a.ldc + ((size_t)head << (a.half_log + 1));
+                if (head >= a.nh) {                                // (nothing reads a key or a value in C)
+                    const bool v = head >= a.nh + a.nkvh;
+                    const long long cell = cell_of[16 * j + lr];
+                    if (cell < 0) continue;
+                    to = (v ? a.vcache : a.kcache) + cell + (((long long)(head - a.nh - (v ? a.nkvh : 0)) * a.page_size) << (a.half_log + 1));
+                }
+                *reinterpret_cast<uint4*>(to + col) = w;
+            } else {
+                *reinterpret_cast<uint4*>(a.C + (size_t)m * a.ldc + n) = w;
+            }
         }
         __builtin_amdgcn_wave_barrier();
     }
@@ -297,7 +376,7 @@ __global__ void __launch_bounds__(T::WAVES * 64, T::BLOCKS_PER_CU) gemm_tiles_ke
 
 template <typename T, int EPI> int launch(TilesArgs a, hipStream_t stream) {
     a.tiles_m = (a.M + T::BM - 1) / T::BM;
-    a.tiles_n = EPI == EPI_SWIGLU ? (a.N / 2 + T::BN / 2 - 1) / (T::BN / 2) : (a.N + T::BN - 1) / T::BN;
+    a.tiles_n = EPI != EPI_BF16 ? (a.N / 2 + T::BN / 2 - 1) / (T::BN / 2) : (a.N + T::BN - 1) / T::BN;
     const int groups = (a.tiles_m + 7) / 8;
     a.group_m = (a.tiles_m + groups - 1) / groups;
     const long long blocks = (long long)a.tiles_m * a.tiles_n;
@@ -337,15 +416,15 @@ template <typename T, int EPI> int launch(TilesArgs a, hipStream_t stream) {
 constexpr int kTiles = 15;
 constexpr double kUnits = 256.0;
 
-struct TileCost { int bm, bn, blocks_per_unit; bool pairs; double fixed, stage, full, round; };
+struct TileCost { int bm, bn, blocks_per_unit; bool takes[3]; double fixed, stage, full, round; };
 constexpr TileCost kCosts[kTiles] = {
-#define X(I, FIXED, STAGE, FULL, ROUND, ...) {Tile<__VA_ARGS__>::BM, Tile<__VA_ARGS__>::BN, Tile<__VA_ARGS__>::BLOCKS_PER_CU, Tile<__VA_ARGS__>::takes(EPI_SWIGLU), FIXED, STAGE, FULL, ROUND},
+#define X(I, FIXED, STAGE, FULL, ROUND, ...) {Tile<__VA_ARGS__>::BM, Tile<__VA_ARGS__>::BN, Tile<__VA_ARGS__>::BLOCKS_PER_CU, {true, Tile<__VA_ARGS__>::takes(EPI_SWIGLU), Tile<__VA_ARGS__>::takes(EPI_ROPE)}, FIXED, STAGE, FULL, ROUND},
     IC_TILES(X)
 #undef X
 };
 
 double cost_of(const TileCost& t, int M, int N, int K, int mode) {
-    const long long tm = (M + t.bm - 1) / t.bm, tn = mode == EPI_SWIGLU ? (N / 2 + t.bn / 2 - 1) / (t.bn / 2) : (N + t.bn - 1) / t.bn;
+    const long long tm = (M + t.bm - 1) / t.bm, tn = mode != EPI_BF16 ? (N / 2 + t.bn / 2 - 1) / (t.bn / 2) : (N + t.bn - 1) / t.bn;
     const double tiles = (double)(tm * tn), x = tiles / kUnits, stages = K / 64;
     double rounds = 1.0, busy = x < 1.0 ? x : 1.0, shared = 1.0;
     if (x > 1.0) {
@@ -362,7 +441,7 @@ double cost_of(const TileCost& t, int M, int N, int K, int mode) {
 int best_tile(int M, int N, int K, int mode, double* cost) {
     int best = 0;
     for (int i = 0; i < kTiles; ++i) {
-        if (mode != EPI_BF16 && !kCosts[i].pairs) continue;
+        if (!kCosts[i].takes[mode]) continue;
         const double c = cost_of(kCosts[i], M, N, K, mode);
         if (i == 0 || c < *cost) { *cost = c; best = i; }
     }
@@ -380,24 +459,52 @@ template <int EPI> int by_number(int tile, const TilesArgs& a, hipStream_t strea
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
-// Whole stages of K, 16-byte pieces of every row, byte offsets within 32 bits.
-bool takes(int M, int N, int K, int lda, int ldw, int ldc, int mode) {
+// Whole stages of K, 16-byte pieces of every row, byte offsets within 32 bits.  cols: columns of C.
+bool takes(int M, int N, int K, int lda, int ldw, int cols, int ldc, int mode) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 64 || lda < K || ldw < K || lda % 8 || ldw % 8) return false;
-    const int cols = mode == EPI_SWIGLU ? N / 2 : N;
-    if (N % (mode == EPI_SWIGLU ? 16 : 8) || ldc < cols || ldc % 8) return false;
-    if ((long long)lda * 2 * 256 >= (1LL << 31) || (long long)ldw * 2 * (mode == EPI_SWIGLU ? N : 256) >= (1LL << 32)) return false;
-    return (long long)((M + 63) / 64) * ((N + 63) / 64) < (1LL << 29);
+    if (N % (mode != EPI_BF16 ? 16 : 8) || ldc < cols || ldc % 8) return false;
+    if ((long long)lda * 2 * 256 >= (1LL << 31) || (long long)ldw * 2 * (mode != EPI_BF16 ? N : 256) >= (1LL << 32)) return false;
+    return (long long)((M + 63) / 64) * ((N + 63) / 64) < (1LL << 28);
 }
 
-int run(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, int mode, int tile, hipStream_t stream) {
-    TilesArgs a{(const uint16_t*)A, (const uint16_t*)W, (uint16_t*)C, M, N, K, lda, ldw, ldc, 0, 0, 0};
+int run(const TilesArgs& a, int mode, int tile, hipStream_t stream) {
+    if (mode == EPI_ROPE) return by_number<EPI_ROPE>(tile, a, stream);
     return mode == EPI_SWIGLU ? by_number<EPI_SWIGLU>(tile, a, stream) : by_number<EPI_BF16>(tile, a, stream);
+}
+
+TilesArgs plain_args(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc) {
+    return TilesArgs{(const uint16_t*)A, (const uint16_t*)W, (uint16_t*)C, M, N, K, lda, ldw, ldc};
+}
+
+int rope_run(const void* A, const void* W, void* C, int M, int K, int lda, int ldw, int ldc, const int* positions, const int* slots, const float* cos_t,
+             const float* sin_t, void* kcache, void* vcache, int nh, int nkvh, int dh, int page_size, int tile, hipStream_t stream) {
+    if (M <= 0) return IC_OK;
+    if (!positions || !slots || tile >= kTiles ||
+        !ic_gemm_tiles_rope_supported(A, W, C, M, K, lda, ldw, ldc, cos_t, sin_t, kcache, vcache, nh, nkvh, dh, page_size)) return IC_ERR_ARG;
+    const int N = (nh + 2 * nkvh) * dh;
+    TilesArgs a = plain_args(A, W, C, M, N, K, lda, ldw, ldc);
+    a.positions = positions, a.slots = slots, a.cos_t = cos_t, a.sin_t = sin_t;
+    a.kcache = (uint16_t*)kcache, a.vcache = (uint16_t*)vcache;
+    a.nh = nh, a.nkvh = nkvh, a.page_size = page_size;
+    while ((2 << a.half_log) < dh) ++a.half_log;
+    double cost = 0.0;
+    return run(a, EPI_ROPE, tile >= 0 ? tile : best_tile(M, N, K, EPI_ROPE, &cost), stream);
 }
 
 }  // namespace
 
 IC_EXPORT int ic_gemm_tiles_supported(int M, int N, int K, int lda, int ldw, int ldc, int mode) {
-    return (mode == EPI_BF16 || mode == EPI_SWIGLU) && takes(M, N, K, lda, ldw, ldc, mode);
+    return (mode == EPI_BF16 || mode == EPI_SWIGLU) && takes(M, N, K, lda, ldw, mode == EPI_SWIGLU ? N / 2 : N, ldc, mode);
+}
+
+// Heads of 32, 64, 128, .. entries, so that 16 neighbouring pairs lie in one head and a pair's head is a shift away.
+IC_EXPORT int ic_gemm_tiles_rope_supported(const void* A, const void* W, const void* C, int M, int K, int lda, int ldw, int ldc, const float* cos_t,
+                                           const float* sin_t, const void* kcache, const void* vcache, int nh, int nkvh, int dh, int page_size) {
+    if (nh <= 0 || nkvh <= 0 || dh < 32 || dh > 1024 || (dh & (dh - 1)) || page_size <= 0 || (long long)(nh + 2LL * nkvh) * dh >= (1LL << 30)) return 0;
+    const void* const all[7] = {A, W, C, cos_t, sin_t, kcache, vcache};
+    for (const void* p : all)
+        if (!p || !aligned16(p)) return 0;
+    return takes(M, (nh + 2 * nkvh) * dh, K, lda, ldw, nh * dh, ldc, EPI_ROPE);
 }
 
 // Whether the library would be faster.  Two kinds of product where it is, fitted to the same sweep (own against library, the choice loses 1.0 % to the
@@ -408,13 +515,17 @@ IC_EXPORT int ic_gemm_tiles_supported(int M, int N, int K, int lda, int ldw, int
 //   product split over the whole chip takes.
 // Elsewhere the own kernel is faster (1,045 x 2,560 x 1,536: 17.0 -> 12.2 us; 871 x 1,536 x 1,536: 12.5 -> 10.0; 2,048 x 2,304 x 2,304: 28 -> 22.6).
 // With the gated unit in the epilogue it is compared with the library's product and the unit's own kernel, and is faster from 33 rows on
-// (1,045 x 7,680 x 1,536: 42.0 -> 28.0; 2,048 x 11,520 x 2,304: 131 -> 97; 16,384 x 32,768 x 4,096: 3,135 -> 2,942).
+// (1,045 x 7,680 x 1,536: 42.0 -> 28.0; 2,048 x 11,520 x 2,304: 131 -> 97; 16,384 x 32,768 x 4,096: 3,135 -> 2,942).  So is QKV with rotary and cache
+// write, against the library's product and their own kernel (64 rows of the 2B shape 19.0 -> 13.9, 1,045 rows of the 1B shape 21.5 -> 15.1, 2,048 of
+// the 8B shape 77 -> 68), but for sizes that the largest tile fits best, which this epilogue does not have.
 IC_EXPORT int ic_gemm_tiles_pays(int M, int N, int K, int mode) {
     if (M <= 32) return 0;
     const double t = (double)((M + 255) / 256) * ((N + 255) / 256), fill = t / (kUnits * __builtin_ceil(t / kUnits));
-    if (mode == EPI_SWIGLU) return K <= 8192 || fill < 0.93;
-    if (t >= 200.0 && fill >= 0.97) return 0;
     double cost = 0.0;
+    if (mode != EPI_BF16 && K > 8192 && fill >= 0.93) return 0;
+    if (mode == EPI_ROPE) return kCosts[best_tile(M, N, K, EPI_SWIGLU, &cost)].takes[EPI_ROPE];
+    if (mode == EPI_SWIGLU) return 1;
+    if (t >= 200.0 && fill >= 0.97) return 0;
     best_tile(M, N, K, mode, &cost);
     const double products = 2.0 * M * N * K / 0.6e9, read = 2.0 * N * K / 4e6;
     return cost <= 1.6 * (6.0 + (products > read ? products : read));
@@ -429,7 +540,7 @@ IC_EXPORT int ic_gemm_tiles(const void* A, const void* W, void* C, int M, int N,
     if (M <= 0) return IC_OK;
     if (!A || !W || !C || !ic_gemm_tiles_supported(M, N, K, lda, ldw, ldc, mode) || !aligned16(A) || !aligned16(W) || !aligned16(C)) return IC_ERR_ARG;
     double cost = 0.0;
-    return run(A, W, C, M, N, K, lda, ldw, ldc, mode, best_tile(M, N, K, mode, &cost), stream);
+    return run(plain_args(A, W, C, M, N, K, lda, ldw, ldc), mode, best_tile(M, N, K, mode, &cost), stream);
 }
 
 IC_EXPORT int ic_gemm_tiles_cfg(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, int mode, int tile,
@@ -437,7 +548,20 @@ IC_EXPORT int ic_gemm_tiles_cfg(const void* A, const void* W, void* C, int M, in
     if (M <= 0) return IC_OK;
     if (!A || !W || !C || tile < 0 || tile >= kTiles || !ic_gemm_tiles_supported(M, N, K, lda, ldw, ldc, mode) || !aligned16(A) || !aligned16(W) ||
         !aligned16(C)) return IC_ERR_ARG;
-    return run(A, W, C, M, N, K, lda, ldw, ldc, mode, tile, stream);
+    return run(plain_args(A, W, C, M, N, K, lda, ldw, ldc), mode, tile, stream);
+}
+
+IC_EXPORT int ic_gemm_tiles_rope(const void* A, const void* W, void* C, int M, int K, int lda, int ldw, int ldc, const int* positions, const int* slots,
+                                 const float* cos_t, const float* sin_t, void* kcache, void* vcache, int nh, int nkvh, int dh, int page_size,
+                                 hipStream_t stream) {
+    return rope_run(A, W, C, M, K, lda, ldw, ldc, positions, slots, cos_t, sin_t, kcache, vcache, nh, nkvh, dh, page_size, -1, stream);
+}
+
+IC_EXPORT int ic_gemm_tiles_rope_cfg(const void* A, const void* W, void* C, int M, int K, int lda, int ldw, int ldc, const int* positions, const int* slots,
+                                     const float* cos_t, const float* sin_t, void* kcache, void* vcache, int nh, int nkvh, int dh, int page_size, int tile,
+                                     hipStream_t stream) {
+    if (tile < 0) return IC_ERR_ARG;
+    return rope_run(A, W, C, M, K, lda, ldw, ldc, positions, slots, cos_t, sin_t, kcache, vcache, nh, nkvh, dh, page_size, tile, stream);
 }
 
 // The product by the kernel that is faster for it: this file's or the library's.

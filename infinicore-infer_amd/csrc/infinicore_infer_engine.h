@@ -169,6 +169,8 @@ int ic_rule_own_product(int a_dtype, int w_dtype, int c_dtype, int rows);
 // 1: the QKV projection runs with rotary and cache write in its epilogue (ic_gemm_qkv_rope); 0: product, then ic_rope_kv_write.
 // kv_heads_written: 0 when the entry writes no cache; row_factors_owed: the rows' norm is half done (IcRowFactor).
 int ic_rule_qkv_fused(int dtype, int rows, int K, int lda, int ldw, int head_dim, int rot_dim, int kv_heads_written, int row_factors_owed);
+// More rows: 1: the same in tiles (ic_gemm_tiles_rope).
+int ic_rule_qkv_tiles(int dtype, const void* A, const void* W, const void* C, int rows, int K, int lda, int ldw, int ldc, const float* cos_t, const float* sin_t, const void* kcache, const void* vcache, int nh, int kv_heads_written, int head_dim, int rot_dim, int page_size);
 // 1: the gate/up projection runs with SwiGLU in its epilogue (ic_gemm_nt, c_mode 1); 0: product, then ic_swiglu.
 int ic_rule_gate_up_fused(int dtype, int rows, int K, int lda, int ldw, int row_factors_owed);
 // More rows: 1: the gate/up projection with SwiGLU in its epilogue in tiles (ic_gemm_tiles, mode 1).  N: rows of W; ldc: the row stride of its result.

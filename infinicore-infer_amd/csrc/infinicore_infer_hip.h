@@ -155,6 +155,10 @@ int ic_splitk_add_rmsnorm(const float* P, int n_slices, int M, float* x, float a
 int ic_gemm_tiles_supported(int M, int N, int K, int lda, int ldw, int ldc, int mode);
 int ic_gemm_tiles_pays(int M, int N, int K, int mode);
 int ic_gemm_tiles(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, int mode, hipStream_t stream);
+// QKV of many rows (W = [q heads; k heads; v heads], full rotary) with rotary and cache write in the epilogue: rotated queries in C[M, nh * dh], rotated
+// keys and values in the cache slots (slot < 0: not stored); keys and values of C are not written.  dh a power of two from 32 on.
+int ic_gemm_tiles_rope_supported(const void* A, const void* W, const void* C, int M, int K, int lda, int ldw, int ldc, const float* cos_t, const float* sin_t, const void* kcache, const void* vcache, int nh, int nkvh, int dh, int page_size);
+int ic_gemm_tiles_rope(const void* A, const void* W, void* C, int M, int K, int lda, int ldw, int ldc, const int* positions, const int* slots, const float* cos_t, const float* sin_t, void* kcache, void* vcache, int nh, int nkvh, int dh, int page_size, hipStream_t stream);
 // C[M, N] = alpha * A[M, K] W[N, K]^T for many rows by the faster of ic_gemm_tiles and ic_matmul; arguments and results as ic_matmul.
 int ic_product(const void* A, int a_dtype, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldw, int ldc, float alpha, void* workspace, long long workspace_bytes, hipStream_t stream);
 

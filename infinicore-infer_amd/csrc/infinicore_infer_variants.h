@@ -21,8 +21,9 @@ int ic_gemm_nt_cfg(const void* A, const void* W, void* C, int c_dtype, int M, in
 // blocks, columns a block) for the kernel of gemm_rows.hip; 0 for the kernels of gemm.hip.
 int ic_gemm_rows_plan(int epi, int M, int N, int K, int blocks, int units, int* plan);
 
-// ic_gemm_tiles with its tile named by the caller (0..14, the order in gemm_tiles.hip), and the tile that it chooses by itself (-1: an argument fault).
+// ic_gemm_tiles and ic_gemm_tiles_rope with their tile named by the caller (0..14, the order in gemm_tiles.hip), and the tile that the former chooses by itself (-1: an argument fault).
 int ic_gemm_tiles_cfg(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, int mode, int tile, hipStream_t stream);
+int ic_gemm_tiles_rope_cfg(const void* A, const void* W, void* C, int M, int K, int lda, int ldw, int ldc, const int* positions, const int* slots, const float* cos_t, const float* sin_t, void* kcache, void* vcache, int nh, int nkvh, int dh, int page_size, int tile, hipStream_t stream);
 int ic_gemm_tiles_plan(int M, int N, int K, int mode);
 
 // key / page_size as the kernels of single tokens compute it; -1: an argument fault.

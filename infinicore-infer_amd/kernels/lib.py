@@ -190,6 +190,10 @@ _SIGNATURES = {
     "ic_gemm_tiles_plan": [_I, _I, _I, _I],
     "ic_gemm_tiles": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
     "ic_gemm_tiles_cfg": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P],
+    "ic_gemm_tiles_rope_supported": [_P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I],
+    "ic_gemm_tiles_rope": [_P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P],
+    "ic_gemm_tiles_rope_cfg": [_P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
+    "ic_rule_qkv_tiles": [_I, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I],
     "ic_product": [_P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _P, _LL, _P],
     "ic_gemm_splitk_supported": [_I, _I, _I, _I, _I],
     "ic_gemm_splitk_slices": [_I, _I],

@@ -401,6 +401,15 @@ def rule_gate_up_fused(dtype, rows: int, a, w, row_factors_owed: bool) -> bool:
                                                                      int(w.stride(0)), int(bool(row_factors_owed))))
 
 
+def rule_qkv_tiles(a, w, qkv, cos, sin, kcache, vcache, n_heads: int, kv_heads_written: int, head_dim: int, rot_dim: int, page_size: int) -> bool:
+    """True when the QKV projection of the many rows a runs with rotary and cache write in its epilogue, in tiles (gemm_tiles_rope)."""
+    code = _code_or_none(a.dtype)
+    return code is not None and a.dtype == w.dtype == qkv.dtype and a.stride(1) == w.stride(1) == qkv.stride(1) == 1 and \
+        bool(get_lib().ic_rule_qkv_tiles(code, a.data_ptr(), w.data_ptr(), qkv.data_ptr(), a.shape[0], a.shape[1], a.stride(0), w.stride(0),
+                                         qkv.stride(0), cos.data_ptr(), sin.data_ptr(), kcache.data_ptr(), vcache.data_ptr(), int(n_heads),
+                                         int(kv_heads_written), int(head_dim), int(rot_dim), int(page_size)))
+
+
 def rule_gate_up_tiles(a, w, out) -> bool:
     """True when the gate/up projection of the many rows a with w runs with SwiGLU in its epilogue, in tiles (gemm_tiles)."""
     code = _code_or_none(a.dtype)
@@ -681,6 +690,31 @@ def gemm_qkv_rope(a, w, qkv, positions, slots, cos, sin, kcache, vcache, n_heads
         check(get_lib().ic_gemm_qkv_rope_variant(*args, int(tile_rows), _stream()), "gemm_qkv_rope")
     else:
         check(get_lib().ic_gemm_qkv_rope(*args, _stream()), "gemm_qkv_rope")
+    return qkv
+
+
+def gemm_tiles_rope(a, w, qkv, positions, slots, cos, sin, kcache, vcache, n_heads, n_kv_heads, head_dim, page_size, tile=None):
+    """gemm_qkv_rope for many rows, in tiles: rotated queries in qkv's q heads, rotated keys and the values in cache slot ``slots[m]``
+    (none for a negative one); qkv's k and v heads are not written.  Head sizes that are powers of two.  tile (tests): as in gemm_tiles."""
+    _dev(a, w, qkv, positions, slots, cos, sin, kcache, vcache)
+    M, K = a.shape
+    _i32(positions, "positions")
+    _i32(slots, "slots")
+    _need(positions.numel() == M and slots.numel() == M, "gemm_tiles_rope: one position and slot each")
+    _need(tuple(w.shape) == ((n_heads + 2 * n_kv_heads) * head_dim, K), "gemm_tiles_rope: weight shape")
+    _need(qkv.shape[0] == M and qkv.shape[1] >= n_heads * head_dim and qkv.stride(1) == 1
+          and a.stride(1) == 1 and w.stride(1) == 1, "gemm_tiles_rope: layout")
+    _need(a.dtype == w.dtype == qkv.dtype == kcache.dtype == vcache.dtype == torch.bfloat16, "gemm_tiles_rope: bfloat16 only")
+    _need(cos.dtype == torch.float32 and sin.dtype == torch.float32 and cos.is_contiguous() and sin.is_contiguous()
+          and cos.shape[-1] == head_dim // 2 and sin.shape == cos.shape, "gemm_tiles_rope: cos/sin must be float32 [max_pos, dh/2]")
+    _need(kcache.is_contiguous() and vcache.is_contiguous() and kcache.shape == vcache.shape
+          and tuple(kcache.shape[1:]) == (n_kv_heads, page_size, head_dim), "gemm_tiles_rope: cache layout")
+    args = (a.data_ptr(), w.data_ptr(), qkv.data_ptr(), M, K, a.stride(0), w.stride(0), qkv.stride(0), positions.data_ptr(),
+            slots.data_ptr(), cos.data_ptr(), sin.data_ptr(), kcache.data_ptr(), vcache.data_ptr(), n_heads, n_kv_heads, head_dim, page_size)
+    if tile is None:
+        check(get_lib().ic_gemm_tiles_rope(*args, _stream()), "gemm_tiles_rope")
+    else:
+        check(get_lib().ic_gemm_tiles_rope_cfg(*args, int(tile), _stream()), "gemm_tiles_rope")
     return qkv
 
 

@@ -110,19 +110,24 @@ class Rotary(PositionEncoding):
 
 
     def project_rotate_store(self, h, w_qkv, qkv, ctx, cache, n_heads, n_kv_heads, head_dim) -> bool:
-        """Few rows in bfloat16 with full rotary: the projection kernel rotates and writes the cache."""
+        """In bfloat16 with full rotary: the projection kernel rotates and writes the cache."""
         rt = self.runtime
         row_factor = None
         if isinstance(h, DeferredRows):
             h, row_factor = h.values, h.row_factor()
-        if (rt.gemm_impl != "auto" or h.dtype != w_qkv.dtype or h.dtype != qkv.dtype
-                or not ops.rule_qkv_fused(h.dtype, h.shape[0], h, w_qkv, head_dim, self.rot_dim, n_kv_heads,
-                                          row_factor is not None)):
+        if rt.gemm_impl != "auto" or h.dtype != w_qkv.dtype or h.dtype != qkv.dtype:
+            return False
+        few = ops.rule_qkv_fused(h.dtype, h.shape[0], h, w_qkv, head_dim, self.rot_dim, n_kv_heads, row_factor is not None)
+        if not few and (row_factor is not None or n_kv_heads <= 0 or not ops.rule_qkv_tiles(
+                h, w_qkv, qkv, self.cos, self.sin, cache.k, cache.v, n_heads, n_kv_heads, head_dim, self.rot_dim, ctx.page_size)):
             return False
         if ctx.max_position >= self.max_positions:
             raise ValueError("position %d is beyond the rotary tables (%d)" % (ctx.max_position, self.max_positions))
-        ops.gemm_qkv_rope(h, w_qkv, qkv, ctx.positions, cache.slots, self.cos, self.sin, cache.k, cache.v,
-                          n_heads, n_kv_heads, head_dim, ctx.page_size, row_factor=row_factor)
+        args = (h, w_qkv, qkv, ctx.positions, cache.slots, self.cos, self.sin, cache.k, cache.v, n_heads, n_kv_heads, head_dim, ctx.page_size)
+        if few:
+            ops.gemm_qkv_rope(*args, row_factor=row_factor)
+        else:
+            ops.gemm_tiles_rope(*args)
         return True
 
 

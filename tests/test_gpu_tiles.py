@@ -121,3 +121,46 @@ def test_refused_operands_go_to_the_library():
             ops.gemm_tiles(ad, w.cuda(), out)
         ops.product(ad, w.cuda(), out)
         _check(a, w, out, False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", [None] + list(range(len(TILES))))
+def test_qkv_with_rotary_and_cache_write(tile):
+    """Queries, keys and values against float64: head sizes whose halves are one matrix tile, two and more, tokens without a slot, slots in any
+    order, page sizes that are no power of two, heads that begin inside a tile."""
+    if tile is not None and TILES[tile] in ((64, 96), (256, 256)):
+        pytest.skip("three column tiles a wave: no pairs; 256 accumulators a lane: no registers")
+    for M, K, nh, nkv, dh, ps in ((70, 128, 3, 1, 64, 16), (33, 64, 2, 2, 32, 7), (197, 192, 5, 2, 128, 64), (1, 320, 1, 1, 256, 3)):
+        a, w = _operands(M, (nh + 2 * nkv) * dh, K, M + dh)
+        g = torch.Generator().manual_seed(M)
+        pos = torch.randint(0, 500, (M,), generator=g, dtype=torch.int32)
+        pages = (M + ps - 1) // ps + 1
+        slots = torch.randperm(pages * ps, generator=g)[:M].to(torch.int32)
+        slots[M // 2:M // 2 + 1] = -1
+        half = dh // 2
+        ang = torch.arange(500).double()[:, None] * 10000.0 ** (-torch.arange(half).double() / half)
+        cos, sin = ang.cos().float(), ang.sin().float()
+        qkv = torch.full((M, (nh + 2 * nkv) * dh), 3.0, dtype=BF16, device="cuda")
+        k = torch.full((pages, nkv, ps, dh), 5.0, dtype=BF16, device="cuda")
+        v = torch.full_like(k, 7.0)
+        ops.gemm_tiles_rope(a.cuda(), w.cuda(), qkv, pos.cuda(), slots.cuda(), cos.cuda(), sin.cuda(), k, v, nh, nkv, dh, ps, tile=tile)
+        ref = (a.double() @ w.double().t()).view(M, nh + 2 * nkv, dh)
+        mag = ((a.double().abs() @ w.double().abs().t()) * K * 2.0 ** -24).view(M, nh + 2 * nkv, dh)
+        c, s = cos.double()[pos.long()][:, None], sin.double()[pos.long()][:, None]
+        rot = nh + nkv
+        x, y, mx, my = ref[:, :rot, :half], ref[:, :rot, half:], mag[:, :rot, :half], mag[:, :rot, half:]
+        want, bound = ref.clone(), mag.clone()
+        want[:, :rot, :half], want[:, :rot, half:] = x * c - y * s, x * s + y * c
+        # two products and a sum in float32 beside the sums' own error
+        bound[:, :rot] = torch.cat([mx + my, mx + my], -1) + 2.0 ** -22 * torch.cat([x.abs() + y.abs()] * 2, -1)
+        bound = bound + want.abs() * 2.0 ** -8
+        got = want.clone()
+        got[:, :nh] = qkv.cpu().double().view(M, -1, dh)[:, :nh]
+        kk, vv = k.cpu().double().transpose(1, 2).reshape(pages * ps, nkv, dh), v.cpu().double().transpose(1, 2).reshape(pages * ps, nkv, dh)
+        have = slots >= 0
+        at = slots[have].long()
+        got[have, nh:rot], got[have, rot:] = kk[at], vv[at]
+        assert ((got - want).abs() - bound).max() <= 0, (M, K, nh, nkv, dh, ps)
+        untouched = torch.ones(pages * ps, dtype=torch.bool)
+        untouched[at] = False
+        assert (kk[untouched] == 5.0).all() and (vv[untouched] == 7.0).all()
