@@ -5,8 +5,9 @@
 // few-row products with their epilogues (rotary and cache write after QKV; residual add, the next norm's
 // weight and sums of squares after O and down; SwiGLU after gate/up), the norm between two products being
 // split over them; more rows take the products in tiles (QKV with rotary and cache write, gate/up with SwiGLU in
-// the epilogue) or the library's, as ic_product chooses, float32 the library's, and the norm, rotary and activation kernels.  Single-token rows go to the split-key attention kernel, prompt portions to the tiled one, what
-// neither takes to the general one.
+// the epilogue) or the library's, as ic_product chooses, float32 the library's, and the norm, rotary and activation kernels.
+// Single-token rows go to the split-key attention kernel, prompt portions to the tiled one, both of a mixed step to one launch
+// where that is faster, what neither takes to the general one.
 #include "common.h"
 #include "infinicore_infer_engine.h"
 #include <algorithm>
@@ -94,6 +95,18 @@ IC_EXPORT int ic_rule_attention(int dtype, int head_dim, int page_size, int n_de
     const bool use_pre = pre_ok && n_tiles > 0 && (dec_ok || n_decode_rows == 0);
     if (!((use_dec || n_decode_rows == 0) && (use_pre || n_tiles == 0))) return IC_ATTN_GENERAL;
     return (use_dec ? IC_ATTN_SINGLE_TOKENS : 0) | (use_pre ? IC_ATTN_PORTIONS : 0);
+}
+
+// Together the two kinds of block fill each other's tails: 40 rows of 100..2,048 keys beside portions of 512 and 463 after 512 (24:8 heads of 64) 39.1 -> 25.2
+// us, 8 rows beside a prompt of 300 18.2 -> 11.0 (36 heads of 64: 20.8 -> 14.6; 32:2 of 128: 23.9 -> 16.5), 60 rows of up to 3,000 keys beside 850
+// tokens 44.2 -> 32.0 (87.6 -> 82.1, 45.1 -> 38.9).  Not where few tiles with long walks would take two wave groups each, which the common kernel does
+// not have: 2 rows beside a portion of 700 after 2,500 (32:2 of 128) 71.2 -> 77.2.
+IC_EXPORT int ic_rule_attention_together(int dtype, int nh, int nkvh, int head_dim, int page_size, int table_stride, int n_decode_rows, int n_tiles,
+                                         int max_position, int window, int parts, int compute_units) {
+    if (n_decode_rows <= 0 || n_tiles <= 0 || !ic_attn_mixed_supported(dtype, nh, nkvh, head_dim, page_size, table_stride)) return 0;
+    const int keys = window > 0 ? std::min(max_position + 1, window + ic_attn_prefill_tile_rows()) : max_position + 1;
+    const bool two_groups = parts <= 1 && (long long)n_tiles * nh <= 2LL * (compute_units > 0 ? compute_units : 256);
+    return !(two_groups && keys >= 24 * 64);
 }
 
 IC_EXPORT int ic_rule_context_bucket(int n_keys) {
@@ -306,6 +319,14 @@ struct IcDecoder {
                 st = ic_attn_generic(qkv, width, attn_out, ow, dt, e.k_cache, e.v_cache, tables, bts, b.token_req, b.positions, T,
                                      A.n_heads, A.n_kv_heads, A.head_dim, ps, A.softmax_scale, A.window, stream);
                 if (st) return fail(st, "attention (general kernel)", i);
+            } else if (int part_len = 0, parts = use_dec && use_pre && decode_rows ? tile_parts_for(b, A, &part_len) : 0;
+                       parts > 0 && ic_rule_attention_together(dt, A.n_heads, A.n_kv_heads, A.head_dim, ps, bts, n_dec, n_tiles, b.max_position, A.window,
+                                                               parts, meta.compute_units)) {
+                st = ic_attn_mixed(qkv, width, attn_out, ow, dt, e.k_cache, e.v_cache, tables, bts, decode_rows, b.token_req, b.positions,
+                                   (float*)(base + ws.part_acc), (float*)(base + ws.part_ml), n_dec, splits_for(b, A), b.prefill_tiles, n_tiles, A.n_heads,
+                                   A.n_kv_heads, A.head_dim, ps, A.softmax_scale, A.window, parts, part_len, (float*)(base + ws.tile_parts),
+                                   ic_attn_prefill_scratch_floats(n_tiles, A.n_heads, A.head_dim, parts), meta.attention_counters, stream);
+                if (st) return fail(st, "attention of single tokens and prompt portions", i);
             } else {
                 if (use_dec) {
                     const int n_split = splits_for(b, A);

@@ -114,6 +114,9 @@ _SIGNATURES = {
     "ic_attn_prefill_parts": [_I, _I, _I, _I, _I, _c.POINTER(_I)],
     "ic_attn_prefill_parts_of_step": [_I, _I, _I, _I, _I, _I, _I, _c.POINTER(_I)],
     "ic_attn_prefill_split": [_P, _I, _P, _I, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _F, _I, _I, _I, _I, _P, _LL, _P, _P],
+    "ic_attn_mixed_supported": [_I, _I, _I, _I, _I, _I],
+    "ic_attn_mixed": [_P, _I, _P, _I, _I, _P, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _P, _I, _I, _I, _I, _I, _F, _I, _I, _I, _P, _LL, _P, _P],
+    "ic_attn_decode_merge": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "ic_attn_prefill_counter_ints": [],
     "ic_embed_sinusoid": [_P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _F, _P],
     "ic_norm_into_stream": [_P, _I, _P, _P, _P, _P, _I, _I, _I, _F, _P],
@@ -208,6 +211,7 @@ _SIGNATURES = {
     "ic_rule_gate_up_tiles": [_I, _P, _P, _P, _I, _I, _I, _I, _I, _I],
     "ic_rule_tail": [_I, _I, _I, _I, _I, _I],
     "ic_rule_attention": [_I, _I, _I, _I, _I],
+    "ic_rule_attention_together": [_I] * 12,
     "ic_rule_context_bucket": [_I],
     "ic_attn_decode_on_matrix_cores": [_I, _I, _I],
     "ic_decoder_create": [_c.POINTER(IcDecoderMeta), _c.POINTER(IcLayer), _c.POINTER(IcRunEntry)],

@@ -318,6 +318,33 @@ def attention_prefill(q, out, kcache, vcache, block_tables, tiles, n_tiles, n_he
         "attention_prefill")
 
 
+def attention_mixed(q, out, kcache, vcache, block_tables, tok_list, n_tok, token_req, positions, part_acc, part_ml, n_split: int, tiles, n_tiles,
+                    n_heads, n_kv_heads, head_dim, page_size, scale: float, window: int = 0, parts: int = 1, part_len: int = 0, scratch=None,
+                    counters=None):
+    """attention_decode of the tokens in tok_list and attention_prefill (one group) of the tiles, in one launch."""
+    _attn_common(q, out, kcache, vcache, block_tables, n_heads, n_kv_heads, head_dim, page_size)
+    for t, what in ((token_req, "token_req"), (positions, "positions"), (tok_list, "tok_list")):
+        _i32(t, what)
+    _need(tok_list.numel() >= n_tok > 0, "attention_mixed: tok_list too short")
+    _need(part_acc.dtype == torch.float32 and part_acc.is_contiguous()
+          and part_acc.numel() >= n_tok * n_heads * n_split * head_dim, "attention_mixed: part_acc too small")
+    _need(part_ml.dtype == torch.float32 and part_ml.is_contiguous()
+          and part_ml.numel() >= n_tok * n_heads * n_split * 2, "attention_mixed: part_ml too small")
+    _need(tiles.dtype == torch.int32 and tiles.is_contiguous() and tiles.dim() == 2 and tiles.shape[1] == 4
+          and tiles.shape[0] >= n_tiles > 0, "attention_mixed: tiles must be int32 [n, 4]")
+    if parts > 1:
+        _dev(scratch)
+        _dev(counters)
+        _need(scratch.dtype == torch.float32 and scratch.is_contiguous() and counters.dtype == torch.int32 and counters.is_contiguous()
+              and counters.numel() >= attention_prefill_counter_ints(), "attention_mixed: a cut walk needs float32 scratch and int32 counters")
+    check(get_lib().ic_attn_mixed(
+        q.data_ptr(), q.stride(0), out.data_ptr(), out.stride(0), dtype_code(q.dtype), kcache.data_ptr(), vcache.data_ptr(), block_tables.data_ptr(),
+        block_tables.stride(0), tok_list.data_ptr(), token_req.data_ptr(), positions.data_ptr(), part_acc.data_ptr(), part_ml.data_ptr(), n_tok,
+        int(n_split), tiles.data_ptr(), n_tiles, n_heads, n_kv_heads, head_dim, page_size, float(scale), int(window or 0), int(parts), int(part_len),
+        scratch.data_ptr() if parts > 1 else None, scratch.numel() if parts > 1 else 0, counters.data_ptr() if parts > 1 else None, _stream()),
+        "attention_mixed")
+
+
 def sample(logits, out, temperature=None, top_k=None, top_p=None, uniform=None):
     """out[r] = token sampled from logits[r] (float32 [R, V]).  temperature None: argmax."""
     _dev(logits, out, temperature, top_k, top_p, uniform)
@@ -429,6 +456,14 @@ def rule_tail(dtype, a, w) -> int:
 def rule_attention(dtype, head_dim: int, page_size: int, n_decode_rows: int, n_tiles: int) -> int:
     """ATTN_GENERAL, or the bits ATTN_SINGLE_TOKENS and ATTN_PORTIONS: which attention kernels a step takes."""
     return int(get_lib().ic_rule_attention(dtype_code(dtype), int(head_dim), int(page_size), int(n_decode_rows), int(n_tiles)))
+
+
+def rule_attention_together(dtype, n_heads: int, n_kv_heads: int, head_dim: int, page_size: int, table_stride: int, n_decode_rows: int, n_tiles: int,
+                            max_position: int, window: int, parts: int, compute_units: int) -> bool:
+    """True when a mixed step's single tokens and prompt tiles run in one launch (attention_mixed)."""
+    return bool(get_lib().ic_rule_attention_together(dtype_code(dtype), int(n_heads), int(n_kv_heads), int(head_dim), int(page_size), int(table_stride),
+                                                     int(n_decode_rows), int(n_tiles), int(max_position), int(window or 0), int(parts),
+                                                     int(compute_units)))
 
 
 def rule_context_bucket(n_keys: int) -> int:
