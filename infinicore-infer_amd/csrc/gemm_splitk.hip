@@ -8,10 +8,10 @@
 // any sensible size for 256 compute units.  Here a block owns 64 weight rows and one slice of K: A
 // goes through LDS once per block (shared by its four waves), the weights stream straight from
 // memory into operand layout, and (N / 64) x S blocks fill most of the chip.  The slices meet in
-// the add + norm kernel, which runs after the library's product too.  Measured on MI355X with cold
+// the add + norm kernel, which runs after unsliced products too.  Measured on MI355X with cold
 // weights at 64 rows (this / the library, us): 2,304 x 2,304: 8.8 / 11.1; 2,304 x 5,760: 13.3 / 25.0.
-// For wide results (QKV, gate/up: N of 7,000 and more) the library is faster and is used: every
-// block re-reads its slice of A, N / 64 times the bytes of A in all, as much as the weights there.
+// Wide results (QKV, gate/up: N of 7,000 and more) do not take this kernel: every block re-reads
+// its slice of A, N / 64 times the bytes of A in all, as much as the weights there.
 //
 // Block: 4 waves; wave w owns weight rows n0 + 16 w .. + 15 and all row tiles of A.  K advances in
 // chunks of 128: the A chunk [16 MT rows, 128] lies in LDS (rows padded to 272 bytes: a wave's 16-byte

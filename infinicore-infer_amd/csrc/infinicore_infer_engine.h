@@ -162,9 +162,9 @@ int ic_decoder_pack(const IcDecoder* decoder, const IcHostBatch* batch, int* sta
 #define IC_ATTN_GENERAL 0     // the general kernel for every row
 #define IC_ATTN_SINGLE_TOKENS 1   // (bit) the split-key kernel for rows that are a request's single new token
 #define IC_ATTN_PORTIONS 2        // (bit) the tiled matrix-core kernel for prompt portions
-int ic_rule_few_rows();           // rows up to which the package's own product runs instead of the library's
+int ic_rule_few_rows();           // rows up to which the package's own few-row product runs
 int ic_rule_sumsq_parts_max();    // column blocks of sums of squares a product takes as row factors
-// 1: a plain product of `rows` rows runs in the package's own kernel (ic_gemm_nt), 0: in the library (ic_matmul).
+// 1: a plain product of `rows` rows runs in the few-row kernel (ic_gemm_nt), 0: in tiles or in the library (ic_product).
 int ic_rule_own_product(int a_dtype, int w_dtype, int c_dtype, int rows);
 // 1: the QKV projection runs with rotary and cache write in its epilogue (ic_gemm_qkv_rope); 0: product, then ic_rope_kv_write.
 // kv_heads_written: 0 when the entry writes no cache; row_factors_owed: the rows' norm is half done (IcRowFactor).

@@ -15,7 +15,7 @@
 //     unit with bounded branches) in its epilogue,
 //   * ic_moe_combine: a token's result is the sum of its pairs' rows (times the weight when it is on the
 //     OUTPUT), plus an optional row of a shared expert; a pair of an identity expert counts the token's own row.
-// For many rows the products between gather and combine are library products over each expert's run of rows.
+// For many rows the products between gather and combine are products in tiles or the library's over each expert's run of rows.
 #include "common.h"
 
 constexpr int kMoeMaxExperts = 1024;

@@ -408,7 +408,7 @@ def _code_or_none(dt):
 
 
 def rule_own_product(a_dtype, w_dtype, c_dtype, rows: int) -> bool:
-    """True when a plain product of ``rows`` rows runs in the package's own kernel (gemm_nt), not in the library."""
+    """True when a plain product of ``rows`` rows runs in the few-row kernel (gemm_nt), not in tiles or the library (product)."""
     codes = (_code_or_none(a_dtype), _code_or_none(w_dtype), _code_or_none(c_dtype))
     return None not in codes and bool(get_lib().ic_rule_own_product(codes[0], codes[1], codes[2], int(rows)))
 

@@ -18,7 +18,7 @@ Tensors: ``router`` [experts + identity, d], ``correction`` [experts + identity]
 A step's (token, choice) pairs are sorted by expert on the device (stable).  For few rows every expert's chunk of rows
 streams that expert's matrices once (``ops.moe_expert_product``, the gated unit in the first product's epilogue): no
 integer leaves the device, so decode steps can be recorded.  For many rows the host reads the experts' row counts and
-runs one library product per expert and matrix over its run of rows.
+runs one product per expert and matrix over its run of rows.
 """
 import torch
 
