@@ -69,6 +69,22 @@ IC_EXPORT int ic_attn_mixed_supported(int dtype, int nh, int nkvh, int dh, int p
            (page_size & (page_size - 1)) == 0 && bt_stride > 0 && bt_stride <= kDecMaxPages && bt_stride <= kPfMaxPages;
 }
 
+// Into how many parts the tiles' walks are cut here, and key tiles per part: as ic_attn_prefill_parts_of_step says for tiles alone, and in two where it
+// leaves walks of 12 key tiles and more whole with up to 1.25 blocks a unit, since there two wave groups share such a walk and here there is one.
+// Whole against two parts, 40 rows of 100..2,048 keys beside portions of 512 and 463 after 512: 24:8 heads of 64 25.9 -> 25.2 us, 36:36 62.9 -> 60.0,
+// 32:2 of 128 41.3 -> 39.4; 6 rows beside a prompt of 1,200: 23.2 -> 20.4, 28.8 -> 24.7, 37.7 -> 36.8.  With 1.5 blocks a unit (32:32 of 128,
+// portions of 700 after 600 and 100) 42.1 -> 44.4.
+IC_EXPORT int ic_attn_mixed_parts_of_step(int dtype, int n_tiles, int nh, int dh, int max_tile_position, int window, int compute_units, int* part_len) {
+    int len = 0, parts = ic_attn_prefill_parts_of_step(dtype, n_tiles, nh, dh, max_tile_position, window, compute_units, &len);
+    const long long blocks = (long long)n_tiles * nh;
+    if (dtype == IC_BF16 && parts == 1 && len >= 12 && blocks > 0 && blocks <= kPfCounters && (dh == 64 || dh == 128) && 4 * blocks <= 5LL * compute_units) {
+        parts = 2;
+        len = (len + 1) / 2;
+    }
+    if (part_len) *part_len = len;
+    return parts;
+}
+
 IC_EXPORT int ic_attn_mixed(const void* q, int q_stride, void* out, int out_stride, int dtype, const void* kcache, const void* vcache,
                             const int* block_tables, int bt_stride, const int* tok_list, const int* token_req, const int* positions, float* part_acc,
                             float* part_ml, int n_tok, int nsplit, const int* tiles, int n_tiles, int nh, int nkvh, int dh, int page_size, float scale,

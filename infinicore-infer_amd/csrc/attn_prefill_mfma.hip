@@ -80,10 +80,10 @@ IC_EXPORT int ic_attn_prefill_parts(int n_tiles, int nh, int dh, int max_keys, i
     return parts;
 }
 
-// The same question for a step: its largest position and the mixer's window (0: none) give the most keys a tile sees.
+// The same question for a step: the largest position of its prompt portions and the mixer's window (0: none) give the most keys a tile sees.
 // (float32 walks are never cut.)
-IC_EXPORT int ic_attn_prefill_parts_of_step(int dtype, int n_tiles, int nh, int dh, int max_position, int window, int compute_units, int* part_len) {
-    int keys = max_position + 1;
+IC_EXPORT int ic_attn_prefill_parts_of_step(int dtype, int n_tiles, int nh, int dh, int max_tile_position, int window, int compute_units, int* part_len) {
+    int keys = max_tile_position + 1;
     if (dtype != IC_BF16) {
         if (part_len) *part_len = (keys + kPfKeys - 1) / kPfKeys;
         return 1;

@@ -102,9 +102,9 @@ IC_EXPORT int ic_rule_attention(int dtype, int head_dim, int page_size, int n_de
 // tokens 44.2 -> 32.0 (87.6 -> 82.1, 45.1 -> 38.9).  Not where few tiles with long walks would take two wave groups each, which the common kernel does
 // not have: 2 rows beside a portion of 700 after 2,500 (32:2 of 128) 71.2 -> 77.2.
 IC_EXPORT int ic_rule_attention_together(int dtype, int nh, int nkvh, int head_dim, int page_size, int table_stride, int n_decode_rows, int n_tiles,
-                                         int max_position, int window, int parts, int compute_units) {
+                                         int max_tile_position, int window, int parts, int compute_units) {
     if (n_decode_rows <= 0 || n_tiles <= 0 || !ic_attn_mixed_supported(dtype, nh, nkvh, head_dim, page_size, table_stride)) return 0;
-    const int keys = window > 0 ? std::min(max_position + 1, window + ic_attn_prefill_tile_rows()) : max_position + 1;
+    const int keys = window > 0 ? std::min(max_tile_position + 1, window + ic_attn_prefill_tile_rows()) : max_tile_position + 1;
     const bool two_groups = parts <= 1 && (long long)n_tiles * nh <= 2LL * (compute_units > 0 ? compute_units : 256);
     return !(two_groups && keys >= 24 * 64);
 }
@@ -147,10 +147,20 @@ struct IcDecoder {
         return split_answer;
     }
 
+    // The largest position of the prompt portions: a long chat that brings one token does not lengthen the tiles' walks.  With the whole step's in its
+    // place parts are too long and too few: 16 chats of 1,073..8,000 keys beside 512 tokens after 2,000 (24:8 heads of 64) 41.6 -> 62.8 us, 12 of up to
+    // 3,000 beside 500 after 400 27.6 -> 31.4; and steps that run best in one launch do not (32:2 of 128, 8 of up to 9,000 beside 700 and 90: 33.1 -> 40.6).
+    // It costs up to 3 % where walks of 40 key tiles of 128 do better in two parts than in four (16 chats of up to 8,000 beside 512 after 2,000: 170 -> 175).
+    static int tiles_end(const IcStepBatch& b) { return b.max_tile_position > 0 ? b.max_tile_position : b.max_position; }
     // into how many parts the walks of a step's prompt tiles are cut (1: not at all), and key tiles per part
     int tile_parts_for(const IcStepBatch& b, const IcAttention& a, int* part_len) const {
         if (!meta.attention_counters) { if (part_len) *part_len = 0; return 1; }     // no counters: no cut
-        return ic_attn_prefill_parts_of_step(meta.dtype, b.n_prefill_tiles, a.n_heads, a.head_dim, b.max_position, a.window, meta.compute_units, part_len);
+        return ic_attn_prefill_parts_of_step(meta.dtype, b.n_prefill_tiles, a.n_heads, a.head_dim, tiles_end(b), a.window, meta.compute_units, part_len);
+    }
+    // the same where they run beside the step's single tokens
+    int mixed_parts_for(const IcStepBatch& b, const IcAttention& a, int* part_len) const {
+        if (!meta.attention_counters) { if (part_len) *part_len = 0; return 1; }
+        return ic_attn_mixed_parts_of_step(meta.dtype, b.n_prefill_tiles, a.n_heads, a.head_dim, tiles_end(b), a.window, meta.compute_units, part_len);
     }
 
     Workspace layout(const IcStepBatch& b) const {
@@ -193,7 +203,7 @@ struct IcDecoder {
         if (meta.dtype == IC_BF16 && b.n_prefill_tiles > 0)
             for (const IcLayer& l : layers) {
                 int len = 0;
-                const int p = tile_parts_for(b, l.attention, &len);
+                const int p = std::max(tile_parts_for(b, l.attention, &len), b.n_decode_rows > 0 ? mixed_parts_for(b, l.attention, &len) : 1);
                 cut = std::max(cut, (size_t)ic_attn_prefill_scratch_floats(b.n_prefill_tiles, l.attention.n_heads, l.attention.head_dim, p));
             }
         w.tile_parts = take(cut * 4);
@@ -319,9 +329,11 @@ struct IcDecoder {
                 st = ic_attn_generic(qkv, width, attn_out, ow, dt, e.k_cache, e.v_cache, tables, bts, b.token_req, b.positions, T,
                                      A.n_heads, A.n_kv_heads, A.head_dim, ps, A.softmax_scale, A.window, stream);
                 if (st) return fail(st, "attention (general kernel)", i);
-            } else if (int part_len = 0, parts = use_dec && use_pre && decode_rows ? tile_parts_for(b, A, &part_len) : 0;
-                       parts > 0 && ic_rule_attention_together(dt, A.n_heads, A.n_kv_heads, A.head_dim, ps, bts, n_dec, n_tiles, b.max_position, A.window,
-                                                               parts, meta.compute_units)) {
+            } else if (use_dec && use_pre && decode_rows &&
+                       ic_rule_attention_together(dt, A.n_heads, A.n_kv_heads, A.head_dim, ps, bts, n_dec, n_tiles, tiles_end(b), A.window,
+                                                  tile_parts_for(b, A, nullptr), meta.compute_units)) {
+                int part_len = 0;
+                const int parts = mixed_parts_for(b, A, &part_len);
                 st = ic_attn_mixed(qkv, width, attn_out, ow, dt, e.k_cache, e.v_cache, tables, bts, decode_rows, b.token_req, b.positions,
                                    (float*)(base + ws.part_acc), (float*)(base + ws.part_ml), n_dec, splits_for(b, A), b.prefill_tiles, n_tiles, A.n_heads,
                                    A.n_kv_heads, A.head_dim, ps, A.softmax_scale, A.window, parts, part_len, (float*)(base + ws.tile_parts),
@@ -618,7 +630,7 @@ IC_EXPORT int ic_decoder_pack(const IcDecoder* decoder, const IcHostBatch* batch
     std::vector<Tile> tiles;
     dec.reserve(h.n_decode);
     tiles.reserve(h.n_tiles);
-    int row0 = 0, w = 0, max_pos = 0, max_ctx = 0;
+    int row0 = 0, w = 0, max_pos = 0, max_tile = 0, max_ctx = 0;
     const int* want = b.want;
     bool identity = h.n_want == b.n_tokens;
     for (int r = 0; r < R; ++r) {
@@ -636,7 +648,10 @@ IC_EXPORT int ic_decoder_pack(const IcDecoder* decoder, const IcHostBatch* batch
         }
         want += nw;
         if (n == 1) { dec.push_back(Row{p0, row0}); max_ctx = std::max(max_ctx, p0 + 1); }
-        else for (int o = 0; o < n; o += b.tile_rows) tiles.push_back(Tile{r, row0 + o, std::min(b.tile_rows, n - o), p0 + o});
+        else {
+            for (int o = 0; o < n; o += b.tile_rows) tiles.push_back(Tile{r, row0 + o, std::min(b.tile_rows, n - o), p0 + o});
+            max_tile = std::max(max_tile, p0 + n - 1);
+        }
         max_pos = std::max(max_pos, p0 + n - 1);
         for (int g = 0; g < decoder->meta.n_groups; ++g) {
             const int* table = b.tables[g * R + r];
@@ -662,6 +677,7 @@ IC_EXPORT int ic_decoder_pack(const IcDecoder* decoder, const IcHostBatch* batch
     s.want_rows_identity = identity ? 1 : 0;
     s.decode_rows_identity = (int)dec.size() == b.n_tokens ? 1 : 0;
     s.max_position = max_pos;
+    s.max_tile_position = max_tile;
     s.max_context = max_ctx ? ic_rule_context_bucket(max_ctx) : 0;
     s.fixed_decode_splits = b.fixed_decode_splits;
     s.tokens = device_ints + h.tokens; s.positions = device_ints + h.positions; s.token_req = device_ints + h.token_req;

@@ -110,6 +110,7 @@ typedef struct {
     const int* group_slots[IC_MAX_CACHE_GROUPS];    // per group: [n_tokens] cache slot (page * page_size + offset) of each token
     const int* group_tables[IC_MAX_CACHE_GROUPS];   // per group: [n_requests, group_table_stride] logical page -> page id
     int group_table_stride[IC_MAX_CACHE_GROUPS];
+    int max_tile_position;   // largest position in the prompt portions (0: not told, max_position stands for it); how their walks over the keys run
 } IcStepBatch;
 
 // A step's batch as host arrays, in the shape of inferBatch (jiuge.h:89-110).
@@ -183,8 +184,9 @@ int ic_rule_attention(int dtype, int head_dim, int page_size, int n_decode_rows,
 // of lengths and splits as an eager one does: to a power of two up to 1,024 (at least 256), above that to a multiple of
 // a quarter of the power of two below (2,560, 3,072, 3,584, 4,096, 5,120 ...).
 int ic_rule_context_bucket(int n_keys);
-// 1: the single tokens and the prompt tiles of a mixed step run in one launch (ic_attn_mixed); parts: into how many the tiles' walks are cut.
-int ic_rule_attention_together(int dtype, int nh, int nkvh, int head_dim, int page_size, int table_stride, int n_decode_rows, int n_tiles, int max_position, int window, int parts, int compute_units);
+// 1: the single tokens and the prompt tiles of a mixed step run in one launch (ic_attn_mixed); parts: into how many the tiles' walks are cut when they run alone;
+// max_tile_position: the largest position in the prompt portions.
+int ic_rule_attention_together(int dtype, int nh, int nkvh, int head_dim, int page_size, int table_stride, int n_decode_rows, int n_tiles, int max_tile_position, int window, int parts, int compute_units);
 
 // How many ways to split the keys of single-token rows (from sweeps on MI355X with caches that do not fit the
 // last-level cache); see the decode attention kernel.  elem_bytes: of a cache element.  matrix_cores: 1 when the

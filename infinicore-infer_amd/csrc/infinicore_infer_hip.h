@@ -72,11 +72,12 @@ int ic_attn_prefill_groups(const void* q, int q_stride, void* out, int out_strid
 long long ic_attn_prefill_scratch_floats(int n_tiles, int nh, int dh, int parts);
 int ic_attn_prefill_counter_ints();
 int ic_attn_prefill_parts(int n_tiles, int nh, int dh, int max_keys, int compute_units, int* part_len);
-int ic_attn_prefill_parts_of_step(int dtype, int n_tiles, int nh, int dh, int max_position, int window, int compute_units, int* part_len);   // max_keys from the step's largest position and the window
+int ic_attn_prefill_parts_of_step(int dtype, int n_tiles, int nh, int dh, int max_tile_position, int window, int compute_units, int* part_len);   // max_keys from where the step's portions end and the window
 int ic_attn_prefill_split(const void* q, int q_stride, void* out, int out_stride, int dtype, const void* kcache, const void* vcache, const int* block_tables, int bt_stride, const int* tiles, int n_tiles, int nh, int nkvh, int dh, int page_size, float scale, int window, int groups, int parts, int part_len, float* scratch, long long scratch_floats, int* counters, hipStream_t stream);
 // A mixed step's attention in one launch: the single tokens of ic_attn_decode beside the prompt tiles of ic_attn_prefill_split (one
 // group), arguments as there; tok_list is needed.  Pages a power of two from 64 on.  With several splits the second pass follows (ic_attn_decode_merge).
 int ic_attn_mixed_supported(int dtype, int nh, int nkvh, int dh, int page_size, int bt_stride);
+int ic_attn_mixed_parts_of_step(int dtype, int n_tiles, int nh, int dh, int max_tile_position, int window, int compute_units, int* part_len);   // as ic_attn_prefill_parts_of_step
 int ic_attn_mixed(const void* q, int q_stride, void* out, int out_stride, int dtype, const void* kcache, const void* vcache, const int* block_tables, int bt_stride, const int* tok_list, const int* token_req, const int* positions, float* part_acc, float* part_ml, int n_tok, int nsplit, const int* tiles, int n_tiles, int nh, int nkvh, int dh, int page_size, float scale, int window, int parts, int part_len, float* scratch, long long scratch_floats, int* counters, hipStream_t stream);
 int ic_attn_decode_merge(const float* part_acc, const float* part_ml, const int* tok_list, void* out, int out_stride, int dtype, int n_tok, int nh, int dh, int nsplit, hipStream_t stream);
 

@@ -112,12 +112,17 @@ class StepContext:
         self.req_ids: List[object] = []
         self.host_state_slots: List[int] = []
         self.max_position = 0            # largest position in the step
+        self.max_tile_position = 0       # largest position in the prompt portions (0: not told)
         self.max_context = 0             # most keys any single-token row sees
         self.cu_count = 256              # compute units of the device, for the parts' launch heuristics
         self.fixed_decode_splits: Optional[int] = None   # a recorded step's fixed way of splitting single-token rows' keys
         self.memo: Dict[str, object] = {}  # scratch of the parts for this step (what several layers would work out alike)
         self.group_views = []            # per cache group: (slots int32 [T], block tables int32 [R, max_blocks])
         self._views: Dict[int, LayerCacheView] = {}
+
+    def tiles_end(self) -> int:
+        """The largest position of the prompt portions, which their walks over the keys reach."""
+        return self.max_tile_position or self.max_position
 
     def cache_view(self, entry) -> LayerCacheView:
         v = self._views[entry.cache]

@@ -528,6 +528,7 @@ class Engine:
         ctx.req_ids = [e.req_id for e in entries]
         ctx.host_state_slots = state_slots
         ctx.max_position = max(p0 + n - 1 for p0, n in zip(starts, lens))
+        ctx.max_tile_position = tiles[0][3] + tiles[0][2] - 1 if tiles else 0      # (they are sorted)
         ctx.max_context = _context_bucket(max_ctx) if max_ctx else 0
         ctx.cu_count = self.cu_count
         group_views = [(view("slots%d" % g), view("tables%d" % g).view(R, group_maxb[g])) for g in range(n_groups)]

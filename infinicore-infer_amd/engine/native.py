@@ -146,7 +146,7 @@ class NativeDecoder:
         b.n_tokens, b.n_requests, b.n_want = ctx.T, ctx.R, ctx.n_want
         b.n_decode_rows, b.n_prefill_tiles = ctx.n_decode_rows, ctx.n_prefill_tiles
         b.want_rows_identity, b.decode_rows_identity = int(ctx.want_rows_identity), int(ctx.decode_rows_identity)
-        b.max_position, b.max_context = ctx.max_position, ctx.max_context
+        b.max_position, b.max_tile_position, b.max_context = ctx.max_position, ctx.max_tile_position, ctx.max_context
         b.fixed_decode_splits = ctx.fixed_decode_splits or 0
         b.tokens, b.positions, b.token_req = ctx.tokens.data_ptr(), ctx.positions.data_ptr(), ctx.token_req.data_ptr()
         b.want_rows = ctx.want_rows.data_ptr() if ctx.n_want else None

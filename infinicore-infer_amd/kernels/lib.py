@@ -76,7 +76,7 @@ class IcStepBatch(_c.Structure):
                 ("want_rows_identity", _I), ("decode_rows_identity", _I), ("max_position", _I), ("max_context", _I),
                 ("fixed_decode_splits", _I), ("tokens", _P), ("positions", _P), ("token_req", _P), ("want_rows", _P),
                 ("decode_rows", _P), ("prefill_tiles", _P), ("group_slots", _P * MAX_CACHE_GROUPS),
-                ("group_tables", _P * MAX_CACHE_GROUPS), ("group_table_stride", _I * MAX_CACHE_GROUPS)]
+                ("group_tables", _P * MAX_CACHE_GROUPS), ("group_table_stride", _I * MAX_CACHE_GROUPS), ("max_tile_position", _I)]
 
 
 class IcHostBatch(_c.Structure):
@@ -114,6 +114,7 @@ _SIGNATURES = {
     "ic_attn_prefill_parts": [_I, _I, _I, _I, _I, _c.POINTER(_I)],
     "ic_attn_prefill_parts_of_step": [_I, _I, _I, _I, _I, _I, _I, _c.POINTER(_I)],
     "ic_attn_prefill_split": [_P, _I, _P, _I, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _F, _I, _I, _I, _I, _P, _LL, _P, _P],
+    "ic_attn_mixed_parts_of_step": [_I, _I, _I, _I, _I, _I, _I, _c.POINTER(_I)],
     "ic_attn_mixed_supported": [_I, _I, _I, _I, _I, _I],
     "ic_attn_mixed": [_P, _I, _P, _I, _I, _P, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _P, _I, _I, _I, _I, _I, _F, _I, _I, _I, _P, _LL, _P, _P],
     "ic_attn_decode_merge": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],

@@ -270,13 +270,22 @@ def attention_prefill_parts(n_tiles: int, n_heads: int, head_dim: int, max_keys:
     return int(parts), int(part_len.value)
 
 
-def attention_prefill_parts_of_step(dtype, n_tiles: int, n_heads: int, head_dim: int, max_position: int, window: int, compute_units: int):
-    """(parts, part_len) for a step whose largest position is ``max_position`` under a mixer's ``window`` (0: none);
+def attention_prefill_parts_of_step(dtype, n_tiles: int, n_heads: int, head_dim: int, max_tile_position: int, window: int, compute_units: int):
+    """(parts, part_len) for a step whose prompt portions end at ``max_tile_position`` under a mixer's ``window`` (0: none);
     float32 walks are never cut."""
+    return _parts_of_step(get_lib().ic_attn_prefill_parts_of_step, dtype, n_tiles, n_heads, head_dim, max_tile_position, window, compute_units)
+
+
+def attention_mixed_parts_of_step(dtype, n_tiles: int, n_heads: int, head_dim: int, max_tile_position: int, window: int, compute_units: int):
+    """The same for portions that run beside single tokens (attention_mixed)."""
+    return _parts_of_step(get_lib().ic_attn_mixed_parts_of_step, dtype, n_tiles, n_heads, head_dim, max_tile_position, window, compute_units)
+
+
+def _parts_of_step(entry, dtype, n_tiles, n_heads, head_dim, max_tile_position, window, compute_units):
     import ctypes
     part_len = ctypes.c_int(0)
-    parts = get_lib().ic_attn_prefill_parts_of_step(dtype_code(dtype), int(n_tiles), int(n_heads), int(head_dim), int(max_position), int(window or 0),
-                                                    int(compute_units), ctypes.byref(part_len))
+    parts = entry(dtype_code(dtype), int(n_tiles), int(n_heads), int(head_dim), int(max_tile_position), int(window or 0), int(compute_units),
+                  ctypes.byref(part_len))
     return int(parts), int(part_len.value)
 
 
@@ -459,10 +468,10 @@ def rule_attention(dtype, head_dim: int, page_size: int, n_decode_rows: int, n_t
 
 
 def rule_attention_together(dtype, n_heads: int, n_kv_heads: int, head_dim: int, page_size: int, table_stride: int, n_decode_rows: int, n_tiles: int,
-                            max_position: int, window: int, parts: int, compute_units: int) -> bool:
-    """True when a mixed step's single tokens and prompt tiles run in one launch (attention_mixed)."""
+                            max_tile_position: int, window: int, parts: int, compute_units: int) -> bool:
+    """True when a mixed step's single tokens and prompt tiles run in one launch (attention_mixed); max_tile_position: where the portions end."""
     return bool(get_lib().ic_rule_attention_together(dtype_code(dtype), int(n_heads), int(n_kv_heads), int(head_dim), int(page_size), int(table_stride),
-                                                     int(n_decode_rows), int(n_tiles), int(max_position), int(window or 0), int(parts),
+                                                     int(n_decode_rows), int(n_tiles), int(max_tile_position), int(window or 0), int(parts),
                                                      int(compute_units)))
 
 

@@ -143,17 +143,22 @@ class Attention(Mixer):
             part_acc = ctx.ws.buffer("attn_part_acc", (n_dec * self.nh * n_split * self.dh,), torch.float32)
             part_ml = ctx.ws.buffer("attn_part_ml", (n_dec * self.nh * n_split * 2,), torch.float32)
             single = (None if ctx.decode_rows_identity else ctx.decode_rows, n_dec, ctx.token_req, ctx.positions, part_acc, part_ml)
+        together = False
         if use_pre:
             # few blocks and long walks over the keys: the tiles' walks are cut into parts (the library's rule)
-            parts, part_len = ops.attention_prefill_parts_of_step(rt.dtype, n_tiles, self.nh, self.dh, ctx.max_position, self.window, ctx.cu_count)
+            step = (rt.dtype, n_tiles, self.nh, self.dh, ctx.tiles_end(), self.window, ctx.cu_count)
+            parts, part_len = ops.attention_prefill_parts_of_step(*step)
+            together = bool(single and single[0] is not None and ops.rule_attention_together(
+                rt.dtype, *args, cache.block_tables.stride(0), n_dec, n_tiles, ctx.tiles_end(), self.window, parts, ctx.cu_count))
+            if together:
+                parts, part_len = ops.attention_mixed_parts_of_step(*step)
             scratch = counters = None
             if parts > 1:
                 scratch = ctx.ws.buffer("attn_tile_parts", (ops.attention_prefill_scratch_floats(n_tiles, self.nh, self.dh, parts),),
                                         torch.float32)
                 counters = ctx.ws.zeroed("attn_tile_arrivals", (ops.attention_prefill_counter_ints(),), torch.int32)
             tiles = dict(parts=parts, part_len=part_len, scratch=scratch, counters=counters)
-        if single and tiles and single[0] is not None and ops.rule_attention_together(
-                rt.dtype, *args, cache.block_tables.stride(0), n_dec, n_tiles, ctx.max_position, self.window, parts, ctx.cu_count):
+        if together:
             ops.attention_mixed(q, out, cache.k, cache.v, cache.block_tables, *single, n_split, ctx.prefill_tiles, n_tiles, *args, self.scale,
                                 self.window, **tiles)
             return

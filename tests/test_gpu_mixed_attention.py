@@ -19,6 +19,55 @@ def test_rule_cpu():
     assert rule(parts=1, tiles=40, pos=3199)
 
 
+def _packed(lens, starts, page_size=64, nh=32, nkv=2, dh=128):
+    """The description of a step of requests with `lens` new tokens from `starts` on, as the C packer lays it out (host code only)."""
+    import ctypes
+    import numpy as np
+    from infinicore_infer_amd.kernels.lib import IcDecoderMeta, IcHostBatch, IcLayer, IcRunEntry, IcStepBatch
+    lib, room = get_lib(), ctypes.create_string_buffer(64)
+    at = ctypes.addressof(room)
+    layer, entry, meta = IcLayer(), IcRunEntry(k_cache=at, v_cache=at, writes_cache=1), IcDecoderMeta()
+    a = layer.attention
+    a.n_heads, a.n_kv_heads, a.head_dim, a.w_qkv, a.w_o = nh, nkv, dh, at, at
+    layer.mixer_norm.weight = layer.ffn_norm.weight = at
+    layer.ffn.intermediate, layer.ffn.w_gate_up, layer.ffn.w_down = 128, at, at
+    meta.dtype, meta.hidden, meta.vocab, meta.page_size, meta.n_layers, meta.n_entries, meta.n_groups = 1, nh * dh, 64, page_size, 1, 1, 1
+    meta.embed_table = meta.head_weight = meta.final_norm.weight = meta.final_norm_scaled = at
+    dec = lib.ic_decoder_create(ctypes.byref(meta), ctypes.byref(layer), ctypes.byref(entry))
+    assert dec, lib.ic_decoder_create_error()
+    try:
+        i32 = lambda x: np.asarray(x, dtype=np.int32)
+        toks, ln, st, want = i32([1] * sum(lens)), i32(lens), i32(starts), i32([0] * len(lens))
+        tables = [i32(range((s + n + page_size - 1) // page_size)) for n, s in zip(lens, starts)]
+        ptrs, tlen = (ctypes.c_void_p * len(lens))(*[t.ctypes.data for t in tables]), i32([len(t) for t in tables])
+        hb = IcHostBatch(len(toks), len(lens), toks.ctypes.data, ln.ctypes.data, st.ctypes.data, want.ctypes.data, None,
+                         ctypes.cast(ptrs, ctypes.c_void_p), tlen.ctypes.data, lib.ic_attn_prefill_tile_rows(), 0)
+        n = lib.ic_decoder_step_ints(dec, ctypes.byref(hb))
+        staging, out = np.zeros(n, dtype=np.int32), IcStepBatch()
+        assert lib.ic_decoder_pack(dec, ctypes.byref(hb), staging.ctypes.data, staging.ctypes.data, n, ctypes.byref(out)) == 0
+        return out
+    finally:
+        lib.ic_decoder_destroy(dec)
+
+
+def test_long_chats_beside_short_prompts_cpu():
+    """How far the prompt tiles walk is told apart from how far the single tokens do: 60 rows of up to 3,000 keys beside portions that
+    end at position 699 (32:2 heads of 128) measured 45.1 us apart and 38.9 together."""
+    b = _packed([1] * 60 + [600, 200, 50], [3000 - 40 * i for i in range(60)] + [100, 0, 0])
+    assert (b.n_decode_rows, b.n_prefill_tiles, b.max_position, b.max_tile_position) == (60, 8, 3000, 699)
+    parts, _ = ops.attention_prefill_parts_of_step(BF16, b.n_prefill_tiles, 32, 128, b.max_tile_position, 0, 256)
+    together = lambda end: ops.rule_attention_together(BF16, 32, 2, 128, 64, 47, b.n_decode_rows, b.n_prefill_tiles, end, 0, parts, 256)
+    assert parts == 1 and together(b.max_tile_position) and not together(b.max_position)
+    assert _packed([1, 1], [5, 700]).max_tile_position == 0
+    # a walk that the tiles alone leave whole is cut in two here from 12 key tiles on, while the blocks are few enough for it
+    cut = lambda nh, dh, tiles, end, entry=ops.attention_mixed_parts_of_step: entry(BF16, tiles, nh, dh, end, 0, 256)
+    alone = ops.attention_prefill_parts_of_step
+    assert cut(24, 64, 8, 1023, alone)[0] == 1 and cut(24, 64, 8, 1023) == (2, 8) and cut(32, 128, 10, 767) == (2, 6)
+    assert cut(24, 64, 8, 703) == cut(24, 64, 8, 703, alone) == (1, 11) and cut(32, 128, 11, 1023)[0] == 1
+    assert cut(24, 64, 4, 1023) == cut(24, 64, 4, 1023, alone) and cut(24, 64, 4, 1023)[0] == 3
+    assert _packed([300, 1], [2000, 7]).max_tile_position == 2299
+
+
 def _case(nh, nkv, dh, ps, held, portions, window, n_split, parts, part_len):
     g = torch.Generator().manual_seed(nh + dh + len(held))
     lens = [p + 1 for p in held] + [a + b for a, b in portions]
@@ -86,3 +135,25 @@ def test_refused_arguments():
     for bad, status in ((dict(dt=0), -2), (dict(dh=80), -2), (dict(ps=32), -2), (dict(bts=2000), -2), (dict(rows=None), -1), (dict(n=0), -1),
                         (dict(nt=0), -1), (dict(ns=65), -1), (dict(q=p + 2), -1), (dict(parts=2, plen=4), -1), (dict(ns=2, acc=None), -1)):
         assert lib.ic_attn_mixed(*dict(good, **bad).values()) == status, bad
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("native", [True, False])
+def test_both_step_paths_ask_with_the_portions_end(native, tmp_path_factory, monkeypatch):
+    import helpers as H
+    from infinicore_infer_amd.engine import Engine, StepEntry
+    folder = H.make_model_dir(tmp_path_factory.getbasetemp(), "C")
+    eng = Engine.from_dir(folder, dtype=BF16, max_tokens=1024, page_size=64, max_requests=4, use_native=native)
+    vocab = H.CONFIGS["C"][0]["vocab_size"]
+    eng.step([StepEntry("a", H.random_tokens(vocab, 400, 1), [399])])
+    seen = []
+    build = Engine._build_context
+    monkeypatch.setattr(Engine, "_build_context", lambda self, *a: seen.append(build(self, *a)) or seen[-1])
+    rule = ops.rule_attention_together
+    asked = []
+    monkeypatch.setattr(ops, "rule_attention_together", lambda *a: asked.append(a[8]) or rule(*a))
+    eng.step([StepEntry("a", [5], [0]), StepEntry("b", H.random_tokens(vocab, 70, 2), [69])])
+    if native:
+        assert eng.native is not None and (eng.native._batch.max_position, eng.native._batch.max_tile_position) == (400, 69)
+    else:
+        assert seen[-1].max_position == 400 and seen[-1].max_tile_position == 69 and asked and set(asked) == {69}
