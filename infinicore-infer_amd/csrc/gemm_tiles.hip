@@ -509,17 +509,19 @@ IC_EXPORT int ic_gemm_tiles_rope_supported(const void* A, const void* W, const v
 
 // Whether the own kernel is the faster one: its cost against what the library's product (and the kernel that follows it, where the epilogue has that) would
 // take.  The library's times jump between neighbouring sizes, so the lines are fitted to 3,900 timed products with weights out of memory (150 pairs of N in
-// 64..32,768 and K in 64..16,384, 33..16,384 rows; the library's first choice of algorithm).  What they choose loses 1.6 % to the faster of the two on
-// average and is over 3 % slower than the library in 3.3 % of the products, over 10 % in 1.0 % (the own kernel everywhere: 3.4 % lost, the library everywhere:
-// 38 %):
-//   up to 512 rows the library splits K over the chip where K is a multiple of 256: about 11 us, the weights and the products at the rates below, however
+// 64..32,768 and K in 64..16,384, 33..16,384 rows; the library's first choice of algorithm).  What they choose loses 1.4 % to the faster of the two on
+// average and is over 3 % slower than the library in 3.7 % of the products, over 10 % in 0.8 % (the own kernel everywhere: 3.3 % lost, the library everywhere:
+// 39 %):
+//   up to 64 rows the library splits K over the chip where K is a multiple of 256: about 11 us, the weights and the products at the rates below, however
 //   long K is, while the own kernel's walk grows with K.  64 x 4,096 x 14,336: 40 us against 52, 48 x 2,048 x 11,264: 20 against 36; on this side of
-//   the line 64 x 2,304 x 2,304: 9.9 -> 7.4, 256 x 1,536 x 3,840: 14.4 -> 10.3.  Other K it does not split, or badly (33 x 2,304 x 5,760: 25.4 -> 17.4, 64 x 128 x
-//   5,248: 18 -> 12.4), and there, and with more rows, only walks far beyond a split over the whole chip go to it (576 x 64 x 14,784: 20 against 31);
+//   the line 64 x 2,304 x 2,304: 9.9 -> 7.4.  Other K it does not split, or badly (33 x 2,304 x 5,760: 25.4 -> 17.4);
+//   there, and up to 512 rows, where its times jump most (4,096 x 16,384: 50 us for 65 rows, 69 for 96, 93 for 160, 65 for 256; own 42, 45, 67, 72), only walks far
+//   beyond a split over the whole chip go to it (256 x 256 x 16,384: 17 against 30; on this side 256 x 1,536 x 3,840: 14.4 -> 10.3);
 //   more rows: where its 256 x 256 tiles, which spend some 6 % less on a stage than the own ones, fit about as well as the own best tile: whole tiles of
 //   columns, K of 1,024 and more (shorter walks are mostly the way out), no ragged last round behind more than four (16,384 x 4,608 x 4,096: 556 -> 452)
 //   (8,192 x 4,096 x 14,336: 615 us against 704; 2,048 x 6,912 x 2,304: 51 against 58; else 1,045 x 2,560 x 1,536: 16.9 -> 12.1, 2,048 x 2,304 x 2,304: 28.0 -> 23.1).
-// The gated unit in the epilogue saves its kernel, 3 us and more, and pays from 33 rows on but for long K as above (48 x 2,048 x 12,288: 24 us against 39; else
+// The gated unit in the epilogue saves its kernel, 3 us and more, and pays from 33 rows on but for long K as above (48 x 2,048 x 12,288: 24 us against 39) and for
+// 190 MB of weights and more in rows of 12 KB and more, which few row tiles read more slowly than the library (96 x 16,384 x 6,144: 54 against 67; else
 // 1,045 x 7,680 x 1,536: 42.8 -> 28.0; 2,048 x 11,520 x 2,304: 130 -> 98; 16,384 x 32,768 x 4,096: 3,195 -> 3,007).  So does rotary and cache write behind QKV
 // (64 rows of the 2B shape 18.3 -> 12.5, 1,045 rows of the 1B shape 21.5 -> 15.5, 2,048 of the 8B shape 78.6 -> 69.6), but for sizes that the largest tile
 // fits best, which this epilogue does not have.
@@ -531,13 +533,11 @@ IC_EXPORT int ic_gemm_tiles_pays(int M, int N, int K, int mode) {
     if (mode == EPI_ROPE) return kCosts[best_tile(M, N, K, EPI_SWIGLU, &cost)].takes[EPI_ROPE];
     best_tile(M, N, K, mode, &cost);
     const double weights = 2.0 * N * K, products = weights * M;            // bytes, operations
-    if (M <= 512 && K % 256 == 0) {
-        const bool one = M <= 64;                                          // one row tile: the weights are read once, by the library too
-        const double read = weights / (one ? 4.6e6 : 2.5e6), unit = mode == EPI_SWIGLU ? 3.0 + 0.75e-6 * M * N : 0.0;
-        const double split = one ? 11.0 + weights / 11.1e6 + products / 4.0e9 : 11.1 + weights / 3.9e6 + products / 1.5e9;
-        return (cost > read ? cost : read) <= split + unit;
+    if (M <= 64 && K % 256 == 0) {
+        const double read = weights / 7.2e6, unit = mode == EPI_SWIGLU ? 3.0 + 0.75e-6 * M * N : 0.0;
+        if ((cost > read ? cost : read) > 11.35 + weights / 9.06e6 + products / 5.0e9 + unit) return 0;
     }
-    if (mode == EPI_SWIGLU) return 1;
+    if (mode == EPI_SWIGLU) return !(M <= 96 && K >= 6144 && K % 256 == 0 && weights >= 1.9e8);
     const double over = 6.0 + (products / 0.6e9 > weights / 4e6 ? products / 0.6e9 : weights / 4e6);
     if (M <= 512) return cost <= 1.6 * over;
     const bool whole = N % 256 == 0 && K >= 1024 && !(t > 4.0 * kUnits && fill < 0.92);

@@ -60,7 +60,8 @@ def test_tile_rule_cpu():
 @pytest.mark.parametrize("M,N,K,swiglu,library,own", [
     # microseconds of the library (swiglu: with the activation's kernel) and of the tiles, weights out of memory
     (64, 4096, 14336, False, 40.0, 52.4), (48, 4096, 16384, False, 38.9, 49.2), (48, 2048, 11264, False, 20.2, 35.6), (33, 4096, 14336, False, 34.9, 41.2),
-    (48, 2048, 12288, True, 24.3, 38.9), (64, 16384, 8192, True, 56.4, 68.2), (56, 768, 12288, False, 17.5, 39.3), (65, 5120, 13824, False, 46.7, 57.0),
+    (48, 2048, 12288, True, 24.3, 38.9), (64, 16384, 8192, True, 56.4, 68.2), (56, 768, 12288, False, 17.5, 39.3), (96, 16384, 6144, True, 54.1, 67.0),
+    (160, 4096, 16384, False, 92.9, 67.2), (65, 4096, 16384, False, 50.0, 42.4), (64, 32768, 4096, True, 64.7, 63.0),
     (2048, 6912, 2304, False, 51.4, 58.1), (4096, 7680, 1536, False, 73.3, 79.4), (8192, 4096, 14336, False, 615.5, 704.4), (576, 64, 14784, False, 19.7, 30.9),
     (33, 2304, 5760, False, 25.4, 17.4), (64, 2304, 2304, False, 9.9, 7.4), (256, 1536, 3840, False, 14.4, 10.3), (256, 2304, 2304, False, 11.5, 9.1),
     (871, 1536, 1536, False, 12.4, 9.0), (1045, 2560, 1536, False, 16.9, 12.1), (2048, 2304, 2304, False, 28.0, 23.1), (2048, 2304, 5760, False, 62.3, 59.2),
