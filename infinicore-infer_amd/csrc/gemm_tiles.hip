@@ -426,12 +426,14 @@ constexpr TileCost kCosts[kTiles] = {
 double cost_of(const TileCost& t, int M, int N, int K, int mode) {
     const long long tm = (M + t.bm - 1) / t.bm, tn = mode != EPI_BF16 ? (N / 2 + t.bn / 2 - 1) / (t.bn / 2) : (N + t.bn - 1) / t.bn;
     const double tiles = (double)(tm * tn), x = tiles / kUnits, stages = K / 64;
-    double rounds = 1.0, busy = x < 1.0 ? x : 1.0, shared = 1.0;
+    double rounds = 1.0, busy = x < 1.0 ? x : 1.0, shared = 1.0, again = 0.0;
     if (x > 1.0) {
         rounds = __builtin_ceil(x / t.blocks_per_unit);
-        if (t.blocks_per_unit > 1) shared = 1.7;
+        // tiles that share a unit have no ROUND of their own, but every further round launches, fetches and stores before and after its stages: 2.3 us
+        // (64 x 64 tiles with K = 64: 4.6 us in one round, 7.3 in two, 10.5 in three, 14.2 in five).  Without it short walks ran in many rounds of them.
+        if (t.blocks_per_unit > 1) { shared = 1.7; again = 2.3 * (rounds - 1.0); }
     }
-    const double walk = t.fixed + rounds * (t.round + stages * t.stage * (1.0 + t.full * busy) * shared);
+    const double walk = t.fixed + rounds * (t.round + stages * t.stage * (1.0 + t.full * busy) * shared) + again;
     // the weights come from memory once, and about half of them again for every further row tile (blocks of one column of tiles seldom run abreast);
     // narrow tiles of pairs read them in pieces of 32 rows and less, which memory serves more slowly (64 x 32,768 x 4,096: 83 us against 63)
     const double read = 3.0 + 2.0 * N * K * (1.0 + 0.5 * (tm < 4 ? tm - 1 : 3)) * (mode != EPI_BF16 && t.bn <= 64 ? 1.35 : 1.0) / 7e6;
@@ -519,7 +521,9 @@ IC_EXPORT int ic_gemm_tiles_rope_supported(const void* A, const void* W, const v
 //   beyond a split over the whole chip go to it (256 x 256 x 16,384: 17 against 30; on this side 256 x 1,536 x 3,840: 14.4 -> 10.3);
 //   more rows: where its 256 x 256 tiles, which spend some 6 % less on a stage than the own ones, fit about as well as the own best tile: whole tiles of
 //   columns, K of 1,024 and more (shorter walks are mostly the way out), no ragged last round behind more than four (16,384 x 4,608 x 4,096: 556 -> 452)
-//   (8,192 x 4,096 x 14,336: 615 us against 704; 2,048 x 6,912 x 2,304: 51 against 58; else 1,045 x 2,560 x 1,536: 16.9 -> 12.1, 2,048 x 2,304 x 2,304: 28.0 -> 23.1).
+//   (8,192 x 4,096 x 14,336: 615 us against 704; 2,048 x 6,912 x 2,304: 51 against 58; else 1,045 x 2,560 x 1,536: 16.9 -> 12.1, 2,048 x 2,304 x 2,304: 28.0 -> 23.1);
+//   a single stage of K in more than one round, where nothing is left to overlap with a tile's way out (3,300 x 4,096 x 64: 10.9 against 15.2; in one round
+//   the own kernel is ahead, 1,300 x 2,304 x 64: 5.7 -> 4.9).
 // The gated unit in the epilogue saves its kernel, 3 us and more, and pays from 33 rows on but for long K as above (48 x 2,048 x 12,288: 24 us against 39) and for
 // 190 MB of weights and more in rows of 12 KB and more, which few row tiles read more slowly than the library (96 x 16,384 x 6,144: 54 against 67; else
 // 1,045 x 7,680 x 1,536: 42.8 -> 28.0; 2,048 x 11,520 x 2,304: 130 -> 98; 16,384 x 32,768 x 4,096: 3,195 -> 3,007).  So does rotary and cache write behind QKV
@@ -531,13 +535,14 @@ IC_EXPORT int ic_gemm_tiles_pays(int M, int N, int K, int mode) {
     if (mode != EPI_BF16 && K > 8192 && fill >= 0.93) return 0;
     double cost = 0.0;
     if (mode == EPI_ROPE) return kCosts[best_tile(M, N, K, EPI_SWIGLU, &cost)].takes[EPI_ROPE];
-    best_tile(M, N, K, mode, &cost);
+    const TileCost& own = kCosts[best_tile(M, N, K, mode, &cost)];
     const double weights = 2.0 * N * K, products = weights * M;            // bytes, operations
     if (M <= 64 && K % 256 == 0) {
         const double read = weights / 7.2e6, unit = mode == EPI_SWIGLU ? 3.0 + 0.75e-6 * M * N : 0.0;
         if ((cost > read ? cost : read) > 11.35 + weights / 9.06e6 + products / 5.0e9 + unit) return 0;
     }
     if (mode == EPI_SWIGLU) return !(M <= 96 && K >= 6144 && K % 256 == 0 && weights >= 1.9e8);
+    if (K == 64 && (double)((M + own.bm - 1) / own.bm) * ((N + own.bn - 1) / own.bn) > kUnits * own.blocks_per_unit) return 0;
     const double over = 6.0 + (products / 0.6e9 > weights / 4e6 ? products / 0.6e9 : weights / 4e6);
     if (M <= 512) return cost <= 1.6 * over;
     const bool whole = N % 256 == 0 && K >= 1024 && !(t > 4.0 * kUnits && fill < 0.92);
