@@ -2,14 +2,17 @@
 // C[M, N] = alpha * A[M, K] W[N, K]^T through hipBLASLt.  A product's descriptors and the
 // algorithm chosen for it are kept per shape, so a call costs a table lookup and one
 // hipblasLtMatmul.  ic_matmul_tune times the algorithms the library proposes for a shape on
-// the device and keeps the fastest.  Host code only: there is no kernel in this file.
+// the device and keeps the fastest, ic_product_tune compares it with the tiles of gemm_tiles.hip as well.  Host
+// code only: there is no kernel in this file.
 //
 // hipBLASLt is column-major.  Row-major C[M, N] = A W^T is column-major C^T[N, M] =
 // (W as [K, N])^T (A as [K, M]): its matrix "A" is W with transposition, its "B" is A.
 #include "common.h"
+#include "infinicore_infer_variants.h"
 #include <hipblaslt/hipblaslt.h>
 #include <hipblaslt/hipblaslt-ext.hpp>
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <unordered_map>
 #include <vector>
@@ -154,16 +157,36 @@ IC_EXPORT int ic_matmul(const void* A, int a_dtype, const void* W, void* C, int 
     return run(*p, p->chosen, A, W, C, alpha, workspace, (size_t)workspace_bytes, stream);
 }
 
-// Times every algorithm the library proposes for this product (reps launches each, after one to warm up) on
-// `stream` and keeps the fastest, if it beats the library's first choice by 3 %, for later ic_matmul calls of the
-// same shape, and of shapes first seen later that differ only by a row count within an eighth of this one.
-// Synchronises the stream.
-// flush (may be nullptr): device memory, larger than the chip's caches, that is overwritten before every timed
-// launch, so that the operands come from memory as a model's weights do and not from the last launch's cache lines.
-// Returns the number of algorithms tried (>= 1) or an error code (< 0).
-IC_EXPORT int ic_matmul_tune(const void* A, int a_dtype, const void* W, void* C, int c_dtype, int M, int N, int K, int lda,
-                             int ldw, int ldc, void* workspace, long long workspace_bytes, void* flush, long long flush_bytes,
-                             int reps, hipStream_t stream) {
+namespace {
+
+// The time of one call as tuning measures it, in milliseconds (< 0: failed): n calls after one to warm up, `flush` overwritten before each.
+template <typename F> float time_calls(F call, int n, void* flush, long long flush_bytes, hipEvent_t e0, hipEvent_t e1, hipStream_t stream) {
+    if (call() != IC_OK) return -1.f;
+    float total = 0.f;
+    for (int r = 0; r < n; ++r) {
+        if (flush_bytes > 0 && hipMemsetAsync(flush, r & 1, (size_t)flush_bytes, stream) != hipSuccess) return -1.f;
+        hipEventRecord(e0, stream);
+        const bool ok = call() == IC_OK;
+        hipEventRecord(e1, stream);
+        float ms = 0.f;
+        if (hipEventSynchronize(e1) != hipSuccess || !ok || hipEventElapsedTime(&ms, e0, e1) != hipSuccess) return -1.f;
+        total += ms;
+    }
+    return total / n;
+}
+
+struct Events {
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+    bool ok = hipEventCreate(&e0) == hipSuccess && hipEventCreate(&e1) == hipSuccess;
+    ~Events() {
+        if (e0) hipEventDestroy(e0);
+        if (e1) hipEventDestroy(e1);
+    }
+};
+
+// ic_matmul_tune; best_ms: the time of the algorithm that is kept.
+int tune(const void* A, int a_dtype, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldw, int ldc, void* workspace,
+                long long workspace_bytes, void* flush, long long flush_bytes, int reps, hipStream_t stream, float* best_ms) {
     if (!args_ok(A, a_dtype, W, C, c_dtype, M, N, K, lda, ldw, ldc) || workspace_bytes < 0 || reps < 1 || flush_bytes < 0) return IC_ERR_ARG;
     if (!flush) flush_bytes = 0;
     std::lock_guard<std::mutex> lock(g_mu);
@@ -189,22 +212,10 @@ IC_EXPORT int ic_matmul_tune(const void* A, int a_dtype, const void* W, void* C,
             }
         }
     }
-    hipEvent_t e0, e1;
-    if (hipEventCreate(&e0) != hipSuccess) return IC_ERR_LIBRARY;
-    if (hipEventCreate(&e1) != hipSuccess) { hipEventDestroy(e0); return IC_ERR_LIBRARY; }
-    auto time_one = [&](int i, int n) -> float {            // ms per launch, < 0: failed
-        if (run(*p, i, A, W, C, 1.0f, workspace, (size_t)workspace_bytes, stream) != IC_OK) return -1.f;
-        float total = 0.f;
-        for (int r = 0; r < n; ++r) {
-            if (flush_bytes > 0 && hipMemsetAsync(flush, r & 1, (size_t)flush_bytes, stream) != hipSuccess) return -1.f;
-            hipEventRecord(e0, stream);
-            const bool ok = run(*p, i, A, W, C, 1.0f, workspace, (size_t)workspace_bytes, stream) == IC_OK;
-            hipEventRecord(e1, stream);
-            float ms = 0.f;
-            if (hipEventSynchronize(e1) != hipSuccess || !ok || hipEventElapsedTime(&ms, e0, e1) != hipSuccess) return -1.f;
-            total += ms;
-        }
-        return total / n;
+    const Events ev;
+    if (!ev.ok) return IC_ERR_LIBRARY;
+    auto time_one = [&](int i, int n) {
+        return time_calls([&] { return run(*p, i, A, W, C, 1.0f, workspace, (size_t)workspace_bytes, stream); }, n, flush, flush_bytes, ev.e0, ev.e1, stream);
     };
     // first round: one timed launch each; second round: the eight best and the first choice, reps launches each
     std::vector<std::pair<float, int>> quick;
@@ -225,11 +236,74 @@ IC_EXPORT int ic_matmul_tune(const void* A, int a_dtype, const void* W, void* C,
         if (best < 0.f || ms < best) { best = ms; best_i = i; }
     }
     if (best < 0.f) tried = 0;
-    hipEventDestroy(e0);
-    hipEventDestroy(e1);
     if (tried == 0) return IC_ERR_LIBRARY;
     // the library's own first choice stays unless another is clearly (3 %) faster: timing noise must not pick
     p->chosen = (first > 0.f && best > 0.97f * first) ? 0 : best_i;
     p->timed = true;
+    *best_ms = p->chosen == 0 ? first : best;
     return tried;
+}
+
+}  // namespace
+
+// Times every algorithm the library proposes for this product (reps launches each, after one to warm up) on
+// `stream` and keeps the fastest, if it beats the library's first choice by 3 %, for later ic_matmul calls of the
+// same shape, and of shapes first seen later that differ only by a row count within an eighth of this one.
+// Synchronises the stream.
+// flush (may be nullptr): device memory, larger than the chip's caches, that is overwritten before every timed
+// launch, so that the operands come from memory as a model's weights do and not from the last launch's cache lines.
+// Returns the number of algorithms tried (>= 1) or an error code (< 0).
+IC_EXPORT int ic_matmul_tune(const void* A, int a_dtype, const void* W, void* C, int c_dtype, int M, int N, int K, int lda,
+                             int ldw, int ldc, void* workspace, long long workspace_bytes, void* flush, long long flush_bytes,
+                             int reps, hipStream_t stream) {
+    float ms = 0.f;
+    return tune(A, a_dtype, W, C, c_dtype, M, N, K, lda, ldw, ldc, workspace, workspace_bytes, flush, flush_bytes, reps, stream, &ms);
+}
+
+// ---- products whose library algorithms were timed, against the tiles of gemm_tiles.hip ---------------------------------
+namespace {
+
+struct TimedProduct { int M, N, K, lda, ldw, ldc; bool tiles; };
+std::vector<TimedProduct> g_timed;           // one a timed shape, guarded by g_mu
+std::atomic<int> g_n_timed{0};               // (most programs time none and ask without the lock)
+
+}  // namespace
+
+IC_EXPORT void ic_product_timing(int M, int N, int K, int lda, int ldw, int ldc, int tiles) {
+    std::lock_guard<std::mutex> lock(g_mu);
+    for (TimedProduct& t : g_timed)
+        if (t.M == M && t.N == N && t.K == K && t.lda == lda && t.ldw == ldw && t.ldc == ldc) { t.tiles = tiles != 0; return; }
+    g_timed.push_back(TimedProduct{M, N, K, lda, ldw, ldc, tiles != 0});
+    g_n_timed.store((int)g_timed.size());
+}
+
+IC_EXPORT int ic_product_timed(int M, int N, int K, int lda, int ldw, int ldc) {
+    if (g_n_timed.load() == 0) return -1;
+    std::lock_guard<std::mutex> lock(g_mu);
+    const TimedProduct* from = nullptr;
+    int dist = 0;
+    for (const TimedProduct& t : g_timed) {
+        if (t.N != N || t.K != K || t.lda != lda || t.ldw != ldw || t.ldc != ldc) continue;
+        const int d = t.M > M ? t.M - M : M - t.M;
+        if (8LL * d <= t.M && (!from || d < dist)) { from = &t; dist = d; }
+    }
+    return from ? (from->tiles ? 1 : 0) : -1;
+}
+
+// As ic_matmul_tune, and where the product could run in tiles those are timed likewise: ic_product then takes, for this shape and the neighbours that
+// take the timed algorithm, the one that the rule names without timing unless the other was 3 % faster.
+IC_EXPORT int ic_product_tune(const void* A, int a_dtype, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldw, int ldc,
+                              void* workspace, long long workspace_bytes, void* flush, long long flush_bytes, int reps, hipStream_t stream) {
+    float library = 0.f;
+    const int tried = tune(A, a_dtype, W, C, c_dtype, M, N, K, lda, ldw, ldc, workspace, workspace_bytes, flush, flush_bytes, reps, stream, &library);
+    if (tried < 0 || a_dtype != IC_BF16 || c_dtype != IC_BF16 || M <= 32 || !ic_gemm_tiles_supported(M, N, K, lda, ldw, ldc, 0) ||
+        (((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) & 15)) return tried;
+    const Events ev;
+    if (!ev.ok) return tried;
+    const float tiles = time_calls([&] { return ic_gemm_tiles(A, W, C, M, N, K, lda, ldw, ldc, 0, stream); }, reps, flush, flush ? flush_bytes : 0, ev.e0,
+                                   ev.e1, stream);
+    if (tiles < 0.f) return tried;
+    const bool rule = ic_gemm_tiles_pays(M, N, K, 0) != 0;
+    ic_product_timing(M, N, K, lda, ldw, ldc, rule ? library >= 0.97f * tiles : tiles < 0.97f * library);
+    return tried + 1;
 }

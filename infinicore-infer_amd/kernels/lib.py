@@ -184,6 +184,9 @@ _SIGNATURES = {
     "ic_gemm_qkv_rope": [_P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _RF, _P],
     "ic_matmul_supported": [_I, _I],
     "ic_matmul": [_P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _P, _LL, _P],
+    "ic_product_tune": [_P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _LL, _P, _LL, _I, _P],
+    "ic_product_timed": [_I] * 6,
+    "ic_product_timing": [_I] * 7,
     "ic_matmul_tune": [_P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _LL, _P, _LL, _I, _P],
     "ic_gemm_qkv_rope_variant": [_P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _RF, _I, _P],
     "ic_gemm_rows_plan": [_I, _I, _I, _I, _I, _I, _c.POINTER(_I)],
@@ -225,7 +228,7 @@ _SIGNATURES = {
     "ic_decoder_pack": [_P, _c.POINTER(IcHostBatch), _P, _P, _LL, _c.POINTER(IcStepBatch)],
     "ic_decoder_step": [_P, _c.POINTER(IcHostBatch), _P, _P, _LL, _P, _LL, _P, _LL, _P, _c.POINTER(IcStepBatch), _P],
 }
-_RESTYPES = {"ic_decoder_create": _P, "ic_decoder_create_error": _c.c_char_p, "ic_decoder_destroy": None,
+_RESTYPES = {"ic_product_timing": None, "ic_decoder_create": _P, "ic_decoder_create_error": _c.c_char_p, "ic_decoder_destroy": None,
              "ic_decoder_last_error": _c.c_char_p, "ic_decoder_workspace_bytes": _LL, "ic_decoder_step_ints": _LL,
              "ic_peak_mfma_bf16": _LL, "ic_attn_prefill_scratch_floats": _LL}
 

@@ -627,7 +627,7 @@ def matmul_library(a, w, out, alpha: float = 1.0):
 
 
 def product(a, w, out, alpha: float = 1.0):
-    """matmul_library, or the package's own product in tiles (gemm_tiles) where that is the faster one."""
+    """matmul_library, or the package's own product in tiles (gemm_tiles) where that is the faster one (by the rule, or as product_tune found)."""
     return _matmul(get_lib().ic_product, a, w, out, alpha, "product")
 
 
@@ -685,17 +685,32 @@ def matmul_library_tune(a, w, out, reps: int = 5, flush=None) -> int:
     """Times the library's algorithms for this product's shape and keeps the fastest; returns how many it tried.
     flush: a device tensor larger than the chip's caches; it is overwritten before every timed launch, so that the
     algorithms are compared with operands that come from memory, as a model's weights do."""
-    M, N, K, ca, cc, sa, sw, so = _matmul_args(a, w, out, "matmul_library_tune")
+    return _tune(get_lib().ic_matmul_tune, a, w, out, reps, flush, "matmul_library_tune")
+
+
+def product_tune(a, w, out, reps: int = 5, flush=None) -> int:
+    """matmul_library_tune, and the product in tiles (gemm_tiles) timed against the algorithm that is kept: ``product`` then takes the
+    faster one for this shape."""
+    return _tune(get_lib().ic_product_tune, a, w, out, reps, flush, "product_tune")
+
+
+def product_timed(m: int, n: int, k: int, lda=None, ldw=None, ldc=None):
+    """What product_tune found for this shape or the nearest row count within an eighth: True the tiles, False the library, None not timed."""
+    found = get_lib().ic_product_timed(int(m), int(n), int(k), int(lda or k), int(ldw or k), int(ldc or n))
+    return None if found < 0 else bool(found)
+
+
+def _tune(entry, a, w, out, reps, flush, what):
+    M, N, K, ca, cc, sa, sw, so = _matmul_args(a, w, out, what)
     ws = _workspace(a.device)
     if flush is not None:
         _dev(a, flush)
-        _need(flush.is_contiguous(), "matmul_library_tune: flush must be contiguous")
-    n = get_lib().ic_matmul_tune(a.data_ptr(), ca, w.data_ptr(), out.data_ptr(), cc, M, N, K, sa, sw, so,
-                                 ws.data_ptr(), ws.numel(),
-                                 flush.data_ptr() if flush is not None else None,
-                                 flush.numel() * flush.element_size() if flush is not None else 0, int(reps), _stream())
+        _need(flush.is_contiguous(), what + ": flush must be contiguous")
+    n = entry(a.data_ptr(), ca, w.data_ptr(), out.data_ptr(), cc, M, N, K, sa, sw, so, ws.data_ptr(), ws.numel(),
+              flush.data_ptr() if flush is not None else None,
+              flush.numel() * flush.element_size() if flush is not None else 0, int(reps), _stream())
     if n < 0:
-        raise KernelError("matmul_library_tune failed with %d for %d x %d x %d" % (n, M, N, K))
+        raise KernelError("%s failed with %d for %d x %d x %d" % (what, n, M, N, K))
     return n
 
 

@@ -20,7 +20,7 @@ torch.backends.cudnn.allow_tf32 = False
 # Which product runs where (own kernel up to some rows, slices over K for the projections into the residual
 # stream, the library beyond) is the kernel library's rule, asked through ops.rule_*: its native step function
 # asks the same functions, so the two ways of issuing a step choose alike.
-TUNE_LIBRARY = False   # while True, every library product times the library's algorithms for its shape first
+TUNE_LIBRARY = False   # while True, every product of many rows first times the library's algorithms for its shape, and the tiles against them
 TUNE_FLUSH = None      # while tuning: a tensor larger than the caches, overwritten before every timed launch
 # Products with a side (N or K) below this keep the library's first choice: timing compares speed alone, and among the
 # algorithms the library lists as taking a product with K = 64 one was met that is fastest and returns NaN.  Products this
@@ -33,11 +33,11 @@ def _library(x, w, out, alpha: float = 1.0, impl: str = "auto"):
     """out = alpha * x w^T of many rows: the product in tiles where the kernel library finds it the faster one (impl "auto"),
     otherwise hipBLASLt called directly; torch's routine if that has no algorithm for the shape."""
     if TUNE_LIBRARY and min(w.shape[0], w.shape[1]) >= TUNE_MIN_SIDE:
-        key = (x.dtype, out.dtype, x.shape[0], w.shape[0], w.shape[1], x.stride(0), w.stride(0), out.stride(0))
+        key = (impl, x.dtype, out.dtype, x.shape[0], w.shape[0], w.shape[1], x.stride(0), w.stride(0), out.stride(0))
         if key not in _tuned:
             _tuned.add(key)
             try:
-                ops.matmul_library_tune(x, w, out, flush=TUNE_FLUSH)
+                (ops.product_tune if impl == "auto" else ops.matmul_library_tune)(x, w, out, flush=TUNE_FLUSH)
             except ops.KernelError:
                 pass
     try:

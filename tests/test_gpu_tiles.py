@@ -81,6 +81,22 @@ def test_short_walks_take_few_rounds_cpu():
     assert TILES[ops.gemm_tiles_plan(871, 2304, 64)] == (64, 64)        # one round of them
 
 
+def test_what_timing_found_cpu():
+    """A timed shape's answer holds for it and for row counts within an eighth of it, the nearest timed one first."""
+    from infinicore_infer_amd.kernels.lib import get_lib
+    note = get_lib().ic_product_timing
+    n, k = 5128, 1088                                  # (no test times this matrix)
+    assert ops.product_timed(800, n, k) is None
+    note(800, n, k, k, k, n, 0)
+    note(1000, n, k, k, k, n, 1)
+    assert ops.product_timed(800, n, k) is False and ops.product_timed(1000, n, k) is True
+    assert ops.product_timed(700, n, k) is False and ops.product_timed(880, n, k) is False and ops.product_timed(920, n, k) is True
+    assert ops.product_timed(699, n, k) is None and ops.product_timed(1126, n, k) is None
+    assert ops.product_timed(800, n, k, ldc=n + 8) is None and ops.product_timed(800, n + 8, k) is None
+    note(800, n, k, k, k, n, 1)
+    assert ops.product_timed(700, n, k) is True
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("tile", range(len(TILES)))
 @pytest.mark.parametrize("swiglu", [False, True])
@@ -188,3 +204,27 @@ def test_qkv_with_rotary_and_cache_write(tile):
         untouched = torch.ones(pages * ps, dtype=torch.bool)
         untouched[at] = False
         assert (kk[untouched] == 5.0).all() and (vv[untouched] == 7.0).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [264, 72])
+def test_products_follow_what_timing_found(rows):
+    """After timing, ops.product runs the kernel that was found the faster one, tiles or the library's kept algorithm, whatever the rule says."""
+    from infinicore_infer_amd.kernels.lib import get_lib
+    M, N, K = rows, 2560, 4032
+    a, w = _operands(M, N, K, 5)
+    ad, wd = a.cuda(), w.cuda()
+    out, tiles, lib = (torch.empty(M, N, dtype=BF16, device="cuda") for _ in range(3))
+    assert ops.product_timed(M, N, K) is None
+    flush = torch.empty(64 << 20, dtype=torch.uint8, device="cuda")
+    assert ops.product_tune(ad, wd, out, reps=3, flush=flush) >= 2
+    found = ops.product_timed(M, N, K)
+    assert found is not None
+    ops.gemm_tiles(ad, wd, tiles)
+    ops.matmul_library(ad, wd, lib)
+    for want in (found, not found):
+        get_lib().ic_product_timing(M, N, K, K, K, N, int(want))
+        ops.product(ad, wd, out)
+        _check(a, w, out, False)
+        assert torch.equal(out, tiles if want else lib)
+    get_lib().ic_product_timing(M, N, K, K, K, N, int(found))
