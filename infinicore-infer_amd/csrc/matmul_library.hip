@@ -159,12 +159,15 @@ IC_EXPORT int ic_matmul(const void* A, int a_dtype, const void* W, void* C, int 
 
 namespace {
 
-// The time of one call as tuning measures it, in milliseconds (< 0: failed): n calls after one to warm up, `flush` overwritten before each.
-template <typename F> float time_calls(F call, int n, void* flush, long long flush_bytes, hipEvent_t e0, hipEvent_t e1, hipStream_t stream) {
+// The time of one call as tuning measures it, in milliseconds (< 0: failed): n calls after one to warm up, `flush` overwritten before each, and
+// then `warm` read (into flush), if it is given.
+template <typename F> float time_calls(F call, int n, void* flush, long long flush_bytes, const void* warm, long long warm_bytes, hipEvent_t e0, hipEvent_t e1,
+                                       hipStream_t stream) {
     if (call() != IC_OK) return -1.f;
     float total = 0.f;
     for (int r = 0; r < n; ++r) {
         if (flush_bytes > 0 && hipMemsetAsync(flush, r & 1, (size_t)flush_bytes, stream) != hipSuccess) return -1.f;
+        if (warm && warm_bytes <= flush_bytes && hipMemcpyAsync(flush, warm, (size_t)warm_bytes, hipMemcpyDeviceToDevice, stream) != hipSuccess) return -1.f;
         hipEventRecord(e0, stream);
         const bool ok = call() == IC_OK;
         hipEventRecord(e1, stream);
@@ -184,9 +187,18 @@ struct Events {
     }
 };
 
-// ic_matmul_tune; best_ms: the time of the algorithm that is kept.
-int tune(const void* A, int a_dtype, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldw, int ldc, void* workspace,
-                long long workspace_bytes, void* flush, long long flush_bytes, int reps, hipStream_t stream, float* best_ms) {
+}  // namespace
+
+// Times every algorithm the library proposes for this product (reps launches each, after one to warm up) on
+// `stream` and keeps the fastest, if it beats the library's first choice by 3 %, for later ic_matmul calls of the
+// same shape, and of shapes first seen later that differ only by a row count within an eighth of this one.
+// Synchronises the stream.
+// flush (may be nullptr): device memory, larger than the chip's caches, that is overwritten before every timed
+// launch, so that the operands come from memory as a model's weights do and not from the last launch's cache lines.
+// Returns the number of algorithms tried (>= 1) or an error code (< 0).
+IC_EXPORT int ic_matmul_tune(const void* A, int a_dtype, const void* W, void* C, int c_dtype, int M, int N, int K, int lda,
+                             int ldw, int ldc, void* workspace, long long workspace_bytes, void* flush, long long flush_bytes,
+                             int reps, hipStream_t stream) {
     if (!args_ok(A, a_dtype, W, C, c_dtype, M, N, K, lda, ldw, ldc) || workspace_bytes < 0 || reps < 1 || flush_bytes < 0) return IC_ERR_ARG;
     if (!flush) flush_bytes = 0;
     std::lock_guard<std::mutex> lock(g_mu);
@@ -215,7 +227,8 @@ int tune(const void* A, int a_dtype, const void* W, void* C, int c_dtype, int M,
     const Events ev;
     if (!ev.ok) return IC_ERR_LIBRARY;
     auto time_one = [&](int i, int n) {
-        return time_calls([&] { return run(*p, i, A, W, C, 1.0f, workspace, (size_t)workspace_bytes, stream); }, n, flush, flush_bytes, ev.e0, ev.e1, stream);
+        return time_calls([&] { return run(*p, i, A, W, C, 1.0f, workspace, (size_t)workspace_bytes, stream); }, n, flush, flush_bytes, nullptr, 0,
+                          ev.e0, ev.e1, stream);
     };
     // first round: one timed launch each; second round: the eight best and the first choice, reps launches each
     std::vector<std::pair<float, int>> quick;
@@ -240,24 +253,7 @@ int tune(const void* A, int a_dtype, const void* W, void* C, int c_dtype, int M,
     // the library's own first choice stays unless another is clearly (3 %) faster: timing noise must not pick
     p->chosen = (first > 0.f && best > 0.97f * first) ? 0 : best_i;
     p->timed = true;
-    *best_ms = p->chosen == 0 ? first : best;
     return tried;
-}
-
-}  // namespace
-
-// Times every algorithm the library proposes for this product (reps launches each, after one to warm up) on
-// `stream` and keeps the fastest, if it beats the library's first choice by 3 %, for later ic_matmul calls of the
-// same shape, and of shapes first seen later that differ only by a row count within an eighth of this one.
-// Synchronises the stream.
-// flush (may be nullptr): device memory, larger than the chip's caches, that is overwritten before every timed
-// launch, so that the operands come from memory as a model's weights do and not from the last launch's cache lines.
-// Returns the number of algorithms tried (>= 1) or an error code (< 0).
-IC_EXPORT int ic_matmul_tune(const void* A, int a_dtype, const void* W, void* C, int c_dtype, int M, int N, int K, int lda,
-                             int ldw, int ldc, void* workspace, long long workspace_bytes, void* flush, long long flush_bytes,
-                             int reps, hipStream_t stream) {
-    float ms = 0.f;
-    return tune(A, a_dtype, W, C, c_dtype, M, N, K, lda, ldw, ldc, workspace, workspace_bytes, flush, flush_bytes, reps, stream, &ms);
 }
 
 // ---- products whose library algorithms were timed, against the tiles of gemm_tiles.hip ---------------------------------
@@ -290,19 +286,22 @@ IC_EXPORT int ic_product_timed(int M, int N, int K, int lda, int ldw, int ldc) {
     return from ? (from->tiles ? 1 : 0) : -1;
 }
 
-// As ic_matmul_tune, and where the product could run in tiles those are timed likewise: ic_product then takes, for this shape and the neighbours that
-// take the timed algorithm, the one that the rule names without timing unless the other was 3 % faster.
+// As ic_matmul_tune, and where the product could run in tiles the two are timed against each other, the rows of A in the caches as the kernel before leaves
+// them (with A out of memory too, 871 x 4,096 x 16,384 seems faster in the library, which takes 150 us where the tiles take 133): ic_product then takes, for
+// this shape and the neighbours that take the timed algorithm, the one that the rule names without timing unless the other was 3 % faster.
 IC_EXPORT int ic_product_tune(const void* A, int a_dtype, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldw, int ldc,
                               void* workspace, long long workspace_bytes, void* flush, long long flush_bytes, int reps, hipStream_t stream) {
-    float library = 0.f;
-    const int tried = tune(A, a_dtype, W, C, c_dtype, M, N, K, lda, ldw, ldc, workspace, workspace_bytes, flush, flush_bytes, reps, stream, &library);
+    const int tried = ic_matmul_tune(A, a_dtype, W, C, c_dtype, M, N, K, lda, ldw, ldc, workspace, workspace_bytes, flush, flush_bytes, reps, stream);
     if (tried < 0 || a_dtype != IC_BF16 || c_dtype != IC_BF16 || M <= 32 || !ic_gemm_tiles_supported(M, N, K, lda, ldw, ldc, 0) ||
         (((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) & 15)) return tried;
     const Events ev;
     if (!ev.ok) return tried;
-    const float tiles = time_calls([&] { return ic_gemm_tiles(A, W, C, M, N, K, lda, ldw, ldc, 0, stream); }, reps, flush, flush ? flush_bytes : 0, ev.e0,
-                                   ev.e1, stream);
-    if (tiles < 0.f) return tried;
+    if (!flush) flush_bytes = 0;
+    const long long rows = 2 * ((long long)(M - 1) * lda + K);
+    auto timed = [&](auto call) { return time_calls(call, reps, flush, flush_bytes, A, rows, ev.e0, ev.e1, stream); };
+    const float library = timed([&] { return ic_matmul(A, a_dtype, W, C, c_dtype, M, N, K, lda, ldw, ldc, 1.0f, workspace, workspace_bytes, stream); });
+    const float tiles = timed([&] { return ic_gemm_tiles(A, W, C, M, N, K, lda, ldw, ldc, 0, stream); });
+    if (library < 0.f || tiles < 0.f) return tried;
     const bool rule = ic_gemm_tiles_pays(M, N, K, 0) != 0;
     ic_product_timing(M, N, K, lda, ldw, ldc, rule ? library >= 0.97f * tiles : tiles < 0.97f * library);
     return tried + 1;
