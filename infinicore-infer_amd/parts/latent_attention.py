@@ -169,7 +169,7 @@ class LatentAttention(Mixer):
         gathered = ctx.ws.buffer("latent_gathered", (keys, D), self.runtime.dtype)
         ops.latent_gather(cache.k, cache.block_tables[r], L, keys, ctx.page_size, R, gathered, key0=key0, first=first)
         kv = ctx.ws.buffer("latent_made", (keys, width), self.runtime.dtype)
-        _library(gathered[:, :R], self.w_ukv, kv)
+        _library(gathered[:, :R], self.w_ukv, kv, self.runtime.gemm_impl)
         mine = q[row0:row0 + n]
         ops.latent_q_rotate(mine, self.dim, self.E, self.dim, H, self.freq, self.rot_dims, ctx.positions[row0:row0 + n], mine, self.rot_mult)
         ops.attention_latent_prefill(q, heads_out, gate, kv, gathered, R, key0, row0, n, pos0, H, self.dim, self.E, self.dv, self.scale,
@@ -200,10 +200,10 @@ class LatentAttention(Mixer):
             c0 = max(0, pos0 + q0 - self.window + 1) // 16 * 16 - key0 if self.window else 0
             cols = min(keys, (pos0 + q0 + qn - key0 + 15) // 16 * 16) - c0
             scores = ctx.ws.buffer("latent_scores", (qn * H, cols), torch.float32)
-            _library(qa[q0:q0 + qn].view(qn * H, D), gathered[c0:c0 + cols], scores)
+            _library(qa[q0:q0 + qn].view(qn * H, D), gathered[c0:c0 + cols], scores, rt.gemm_impl)
             probs = ctx.ws.buffer("latent_probs", (qn * H, cols), rt.dtype)
             ops.latent_softmax(scores, probs, H, pos0 + q0, self.scale, window=self.window, sinks=self.sinks, key0=key0 + c0)
-            _library(probs, gathered_t[:, c0:c0 + cols], walked[q0:q0 + qn].view(qn * H, R))
+            _library(probs, gathered_t[:, c0:c0 + cols], walked[q0:q0 + qn].view(qn * H, R), rt.gemm_impl)
         ops.blocked_product(walked.view(n, H, R), self.w_uv, heads_out[rows].view(n, H, self.dv),
                             gate=None if gate is None else gate[rows].view(n, H, self.dv))
 

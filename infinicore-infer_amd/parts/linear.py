@@ -29,7 +29,7 @@ TUNE_MIN_SIDE = 256
 _tuned = set()
 
 
-def _library(x, w, out, alpha: float = 1.0, impl: str = "auto"):
+def _library(x, w, out, impl: str, alpha: float = 1.0):
     """out = alpha * x w^T of many rows: the product in tiles where the kernel library finds it the faster one (impl "auto"),
     otherwise hipBLASLt called directly; torch's routine if that has no algorithm for the shape."""
     if TUNE_LIBRARY and min(w.shape[0], w.shape[1]) >= TUNE_MIN_SIDE:
@@ -73,14 +73,14 @@ def linear(x, w, out, impl: str = "auto", alpha: float = 1.0, ws=None):
         x32 = x if x.dtype == torch.float32 else scratch("linear_x32", tuple(x.shape)).copy_(x)
         w32 = w if w.dtype == torch.float32 else w.to(torch.float32)
         if out.dtype == torch.float32:
-            return _library(x32, w32, out, alpha, impl)
+            return _library(x32, w32, out, impl, alpha)
         tmp = scratch("linear_out32", tuple(out.shape))
-        _library(x32, w32, tmp, alpha, impl)
+        _library(x32, w32, tmp, impl, alpha)
         out.copy_(tmp)
         return out
     if own_kernel_applies(x.shape[0], x.dtype, w.dtype, out.dtype, impl):
         return ops.gemm_nt(x, w, out, alpha=alpha)
-    return _library(x, w, out, alpha, impl)
+    return _library(x, w, out, impl, alpha)
 
 
 def linear_tail(x, w, tail, ws, name: str, impl: str = "auto"):

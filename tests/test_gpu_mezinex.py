@@ -657,3 +657,34 @@ def test_drawn_configurations(tmp_path_factory, seed):
         _compare(H.run_trace(engine, steps), ref, dtype, tol if dtype == torch.float32 else 1.5, "drawn %d %s" % (seed, dname), steps, median_only=True)
         engine.cache.check_invariants()
         assert not engine.cache.requests
+
+
+@pytest.mark.parametrize("makes_keys", [True, False])
+def test_library_products_only(tmp_path_factory, monkeypatch, makes_keys):
+    """gemm_impl "library": no product of a step runs in the package's own tiles, those over latent rows included (keys and values made for a
+    portion; scores and probabilities times values), and the logits are those of the own kernels up to rounding."""
+    from infinicore_infer_amd.engine import Engine, StepEntry
+    from infinicore_infer_amd.kernels import ops
+    from infinicore_infer_amd.parts.latent_attention import LatentAttention
+    CONFIGS["wide"] = {"architecture": "Mezinex", "vocab": 160, "width": 256, "norm": {"eps": 1e-5}, "logit_scale": 1.0, "streams": 2,
+                       "layers": [_latent(4, 64, 32, 32, 64, 128, 256, 0.1, 10000.0, 512), _rglru(256, 4, 4, 512)]}
+    folder, _ = _model(tmp_path_factory, "wide")
+    toks = H.random_tokens(160, 300, 9)
+    logits = {}
+    if not makes_keys:
+        monkeypatch.setattr(LatentAttention, "_makes_keys", lambda self: False)
+    for impl in ("auto", "library"):
+        eng = Engine.from_dir(folder, dtype=torch.bfloat16, max_tokens=1024, page_size=16, max_requests=2, gemm_impl=impl)
+        asked = []
+        made = LatentAttention._portion_by_keys
+        monkeypatch.setattr(LatentAttention, "_portion_by_keys", lambda self, *a: asked.append(1) or made(self, *a))
+        if impl == "library":
+            def refuse(*a, **k):
+                raise AssertionError("a product in tiles under gemm_impl library")
+            for name in ("product", "product_tune", "gemm_tiles", "gemm_tiles_rope"):
+                monkeypatch.setattr(ops, name, refuse)
+        logits[impl] = eng.step([StepEntry("a", toks, [100, 299])]).float().cpu()
+        assert bool(asked) == makes_keys
+        monkeypatch.setattr(LatentAttention, "_portion_by_keys", made)
+    scale = float(logits["library"].abs().max())
+    assert float((logits["auto"] - logits["library"]).abs().max()) <= 3e-2 * scale
