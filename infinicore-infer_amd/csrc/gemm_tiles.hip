@@ -73,12 +73,22 @@ template <int N, typename F> __device__ __forceinline__ void each(F&& f) { each_
 // acc += w a.  OWN: with 256 accumulators a lane, all of the second half of its 512 registers, the compiler's own product copies them from product to
 // product (192 copies a stage; with ROPE's way out, which needs more registers, in all tiles of 32 accumulators and more); written as assembly, with
 // an operand that is read and written, it does not.  The compiler does not know such a product for one and adds no wait before an instruction that
-// reads its result: LAST, on the last product of a stage, waits here (11 wait states after eight passes), so that whatever follows the stage may read
-// any accumulator.
+// reads its result: LAST, on the last product of a k-step, waits here (11 wait states after eight passes), so that whatever follows the k-step may read
+// any accumulator.  settled() ties the accumulators to a place between the volatile products: what writes or reads them stays on its side of it.
 template <bool OWN, bool LAST> __device__ __forceinline__ void product(v4f& acc, const v8b& w, const v8b& a) {
     if constexpr (!OWN) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, a, acc, 0, 0, 0);
     else if constexpr (LAST) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\ts_nop 15" : "+a"(acc) : "v"(w), "v"(a));
     else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(w), "v"(a));
+}
+
+template <bool OWN, int N, int M> __device__ __forceinline__ void settled(v4f (&acc)[N][M]) {
+    if constexpr (OWN) {
+#pragma unroll
+        for (int n = 0; n < N; ++n)
+#pragma unroll
+            for (int m = 0; m < M; ++m) asm volatile("" : "+a"(acc[n][m]));
+        asm volatile("s_nop 7");
+    }
 }
 
 template <int BM_, int BN_, int WM_, int WN_, int WK_, int STAGES_> struct Tile {
@@ -170,7 +180,7 @@ __global__ void __launch_bounds__(T::WAVES * 64, T::BLOCKS_PER_CU) gemm_tiles_ke
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = v4f{0.f, 0.f, 0.f, 0.f};
-    if constexpr (T::own_product(EPI)) asm volatile("s_nop 7");         // (and none between these writes and the first products)
+    settled<T::own_product(EPI)>(acc);                             // (the compiler waits neither between these writes and the first products)
 
     // operand registers of two k-steps: one is multiplied while the other is read
     v8b fa[2][MT], fw[2][NT];
@@ -254,6 +264,7 @@ __global__ void __launch_bounds__(T::WAVES * 64, T::BLOCKS_PER_CU) gemm_tiles_ke
     } else {
         for (; s < n_stages; ++s) buf = whole_stage(s, buf, std::integral_constant<int, 0>{});
     }
+    settled<T::own_product(EPI)>(acc);
     wait_loads<0>();
     __syncthreads();                                               // LDS is free
 

@@ -115,6 +115,21 @@ def test_tiles_at_their_edges(tile, swiglu):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("tile", range(len(TILES)))
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_tiles_over_long_walks(tile, swiglu):
+    """41 and 128 stages, an odd and an even number of rounds of every tile's buffers: the products written as assembly (256 x 256) and the compiler's."""
+    bm, bn = TILES[tile]
+    if swiglu and bn == 96:
+        pytest.skip("three column tiles a wave: no pairs of gate and up")
+    for M, N, K in ((bm + 5, bn + 16, 2624), (bm, 2 * bn, 8192)):
+        a, w = _operands(M, N, K, 100 + tile)
+        out = torch.empty(M, N // 2 if swiglu else N, dtype=BF16, device="cuda")
+        ops.gemm_tiles(a.cuda(), w.cuda(), out, swiglu_output=swiglu, tile=tile)
+        _check(a, w, out, swiglu)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(33, 7680, 1536), (65, 512, 512), (129, 1536, 3840), (871, 2560, 1536), (1045, 1536, 1536), (2049, 2304, 2304)])
 def test_chosen_tiles_and_their_replays(M, N, K):
     """The tile that the rule names, recorded and replayed with other rows in between."""
@@ -170,7 +185,7 @@ def test_qkv_with_rotary_and_cache_write(tile):
     order, page sizes that are no power of two, heads that begin inside a tile."""
     if tile is not None and TILES[tile] in ((64, 96), (256, 256)):
         pytest.skip("three column tiles a wave: no pairs; 256 accumulators a lane: no registers")
-    for M, K, nh, nkv, dh, ps in ((70, 128, 3, 1, 64, 16), (33, 64, 2, 2, 32, 7), (197, 192, 5, 2, 128, 64), (1, 320, 1, 1, 256, 3)):
+    for M, K, nh, nkv, dh, ps in ((70, 128, 3, 1, 64, 16), (33, 64, 2, 2, 32, 7), (197, 192, 5, 2, 128, 64), (1, 320, 1, 1, 256, 3), (130, 2624, 4, 2, 64, 16)):
         a, w = _operands(M, (nh + 2 * nkv) * dh, K, M + dh)
         g = torch.Generator().manual_seed(M)
         pos = torch.randint(0, 500, (M,), generator=g, dtype=torch.int32)
