@@ -123,14 +123,7 @@ IC_EXPORT int ic_attn_prefill_split(const void* q, int q_stride, void* out, int 
     // Few blocks (up to 2 per compute unit; measured with 16..64 heads of 64 and 32..40 of 128 over 512..4,096
     // tokens: two groups win up to 2.0 blocks a unit by 5..25 %, one group from 2.25 on by 2..25 %): the longest
     // tile's walk over the keys sets the time, so two wave groups share it.  Many blocks: one group, more blocks resident.
-    static int cus = 0;                                 // compute units of the device, asked once
-    if (cus == 0) {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) cus = n;
-        else cus = 256;
-    }
-    const bool two_groups = groups ? groups == 2 : (long long)nh * n_tiles <= 2LL * cus;
+    const bool two_groups = groups ? groups == 2 : (long long)nh * n_tiles <= 2LL * compute_units();
     dim3 grid((unsigned)nh * (unsigned)n_tiles * (unsigned)parts);
     const bool page64 = page_size >= kPfKeys;            // (a power of two) a 64-key tile lies in one page
 #define IC_PF_LAUNCH(DD, ST, GG, PP)                                                                                   \

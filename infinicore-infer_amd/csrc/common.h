@@ -127,6 +127,18 @@ __device__ __forceinline__ float block_max(float v, float* red) {
     return t;
 }
 
+// Compute units of the current device, asked once.
+static inline int compute_units() {
+    static int cus = 0;
+    if (cus == 0) {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) == hipSuccess &&
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) cus = n;
+        else cus = 256;
+    }
+    return cus;
+}
+
 static inline int ic_launch_status() {
     hipError_t e = hipGetLastError();
     return (int)e;

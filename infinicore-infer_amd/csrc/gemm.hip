@@ -503,17 +503,6 @@ static void launch_gemm_swiglu_two_tiles(const void* A, const void* W, void* C, 
                        (const uint16_t*)A, (const uint16_t*)W, (bf16*)C, M, N, K, lda, ldw, ldc, 1.0f, RopeEpilogue{}, nf);
 }
 
-// Compute units of the current device, asked once.
-static int compute_units() {
-    static int cus = 0;
-    if (cus == 0) {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) cus = n;
-        else cus = 256;
-    }
-    return cus;
-}
 
 // Very many weight rows and at most 16 token rows (the output head over the vocabulary): there are enough 16-row
 // weight tiles for every wave to own whole tiles, so nothing is summed across waves.  The token rows are staged in
@@ -834,7 +823,6 @@ static bool norm_fuse_args(const IcRowFactor* rf, const IcResidualNorm* tail, in
 
 // Column blocks (= sums of squares per row) that c_mode 2 writes for an N wide product.
 // (one block per compute unit when 16-column tiles would be fewer than the units)
-static int compute_units();
 IC_EXPORT int ic_gemm_nt_residual_parts(int N) {
     const int tiles = (N + 15) / 16, cus = compute_units();
     if (tiles >= cus || N <= 0) return tiles;

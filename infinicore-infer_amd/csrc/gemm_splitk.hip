@@ -264,16 +264,6 @@ __global__ void splitk_add_norm_kernel(const float* __restrict__ P, int S, int M
     }
 }
 
-int compute_units_sk() {
-    static int cus = 0;
-    if (cus == 0) {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) cus = n;
-        else cus = 256;
-    }
-    return cus;
-}
-
 bool splits_ok(const float* P, int S, int M, int N) {
     return P && S >= 1 && S <= 64 && M >= 1 && M <= 64 && N >= 1 && (((uintptr_t)P & 15) == 0) && ((size_t)M * N) % 4 == 0;
 }
@@ -294,7 +284,7 @@ IC_EXPORT int ic_gemm_splitk_supported(int M, int N, int K, int lda, int ldw) {
 IC_EXPORT int ic_gemm_splitk_slices(int N, int K) {
     if (N <= 0 || K <= 0) return 1;
     const int col_blocks = (N + kSkCols - 1) / kSkCols, chunks = (K + kSkChunk - 1) / kSkChunk;
-    const int cus = compute_units_sk();
+    const int cus = compute_units();
     int want = (7 * cus / 8) / col_blocks;
     const int full = cus / col_blocks;
     if (4 * full >= 5 * want) want = full;
@@ -314,7 +304,7 @@ IC_EXPORT int ic_gemm_splitk_pays(int M, int N, int K) {
     if (M <= 0 || M > 64 || N <= 0 || K <= 0 || N > 8192) return 0;
     if (M <= 16 && (M <= 12 || K < 8192)) return 0;
     const int col_blocks = (N + kSkCols - 1) / kSkCols;
-    return 2 * col_blocks * ic_gemm_splitk_slices(N, K) >= compute_units_sk();
+    return 2 * col_blocks * ic_gemm_splitk_slices(N, K) >= compute_units();
 }
 
 // P[s, m, n] (float32 [n_slices, M, N]) = A[m, K_s] . W[n, K_s] for the n_slices slices of K (whole chunks of 128).

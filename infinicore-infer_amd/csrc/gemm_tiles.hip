@@ -400,7 +400,7 @@ template <typename T, int EPI> int launch(TilesArgs a, hipStream_t stream) {
 }
 
 // The tiles, smallest first, and what one costs in microseconds: FIXED + rounds * (ROUND + stages * STAGE * (1 + FULL * x)), where x is the part of
-// the 256 compute units that have a block and a round is one block a unit (two of 64 x 32 and 64 x 64, which then share it: 1.7 times the stage).
+// the compute units (256 of them where this was fitted) that have a block and a round is one block a unit (two of 64 x 32 and 64 x 64, which then share it: 1.7 times the stage).
 // Fitted to 6,900 timed products (17 pairs of N in 512..32,768 and K in 512..16,384, 33..16,384 rows, weights out of memory); the tile with the least
 // cost loses 0.7 % to the best one on average and 5 % at the 95th percentile.  64 x 32 is for few rows of narrow matrices, where only many small tiles
 // reach all units (64 x 6,912 x 2,304: 15.0 us with 64 x 64, 11.8), 64 x 96 and 128 x 64 likewise (200 x 4,608 x 4,096: 25.4 -> 21.3).  Tried and not
@@ -425,7 +425,6 @@ template <typename T, int EPI> int launch(TilesArgs a, hipStream_t stream) {
     X(14, 6.27, 1.084, 0.30, 0.00, 256, 256, 2, 2, 1, 2)
 
 constexpr int kTiles = 15;
-constexpr double kUnits = 256.0;
 
 struct TileCost { int bm, bn, blocks_per_unit; bool takes[3]; double fixed, stage, full, round; };
 constexpr TileCost kCosts[kTiles] = {
@@ -434,9 +433,10 @@ constexpr TileCost kCosts[kTiles] = {
 #undef X
 };
 
-double cost_of(const TileCost& t, int M, int N, int K, int mode) {
+// units: compute units of the device or partition; memory serves each its share of the whole chip's rate.
+double cost_of(const TileCost& t, int M, int N, int K, int mode, int units) {
     const long long tm = (M + t.bm - 1) / t.bm, tn = mode != EPI_BF16 ? (N / 2 + t.bn / 2 - 1) / (t.bn / 2) : (N + t.bn - 1) / t.bn;
-    const double tiles = (double)(tm * tn), x = tiles / kUnits, stages = K / 64;
+    const double tiles = (double)(tm * tn), x = tiles / units, stages = K / 64;
     double rounds = 1.0, busy = x < 1.0 ? x : 1.0, shared = 1.0, again = 0.0;
     if (x > 1.0) {
         rounds = __builtin_ceil(x / t.blocks_per_unit);
@@ -447,15 +447,15 @@ double cost_of(const TileCost& t, int M, int N, int K, int mode) {
     const double walk = t.fixed + rounds * (t.round + stages * t.stage * (1.0 + t.full * busy) * shared) + again;
     // the weights come from memory once, and about half of them again for every further row tile (blocks of one column of tiles seldom run abreast);
     // narrow tiles of pairs read them in pieces of 32 rows and less, which memory serves more slowly (64 x 32,768 x 4,096: 83 us against 63)
-    const double read = 3.0 + 2.0 * N * K * (1.0 + 0.5 * (tm < 4 ? tm - 1 : 3)) * (mode != EPI_BF16 && t.bn <= 64 ? 1.35 : 1.0) / 7e6;
+    const double read = 3.0 + 2.0 * N * K * (1.0 + 0.5 * (tm < 4 ? tm - 1 : 3)) * (mode != EPI_BF16 && t.bn <= 64 ? 1.35 : 1.0) / (7e6 * units / 256.0);
     return walk > read ? walk : read;
 }
 
-int best_tile(int M, int N, int K, int mode, double* cost) {
+int best_tile(int M, int N, int K, int mode, int units, double* cost) {
     int best = 0;
     for (int i = 0; i < kTiles; ++i) {
         if (!kCosts[i].takes[mode]) continue;
-        const double c = cost_of(kCosts[i], M, N, K, mode);
+        const double c = cost_of(kCosts[i], M, N, K, mode, units);
         if (i == 0 || c < *cost) { *cost = c; best = i; }
     }
     return best;
@@ -501,7 +501,7 @@ int rope_run(const void* A, const void* W, void* C, int M, int K, int lda, int l
     a.nh = nh, a.nkvh = nkvh, a.page_size = page_size;
     while ((2 << a.half_log) < dh) ++a.half_log;
     double cost = 0.0;
-    return run(a, EPI_ROPE, tile >= 0 ? tile : best_tile(M, N, K, EPI_ROPE, &cost), stream);
+    return run(a, EPI_ROPE, tile >= 0 ? tile : best_tile(M, N, K, EPI_ROPE, compute_units(), &cost), stream);
 }
 
 }  // namespace
@@ -540,36 +540,40 @@ IC_EXPORT int ic_gemm_tiles_rope_supported(const void* A, const void* W, const v
 // 1,045 x 7,680 x 1,536: 42.8 -> 28.0; 2,048 x 11,520 x 2,304: 130 -> 98; 16,384 x 32,768 x 4,096: 3,195 -> 3,007).  So does rotary and cache write behind QKV
 // (64 rows of the 2B shape 18.3 -> 12.5, 1,045 rows of the 1B shape 21.5 -> 15.5, 2,048 of the 8B shape 78.6 -> 69.6), but for sizes that the largest tile
 // fits best, which this epilogue does not have.
-IC_EXPORT int ic_gemm_tiles_pays(int M, int N, int K, int mode) {
+IC_EXPORT int ic_gemm_tiles_pays_on(int M, int N, int K, int mode, int units) {
     if (M <= 32) return 0;
-    const double t = (double)((M + 255) / 256) * ((N + 255) / 256), fill = t / (kUnits * __builtin_ceil(t / kUnits));
+    const double t = (double)((M + 255) / 256) * ((N + 255) / 256), fill = t / (units * __builtin_ceil(t / units)), part = units / 256.0;
     if (mode != EPI_BF16 && K > 8192 && fill >= 0.93) return 0;
     double cost = 0.0;
-    if (mode == EPI_ROPE) return kCosts[best_tile(M, N, K, EPI_SWIGLU, &cost)].takes[EPI_ROPE];
-    const TileCost& own = kCosts[best_tile(M, N, K, mode, &cost)];
-    const double weights = 2.0 * N * K, products = weights * M;            // bytes, operations
+    if (mode == EPI_ROPE) return kCosts[best_tile(M, N, K, EPI_SWIGLU, units, &cost)].takes[EPI_ROPE];
+    const TileCost& own = kCosts[best_tile(M, N, K, mode, units, &cost)];
+    const double weights = 2.0 * N * K / part, products = weights * M;     // bytes, operations for the whole chip's rates below
     if (M <= 64 && K % 256 == 0) {
         const double read = weights / 7.2e6, unit = mode == EPI_SWIGLU ? 3.0 + 0.75e-6 * M * N : 0.0;
         if ((cost > read ? cost : read) > 11.35 + weights / 9.06e6 + products / 5.0e9 + unit) return 0;
     }
-    if (mode == EPI_SWIGLU) return !(M <= 96 && K >= 6144 && K % 256 == 0 && weights >= 1.9e8);
-    if (K == 64 && (double)((M + own.bm - 1) / own.bm) * ((N + own.bn - 1) / own.bn) > kUnits * own.blocks_per_unit) return 0;
+    if (mode == EPI_SWIGLU) return !(M <= 96 && K >= 6144 && K % 256 == 0 && 2.0 * N * K >= 1.9e8);
+    if (K == 64 && (double)((M + own.bm - 1) / own.bm) * ((N + own.bn - 1) / own.bn) > (double)units * own.blocks_per_unit) return 0;
     const double over = 6.0 + (products / 0.6e9 > weights / 4e6 ? products / 0.6e9 : weights / 4e6);
     if (M <= 512) return cost <= 1.6 * over;
-    const bool whole = N % 256 == 0 && K >= 1024 && !(t > 4.0 * kUnits && fill < 0.92);
-    return cost <= 2.0 * over && !(whole && cost > 0.94 * cost_of(kCosts[kTiles - 1], M, N, K, EPI_BF16));
+    const bool whole = N % 256 == 0 && K >= 1024 && !(t > 4.0 * units && fill < 0.92);
+    return cost <= 2.0 * over && !(whole && cost > 0.94 * cost_of(kCosts[kTiles - 1], M, N, K, EPI_BF16, units));
 }
 
-IC_EXPORT int ic_gemm_tiles_plan(int M, int N, int K, int mode) {
+IC_EXPORT int ic_gemm_tiles_pays(int M, int N, int K, int mode) { return ic_gemm_tiles_pays_on(M, N, K, mode, compute_units()); }
+
+IC_EXPORT int ic_gemm_tiles_plan_on(int M, int N, int K, int mode, int units) {
     double cost = 0.0;
-    return M > 0 && N > 0 && K > 0 ? best_tile(M, N, K, mode, &cost) : -1;
+    return M > 0 && N > 0 && K > 0 && units > 0 ? best_tile(M, N, K, mode, units, &cost) : -1;
 }
+
+IC_EXPORT int ic_gemm_tiles_plan(int M, int N, int K, int mode) { return ic_gemm_tiles_plan_on(M, N, K, mode, compute_units()); }
 
 IC_EXPORT int ic_gemm_tiles(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, int mode, hipStream_t stream) {
     if (M <= 0) return IC_OK;
     if (!A || !W || !C || !ic_gemm_tiles_supported(M, N, K, lda, ldw, ldc, mode) || !aligned16(A) || !aligned16(W) || !aligned16(C)) return IC_ERR_ARG;
     double cost = 0.0;
-    return run(plain_args(A, W, C, M, N, K, lda, ldw, ldc), mode, best_tile(M, N, K, mode, &cost), stream);
+    return run(plain_args(A, W, C, M, N, K, lda, ldw, ldc), mode, best_tile(M, N, K, mode, compute_units(), &cost), stream);
 }
 
 IC_EXPORT int ic_gemm_tiles_cfg(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, int mode, int tile,

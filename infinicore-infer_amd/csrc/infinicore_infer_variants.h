@@ -25,6 +25,9 @@ int ic_gemm_rows_plan(int epi, int M, int N, int K, int blocks, int units, int* 
 int ic_gemm_tiles_cfg(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, int mode, int tile, hipStream_t stream);
 int ic_gemm_tiles_rope_cfg(const void* A, const void* W, void* C, int M, int K, int lda, int ldw, int ldc, const int* positions, const int* slots, const float* cos_t, const float* sin_t, void* kcache, void* vcache, int nh, int nkvh, int dh, int page_size, int tile, hipStream_t stream);
 int ic_gemm_tiles_plan(int M, int N, int K, int mode);
+// The same, and ic_gemm_tiles_pays, for a device or partition of `units` compute units.
+int ic_gemm_tiles_plan_on(int M, int N, int K, int mode, int units);
+int ic_gemm_tiles_pays_on(int M, int N, int K, int mode, int units);
 // Notes what timing a product found (ic_product_tune does).
 void ic_product_timing(int M, int N, int K, int lda, int ldw, int ldc, int tiles);
 

@@ -195,6 +195,8 @@ _SIGNATURES = {
     "ic_gemm_tiles_supported": [_I, _I, _I, _I, _I, _I, _I],
     "ic_gemm_tiles_pays": [_I, _I, _I, _I],
     "ic_gemm_tiles_plan": [_I, _I, _I, _I],
+    "ic_gemm_tiles_plan_on": [_I] * 5,
+    "ic_gemm_tiles_pays_on": [_I] * 5,
     "ic_gemm_tiles": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
     "ic_gemm_tiles_cfg": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P],
     "ic_gemm_tiles_rope_supported": [_P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I],

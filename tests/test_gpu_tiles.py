@@ -81,6 +81,20 @@ def test_short_walks_take_few_rounds_cpu():
     assert TILES[ops.gemm_tiles_plan(871, 2304, 64)] == (64, 64)        # one round of them
 
 
+def test_rules_of_a_partition_cpu():
+    """The tiles and the choice against the library follow the units there are: 512 x 1,536 x 1,536 runs as 192 tiles of 64 x 64 on 256 units and as 32
+    of 128 x 192 on 32."""
+    from infinicore_infer_amd.kernels.lib import get_lib
+    lib = get_lib()
+    tiles = lambda units, M, N, K: (lambda bm, bn: (bm, bn, -(-M // bm) * -(-N // bn)))(*TILES[lib.ic_gemm_tiles_plan_on(M, N, K, 0, units)])
+    for M, N, K in ((512, 1536, 1536), (256, 2048, 2048), (1024, 1024, 4096)):
+        whole, part = tiles(256, M, N, K), tiles(32, M, N, K)
+        assert whole[2] <= 256 and part[2] <= 32 and part[0] * part[1] > whole[0] * whole[1], (whole, part)
+    # what a chip of 256 units does with 256 rounds' worth of work, 32 units do with an eighth of it
+    assert not lib.ic_gemm_tiles_pays_on(4096, 4096, 4096, 0, 256) and lib.ic_gemm_tiles_pays_on(512, 4096, 4096, 0, 256)
+    assert not lib.ic_gemm_tiles_pays_on(1024, 2048, 4096, 0, 32) and lib.ic_gemm_tiles_pays_on(1024, 2048, 4096, 0, 256)
+
+
 def test_what_timing_found_cpu():
     """A timed shape's answer holds for it and for row counts within an eighth of it, the nearest timed one first."""
     from infinicore_infer_amd.kernels.lib import get_lib
