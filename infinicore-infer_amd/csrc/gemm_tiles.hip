@@ -474,7 +474,7 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 // Whole stages of K, 16-byte pieces of every row, byte offsets within 32 bits.  cols: columns of C.
 bool takes(int M, int N, int K, int lda, int ldw, int cols, int ldc, int mode) {
-    if (M <= 0 || N <= 0 || K <= 0 || K % 64 || lda < K || ldw < K || lda % 8 || ldw % 8) return false;
+    if (M <= 0 || M > (1 << 30) || N <= 0 || N > (1 << 30) || K <= 0 || K % 64 || lda < K || ldw < K || lda % 8 || ldw % 8) return false;
     if (N % (mode != EPI_BF16 ? 16 : 8) || ldc < cols || ldc % 8) return false;
     if ((long long)lda * 2 * 256 >= (1LL << 31) || (long long)ldw * 2 * (mode != EPI_BF16 ? N : 256) >= (1LL << 32)) return false;
     return (long long)((M + 63) / 64) * ((N + 63) / 64) < (1LL << 28);
@@ -541,7 +541,7 @@ IC_EXPORT int ic_gemm_tiles_rope_supported(const void* A, const void* W, const v
 // (64 rows of the 2B shape 18.3 -> 12.5, 1,045 rows of the 1B shape 21.5 -> 15.5, 2,048 of the 8B shape 78.6 -> 69.6), but for sizes that the largest tile
 // fits best, which this epilogue does not have.
 IC_EXPORT int ic_gemm_tiles_pays_on(int M, int N, int K, int mode, int units) {
-    if (M <= 32) return 0;
+    if (M <= 32 || M > (1 << 30) || N <= 0 || N > (1 << 30) || K <= 0 || units <= 0 || mode < EPI_BF16 || mode > EPI_ROPE) return 0;
     const double t = (double)((M + 255) / 256) * ((N + 255) / 256), fill = t / (units * __builtin_ceil(t / units)), part = units / 256.0;
     if (mode != EPI_BF16 && K > 8192 && fill >= 0.93) return 0;
     double cost = 0.0;
@@ -564,7 +564,7 @@ IC_EXPORT int ic_gemm_tiles_pays(int M, int N, int K, int mode) { return ic_gemm
 
 IC_EXPORT int ic_gemm_tiles_plan_on(int M, int N, int K, int mode, int units) {
     double cost = 0.0;
-    return M > 0 && N > 0 && K > 0 && units > 0 ? best_tile(M, N, K, mode, units, &cost) : -1;
+    return M > 0 && N > 0 && K > 0 && units > 0 && mode >= EPI_BF16 && mode <= EPI_ROPE ? best_tile(M, N, K, mode, units, &cost) : -1;
 }
 
 IC_EXPORT int ic_gemm_tiles_plan(int M, int N, int K, int mode) { return ic_gemm_tiles_plan_on(M, N, K, mode, compute_units()); }

@@ -54,6 +54,9 @@ def test_tile_rule_cpu():
     assert not sup(100, 64, 128, 132, 128, 64, 0) and not sup(100, 64, 128, 128, 132, 64, 0) and not sup(100, 64, 128, 128, 128, 68, 0)
     assert not sup(100, 72, 128, 128, 128, 40, 1)            # gate and up in 16-byte pieces each
     assert not sup(100, 64, 128, 120, 128, 64, 0) and not sup(100, 64, 128, 128, 128, 56, 0) and not sup(0, 64, 128, 128, 128, 64, 0)
+    assert not sup((1 << 31) - 1, 64, 64, 64, 64, 64, 0) and not sup(100, (1 << 31) - 8, 64, 64, 64, (1 << 31) - 8, 0)     # sums with a tile's rows stay in range
+    assert lib.ic_gemm_tiles_plan(100, 64, 64, 3) == -1 and lib.ic_gemm_tiles_plan(100, 64, 64, -1) == -1 and lib.ic_gemm_tiles_plan(100, 64, 64, 2) >= 0
+    assert not lib.ic_gemm_tiles_pays(100, 64, 64, 3) and not lib.ic_gemm_tiles_pays((1 << 31) - 1, 64, 64, 0)
     assert not sup(100, 1 << 16, 1 << 15, 1 << 15, 1 << 15, 1 << 15, 1)     # gate and up rows more than 32 bits of bytes apart
 
 
