@@ -209,7 +209,7 @@ def test_fourteen_rows_of_16_kb_go_through_the_sliced_product(tmp_path_factory, 
 def test_seventeen_to_sixty_four_rows_at_a_width_where_the_slices_pay(tmp_path_factory, n_req):
     """20 and 40 requests decode together on two layers of the benchmark's sizes, where the O and the down projection
     both run as slices over K (hidden 2,304, inner size 5,760): sliced O with the whole norm applied, the gate/up product fed fully normed rows
-    (with the SwiGLU epilogue at 20 rows, the library's product and the activation kernel at 40), sliced down, and the
+    (with the SwiGLU epilogue, in the few-row kernel at 20 rows and in tiles at 40), sliced down, and the
     head fed normed rows.  The logits equal the plain model's, and the step issued by native code and the one issued
     by the parts' Python forward launch the same kernels: their logits are equal to the bit."""
     from infinicore_infer_amd.engine import Engine, StepEntry
@@ -297,8 +297,9 @@ def test_recorded_decode_steps_equal_eager_ones(tmp_path_factory, dname, dtype, 
 
 @pytest.mark.parametrize("shape", ["2b", "1b", "8b"])
 def test_recorded_steps_with_library_products_equal_eager_ones(tmp_path_factory, shape):
-    """From 17 rows on a decode step's matrix products are the library's, and they are recorded into
-    the graph with everything else.  Two layers of each benchmark shape, bfloat16, 20 and 64
+    """A decode step of 20 requests takes library products (the head, and whatever neither slices nor an
+    epilogue takes), one of 64 products in tiles besides, and both are recorded into the graph with everything
+    else.  Two layers of each benchmark shape, bfloat16, 20 and 64
     requests: every replay against the same step run eagerly by a second engine, with eager work
     (a prompt, synchronising copies) between the replays."""
     from infinicore_infer_amd.engine import Engine, StepEntry

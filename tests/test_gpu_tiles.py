@@ -44,9 +44,9 @@ def test_tile_rule_cpu():
     for m in (1, 33, 64, 65, 871, 4096, 100000):
         for n in (8, 64, 2304, 32768):
             for k in (64, 1536, 16384):
-                for mode in (0, 1):
-                    assert 0 <= lib.ic_gemm_tiles_plan(m, n, k, mode) < len(TILES)
-                    assert not (m <= 32 and lib.ic_gemm_tiles_pays(m, n, k, mode))
+                for mode in (False, True):
+                    assert 0 <= ops.gemm_tiles_plan(m, n, k, mode) < len(TILES)
+                    assert not (m <= 32 and ops.gemm_tiles_pays(m, n, k, mode))
     sup = lib.ic_gemm_tiles_supported
     assert sup(100, 64, 128, 128, 128, 64, 0) and sup(100, 64, 128, 136, 144, 72, 0) and sup(100, 64, 128, 128, 128, 32, 1)
     assert not sup(100, 64, 96, 96, 96, 64, 0)               # K in whole stages
@@ -149,17 +149,21 @@ def test_tiles_over_long_walks(tile, swiglu):
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(33, 7680, 1536), (65, 512, 512), (129, 1536, 3840), (871, 2560, 1536), (1045, 1536, 1536), (2049, 2304, 2304)])
 def test_chosen_tiles_and_their_replays(M, N, K):
-    """The tile that the rule names, recorded and replayed with other rows in between."""
+    """ops.product runs the tile that the rule names, and that recorded and replayed with other rows in between."""
+    assert ops.gemm_tiles_pays(M, N, K)
     a, w = _operands(M, N, K, M)
-    ad, wd, out = a.cuda(), w.cuda(), torch.empty(M, N, dtype=BF16, device="cuda")
+    ad, wd, out, chosen = a.cuda(), w.cuda(), *(torch.empty(M, N, dtype=BF16, device="cuda") for _ in range(2))
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):
-        ops.product(ad, wd, out)
+        ops.product(ad, wd, chosen)
+        ops.gemm_tiles(ad, wd, out, tile=ops.gemm_tiles_plan(M, N, K))
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph, stream=side):
             ops.gemm_tiles(ad, wd, out)
     torch.cuda.current_stream().wait_stream(side)
+    _check(a, w, chosen, False)
+    assert torch.equal(chosen, out)
     for _ in range(3):
         a = a.roll(1, 0)
         ad.copy_(a)

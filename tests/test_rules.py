@@ -62,6 +62,27 @@ def test_products_of_a_layer_at_the_benchmark_sizes():
     assert ops.rule_tail(BF16, _Mat(20, 64), _Mat(64, 64)) == ops.TAIL_PLAIN
 
 
+def test_products_in_tiles_and_their_guards():
+    """Gate/up with SwiGLU and QKV with rotary and cache write in tiles: taken for many rows, and every operand that the tiles' epilogues cannot take is
+    refused by itself (the caller then runs the product and the following kernel apart)."""
+    from infinicore_infer_amd.kernels.lib import get_lib
+    lib, at = get_lib(), 1 << 20                             # addresses that are never read: 16-byte aligned
+    gu = dict(dtype=1, a=at, w=at, c=at, rows=871, n=7680, k=1536, lda=1536, ldw=1536, ldc=3840)
+    ask = lambda **k: lib.ic_rule_gate_up_tiles(*dict(gu, **k).values())
+    assert ask() == 1 and ask(rows=33) == 1 and ask(lda=1544, ldw=1600, ldc=3848) == 1
+    for bad in (dict(dtype=0), dict(a=at + 2), dict(w=at + 8), dict(c=at + 4), dict(rows=32), dict(rows=0), dict(n=7688), dict(k=1504), dict(lda=1540),
+                dict(ldw=1540), dict(ldc=3844), dict(ldc=3832), dict(lda=1528), dict(n=1 << 20, ldc=1 << 19, k=4096, lda=4096, ldw=4096)):
+        assert ask(**bad) == 0, bad
+    qkv = dict(dtype=1, a=at, w=at, c=at, rows=871, k=1536, lda=1536, ldw=1536, ldc=2560, cos=at, sin=at, kc=at, vc=at, nh=24, nkv=8, dh=64, rot=64, ps=64)
+    ask = lambda **k: lib.ic_rule_qkv_tiles(*dict(qkv, **k).values())
+    assert ask() == 1 and ask(rows=33) == 1 and ask(ps=7) == 1 and ask(nh=12, nkv=4, dh=128, rot=128) == 1 and ask(ldc=1536) == 1
+    for bad in (dict(dtype=0), dict(rot=32), dict(rot=0), dict(nkv=0), dict(dh=80, rot=80), dict(dh=16, rot=16), dict(rows=32), dict(k=1504), dict(lda=1540),
+                dict(ldw=1540), dict(ldc=2564), dict(ldc=1528), dict(ps=0), dict(nh=0), dict(a=at + 2), dict(w=at + 2), dict(c=at + 2), dict(cos=at + 4),
+                dict(sin=at + 4), dict(kc=at + 8), dict(vc=at + 8), dict(cos=None), dict(kc=None), dict(vc=None)):
+        assert ask(**bad) == 0, bad
+    assert ask(rows=2048, nh=36, nkv=36, k=2304, lda=2304, ldw=2304, ldc=6912) == 0          # the largest tile fits best, and has no room for this
+
+
 def test_attention_kernels_of_a_step():
     ops = _ops()
     both = ops.ATTN_SINGLE_TOKENS | ops.ATTN_PORTIONS
