@@ -79,7 +79,7 @@ IC_EXPORT int ic_attn_mixed_parts_of_step(int dtype, int n_tiles, int nh, int dh
     const long long blocks = (long long)n_tiles * nh;
     if (dtype == IC_BF16 && parts == 1 && len >= 12 && blocks > 0 && blocks <= kPfCounters && (dh == 64 || dh == 128) && 4 * blocks <= 5LL * compute_units) {
         parts = 2;
-        len = (len + 1) / 2;
+        len = len > 22 ? (len + 1) / 2 : 11;                // (a shorter walk of the same step stays whole)
     }
     if (part_len) *part_len = len;
     return parts;

@@ -15,9 +15,10 @@
 // have no register results, so nothing but LDS is written while they are in flight.
 //
 // What bounds it.  Few tiles (up to one a compute unit): a stage's products at the matrix cores' rate plus its barrier and what the loads hold up the
-// products: 256 x 256 0.96 us a stage (0.87 with products alone), 192 x 192 0.58 (0.49), 128 x 128 0.30 (0.23), and about 4 us for launch, first
+// products: 256 x 256 0.96 us a stage (0.87 with products alone), 128 x 128 0.30 (0.23), and about 4 us for launch, first
 // loads and the way out.  128 x 128 tiles take all of a unit's 64 bytes a cycle from L2 for their loads, 256 x 256 half of it, hence the large
-// tiles where there are rows and columns enough.  The whole chip busy for long: its power, the clock gives way (256 x 256: 1.38..1.5 us a stage).
+// tiles where there are rows and columns enough.  The whole chip busy for long: its power, the clock gives way (256 x 256: 1.43 us a stage in gate/up of
+// 16,384 x 32,768 x 4,096, 1.68 in 16,384 x 4,096 x 16,384).
 // Large tiles take four waves of up to 512 registers a block: eight waves of half the size read 1.5 times as much from LDS
 // (256 x 256: 1.07 us a stage).  v_mfma_f32_32x32x16_bf16 instead of 16x16x32 is no faster (0.96 and 0.97).
 //
@@ -192,7 +193,7 @@ __global__ void __launch_bounds__(T::WAVES * 64, T::BLOCKS_PER_CU) gemm_tiles_ke
 
     // The loads of stage s + STAGES go into the buffer of stage s from that stage's barrier on: with more than two stages SPREAD of them in each
     // k-step up to the next barrier, so that they do not queue up behind one another (a 1 KB load takes the unit 16 cycles, and a wave that
-    // waits to issue one issues no products: 192 x 192 tiles 0.72 -> 0.58 us a stage); with two the last ones would have to arrive too soon.
+    // waits to issue one issues no products: 128 x 128 tiles 0.40 -> 0.30 us a stage); with two the last ones would have to arrive too soon.
     constexpr int SPREAD = STAGES > 2 ? (LOADS + STEPS - 1) / STEPS : LOADS;
     // the first stages, the last of them without what the first stage's steps load
     each<STAGES>([&](auto sc) {

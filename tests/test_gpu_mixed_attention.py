@@ -62,7 +62,7 @@ def test_long_chats_beside_short_prompts_cpu():
     # a walk that the tiles alone leave whole is cut in two here from 12 key tiles on, while the blocks are few enough for it
     cut = lambda nh, dh, tiles, end, entry=ops.attention_mixed_parts_of_step: entry(BF16, tiles, nh, dh, end, 0, 256)
     alone = ops.attention_prefill_parts_of_step
-    assert cut(24, 64, 8, 1023, alone)[0] == 1 and cut(24, 64, 8, 1023) == (2, 8) and cut(32, 128, 10, 767) == (2, 6)
+    assert cut(24, 64, 8, 1023, alone)[0] == 1 and cut(24, 64, 8, 1023) == (2, 11) and cut(32, 128, 10, 767) == (2, 11) and cut(32, 128, 10, 2047) == (2, 16)
     assert cut(24, 64, 8, 703) == cut(24, 64, 8, 703, alone) == (1, 11) and cut(32, 128, 11, 1023)[0] == 1
     assert cut(24, 64, 4, 1023) == cut(24, 64, 4, 1023, alone) and cut(24, 64, 4, 1023)[0] == 3
     assert _packed([300, 1], [2000, 7]).max_tile_position == 2299
