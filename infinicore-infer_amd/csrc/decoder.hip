@@ -5,7 +5,7 @@
 // few-row products with their epilogues (rotary and cache write after QKV; residual add, the next norm's
 // weight and sums of squares after O and down; SwiGLU after gate/up), the norm between two products being
 // split over them; more rows take the products in tiles (QKV with rotary and cache write, gate/up with SwiGLU in
-// the epilogue) or the library's, as ic_product chooses, float32 the library's, and the norm, rotary and activation kernels.
+// the epilogue) or the library's, float32 the product of bfloat16 parts or the library's, as ic_product chooses, and the norm, rotary and activation kernels.
 // Single-token rows go to the split-key attention kernel, prompt portions to the tiled one, both of a mixed step to one launch
 // where that is faster, what neither takes to the general one.
 #include "common.h"

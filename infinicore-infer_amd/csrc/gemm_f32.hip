@@ -1,0 +1,425 @@
+// C[M, N] = alpha * A[M, K] * W[N, K]^T in float32 for many rows M, on the bfloat16 matrix cores.
+//
+// A float32 number is the sum of three bfloat16 numbers: its upper 16 bits, those of what is left, and the rest, which has 8 bits at most; every
+// subtraction is exact.  Of the nine products of parts the six of 2^-16 and more are summed in float32, a0 w0 + a0 w1 + a1 w0 + a1 w1 + a0 w2 + a2 w0, the
+// small ones first; the three left out are some 2^-25 of a product, under the rounding of its float32 sum.  Six bfloat16 products take 96 cycles where
+// the float32 instruction takes 256.  a0 w0 has a sum of its own, which is rounded once per 32 k; the five others are summed beside it.  Error against 64 bits
+// (relative, 2-norm; normal values, 1,536 / 3,840 / 5,760 k, 33..2,048 rows): 1.3..2.4e-7 / 1.9..3.9e-7 / 2.3..4.8e-7, the library's float32 product 3.5..7.1e-7 / 0.56..1.1e-6 / 0.67..1.4e-6
+// (with all six in one sum 2.9..6.1e-7 / 4.8..9.8e-7).  A result that is not finite is summed again in plain float32, since inf - inf is no part of infinity.
+//
+// A is split once per product by a kernel before (3.7 us and 10 bytes a value), into the order of the matrix cores' operands: 1 KB per 16 rows, 32 k and part, which go to LDS and
+// into registers as they lie.  W stays float32 in memory and in LDS (rows of 128 bytes, the 16-byte chunk c of row r at c ^ (r / 2 % 8)) and is split in registers by the
+// one wave that multiplies it: 22 vector instructions per 4 values and 6 MT products, where MT row tiles of 16 share the split.  The matrix cores hide two
+// vector instructions per product of 16 cycles (measured: 8.3 ns a product with none to two, 10.3 with three, 12.1 with four), hence no split of A in the loop
+// (2.7 per product, 11.5 ns) and blocks of four waves side by side over all rows of the tile, not two by two (W split twice).
+// Loads are sent STAGES - 1 stages of 32 k ahead (two stages of 57 KB: 1.7 us a stage that multiplies for 0.85; three of 41 KB: 0.96).
+//
+// What bounds it: the products' rate, 8.9 ns each (a lone wave a SIMD, power), some 5 us for launch, first loads and way out; the fill of the last round of blocks.  Few rows:
+// the weights' bytes.  517 x 7,680 x 1,536: 61.6 us and 4.2 for the split, 1.19 PFLOP/s of parts (library 99); 517 x 1,536 x 3,840 in 4 slices 33.9 (library 61); 2,048 x 7,680 x 1,536 233 (391).
+//
+// Few tiles: K in slices, blocks of their own, whose sums a second kernel adds up.
+#include "common.h"
+#include "infinicore_infer_variants.h"
+#include <type_traits>
+#include <utility>
+
+namespace {
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
+typedef __bf16 v8b __attribute__((ext_vector_type(8)));
+
+struct F32Args {
+    const float* A;
+    const float* W;
+    float* C;                       // slice s at C + s * slice_stride
+    const unsigned char* parts;     // A in three parts (split_rows_kernel)
+    int M, N, K, lda, ldw, ldc;
+    int tiles_m, tiles_n, slices;
+    long long slice_stride;
+    float alpha;
+};
+
+template <typename F, int... Is> __device__ __forceinline__ void each_of(F&& f, std::integer_sequence<int, Is...>) {
+    (f(std::integral_constant<int, Is>{}), ...);
+}
+template <int N, typename F> __device__ __forceinline__ void each(F&& f) { each_of(f, std::make_integer_sequence<int, N>{}); }
+
+// 16 bytes a lane from base + off to LDS at lds + 16 * lane.
+__device__ __forceinline__ void load_to_lds(unsigned lds, unsigned off, const char* base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+}
+// waits until at most N of this wave's loads are on their way and all its LDS reads are done
+template <int N> __device__ __forceinline__ void wait_loads() {
+    static_assert(N >= 0 && N < 64, "vmcnt has six bits");
+    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (0 << 8));
+}
+
+// Ties the accumulators to a place between the products written as assembly, whose results the compiler does not know to wait for.
+template <int N, int M> __device__ __forceinline__ void settled(v4f (&acc)[N][M]) {
+    asm volatile("s_nop 15");
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+#pragma unroll
+        for (int m = 0; m < M; ++m) asm volatile("" : "+a"(acc[n][m]));
+    asm volatile("s_nop 7");
+}
+
+// Four values in three bfloat16 parts each: step O of 22 (level O / 10: the parts' upper halves are packed, then taken off).
+struct Split4 {
+    float y[4], t[4];
+    unsigned p[3][2];
+};
+template <int O> __device__ __forceinline__ void split_step(Split4& s) {
+    constexpr int L = O / 10, Q = O % 10;
+    if constexpr (Q < 2) s.p[L][Q] = __builtin_amdgcn_perm(__float_as_uint(s.y[2 * Q + 1]), __float_as_uint(s.y[2 * Q]), 0x07060302);
+    else if constexpr (Q < 6) s.t[Q - 2] = __uint_as_float(__float_as_uint(s.y[Q - 2]) & 0xffff0000u);
+    else s.y[Q - 6] -= s.t[Q - 6];
+}
+constexpr int kSplitSteps = 22;
+
+template <int MT_, int NT_, int STAGES_> struct Shape {
+    static constexpr int MT = MT_, NT = NT_, STAGES = STAGES_, BM = 16 * MT, BN = 64 * NT;
+    static constexpr int PIECES = 3 * MT + 8 * NT, LOADS = (PIECES + 3) / 4, STAGE_BYTES = 1024 * PIECES;
+    static_assert(STAGES >= 2 && STAGES * STAGE_BYTES <= 160 * 1024 && LOADS * (STAGES - 1) < 64, "limits");
+};
+
+template <typename T>
+__global__ void __launch_bounds__(256, 1) gemm_f32_kernel(F32Args a) {
+    constexpr int MT = T::MT, NT = T::NT, STAGES = T::STAGES, LOADS = T::LOADS, PIECES = T::PIECES;
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[STAGES * T::STAGE_BYTES];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, kq = lane >> 4;
+
+    const int tiles = a.tiles_m * a.tiles_n, total = tiles * a.slices;
+    const int xcd = blockIdx.x & 7, nth = blockIdx.x >> 3;
+    const int v = xcd * (total >> 3) + min(xcd, total & 7) + nth;
+    const int slice = v / tiles, t = v - slice * tiles;
+    const int bn = t / a.tiles_m, bm = t - bn * a.tiles_m;
+    const int m0 = bm * T::BM, n0 = bn * T::BN;
+    const int KG = a.K / 32, RT = (a.M + 15) / 16;
+    const int s_first = (int)((long long)slice * KG / a.slices), s_end = (int)((long long)(slice + 1) * KG / a.slices), n_stages = s_end - s_first;
+
+    const char* const base_a = (const char*)a.parts + ((size_t)bm * MT * KG + s_first) * 3072;
+    const char* const base_w = (const char*)(a.W + (size_t)n0 * a.ldw) + (size_t)s_first * 128;
+    // this wave's pieces of a stage: of 1 KB, the rows of A's parts first
+    unsigned off[LOADS];
+    each<LOADS>([&](auto at) {
+        constexpr int I = decltype(at)::value;
+        const int piece = min(wave + 4 * I, PIECES - 1);
+        if (piece < 3 * MT) {
+            const int rt = piece / 3;
+            off[I] = (unsigned)min(rt, RT - 1 - bm * MT) * (unsigned)(KG * 3072) + (piece - 3 * rt) * 1024 + lane * 16;
+        } else {
+            const int row = 8 * (piece - 3 * MT) + (lane >> 3);
+            off[I] = (unsigned)min(row, a.N - 1 - n0) * (unsigned)(a.ldw * 4) + 16 * ((lane & 7) ^ ((row >> 1) & 7));
+        }
+    });
+    const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds;
+    auto fetch = [&](auto at, unsigned s, unsigned into) {
+        constexpr int I = decltype(at)::value;
+        const int piece = min(wave + 4 * I, PIECES - 1);
+        const bool is_a = 4 * I + 3 < 3 * MT || (4 * I < 3 * MT && piece < 3 * MT);
+        load_to_lds(into + 1024 * piece, off[I], is_a ? base_a + (size_t)(s * 3072) : base_w + (size_t)(s * 128));
+    };
+    auto clamped = [&](int s) { return (unsigned)min(s, n_stages - 1); };
+
+    v4f acc[NT][MT], low[NT][MT];                                  // the sums of a0 w0, and of the five smaller products
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = low[nt][mt] = v4f{0.f, 0.f, 0.f, 0.f};
+
+    settled(acc);
+    settled(low);
+    each<STAGES>([&](auto sc) { each<LOADS>([&](auto i) { fetch(i, clamped(sc), lds0 + decltype(sc)::value * T::STAGE_BYTES); }); });
+    const unsigned char* const pa_ = lds + lane * 16;
+    const unsigned char* const pw_ = lds + MT * 3072 + (wave * (16 * NT) + r) * 128;
+    const int sw = (r >> 1) & 7, place0 = 16 * (kq ^ sw), place1 = 16 * ((4 + kq) ^ sw);
+    constexpr int U = 2 * NT;                                      // halves of a wave's operands of W
+    v8b pa[2][MT][3];
+    Split4 pw[2][U];
+    auto w_of = [&](auto uc, auto cur, int buf) {
+        constexpr int u = decltype(uc)::value;
+        const v4f x = *reinterpret_cast<const v4f*>(pw_ + (u / 2) * 2048 + buf * T::STAGE_BYTES + (u % 2 ? place1 : place0));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) pw[decltype(cur)::value][u].y[e] = x[e];
+    };
+    auto a_of = [&](auto ic, auto cur, int buf) {
+        constexpr int i = decltype(ic)::value;
+        pa[decltype(cur)::value][i / 3][i % 3] = *reinterpret_cast<const v8b*>(pa_ + i * 1024 + buf * T::STAGE_BYTES);
+    };
+    using Zero = std::integral_constant<int, 0>;
+    wait_loads<LOADS * (STAGES - 1)>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    each<3 * MT>([&](auto i) { a_of(i, Zero{}, 0); });
+    each<U>([&](auto u) {
+        w_of(u, Zero{}, 0);
+        each<kSplitSteps>([&](auto o) { split_step<decltype(o)::value>(pw[0][decltype(u)::value]); });
+    });
+
+    // One k-step of 32: the operands CUR are multiplied; those of the next step are read from LDS and W's split; the loads of stage s + STAGES go out.
+    auto step = [&](int s, int buf, auto cur) {
+        constexpr int CUR = decltype(cur)::value, P = 6 * MT * NT, D = U < 2 ? U : 2;
+        using Next = std::integral_constant<int, CUR ^ 1>;
+        const int next = buf + 1 == STAGES ? 0 : buf + 1;
+        wait_loads<LOADS * (STAGES - 2)>();
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        const unsigned from = clamped(s + STAGES), into = lds0 + buf * T::STAGE_BYTES;
+        each<D>([&](auto u) { w_of(u, Next{}, next); });
+        __builtin_amdgcn_sched_barrier(0);
+        each<P>([&](auto pc) {
+            constexpr int p = decltype(pc)::value, n = p / (6 * MT), term = p / MT % 6, mt = p % MT;
+            constexpr int X[6] = {2, 0, 1, 1, 0, 0}, Y[6] = {0, 2, 1, 0, 1, 0};
+            const Split4 &lo = pw[CUR][2 * n], &hi = pw[CUR][2 * n + 1];
+            const v8b w = __builtin_bit_cast(v8b, v4u{lo.p[X[term]][0], lo.p[X[term]][1], hi.p[X[term]][0], hi.p[X[term]][1]});
+            asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(term == 5 ? acc[n][mt] : low[n][mt]) : "v"(w), "v"(pa[CUR][mt][Y[term]]));
+            // the splits are dealt over the products but for the first few, which the reads from LDS have to arrive
+            constexpr int HOLD = P / 8, O0 = p < HOLD ? 0 : (p - HOLD) * U * kSplitSteps / (P - HOLD), O1 = p < HOLD ? 0 : (p + 1 - HOLD) * U * kSplitSteps / (P - HOLD);
+            constexpr int A0 = p * 3 * MT / P, A1 = (p + 1) * 3 * MT / P, L0 = p * LOADS / P, L1 = (p + 1) * LOADS / P;
+            each<A1 - A0>([&](auto k) { a_of(std::integral_constant<int, A0 + decltype(k)::value>{}, Next{}, next); });
+            each<L1 - L0>([&](auto k) { fetch(std::integral_constant<int, L0 + decltype(k)::value>{}, from, into); });
+            each<O1 - O0>([&](auto k) {
+                constexpr int o = O0 + decltype(k)::value, u = o / kSplitSteps;
+                if constexpr (o % kSplitSteps == 0 && u + D < U) w_of(std::integral_constant<int, u + D>{}, Next{}, next);
+                split_step<o % kSplitSteps>(pw[CUR ^ 1][u]);
+            });
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        return next;
+    };
+    int s = 0, buf = 0;
+    for (; s + 1 < n_stages; s += 2) {
+        buf = step(s, buf, Zero{});
+        buf = step(s + 1, buf, std::integral_constant<int, 1>{});
+    }
+    if (s < n_stages) step(s, buf, Zero{});
+    settled(acc);
+    settled(low);
+    wait_loads<0>();                                               // (nothing may land in LDS after the block)
+
+    float* const C = a.C + (size_t)slice * a.slice_stride;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        const int m = m0 + 16 * mt + r;
+        if (m >= a.M) continue;
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            const int n = n0 + (wave * NT + nt) * 16 + 4 * kq;
+            if (n >= a.N) continue;
+            v4f x = acc[nt][mt] + low[nt][mt];
+            bool odd = false;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) odd = odd || !(fabsf(x[e]) <= 3.402823466e38f);
+            if (odd) {
+                for (int e = 0; e < 4 && n + e < a.N; ++e) {
+                    const float *pa1 = a.A + (size_t)m * a.lda, *pw1 = a.W + (size_t)(n + e) * a.ldw;
+                    float d = 0.f;
+                    for (int k = 32 * s_first; k < 32 * s_end; ++k) d = fmaf(pa1[k], pw1[k], d);
+                    x[e] = d;
+                }
+            }
+            x *= a.alpha;
+            float* const to = C + (size_t)m * a.ldc + n;
+            if (n + 4 <= a.N) *reinterpret_cast<v4f*>(to) = x;
+            else
+                for (int e = 0; n + e < a.N; ++e) to[e] = x[e];
+        }
+    }
+}
+
+// The rows of A in three parts, in the order of the matrix cores' operands: [row / 16][k / 32][part][lane][8], lane l row l % 16, k 4 (l / 16) .. + 3 and 16 on.
+__global__ void __launch_bounds__(256) split_rows_kernel(const float* A, int lda, int M, int K, uint4* out) {
+    const int lane = threadIdx.x & 63, r = lane & 15, kq = lane >> 4, KG = K / 32;
+    const int w = blockIdx.x * 4 + (threadIdx.x >> 6), rt = w / KG, kg = w - rt * KG;
+    if (rt >= (M + 15) / 16) return;
+    const float* const from = A + (size_t)min(16 * rt + r, M - 1) * lda + 32 * kg + 4 * kq;
+    Split4 s[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const v4f x = *reinterpret_cast<const v4f*>(from + 16 * h);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[h].y[e] = x[e];
+        each<kSplitSteps>([&](auto o) { split_step<decltype(o)::value>(s[h]); });
+    }
+#pragma unroll
+    for (int p = 0; p < 3; ++p) out[(size_t)w * 192 + p * 64 + lane] = uint4{s[0].p[p][0], s[0].p[p][1], s[1].p[p][0], s[1].p[p][1]};
+}
+
+// C = alpha * the sum of the slices P [S][M][N]; N a multiple of 4.
+__global__ void __launch_bounds__(256) sum_slices_kernel(const v4f* P, int S, int M, int N4, float* C, int ldc, float alpha) {
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x, n = (long long)M * N4;
+    if (i >= n) return;
+    v4f x = P[i];
+    for (int s = 1; s < S; ++s) x += P[i + s * n];
+    const int m = (int)(i / N4);
+    *reinterpret_cast<v4f*>(C + (size_t)m * ldc + 4 * (int)(i - (long long)m * N4)) = alpha * x;
+}
+
+template <typename T> int launch(F32Args a, hipStream_t stream) {
+    a.tiles_m = (a.M + T::BM - 1) / T::BM;
+    a.tiles_n = (a.N + T::BN - 1) / T::BN;
+    const long long blocks = (long long)a.tiles_m * a.tiles_n * a.slices;
+    if (blocks > (1LL << 30)) return IC_ERR_ARG;
+    hipLaunchKernelGGL((gemm_f32_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+    return ic_launch_status();
+}
+
+// The shapes of a block, smallest first, and what one costs in microseconds: FIXED + rounds * (ROUND + k-steps of 32 * STAGE * (1 + FULL * x)), x the part of the units
+// (256 where this was fitted) that have a block, or the weights' bytes at 6 TB/s where those take longer.  Fitted to 11,700 timed products (13 pairs of N in 512..12,288 and K in
+// 768..5,760, 1..2,048 rows, one to four slices, weights out of memory): the shape and slices with the least cost lose 0.5 % to the best on average, 3 % at the 95th percentile.
+#define IC_F32_SHAPES(X) \
+    /* number, FIXED, STAGE, FULL, ROUND, shape: row tiles of 16, column tiles of 64, stages */ \
+    X(0, 1.69, 0.226, 0.13, 1.80, 1, 1, 8) \
+    X(1, 1.80, 0.232, 0.26, 2.01, 2, 1, 8) \
+    X(2, 1.90, 0.280, 0.15, 2.41, 3, 1, 8) \
+    X(3, 1.92, 0.294, 0.20, 2.50, 4, 1, 7) \
+    X(4, 1.73, 0.341, 0.20, 2.81, 5, 1, 6) \
+    X(5, 1.82, 0.383, 0.22, 3.13, 6, 1, 6) \
+    X(6, 1.65, 0.416, 0.26, 3.23, 7, 1, 5) \
+    X(7, 1.89, 0.483, 0.23, 3.45, 4, 2, 5) \
+    X(8, 1.87, 0.560, 0.24, 3.97, 5, 2, 5) \
+    X(9, 1.95, 0.647, 0.24, 4.16, 6, 2, 4) \
+    X(10, 1.61, 0.705, 0.28, 4.92, 7, 2, 4) \
+    X(11, 1.93, 0.759, 0.29, 5.20, 8, 2, 4) \
+    X(12, 1.87, 0.670, 0.23, 4.22, 4, 3, 4) \
+    X(13, 1.81, 0.874, 0.24, 5.38, 6, 3, 3) \
+    X(14, 1.91, 1.106, 0.28, 6.44, 8, 3, 3)
+
+constexpr int kShapes = 15, kMaxSlices = 4;
+struct ShapeCost { int bm, bn; double fixed, stage, full, round; };
+constexpr ShapeCost kCosts[kShapes] = {
+#define X(I, FIXED, STAGE, FULL, ROUND, MT, NT, ST) {16 * MT, 64 * NT, FIXED, STAGE, FULL, ROUND},
+    IC_F32_SHAPES(X)
+#undef X
+};
+
+double cost_of(const ShapeCost& c, int M, int N, int K, int slices, int units) {
+    const double tm = (M + c.bm - 1) / c.bm, x = tm * ((N + c.bn - 1) / c.bn) * slices / units, steps = (double)(K / 32) / slices;
+    const double walk = c.fixed + __builtin_ceil(x) * (c.round + steps * c.stage * (1.0 + c.full * (x < 1.0 ? x : 1.0)));
+    const double read = 3.0 + 4.0 * N * K * (1.0 + 0.3 * (tm < 5 ? tm - 1 : 4)) / (6e6 * units / 256.0);
+    return walk > read ? walk : read;
+}
+
+struct Plan { int shape, slices; double cost; };
+// adds_slices: whoever follows adds the slices up (else a kernel of its own does).
+Plan plan_for(int M, int N, int K, bool adds_slices, int max_slices, int units) {
+    Plan best{-1, 1, 0.0};
+    for (int s = 1; s <= max_slices && s <= kMaxSlices && s <= K / 32 && (s == 1 || N % 4 == 0); ++s) {
+        const double bytes = 4.0 * M * N, extra = s == 1 ? 0.0 : adds_slices ? (s - 1) * bytes / 5e6 : 3.5 + (s + 1) * bytes / 6e6;
+        for (int i = 0; i < kShapes; ++i) {
+            const double c = cost_of(kCosts[i], M, N, K, s, units) + extra;
+            if (best.shape < 0 || c < best.cost) best = Plan{i, s, c};
+        }
+    }
+    return best;
+}
+
+bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+
+// Whole k-steps, 16-byte pieces of every row, byte offsets within 32 bits.
+bool takes(int M, int N, int K, int lda, int ldw, int ldc) {
+    if (M <= 0 || M > (1 << 26) || N <= 0 || N > (1 << 30) || K <= 0 || K > (1 << 20) || K % 32 || lda < K || ldw < K || ldc < N || lda % 4 || ldw % 4 || ldc % 4) return false;
+    return (long long)ldw * 4 * 192 < (1LL << 32) && (long long)((M + 15) / 16) * (K / 32) < (1LL << 30) && (long long)((M + 15) / 16) * ((N + 63) / 64) * kMaxSlices < (1LL << 30);
+}
+
+long long parts_bytes(int M, int K) { return (long long)((M + 15) / 16) * (K / 32) * 3072; }
+
+int split_rows(const float* A, int lda, int M, int K, void* parts, hipStream_t stream) {
+    const long long waves = (long long)((M + 15) / 16) * (K / 32);
+    hipLaunchKernelGGL(split_rows_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream, A, lda, M, K, (uint4*)parts);
+    return ic_launch_status();
+}
+
+int run(const F32Args& a, int shape, hipStream_t stream) {
+    switch (shape) {
+#define X(I, FIXED, STAGE, FULL, ROUND, ...) case I: return launch<Shape<__VA_ARGS__>>(a, stream);
+        IC_F32_SHAPES(X)
+#undef X
+    }
+    return IC_ERR_ARG;
+}
+
+// Rows that are split and multiplied at a time: all, or equal runs of whole row tiles, as many as the workspace holds.
+int rows_at_once(int M, int K, long long workspace_bytes) {
+    const long long most = workspace_bytes / ((K / 32) * 3072LL) * 16;
+    if (most >= M) return M;
+    if (most < 16) return 0;
+    const long long runs = (M + most - 1) / most;
+    return (int)(((M + runs - 1) / runs + 15) / 16 * 16);
+}
+
+int product(const float* A, const float* W, float* C, int M, int N, int K, int lda, int ldw, int ldc, float alpha, int shape, int slices, void* workspace,
+            long long workspace_bytes, hipStream_t stream) {
+    const int at_once = rows_at_once(M, K, workspace_bytes);
+    if (at_once <= 0) return IC_ERR_ARG;
+    if (slices > 1 && (at_once < M || parts_bytes(M, K) + 4LL * slices * M * N > workspace_bytes)) return IC_ERR_ARG;
+    for (int m = 0; m < M; m += at_once) {
+        const int rows = M - m < at_once ? M - m : at_once;
+        const float* const a0 = A + (size_t)m * lda;
+        float* const sums = slices > 1 ? (float*)((char*)workspace + parts_bytes(M, K)) : C + (size_t)m * ldc;
+        int st = split_rows(a0, lda, rows, K, workspace, stream);
+        if (st) return st;
+        st = run(F32Args{a0, W, sums, (const unsigned char*)workspace, rows, N, K, lda, ldw, slices > 1 ? N : ldc, 0, 0, slices, (long long)rows * N,
+                         slices > 1 ? 1.0f : alpha}, shape, stream);
+        if (st) return st;
+    }
+    if (slices > 1) {
+        const long long n = (long long)M * (N / 4);
+        if (n > (1LL << 38)) return IC_ERR_ARG;
+        hipLaunchKernelGGL(sum_slices_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream,
+                           (const v4f*)((const char*)workspace + parts_bytes(M, K)), slices, M, N / 4, C, ldc, alpha);
+        return ic_launch_status();
+    }
+    return IC_OK;
+}
+
+int most_slices(int M, int N, int K, long long workspace_bytes) {
+    int s = kMaxSlices;                                            // (none where the rows do not fit at once)
+    while (s > 1 && parts_bytes(M, K) + 4LL * s * M * N > workspace_bytes) --s;
+    return s;
+}
+
+}  // namespace
+
+IC_EXPORT int ic_gemm_f32_supported(int M, int N, int K, int lda, int ldw, int ldc) { return takes(M, N, K, lda, ldw, ldc); }
+
+IC_EXPORT int ic_gemm_f32_plan_on(int M, int N, int K, int adds_slices, int units, int* slices) {
+    if (M <= 0 || N <= 0 || K < 32 || units <= 0) return -1;
+    const Plan p = plan_for(M, N, K, adds_slices != 0, kMaxSlices, units);
+    if (slices) *slices = p.slices;
+    return p.shape;
+}
+
+// Whether the split, the product and the sum of its slices beat the library's float32 product, whose time is within 17 % (rms) of 12 us or 8.7 us and 127 TFLOP/s; from 33 rows on,
+// since fewer are a matter of the weights' bytes, which it reads as fast (8 x 7,680 x 1,536: 13 us, the split alone 4).  Over the sweep above the choice loses 1.1 % to the
+// better of the two.  130 x 7,680 x 1,536: 35 -> 29, 256 x 2,560 x 1,536: 28 -> 22, on the other side 96 x 2,560 x 1,536: 11 against 18.
+IC_EXPORT int ic_gemm_f32_pays_on(int M, int N, int K, int units) {
+    if (M <= 32 || N <= 0 || K < 32 || units <= 0) return 0;
+    const double products = 2.0 * M * N * K / (127e6 * units / 256.0) + 8.7;
+    return 3.73 + 10.0 * M * K / (14.8e6 * units / 256.0) + plan_for(M, N, K, false, kMaxSlices, units).cost < (products > 12.0 ? products : 12.0);
+}
+
+IC_EXPORT int ic_gemm_f32_pays(int M, int N, int K) { return ic_gemm_f32_pays_on(M, N, K, compute_units()); }
+
+IC_EXPORT long long ic_gemm_f32_parts_bytes(int M, int K) { return M > 0 && K >= 32 ? parts_bytes(M, K) : 0; }
+
+// The whole product.  workspace (16-byte aligned): A's parts, or as many rows of them at a time as it holds (16 at least), and the slices where they fit too.
+IC_EXPORT int ic_gemm_f32(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, float alpha, void* workspace,
+                          long long workspace_bytes, hipStream_t stream) {
+    if (M <= 0) return IC_OK;
+    if (!A || !W || !C || !workspace || !takes(M, N, K, lda, ldw, ldc) || !aligned16(A) || !aligned16(W) || !aligned16(C) || !aligned16(workspace)) return IC_ERR_ARG;
+    const Plan p = plan_for(rows_at_once(M, K, workspace_bytes), N, K, false, most_slices(M, N, K, workspace_bytes), compute_units());
+    return product((const float*)A, (const float*)W, (float*)C, M, N, K, lda, ldw, ldc, alpha, p.shape, p.slices, workspace, workspace_bytes, stream);
+}
+
+IC_EXPORT int ic_gemm_f32_cfg(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, float alpha, int shape, int slices, void* workspace,
+                              long long workspace_bytes, hipStream_t stream) {
+    if (M <= 0) return IC_OK;
+    if (!A || !W || !C || !workspace || !takes(M, N, K, lda, ldw, ldc) || !aligned16(A) || !aligned16(W) || !aligned16(C) || !aligned16(workspace) || shape < 0 ||
+        shape >= kShapes || slices < 1 || slices > kMaxSlices || slices > K / 32 || (slices > 1 && N % 4)) return IC_ERR_ARG;
+    return product((const float*)A, (const float*)W, (float*)C, M, N, K, lda, ldw, ldc, alpha, shape, slices, workspace, workspace_bytes, stream);
+}

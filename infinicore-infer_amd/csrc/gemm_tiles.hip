@@ -598,7 +598,7 @@ IC_EXPORT int ic_gemm_tiles_rope_cfg(const void* A, const void* W, void* C, int 
     return rope_run(A, W, C, M, K, lda, ldw, ldc, positions, slots, cos_t, sin_t, kcache, vcache, nh, nkvh, dh, page_size, tile, stream);
 }
 
-// The product by the kernel that is faster for it, as timed (ic_product_tune) or by the rule: this file's or the library's.
+// The product by the kernel that is faster for it, as timed (ic_product_tune) or by the rule: this file's or the library's; in float32, by the rule, gemm_f32.hip's or the library's.
 IC_EXPORT int ic_product(const void* A, int a_dtype, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldw, int ldc, float alpha,
                          void* workspace, long long workspace_bytes, hipStream_t stream) {
     if (a_dtype == IC_BF16 && c_dtype == IC_BF16 && alpha == 1.0f && A && W && C && ic_gemm_tiles_supported(M, N, K, lda, ldw, ldc, EPI_BF16) &&
@@ -606,5 +606,8 @@ IC_EXPORT int ic_product(const void* A, int a_dtype, const void* W, void* C, int
         const int timed = ic_product_timed(M, N, K, lda, ldw, ldc);
         if (timed >= 0 ? timed : ic_gemm_tiles_pays(M, N, K, EPI_BF16)) return ic_gemm_tiles(A, W, C, M, N, K, lda, ldw, ldc, EPI_BF16, stream);
     }
+    if (a_dtype == IC_F32 && c_dtype == IC_F32 && A && W && C && workspace && aligned16(A) && aligned16(W) && aligned16(C) && aligned16(workspace) &&
+        ic_gemm_f32_supported(M, N, K, lda, ldw, ldc) && ic_gemm_f32_parts_bytes(16, K) <= workspace_bytes && ic_gemm_f32_pays(M, N, K))
+        return ic_gemm_f32(A, W, C, M, N, K, lda, ldw, ldc, alpha, workspace, workspace_bytes, stream);
     return ic_matmul(A, a_dtype, W, C, c_dtype, M, N, K, lda, ldw, ldc, alpha, workspace, workspace_bytes, stream);
 }

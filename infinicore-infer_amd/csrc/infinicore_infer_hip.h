@@ -165,9 +165,18 @@ int ic_gemm_tiles(const void* A, const void* W, void* C, int M, int N, int K, in
 // keys and values in the cache slots (slot < 0: not stored); keys and values of C are not written.  dh a power of two from 32 on.
 int ic_gemm_tiles_rope_supported(const void* A, const void* W, const void* C, int M, int K, int lda, int ldw, int ldc, const float* cos_t, const float* sin_t, const void* kcache, const void* vcache, int nh, int nkvh, int dh, int page_size);
 int ic_gemm_tiles_rope(const void* A, const void* W, void* C, int M, int K, int lda, int ldw, int ldc, const int* positions, const int* slots, const float* cos_t, const float* sin_t, void* kcache, void* vcache, int nh, int nkvh, int dh, int page_size, hipStream_t stream);
-// C[M, N] = alpha * A[M, K] W[N, K]^T for many rows by the faster of ic_gemm_tiles and ic_matmul; arguments and results as ic_matmul.  Which is the faster one
-// ic_gemm_tiles_pays says, or ic_product_tune found (matmul_library.hip).
+// C[M, N] = alpha * A[M, K] W[N, K]^T for many rows by the faster of ic_gemm_tiles, ic_gemm_f32 and ic_matmul; arguments and results as ic_matmul.  Which is the
+// faster one ic_gemm_tiles_pays and ic_gemm_f32_pays say, or ic_product_tune found (bfloat16; matmul_library.hip).
 int ic_product(const void* A, int a_dtype, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldw, int ldc, float alpha, void* workspace, long long workspace_bytes, hipStream_t stream);
+
+// ---- gemm_f32.hip ---------------------------------------------------------------------------------------
+// C[M, N] = alpha * A[M, K] W[N, K]^T in float32 on the bfloat16 matrix cores, every number as the sum of three bfloat16 numbers (errors as a float32 product's or smaller).  K a multiple
+// of 32, strides multiples of 4, operands and workspace 16-byte aligned; workspace: ic_gemm_f32_parts_bytes(M, K) bytes, or any smaller number from
+// ic_gemm_f32_parts_bytes(16, K) on (then the rows are taken in several launches).  ic_gemm_f32_pays: whether it beats ic_matmul.
+int ic_gemm_f32_supported(int M, int N, int K, int lda, int ldw, int ldc);
+int ic_gemm_f32_pays(int M, int N, int K);
+long long ic_gemm_f32_parts_bytes(int M, int K);
+int ic_gemm_f32(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, float alpha, void* workspace, long long workspace_bytes, hipStream_t stream);
 
 // ---- matmul_library.hip ------------------------------------------------------------------------------
 // The library (hipBLASLt) matrix product for many rows: C[M, N] = alpha * A[M, K] W[N, K]^T, bfloat16 operands with a

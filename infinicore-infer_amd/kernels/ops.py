@@ -627,7 +627,8 @@ def matmul_library(a, w, out, alpha: float = 1.0):
 
 
 def product(a, w, out, alpha: float = 1.0):
-    """matmul_library, or the package's own product in tiles (gemm_tiles) where that is the faster one (by the rule, or as product_tune found)."""
+    """matmul_library, or the package's own product where that is the faster one: in tiles (gemm_tiles; by the rule, or as product_tune found), in
+    float32 gemm_f32 (by the rule)."""
     return _matmul(get_lib().ic_product, a, w, out, alpha, "product")
 
 
@@ -646,6 +647,22 @@ def _matmul(entry, a, w, out, alpha, what):
     if st == -3:
         raise KernelError("%s: the library refused the product %d x %d x %d" % (what, M, N, K))
     check(st, what)
+    return out
+
+
+def gemm_f32(a, w, out, alpha: float = 1.0, shape=None, slices: int = 1, workspace=None):
+    """out[M, N] = alpha * a[M, K] @ w[N, K]^T in float32 on the bfloat16 matrix cores (csrc/gemm_f32.hip), K a multiple of 32.  shape, slices (tests): the
+    block's shape and the slices of K, which it chooses itself otherwise; workspace (tests): a uint8 tensor in place of the library's."""
+    _dev(a, w, out)
+    (M, K), N = a.shape, w.shape[0]
+    _need(a.dtype == w.dtype == out.dtype == torch.float32, "gemm_f32: float32 only")
+    _need(w.shape[1] == K and tuple(out.shape) == (M, N) and a.stride(1) == w.stride(1) == out.stride(1) == 1, "gemm_f32: shape or layout")
+    ws = _workspace(a.device) if workspace is None else workspace
+    args = (a.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K, a.stride(0), w.stride(0), out.stride(0), float(alpha))
+    if shape is None:
+        check(get_lib().ic_gemm_f32(*args, ws.data_ptr(), ws.numel(), _stream()), "gemm_f32")
+    else:
+        check(get_lib().ic_gemm_f32_cfg(*args, int(shape), int(slices), ws.data_ptr(), ws.numel(), _stream()), "gemm_f32")
     return out
 
 

@@ -5,8 +5,9 @@ The matrix product itself is the package's own matrix-core kernel for few rows
 (decoding, the output head) and for most many-row products, and a library
 routine for the rest (the reference calls the library's Gemm for every product,
 inference_context.cpp:59-79).
-float32 operands always go to the library with reduced-precision matrix modes
-switched off.
+float32 operands go to the package's product of bfloat16 parts (``ops.gemm_f32``, errors as a
+float32 product's or smaller) where it is the faster one, else to the library with reduced-precision
+matrix modes switched off.
 """
 import torch
 
@@ -30,7 +31,7 @@ _tuned = set()
 
 
 def _library(x, w, out, impl: str, alpha: float = 1.0):
-    """out = alpha * x w^T of many rows: the product in tiles where the kernel library finds it the faster one (impl "auto"),
+    """out = alpha * x w^T of many rows: the package's own product where the kernel library finds it the faster one (impl "auto"),
     otherwise hipBLASLt called directly; torch's routine if that has no algorithm for the shape."""
     if TUNE_LIBRARY and min(w.shape[0], w.shape[1]) >= TUNE_MIN_SIDE:
         key = (impl, x.dtype, out.dtype, x.shape[0], w.shape[0], w.shape[1], x.stride(0), w.stride(0), out.stride(0))

@@ -1,0 +1,117 @@
+"""Float32 products on the bfloat16 matrix cores against 64-bit sums.
+
+The bound of an element is (K + 16) 2^-24 sum |a| |w|: K roundings of a float32 sum in any order, and 2^-21 for the three products of parts that are left out
+(a second part is under 2^-7 of its number, a third under 2^-15)."""
+import ctypes
+
+import pytest
+import torch
+
+from infinicore_infer_amd.kernels import ops
+from infinicore_infer_amd.kernels.lib import get_lib
+
+# row tiles of 16, column tiles of 64: the order of the kernel's list
+SHAPES = [(1, 1), (2, 1), (3, 1), (4, 1), (5, 1), (6, 1), (7, 1), (4, 2), (5, 2), (6, 2), (7, 2), (8, 2), (4, 3), (6, 3), (8, 3)]
+
+
+def _inputs(M, N, K, pad=0, seed=1):
+    g = torch.Generator().manual_seed(seed * 1000003 + M * 7919 + N * 31 + K)
+    a = torch.randn(M, K + pad, generator=g) * torch.exp(2.0 * torch.randn(M, 1, generator=g))
+    w = torch.randn(N, K + pad, generator=g) * torch.exp(2.0 * torch.randn(N, 1, generator=g))
+    return a[:, :K], w[:, :K]
+
+
+def _check(got, a, w, alpha=1.0):
+    A, W = a.double(), w.double()
+    bound = (a.shape[1] + 16) * 2.0 ** -24 * abs(alpha) * (A.abs() @ W.abs().t())
+    assert bool(((got.double().cpu() - alpha * (A @ W.t())).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("units", [256, 64])
+def test_plans(units):
+    """Every plan names a shape and slices that the kernel takes; up to 32 rows the library's product stays."""
+    lib, n = get_lib(), ctypes.c_int()
+    for M in (1, 32, 33, 130, 517, 2048, 30000):
+        for N, K in ((4, 32), (65, 64), (1536, 1536), (7680, 1536), (1536, 3840), (73440, 4096)):
+            for adds in (0, 1):
+                assert 0 <= lib.ic_gemm_f32_plan_on(M, N, K, adds, units, n) < len(SHAPES)
+                assert 1 <= n.value <= min(4, K // 32) and (n.value == 1 or N % 4 == 0)
+            assert not (M <= 32 and lib.ic_gemm_f32_pays_on(M, N, K, units))
+    assert lib.ic_gemm_f32_plan_on(0, 64, 64, 0, units, n) == -1 and not lib.ic_gemm_f32_pays_on(100, 0, 64, units)
+    sup = lib.ic_gemm_f32_supported
+    assert sup(100, 64, 64, 64, 64, 64) and not sup(100, 64, 48, 64, 64, 64) and not sup(100, 64, 64, 66, 64, 64)
+    assert not sup(100, 64, 64, 64, 60, 64) and not sup(100, 64, 64, 64, 64, 60) and not sup(0, 64, 64, 64, 64, 64)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", range(len(SHAPES)))
+def test_edges(shape):
+    """Rows and columns around a tile's edges, one k-step and odd numbers of them, padded strides, slices; nothing beyond the matrix is written."""
+    bm, bn = 16 * SHAPES[shape][0], 64 * SHAPES[shape][1]
+    for M, N, K, pad, slices, alpha in ((1, 4, 32, 0, 1, 1.0), (bm, bn, 64, 4, 1, 1.0), (bm + 1, bn + 1, 96, 0, 1, -0.5), (2 * bm - 1, 3 * bn - 1, 288, 8, 1, 1.0),
+                                        (bm - 1, bn + 4, 64, 0, 2, 1.0), (3 * bm + 5, bn - 4, 416, 4, 3, 2.0), (17, 2 * bn, 128, 0, 4, 1.0), (bm, 68, 1056, 0, 4, 1.0)):
+        a, w = _inputs(M, N, K, pad, shape)
+        ldc = (N + 3) // 4 * 4 + 8
+        out = torch.full((M + 2, ldc), 7.0, device="cuda")
+        A, W = torch.empty(M, K + pad, device="cuda"), torch.empty(N, K + pad, device="cuda")
+        A[:, :K], W[:, :K] = a.cuda(), w.cuda()
+        ops.gemm_f32(A[:, :K], W[:, :K], out[:M, :N], alpha, shape, slices)
+        _check(out[:M, :N], a, w, alpha)
+        assert bool((out[M:] == 7.0).all()) and bool((out[:, N:] == 7.0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(40, 260, 96), (257, 1536, 1536), (130, 2304, 2304), (517, 512, 3840)])
+def test_chosen(M, N, K):
+    """The plan it makes itself, the product by the rule, and rows in several runs where the workspace is small."""
+    a, w = _inputs(M, N, K)
+    A, W, out = a.cuda(), w.cuda(), torch.empty(M, N, device="cuda")
+    _check(ops.gemm_f32(A, W, out), a, w)
+    _check(ops.product(A, W, out, 0.25), a, w, 0.25)
+    small = torch.empty(int(get_lib().ic_gemm_f32_parts_bytes(48, K)) + 16, dtype=torch.uint8, device="cuda")
+    _check(ops.gemm_f32(A, W, out.zero_(), workspace=small), a, w)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,lda,off", [(300, 2560, 1536, 1538, 0), (300, 2560, 1528, 1528, 0), (300, 2560, 1536, 1540, 1), (300, 2557, 1536, 1536, 0)])
+def test_product_of_forms_the_kernel_does_not_take(M, N, K, lda, off):
+    """Odd strides, rows that are no whole k-steps, misaligned operands: the product by the rule is right as ever."""
+    a, w = _inputs(M, N, K)
+    store = torch.zeros(M * lda + 8, device="cuda")
+    A = store[off:off + M * lda].view(M, lda)[:, :K]
+    A.copy_(a)
+    _check(ops.product(A, w.cuda(), torch.empty(M, N, device="cuda")), a, w)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("slices", [1, 3])
+def test_values_that_are_not_finite(slices):
+    """Infinities, NaN and the largest numbers come out as a float32 sum has them, and touch only their own row or column."""
+    M, N, K = 37, 132, 192
+    a, w = _inputs(M, N, K)
+    w = w.abs() / w.norm(dim=1, keepdim=True)
+    a[3, 5], a[4, 7], a[5, 9], a[6, 11] = float("inf"), float("-inf"), float("nan"), 3.4028234e38
+    w[8, 100], w[9, 0] = float("inf"), -3.4e38
+    a[:, 0] = 0.5                                   # (no sum overflows on its way)
+    A, W, out = a.cuda(), w.cuda(), torch.empty(M, N, device="cuda")
+    ops.gemm_f32(A, W, out, 1.0, 3, slices)
+    want = (a.double() @ w.double().t()).float()
+    same = (out.cpu() == want) | (out.cpu().isnan() & want.isnan())
+    finite = want.isfinite() & out.cpu().isfinite()
+    assert bool((same | finite).all())
+    rows = [m for m in range(M) if m not in (3, 4, 5, 6)]
+    cols = [n for n in range(N) if n not in (8, 9)]
+    _check(out[rows][:, cols], a[rows], w[cols])
+    _check(out[[6]][:, cols], a[[6]], w[cols])
+
+
+@pytest.mark.gpu
+def test_smaller_error_than_the_library():
+    """Against 64 bits the parts' error is no larger than the library's float32 product has it."""
+    for M, N, K in ((40, 1536, 1536), (256, 2560, 1536), (517, 1536, 3840)):
+        a, w = _inputs(M, N, K, seed=9)
+        A, W, own, lib = a.cuda(), w.cuda(), torch.empty(M, N, device="cuda"), torch.empty(M, N, device="cuda")
+        ops.gemm_f32(A, W, own)
+        ops.matmul_library(A, W, lib)
+        want = A.double() @ W.double().t()
+        assert (own.double() - want).norm() <= (lib.double() - want).norm()
