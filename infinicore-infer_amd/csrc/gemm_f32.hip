@@ -19,15 +19,14 @@
 //
 // Few tiles: K in slices, blocks of their own, whose sums a second kernel adds up.
 #include "common.h"
+#include "float_parts.h"
 #include "infinicore_infer_variants.h"
-#include <type_traits>
-#include <utility>
 
 namespace {
 
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef unsigned v4u __attribute__((ext_vector_type(4)));
-typedef __bf16 v8b __attribute__((ext_vector_type(8)));
+typedef parts_v4f v4f;
+typedef parts_v4u v4u;
+typedef parts_v8b v8b;
 
 struct F32Args {
     const float* A;
@@ -39,11 +38,6 @@ struct F32Args {
     long long slice_stride;
     float alpha;
 };
-
-template <typename F, int... Is> __device__ __forceinline__ void each_of(F&& f, std::integer_sequence<int, Is...>) {
-    (f(std::integral_constant<int, Is>{}), ...);
-}
-template <int N, typename F> __device__ __forceinline__ void each(F&& f) { each_of(f, std::make_integer_sequence<int, N>{}); }
 
 // 16 bytes a lane from base + off to LDS at lds + 16 * lane.
 __device__ __forceinline__ void load_to_lds(unsigned lds, unsigned off, const char* base) {
@@ -64,19 +58,6 @@ template <int N, int M> __device__ __forceinline__ void settled(v4f (&acc)[N][M]
         for (int m = 0; m < M; ++m) asm volatile("" : "+a"(acc[n][m]));
     asm volatile("s_nop 7");
 }
-
-// Four values in three bfloat16 parts each: step O of 22 (level O / 10: the parts' upper halves are packed, then taken off).
-struct Split4 {
-    float y[4], t[4];
-    unsigned p[3][2];
-};
-template <int O> __device__ __forceinline__ void split_step(Split4& s) {
-    constexpr int L = O / 10, Q = O % 10;
-    if constexpr (Q < 2) s.p[L][Q] = __builtin_amdgcn_perm(__float_as_uint(s.y[2 * Q + 1]), __float_as_uint(s.y[2 * Q]), 0x07060302);
-    else if constexpr (Q < 6) s.t[Q - 2] = __uint_as_float(__float_as_uint(s.y[Q - 2]) & 0xffff0000u);
-    else s.y[Q - 6] -= s.t[Q - 6];
-}
-constexpr int kSplitSteps = 22;
 
 template <int MT_, int NT_, int STAGES_> struct Shape {
     static constexpr int MT = MT_, NT = NT_, STAGES = STAGES_, BM = 16 * MT, BN = 64 * NT;
@@ -173,7 +154,7 @@ __global__ void __launch_bounds__(256, 1) gemm_f32_kernel(F32Args a) {
         __builtin_amdgcn_sched_barrier(0);
         each<P>([&](auto pc) {
             constexpr int p = decltype(pc)::value, n = p / (6 * MT), term = p / MT % 6, mt = p % MT;
-            constexpr int X[6] = {2, 0, 1, 1, 0, 0}, Y[6] = {0, 2, 1, 0, 1, 0};
+            constexpr auto &X = kPartX, &Y = kPartY;
             const Split4 &lo = pw[CUR][2 * n], &hi = pw[CUR][2 * n + 1];
             const v8b w = __builtin_bit_cast(v8b, v4u{lo.p[X[term]][0], lo.p[X[term]][1], hi.p[X[term]][0], hi.p[X[term]][1]});
             asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(term == 5 ? acc[n][mt] : low[n][mt]) : "v"(w), "v"(pa[CUR][mt][Y[term]]));

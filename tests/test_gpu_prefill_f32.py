@@ -15,3 +15,32 @@ def test_key_groups(nh, nkvh, dh, page, window):
     lens = [(0, 2), (0, 31), (0, 129), (130, 65), (257, 160), (31, 97), (700, 33)]          # nine tiles
     got, want = _attention_case(torch.float32, nh, nkvh, dh, page, lens, window, 61, "prefill")
     _close(got, want, torch.float32, factor=3)
+
+
+@pytest.mark.parametrize("nh,nkvh,dh,lens", [(2, 1, 64, [(40, 150)]), (26, 13, 64, [(0, 640)]), (72, 9, 64, [(3, 1300)]), (4, 2, 128, [(40, 150)]), (41, 41, 128, [(0, 1300)])])
+def test_products_of_parts(nh, nkvh, dh, lens):
+    """Error against 64 bits with one, two and four key groups: under that of the same sums in float32, where every product and sum is rounded (2^-24 a term, over the
+    square root of the head size and of the keys).  A key with an infinity, whose parts are no numbers, counts as a score of -inf."""
+    from infinicore_infer_amd.kernels import ops
+    dev, ps, (past, n) = "cuda", 64, lens[0]
+    g = torch.Generator().manual_seed(dh + n)
+    pages = -(-(past + n) // ps)
+    for infinite in (False, True):
+        k, v = (torch.randn(pages, nkvh, ps, dh, generator=g).to(dev) for _ in range(2))
+        q = torch.randn(n, (nh + 2 * nkvh) * dh, generator=g).to(dev)
+        if infinite:
+            q[:, :nh * dh:dh] = q[:, :nh * dh:dh].abs() + 0.5
+            k[pages // 2, :, 5, 0] = float("-inf")
+        tiles = torch.tensor([(0, i, min(128, n - i), past + i) for i in range(0, n, 128)][::-1], dtype=torch.int32, device=dev)
+        table = torch.arange(pages, dtype=torch.int32, device=dev)[None]
+        out = torch.empty(n, nh * dh, device=dev)
+        ops.attention_prefill(q, out, k, v, table, tiles, len(tiles), nh, nkvh, dh, ps, dh ** -0.5, 0)
+        seen = torch.arange(past + n)[None] <= past + torch.arange(n)[:, None]
+        wrong = total = 0.0
+        for h in range(0, nh, max(1, nh // 4)):
+            kh, vh = (x[:, h // (nh // nkvh)].reshape(-1, dh)[:past + n].double().cpu() for x in (k, v))
+            s = (q[:, h * dh:(h + 1) * dh].double().cpu() @ kh.t() * dh ** -0.5).masked_fill(~seen, float("-inf"))
+            want = torch.softmax(s, -1) @ vh
+            wrong += float((out[:, h * dh:(h + 1) * dh].double().cpu() - want).square().sum())
+            total += float(want.square().sum())
+        assert (wrong / total) ** 0.5 < 2 ** -24 * (dh ** 0.5 + (past + n) ** 0.5)
