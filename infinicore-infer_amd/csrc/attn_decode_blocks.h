@@ -187,11 +187,11 @@ __device__ __forceinline__ void split_block(const T* __restrict__ q, int q_strid
         for (int j = 0; j < GQ; ++j) {
 #pragma unroll
             for (int o = LPK; o < 64; o <<= 1) {
-                const float mb = __shfl_xor(m[j], o, kWave);
-                const float lb = __shfl_xor(l[j], o, kWave);
+                const float mb = lane_xor(m[j], o);
+                const float lb = lane_xor(l[j], o);
                 float ab[VEC];
 #pragma unroll
-                for (int i = 0; i < VEC; ++i) ab[i] = __shfl_xor(acc[j][i], o, kWave);
+                for (int i = 0; i < VEC; ++i) ab[i] = lane_xor(acc[j][i], o);
                 merge_state(m[j], l[j], acc[j], VEC, mb, lb, ab);
             }
         }

@@ -389,7 +389,7 @@ attn_latent_mfma_kernel(const bf16* __restrict__ qa, int qa_stride, bf16* __rest
         float mloc = sacc[0];
 #pragma unroll
         for (int r = 1; r < 16; ++r) mloc = fmaxf(mloc, sacc[r]);
-        mloc = fmaxf(mloc, __shfl_xor(mloc, 32, kWave));
+        mloc = swap_max<32>(mloc);
         const float m_new = fmaxf(m, mloc);                     // finite: some key of every step is visible
         const float mc = m_new * scale_log2e;
         const float corr = (m == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m * scale_log2e - mc);
@@ -400,7 +400,7 @@ attn_latent_mfma_kernel(const bf16* __restrict__ qa, int qa_stride, bf16* __rest
             sacc[r] = p;
             rs += p;
         }
-        rs += __shfl_xor(rs, 32, kWave);
+        rs = swap_add<32>(rs);
         l = l * corr + rs;
         m = m_new;
 #pragma unroll

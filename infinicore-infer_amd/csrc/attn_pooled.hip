@@ -374,7 +374,7 @@ attn_pooled_decode_kernel(const T* __restrict__ q, int q_stride, const T* __rest
                 for (int j = 0; j < VEC; ++j) {
                     float v = acc[g][n][j];
 #pragma unroll
-                    for (int o = LPK; o < 64; o <<= 1) v += __shfl_xor(v, o, kWave);
+                    for (int o = LPK; o < 64; o <<= 1) v += lane_xor(v, o);
                     acc[g][n][j] = v;
                 }
         if (grp == 0) {

@@ -320,14 +320,14 @@ attn_span_decode_kernel(const T* __restrict__ q, int q_stride, const T* __restri
         for (int j = 0; j < GQ; ++j) {
 #pragma unroll
             for (int o = LPK; o < 64; o <<= 1) {
-                const float mb = __shfl_xor(m[j], o, kWave);
-                const float lb = __shfl_xor(l[j], o, kWave);
+                const float mb = lane_xor(m[j], o);
+                const float lb = lane_xor(l[j], o);
                 const float mn = fmaxf(m[j], mb);
                 const float ca = (mn == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m[j] - mn);
                 const float cb = (mn == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(mb - mn);
                 l[j] = l[j] * ca + lb * cb;
 #pragma unroll
-                for (int i = 0; i < NVS * VEC; ++i) acc[j][i] = acc[j][i] * ca + __shfl_xor(acc[j][i], o, kWave) * cb;
+                for (int i = 0; i < NVS * VEC; ++i) acc[j][i] = acc[j][i] * ca + lane_xor(acc[j][i], o) * cb;
                 m[j] = mn;
             }
         }

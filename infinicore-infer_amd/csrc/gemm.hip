@@ -322,8 +322,8 @@ gemm_nt_bf16_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__
         float t = 0.f;
 #pragma unroll
         for (int j = 0; j < WPB; ++j) t += ssum[4 * j + kq][r];
-        t += __shfl_xor(t, 16, kWave);
-        t += __shfl_xor(t, 32, kWave);
+        t = swap_add<16>(t);
+        t = swap_add<32>(t);
         rowf = rsqrtf(t * nf.inv_width + nf.eps);
     }
     alpha *= rowf;
@@ -409,8 +409,8 @@ gemm_nt_bf16_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__
                 ss += h * h;
             }
         }
-        ss += __shfl_xor(ss, 16, kWave);
-        ss += __shfl_xor(ss, 32, kWave);
+        ss = swap_add<16>(ss);
+        ss = swap_add<32>(ss);
         if (kq == 0) nf.ss_out[blockIdx.x * 16 + r] = ss;
         return;
     }

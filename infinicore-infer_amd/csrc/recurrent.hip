@@ -788,9 +788,9 @@ blocked_product_rows_kernel(const T* __restrict__ A, int lda, int a_step, const 
 #pragma unroll
     for (int mm = 0; mm < MT; ++mm) {
         float v = acc[mm];
-        v += __shfl_xor(v, 4, kWave);
-        v += __shfl_xor(v, 2, kWave);
-        v += __shfl_xor(v, 1, kWave);
+        v += lane_xor(v, 4);
+        v += lane_xor(v, 2);
+        v += lane_xor(v, 1);
         if (sub == 0 && n < N && mm < M) {
             v = ep(v, mm, b * c_step + n, n);
             C[(size_t)mm * ldc + (size_t)b * c_step + n] = from_f32<TC>(v);
