@@ -31,7 +31,7 @@ attn_decode_split_kernel(const T* __restrict__ q, int q_stride,
 }
 
 // Grid (tokens * heads), four waves.  Lane s of every wave holds split s (at most 64 splits): the
-// weights exp(m_s - max) come from one wave reduction.  Thread (d, g) sums output dim d over
+// weights exp(m_s - max) come from one wave reduction, which every wave does for itself (through LDS: a barrier, 0.1..0.2 us).  Thread (d, g) sums output dim d over
 // the splits g, g + G, .. (G = 256 / DH groups, CNT = ceil(splits / G) of them a thread), and the
 // groups meet in LDS: with many splits (few kv heads, few requests) one wave alone would walk them
 // one after the other.  The partial sums are loaded first, without condition (a slot beyond the
@@ -45,11 +45,10 @@ attn_decode_reduce_kernel(const float* __restrict__ part_acc, const float* __res
                           int out_stride, int nh, int nsplit) {
     constexpr int G = kRedThreads / DH;
     static_assert(kRedThreads % DH == 0, "every thread has a (dim, group) place");
-    __shared__ float wgt[64];
     __shared__ float grp[kRedThreads];
     const int n = blockIdx.x / nh, h = blockIdx.x % nh, tid = threadIdx.x, lane = tid & 63;
     const size_t base = ((size_t)n * nh + h) * nsplit;
-    const int g = tid / DH, d = tid - g * DH;
+    const int g = __builtin_amdgcn_readfirstlane(tid / DH), d = tid - g * DH;     // (a wave is of one group)
     float pa[CNT];
 #pragma unroll
     for (int i = 0; i < CNT; ++i) {
@@ -63,12 +62,10 @@ attn_decode_reduce_kernel(const float* __restrict__ part_acc, const float* __res
     const float mm = wave_max(ms);
     const float w = (ms == -INFINITY) ? 0.f : expf(ms - mm);
     const float inv = 1.0f / wave_sum(ls * w);
-    if (tid < 64) wgt[lane] = w;
-    __syncthreads();
     float a = 0.f;
 #pragma unroll
     for (int i = 0; i < CNT; ++i)
-        if (g + i * G < nsplit) a += pa[i] * wgt[g + i * G];
+        if (g + i * G < nsplit) a += pa[i] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), g + i * G));
     grp[tid] = a;
     __syncthreads();
     if (tid < DH) {
