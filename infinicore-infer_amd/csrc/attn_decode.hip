@@ -61,7 +61,7 @@ attn_decode_reduce_kernel(const float* __restrict__ part_acc, const float* __res
     if (lane >= nsplit) { ms = -INFINITY; ls = 0.f; }
     const float mm = wave_max(ms);
     const float w = (ms == -INFINITY) ? 0.f : expf(ms - mm);
-    const float inv = 1.0f / wave_sum(ls * w);
+    const float inv = 1.0f / wave_sum_of_products(ls, w);
     float a = 0.f;
 #pragma unroll
     for (int i = 0; i < CNT; ++i)

@@ -43,14 +43,14 @@ template <> struct Vec16<bf16> {
     __device__ static void load(const bf16* p, float* o) { unpack(raw(p), o); }
 };
 
-// merge running-softmax state b into a
+// merge running-softmax state b into a (which product of a sum is rounded first is written out: left to the compiler it differs from kernel to kernel)
 __device__ __forceinline__ void merge_state(float& m, float& l, float* acc, int n,
                                             float mb, float lb, const float* accb) {
     const float mn = fmaxf(m, mb);
     if (mn == -INFINITY) return;                 // both empty
     const float ca = __builtin_amdgcn_exp2f(m - mn), cb = __builtin_amdgcn_exp2f(mb - mn);   // maxima in units of log 2
-    l = l * ca + lb * cb;
-    for (int i = 0; i < n; ++i) acc[i] = acc[i] * ca + accb[i] * cb;
+    l = fmaf(lb, cb, l * ca);
+    for (int i = 0; i < n; ++i) acc[i] = fmaf(acc[i], ca, accb[i] * cb);
     m = mn;
 }
 

@@ -477,7 +477,7 @@ attn_latent_merge_kernel(const float* __restrict__ part_acc, const float* __rest
         float m = wave_max(ms);
         if (sinks) m = fmaxf(m, sinks[h]);
         const float e = ms > -INFINITY ? expf(ms - m) : 0.f;
-        const float l = wave_sum(ls * e) + (sinks ? expf(sinks[h] - m) : 0.f);
+        const float l = wave_sum_of_products(ls, e) + (sinks ? expf(sinks[h] - m) : 0.f);
         wgt[sp] = e / l;
     }
     __syncthreads();

@@ -325,9 +325,9 @@ attn_span_decode_kernel(const T* __restrict__ q, int q_stride, const T* __restri
                 const float mn = fmaxf(m[j], mb);
                 const float ca = (mn == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m[j] - mn);
                 const float cb = (mn == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(mb - mn);
-                l[j] = l[j] * ca + lb * cb;
+                l[j] = fmaf(l[j], ca, lb * cb);             // (written out, as merge_state in attn_decode_blocks.h)
 #pragma unroll
-                for (int i = 0; i < NVS * VEC; ++i) acc[j][i] = acc[j][i] * ca + lane_xor(acc[j][i], o) * cb;
+                for (int i = 0; i < NVS * VEC; ++i) acc[j][i] = fmaf(acc[j][i], ca, lane_xor(acc[j][i], o) * cb);
                 m[j] = mn;
             }
         }

@@ -102,10 +102,13 @@ template <int D> __device__ __forceinline__ float swap_max(float v) {
     return fmaxf(__int_as_float((int)r[0]), __int_as_float((int)r[1]));
 }
 // Over a wave; halves first, in the order of a shuffle by 32, 16, 8, 4, 2 and 1.
-__device__ __forceinline__ float wave_sum(float v) {
-    v = dpp_add<0x128>(swap_add<16>(swap_add<32>(v)));
+__device__ __forceinline__ float sum_of_halves(float v) {
+    v = dpp_add<0x128>(swap_add<16>(v));
     return dpp_add<0xB1>(dpp_add<0x4E>(v + lane_xor(v, 4)));
 }
+__device__ __forceinline__ float wave_sum(float v) { return sum_of_halves(swap_add<32>(v)); }
+// Of a * b over a wave, the lane's own product not rounded before the first sum.
+__device__ __forceinline__ float wave_sum_of_products(float a, float b) { return sum_of_halves(fmaf(a, b, lane_xor(a * b, 32))); }
 __device__ __forceinline__ float wave_max(float v) {
     v = swap_max<16>(swap_max<32>(v));
 #pragma unroll
