@@ -32,7 +32,7 @@ inline int dtype_size(int dtype) { return dtype == IC_BF16 ? 2 : 4; }
 struct Workspace {
     // byte offsets into the caller's workspace
     size_t residual, normed, qkv, attn_out, mixer_out, ffn_out, mixer_tail, mixer_sumsq, ffn_tail, ffn_sumsq, gate_up, act,
-        part_acc, part_ml, decode_order, head_in, tail_parts, tile_parts, total;
+        part_acc, part_ml, decode_order, head_in, tail_parts, tile_parts, f32_parts, total;
 };
 
 // Rows whose norm is half done: values = x * w, sums of squares per column block; the row factor
@@ -207,12 +207,22 @@ struct IcDecoder {
                 cut = std::max(cut, (size_t)ic_attn_prefill_scratch_floats(b.n_prefill_tiles, l.attention.n_heads, l.attention.head_dim, p));
             }
         w.tile_parts = take(cut * 4);
+        long long f32 = 0;           // float32 products of many rows (this engine's own: another's must not write there between two launches)
+        if (meta.dtype == IC_F32) {
+            for (const IcLayer& l : layers) {
+                const int heads = l.attention.n_heads * l.attention.head_dim, di = l.ffn.intermediate;
+                f32 = std::max({f32, ic_gemm_f32_workspace_bytes(b.n_tokens, max_qkv_width, meta.hidden), ic_gemm_f32_workspace_bytes(b.n_tokens, meta.hidden, heads),
+                                ic_gemm_f32_workspace_bytes(b.n_tokens, 2 * di, meta.hidden), ic_gemm_f32_workspace_bytes(b.n_tokens, meta.hidden, di)});
+            }
+            f32 = std::max(f32, ic_gemm_f32_workspace_bytes(b.n_want, meta.vocab, meta.hidden));
+        }
+        w.f32_parts = take((size_t)f32);
         w.total = o;
         return w;
     }
     // out[M, N] = alpha * a w^T: the few-row product, or what ic_product takes.
     int linear(const void* a, int lda, const void* w, void* out, int out_dtype, int M, int N, int K, float alpha,
-               const Deferred* rows, void* lib_ws, long long lib_ws_bytes, hipStream_t stream) const {
+               const Deferred* rows, void* f32_parts, void* lib_ws, long long lib_ws_bytes, hipStream_t stream) const {
         if (ic_rule_own_product(meta.dtype, meta.dtype, out_dtype, M)) {
             IcRowFactor rf{};
             if (rows) rf = IcRowFactor{rows->sumsq, rows->parts, rows->width, rows->eps};
@@ -220,6 +230,8 @@ struct IcDecoder {
                               nullptr, stream);
         }
         if (rows) return IC_ERR_ARG;      // half-normed rows exist only where the few-row product runs
+        if (meta.dtype == IC_F32)
+            return ic_product_f32(a, w, out, M, N, K, lda, K, N, alpha, f32_parts, ic_gemm_f32_workspace_bytes(M, N, K), lib_ws, lib_ws_bytes, stream);
         return ic_product(a, meta.dtype, w, out, out_dtype, M, N, K, lda, K, N, alpha, lib_ws, lib_ws_bytes, stream);
     }
 
@@ -249,6 +261,7 @@ struct IcDecoder {
         void* normed = base + ws.normed;
         void* qkv = base + ws.qkv;
         void* attn_out = base + ws.attn_out;
+        void* f32_parts = base + ws.f32_parts;
         const int parts = ic_gemm_nt_residual_parts(d);
         int st;
 
@@ -308,7 +321,7 @@ struct IcDecoder {
                                         A.head_dim, ps, stream);
                 if (st) return fail(st, "the QKV product with rotary and cache write, in tiles", i);
             } else {
-                st = linear(h, d, A.w_qkv, qkv, dt, T, width, d, 1.0f, h_def, lib_ws, lib_ws_bytes, stream);
+                st = linear(h, d, A.w_qkv, qkv, dt, T, width, d, 1.0f, h_def, f32_parts, lib_ws, lib_ws_bytes, stream);
                 if (st) return fail(st, "the QKV product", i);
                 if (A.rot_dim > 0 || nkv > 0) {
                     st = ic_rope_kv_write(qkv, dt, b.positions, A.rot_dim > 0 ? A.cos : nullptr, A.rot_dim > 0 ? A.sin : nullptr,
@@ -382,7 +395,7 @@ struct IcDecoder {
                 mid = Deferred{base + ws.mixer_tail, (const float*)(base + ws.mixer_sumsq), parts, d, L.ffn_norm.eps};
                 g_def = &mid;
             } else {
-                st = linear(attn_out, ow, A.w_o, base + ws.mixer_out, dt, T, d, ow, 1.0f, nullptr, lib_ws, lib_ws_bytes, stream);
+                st = linear(attn_out, ow, A.w_o, base + ws.mixer_out, dt, T, d, ow, 1.0f, nullptr, f32_parts, lib_ws, lib_ws_bytes, stream);
                 if (st) return fail(st, "the O product", i);
                 st = ic_add_rmsnorm(x, base + ws.mixer_out, dt, L.residual_scale, L.ffn_norm.weight, normed, dt, T, d, L.ffn_norm.eps, stream);
                 if (st) return fail(st, "the residual add and norm before the feed-forward", i);
@@ -402,7 +415,7 @@ struct IcDecoder {
                 st = ic_gemm_tiles(g, L.ffn.w_gate_up, act, T, 2 * di, d, d, d, di, 1, stream);
                 if (st) return fail(st, "the gate/up product with SwiGLU, in tiles", i);
             } else {
-                st = linear(g, d, L.ffn.w_gate_up, base + ws.gate_up, dt, T, 2 * di, d, 1.0f, nullptr, lib_ws, lib_ws_bytes, stream);
+                st = linear(g, d, L.ffn.w_gate_up, base + ws.gate_up, dt, T, 2 * di, d, 1.0f, nullptr, f32_parts, lib_ws, lib_ws_bytes, stream);
                 if (st) return fail(st, "the gate/up product", i);
                 st = ic_swiglu(base + ws.gate_up, act, dt, T, di, stream);
                 if (st) return fail(st, "SwiGLU", i);
@@ -421,7 +434,7 @@ struct IcDecoder {
                 def = Deferred{base + ws.ffn_tail, (const float*)(base + ws.ffn_sumsq), parts, d, succ->eps};
                 owed = DEFERRED;
             } else {
-                st = linear(act, di, L.ffn.w_down, base + ws.ffn_out, dt, T, d, di, 1.0f, nullptr, lib_ws, lib_ws_bytes, stream);
+                st = linear(act, di, L.ffn.w_down, base + ws.ffn_out, dt, T, d, di, 1.0f, nullptr, f32_parts, lib_ws, lib_ws_bytes, stream);
                 if (st) return fail(st, "the down product", i);
                 branch = base + ws.ffn_out;
                 branch_alpha = L.residual_scale;
@@ -432,12 +445,12 @@ struct IcDecoder {
         // ---- final norm and head, on the wanted rows only -----------------------------------------------------
         if (b.n_want == 0) return IC_OK;
         if (owed == NORMED) {        // every row in order, the final norm (with the logit scale in its weight) applied
-            st = linear(normed, d, meta.head_weight, logits, IC_F32, T, meta.vocab, d, 1.0f, nullptr, lib_ws, lib_ws_bytes, stream);
+            st = linear(normed, d, meta.head_weight, logits, IC_F32, T, meta.vocab, d, 1.0f, nullptr, f32_parts, lib_ws, lib_ws_bytes, stream);
             if (st) return fail(st, "the head product", -1);
             return IC_OK;
         }
         if (owed == DEFERRED) {      // every row in order, the final norm half done: its row factors go into the product
-            st = linear(def.values, d, meta.head_weight, logits, IC_F32, T, meta.vocab, d, 1.0f, &def, lib_ws, lib_ws_bytes, stream);
+            st = linear(def.values, d, meta.head_weight, logits, IC_F32, T, meta.vocab, d, 1.0f, &def, f32_parts, lib_ws, lib_ws_bytes, stream);
             if (st) return fail(st, "the head product", -1);
             return IC_OK;
         }
@@ -448,7 +461,7 @@ struct IcDecoder {
         void* head_in = base + ws.head_in;
         st = ic_rmsnorm(x, b.want_rows, meta.final_norm.weight, head_in, dt, b.n_want, d, meta.final_norm.eps, meta.logit_scale, stream);
         if (st) return fail(st, "the final norm", -1);
-        st = linear(head_in, d, meta.head_weight, logits, IC_F32, b.n_want, meta.vocab, d, 1.0f, nullptr, lib_ws, lib_ws_bytes, stream);
+        st = linear(head_in, d, meta.head_weight, logits, IC_F32, b.n_want, meta.vocab, d, 1.0f, nullptr, f32_parts, lib_ws, lib_ws_bytes, stream);
         if (st) return fail(st, "the head product", -1);
         return IC_OK;
     }

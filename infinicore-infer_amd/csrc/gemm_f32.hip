@@ -21,6 +21,7 @@
 #include "common.h"
 #include "float_parts.h"
 #include "infinicore_infer_variants.h"
+#include "workspace_lock.h"
 
 namespace {
 
@@ -270,7 +271,7 @@ template <typename T> int launch(F32Args a, hipStream_t stream) {
     X(13, 1.81, 0.874, 0.24, 5.38, 6, 3, 3) \
     X(14, 1.91, 1.106, 0.28, 6.44, 8, 3, 3)
 
-constexpr int kShapes = 15, kMaxSlices = 4;
+constexpr int kShapes = 15, kMaxSlices = 4, kFewRows = 32;
 struct ShapeCost { int bm, bn; double fixed, stage, full, round; };
 constexpr ShapeCost kCosts[kShapes] = {
 #define X(I, FIXED, STAGE, FULL, ROUND, MT, NT, ST) {16 * MT, 64 * NT, FIXED, STAGE, FULL, ROUND},
@@ -338,6 +339,7 @@ int product(const float* A, const float* W, float* C, int M, int N, int K, int l
     const int at_once = rows_at_once(M, K, workspace_bytes);
     if (at_once <= 0) return IC_ERR_ARG;
     if (slices > 1 && (at_once < M || parts_bytes(M, K) + 4LL * slices * M * N > workspace_bytes)) return IC_ERR_ARG;
+    std::lock_guard<std::mutex> lock(workspace_lock());
     for (int m = 0; m < M; m += at_once) {
         const int rows = M - m < at_once ? M - m : at_once;
         const float* const a0 = A + (size_t)m * lda;
@@ -379,7 +381,7 @@ IC_EXPORT int ic_gemm_f32_plan_on(int M, int N, int K, int adds_slices, int unit
 // since fewer are a matter of the weights' bytes, which it reads as fast (8 x 7,680 x 1,536: 13 us, the split alone 4).  Over the sweep above the choice loses 1.1 % to the
 // better of the two.  130 x 7,680 x 1,536: 35 -> 29, 256 x 2,560 x 1,536: 28 -> 22, on the other side 96 x 2,560 x 1,536: 11 against 18.
 IC_EXPORT int ic_gemm_f32_pays_on(int M, int N, int K, int units) {
-    if (M <= 32 || N <= 0 || K < 32 || units <= 0) return 0;
+    if (M <= kFewRows || N <= 0 || K < 32 || units <= 0) return 0;
     const double products = 2.0 * M * N * K / (127e6 * units / 256.0) + 8.7;
     return 3.73 + 10.0 * M * K / (14.8e6 * units / 256.0) + plan_for(M, N, K, false, kMaxSlices, units).cost < (products > 12.0 ? products : 12.0);
 }
@@ -387,6 +389,22 @@ IC_EXPORT int ic_gemm_f32_pays_on(int M, int N, int K, int units) {
 IC_EXPORT int ic_gemm_f32_pays(int M, int N, int K) { return ic_gemm_f32_pays_on(M, N, K, compute_units()); }
 
 IC_EXPORT long long ic_gemm_f32_parts_bytes(int M, int K) { return M > 0 && K >= 32 ? parts_bytes(M, K) : 0; }
+
+// Memory for any plan of the product: A's parts and all slices, up to 64 MB; grows with M.  None where the rule takes the library's product in any case.
+IC_EXPORT long long ic_gemm_f32_workspace_bytes(int M, int N, int K) {
+    if (M <= kFewRows || N <= 0 || K < 32) return 0;
+    const long long need = parts_bytes(M, K) + 4LL * kMaxSlices * M * N, most = 64LL << 20;
+    return need < most ? need : most;
+}
+
+// The product by this file's kernels or the library's, by the rule: parts is the caller's own memory for the former, workspace the library's.
+IC_EXPORT int ic_product_f32(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, float alpha, void* parts, long long parts_bytes,
+                             void* workspace, long long workspace_bytes, hipStream_t stream) {
+    if (A && W && C && parts && aligned16(A) && aligned16(W) && aligned16(C) && aligned16(parts) && takes(M, N, K, lda, ldw, ldc) &&
+        rows_at_once(M, K, parts_bytes) > 0 && ic_gemm_f32_pays(M, N, K))
+        return ic_gemm_f32(A, W, C, M, N, K, lda, ldw, ldc, alpha, parts, parts_bytes, stream);
+    return ic_matmul(A, IC_F32, W, C, IC_F32, M, N, K, lda, ldw, ldc, alpha, workspace, workspace_bytes, stream);
+}
 
 // The whole product.  workspace (16-byte aligned): A's parts, or as many rows of them at a time as it holds (16 at least), and the slices where they fit too.
 IC_EXPORT int ic_gemm_f32(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, float alpha, void* workspace,

@@ -606,8 +606,7 @@ IC_EXPORT int ic_product(const void* A, int a_dtype, const void* W, void* C, int
         const int timed = ic_product_timed(M, N, K, lda, ldw, ldc);
         if (timed >= 0 ? timed : ic_gemm_tiles_pays(M, N, K, EPI_BF16)) return ic_gemm_tiles(A, W, C, M, N, K, lda, ldw, ldc, EPI_BF16, stream);
     }
-    if (a_dtype == IC_F32 && c_dtype == IC_F32 && A && W && C && workspace && aligned16(A) && aligned16(W) && aligned16(C) && aligned16(workspace) &&
-        ic_gemm_f32_supported(M, N, K, lda, ldw, ldc) && ic_gemm_f32_parts_bytes(16, K) <= workspace_bytes && ic_gemm_f32_pays(M, N, K))
-        return ic_gemm_f32(A, W, C, M, N, K, lda, ldw, ldc, alpha, workspace, workspace_bytes, stream);
+    if (a_dtype == IC_F32 && c_dtype == IC_F32)
+        return ic_product_f32(A, W, C, M, N, K, lda, ldw, ldc, alpha, workspace, workspace_bytes, workspace, workspace_bytes, stream);
     return ic_matmul(A, a_dtype, W, C, c_dtype, M, N, K, lda, ldw, ldc, alpha, workspace, workspace_bytes, stream);
 }

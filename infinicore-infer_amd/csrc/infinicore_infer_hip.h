@@ -176,7 +176,12 @@ int ic_product(const void* A, int a_dtype, const void* W, void* C, int c_dtype, 
 int ic_gemm_f32_supported(int M, int N, int K, int lda, int ldw, int ldc);
 int ic_gemm_f32_pays(int M, int N, int K);
 long long ic_gemm_f32_parts_bytes(int M, int K);
+// ic_gemm_f32_workspace_bytes: what ic_product_f32 has use for, at most 64 MB; none up to 32 rows.  Threads may share a workspace on one stream.
+long long ic_gemm_f32_workspace_bytes(int M, int N, int K);
 int ic_gemm_f32(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, float alpha, void* workspace, long long workspace_bytes, hipStream_t stream);
+
+// ic_product in float32 with memory of the caller's own for ic_gemm_f32 (parts, 16-byte aligned) beside ic_matmul's workspace.
+int ic_product_f32(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, float alpha, void* parts, long long parts_bytes, void* workspace, long long workspace_bytes, hipStream_t stream);
 
 // ---- matmul_library.hip ------------------------------------------------------------------------------
 // The library (hipBLASLt) matrix product for many rows: C[M, N] = alpha * A[M, K] W[N, K]^T, bfloat16 operands with a

@@ -9,11 +9,11 @@
 // (W as [K, N])^T (A as [K, M]): its matrix "A" is W with transposition, its "B" is A.
 #include "common.h"
 #include "infinicore_infer_variants.h"
+#include "workspace_lock.h"
 #include <hipblaslt/hipblaslt.h>
 #include <hipblaslt/hipblaslt-ext.hpp>
 #include <algorithm>
 #include <atomic>
-#include <mutex>
 #include <unordered_map>
 #include <vector>
 
@@ -46,7 +46,7 @@ struct Plan {
     bool timed = false;                                          // `chosen` comes from timing on the device
 };
 
-std::mutex g_mu;
+std::mutex g_mu;       // the plans, and the workspace while a product is enqueued (workspace_lock.h)
 hipblasLtHandle_t g_handle = nullptr;
 std::unordered_map<Key, Plan, KeyHash> g_plans;
 
@@ -139,6 +139,8 @@ bool args_ok(const void* A, int a_dtype, const void* W, void* C, int c_dtype, in
 }
 
 }  // namespace
+
+std::mutex& workspace_lock() { return g_mu; }
 
 // 1 when the direct path takes these types (bfloat16 operands with a bfloat16 or float32 result; all float32).
 IC_EXPORT int ic_matmul_supported(int a_dtype, int c_dtype) {

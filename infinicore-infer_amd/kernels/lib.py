@@ -208,6 +208,8 @@ _SIGNATURES = {
     "ic_gemm_f32_pays_on": [_I] * 4,
     "ic_gemm_f32_plan_on": [_I] * 5 + [_c.POINTER(_I)],
     "ic_gemm_f32_parts_bytes": [_I, _I],
+    "ic_gemm_f32_workspace_bytes": [_I] * 3,
+    "ic_product_f32": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P, _LL, _P, _LL, _P],
     "ic_gemm_f32": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P, _LL, _P],
     "ic_gemm_f32_cfg": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _I, _P, _LL, _P],
     "ic_product": [_P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _P, _LL, _P],
@@ -239,7 +241,7 @@ _SIGNATURES = {
 }
 _RESTYPES = {"ic_product_timing": None, "ic_decoder_create": _P, "ic_decoder_create_error": _c.c_char_p, "ic_decoder_destroy": None,
              "ic_decoder_last_error": _c.c_char_p, "ic_decoder_workspace_bytes": _LL, "ic_decoder_step_ints": _LL,
-             "ic_peak_mfma_bf16": _LL, "ic_attn_prefill_scratch_floats": _LL, "ic_gemm_f32_parts_bytes": _LL}
+             "ic_peak_mfma_bf16": _LL, "ic_attn_prefill_scratch_floats": _LL, "ic_gemm_f32_parts_bytes": _LL, "ic_gemm_f32_workspace_bytes": _LL}
 
 
 def get_lib():

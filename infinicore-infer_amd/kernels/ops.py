@@ -626,20 +626,30 @@ def matmul_library(a, w, out, alpha: float = 1.0):
     return _matmul(get_lib().ic_matmul, a, w, out, alpha, "matmul_library")
 
 
-def product(a, w, out, alpha: float = 1.0):
+def product(a, w, out, alpha: float = 1.0, parts=None):
     """matmul_library, or the package's own product where that is the faster one: in tiles (gemm_tiles; by the rule, or as product_tune found), in
-    float32 gemm_f32 (by the rule)."""
-    return _matmul(get_lib().ic_product, a, w, out, alpha, "product")
+    float32 gemm_f32 (by the rule).  parts (float32): a uint8 tensor of product_parts_bytes(M, N, K) for gemm_f32, in place of the library's scratch memory."""
+    return _matmul(get_lib().ic_product, a, w, out, alpha, "product", parts)
 
 
-def _matmul(entry, a, w, out, alpha, what):
+def product_parts_bytes(m: int, n: int, k: int) -> int:
+    """Bytes of scratch memory that a float32 ``product`` has use for besides the library's (0: none)."""
+    return int(get_lib().ic_gemm_f32_workspace_bytes(m, n, k))
+
+
+def _matmul(entry, a, w, out, alpha, what, parts=None):
     M, N, K, ca, cc, sa, sw, so = _matmul_args(a, w, out, what)
     stream = _stream()
     ws = _matmul_workspace.get((a.device, stream))
     if ws is None:
         ws = _workspace(a.device)
-    st = entry(a.data_ptr(), ca, w.data_ptr(), out.data_ptr(), cc, M, N, K, sa, sw, so, alpha,
-               ws.data_ptr(), MATMUL_WORKSPACE_BYTES, stream)
+    if parts is None:
+        st = entry(a.data_ptr(), ca, w.data_ptr(), out.data_ptr(), cc, M, N, K, sa, sw, so, alpha,
+                   ws.data_ptr(), MATMUL_WORKSPACE_BYTES, stream)
+    else:
+        _need(ca == cc == 0 and parts.device == a.device and parts.dtype == torch.uint8 and parts.is_contiguous(), what + ": parts")
+        st = get_lib().ic_product_f32(a.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K, sa, sw, so, alpha, parts.data_ptr(), parts.numel(),
+                                      ws.data_ptr(), MATMUL_WORKSPACE_BYTES, stream)
     if st == 0:
         return out
     if st == -4:

@@ -30,9 +30,9 @@ TUNE_MIN_SIDE = 256
 _tuned = set()
 
 
-def _library(x, w, out, impl: str, alpha: float = 1.0):
-    """out = alpha * x w^T of many rows: the package's own product where the kernel library finds it the faster one (impl "auto"),
-    otherwise hipBLASLt called directly; torch's routine if that has no algorithm for the shape."""
+def _library(x, w, out, impl: str, alpha: float = 1.0, ws=None):
+    """out = alpha * x w^T of many rows: the package's own product where the kernel library finds it the faster one (impl "auto"; its float32 scratch memory
+    is the step's own, since its kernels hand numbers on there), otherwise hipBLASLt called directly; torch's routine if that has no algorithm for the shape."""
     if TUNE_LIBRARY and min(w.shape[0], w.shape[1]) >= TUNE_MIN_SIDE:
         key = (impl, x.dtype, out.dtype, x.shape[0], w.shape[0], w.shape[1], x.stride(0), w.stride(0), out.stride(0))
         if key not in _tuned:
@@ -42,7 +42,14 @@ def _library(x, w, out, impl: str, alpha: float = 1.0):
             except ops.KernelError:
                 pass
     try:
-        return (ops.product if impl == "auto" else ops.matmul_library)(x, w, out, alpha)
+        if impl != "auto":
+            return ops.matmul_library(x, w, out, alpha)
+        parts = None
+        if ws is not None and x.dtype == torch.float32:
+            n = ops.product_parts_bytes(x.shape[0], w.shape[0], w.shape[1])
+            if n:
+                parts = ws.buffer("product_parts", (n,), torch.uint8)
+        return ops.product(x, w, out, alpha, parts)
     except ops.NoLibraryAlgorithm:
         if out.dtype == x.dtype:
             torch.mm(x, w.t(), out=out)
@@ -59,7 +66,7 @@ def linear(x, w, out, impl: str = "auto", alpha: float = 1.0, ws=None):
     """out[M, N] = alpha * x[M, K] @ w[N, K]^T.  out may be float32 when x is bfloat16.  x may be
     ``DeferredRows``: the row factors are applied to the result by the own kernel, or to x first.
     ``ws``: the step's workspace, for the float32 copies that a matrix stored in 32-bit under a bfloat16
-    model needs (without it they are allocated by the call)."""
+    model needs (without it they are allocated by the call) and for float32 products' scratch memory."""
     if isinstance(x, DeferredRows):
         if own_kernel_applies(x.shape[0], x.dtype, w.dtype, out.dtype, impl):
             return ops.gemm_nt(x.values, w, out, alpha=alpha, row_factor=x.row_factor())
@@ -74,14 +81,14 @@ def linear(x, w, out, impl: str = "auto", alpha: float = 1.0, ws=None):
         x32 = x if x.dtype == torch.float32 else scratch("linear_x32", tuple(x.shape)).copy_(x)
         w32 = w if w.dtype == torch.float32 else w.to(torch.float32)
         if out.dtype == torch.float32:
-            return _library(x32, w32, out, impl, alpha)
+            return _library(x32, w32, out, impl, alpha, ws)
         tmp = scratch("linear_out32", tuple(out.shape))
-        _library(x32, w32, tmp, impl, alpha)
+        _library(x32, w32, tmp, impl, alpha, ws)
         out.copy_(tmp)
         return out
     if own_kernel_applies(x.shape[0], x.dtype, w.dtype, out.dtype, impl):
         return ops.gemm_nt(x, w, out, alpha=alpha)
-    return _library(x, w, out, impl, alpha)
+    return _library(x, w, out, impl, alpha, ws)
 
 
 def linear_tail(x, w, tail, ws, name: str, impl: str = "auto"):
