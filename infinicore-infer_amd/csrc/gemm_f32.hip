@@ -5,7 +5,8 @@
 // small ones first; the three left out are some 2^-25 of a product, under the rounding of its float32 sum.  Six bfloat16 products take 96 cycles where
 // the float32 instruction takes 256.  a0 w0 has a sum of its own, which is rounded once per 32 k; the five others are summed beside it.  Error against 64 bits
 // (relative, 2-norm; normal values, 1,536 / 3,840 / 5,760 k, 33..2,048 rows): 1.3..2.4e-7 / 1.9..3.9e-7 / 2.3..4.8e-7, the library's float32 product 3.5..7.1e-7 / 0.56..1.1e-6 / 0.67..1.4e-6
-// (with all six in one sum 2.9..6.1e-7 / 4.8..9.8e-7).  A result that is not finite is summed again in plain float32, since inf - inf is no part of infinity.
+// (with all six in one sum 2.9..6.1e-7 / 4.8..9.8e-7).  The 16 rows of a result that is not finite are summed again with the float32
+// instructions, since inf - inf is no part of infinity.
 //
 // A is split once per product by a kernel before (3.7 us and 10 bytes a value), into the order of the matrix cores' operands: 1 KB per 16 rows, 32 k and part, which go to LDS and
 // into registers as they lie.  W stays float32 in memory and in LDS (rows of 128 bytes, the 16-byte chunk c of row r at c ^ (r / 2 % 8)) and is split in registers by the
@@ -65,6 +66,32 @@ template <int MT_, int NT_, int STAGES_> struct Shape {
     static constexpr int PIECES = 3 * MT + 8 * NT, LOADS = (PIECES + 3) / 4, STAGE_BYTES = 1024 * PIECES;
     static_assert(STAGES >= 2 && STAGES * STAGE_BYTES <= 160 * 1024 && LOADS * (STAGES - 1) < 64, "limits");
 };
+
+// What is summed again is bound by the loads' latency.  One row of 517 (130) with a NaN, 7,680 x 1,536: the product 83 -> 114 us (29 -> 57); with a result summed by its lane, k after k,
+// 1,623 (526).
+// 16 rows of A times NT tiles of 16 rows of W over k0 .. k1 - 1 (multiples of 32) with the float32 instructions: a lane's pointers are at k 4 (lane / 16) of row lane % 16, and
+// instruction e takes k e, 4 + e, 8 + e and 12 + e of a run of 16.
+template <int NT> __device__ __forceinline__ void sum_again(const float* pa, const float* const (&pw)[NT], int k0, int k1, v4f (&x)[NT]) {
+    constexpr int RUNS = NT > 2 ? 4 : 8;
+    for (int k = k0; k < k1; k += 16 * RUNS) {
+        v4f va[RUNS], vw[NT][RUNS];
+#pragma unroll
+        for (int u = 0; u < RUNS; ++u) {
+            const int from = min(k + 16 * u, k1 - 16);
+            va[u] = *reinterpret_cast<const v4f*>(pa + from);
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) vw[nt][u] = *reinterpret_cast<const v4f*>(pw[nt] + from);
+        }
+#pragma unroll
+        for (int u = 0; u < RUNS; ++u) {
+            if (k + 16 * u >= k1) break;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) x[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vw[nt][u][e], va[u][e], x[nt], 0, 0, 0);
+        }
+    }
+}
 
 template <typename T>
 __global__ void __launch_bounds__(256, 1) gemm_f32_kernel(F32Args a) {
@@ -184,32 +211,46 @@ __global__ void __launch_bounds__(256, 1) gemm_f32_kernel(F32Args a) {
     wait_loads<0>();                                               // (nothing may land in LDS after the block)
 
     float* const C = a.C + (size_t)slice * a.slice_stride;
+    const int n_lane = n0 + wave * 16 * NT + 4 * kq;
+    auto store = [&](v4f x, int m, int n) {
+        float* const to = C + (size_t)m * a.ldc + n;
+        x *= a.alpha;
+        if (n + 4 <= a.N) *reinterpret_cast<v4f*>(to) = x;
+        else
+            for (int e = 0; n + e < a.N; ++e) to[e] = x[e];
+    };
+    unsigned again = 0;                                            // row tiles of this wave that are summed again
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
         const int m = m0 + 16 * mt + r;
-        if (m >= a.M) continue;
+        bool odd = false;
+        if (m < a.M) {
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                const int n = n_lane + 16 * nt;
+                if (n >= a.N) continue;
+                const v4f x = acc[nt][mt] + low[nt][mt];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) odd = odd || !(fabsf(x[e]) <= 3.402823466e38f);
+                store(x, m, n);
+            }
+        }
+        if (__builtin_amdgcn_ballot_w64(odd)) again |= 1u << mt;
+    }
+    for (; again; again &= again - 1) {
+        const int m = m0 + 16 * __builtin_ctz(again) + r;
+        v4f x[NT];
+        const float *pa1 = a.A + (size_t)min(m, a.M - 1) * a.lda + 4 * kq, *pw1[NT];
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
-            const int n = n0 + (wave * NT + nt) * 16 + 4 * kq;
-            if (n >= a.N) continue;
-            v4f x = acc[nt][mt] + low[nt][mt];
-            bool odd = false;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) odd = odd || !(fabsf(x[e]) <= 3.402823466e38f);
-            if (odd) {
-                for (int e = 0; e < 4 && n + e < a.N; ++e) {
-                    const float *pa1 = a.A + (size_t)m * a.lda, *pw1 = a.W + (size_t)(n + e) * a.ldw;
-                    float d = 0.f;
-                    for (int k = 32 * s_first; k < 32 * s_end; ++k) d = fmaf(pa1[k], pw1[k], d);
-                    x[e] = d;
-                }
-            }
-            x *= a.alpha;
-            float* const to = C + (size_t)m * a.ldc + n;
-            if (n + 4 <= a.N) *reinterpret_cast<v4f*>(to) = x;
-            else
-                for (int e = 0; n + e < a.N; ++e) to[e] = x[e];
+            pw1[nt] = a.W + (size_t)min(n0 + (wave * NT + nt) * 16 + r, a.N - 1) * a.ldw + 4 * kq;
+            x[nt] = v4f{0.f, 0.f, 0.f, 0.f};
         }
+        sum_again<NT>(pa1, pw1, 32 * s_first, 32 * s_end, x);
+        if (m >= a.M) continue;
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+            if (n_lane + 16 * nt < a.N) store(x[nt], m, n_lane + 16 * nt);
     }
 }
 

@@ -115,3 +115,36 @@ def test_smaller_error_than_the_library():
         ops.matmul_library(A, W, lib)
         want = A.double() @ W.double().t()
         assert (own.double() - want).norm() <= (lib.double() - want).norm()
+
+
+def _fastest(call, n=7):
+    times = []
+    for _ in range(n):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(5):
+            call()
+        b.record()
+        b.synchronize()
+        times.append(a.elapsed_time(b))
+    return min(times)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("slices", [1, 2])
+def test_a_row_that_is_not_finite_costs_others_little(slices):
+    """A request whose row holds a NaN shares its step with others: their results keep their bits outside the row's 16, and the product takes at most three times as long
+    (with a result summed by one lane, k after k, it took twenty times)."""
+    M, N, K = 517, 7680, 1536
+    a, w = _inputs(M, N, K)
+    A, W, out, want = a.cuda(), w.cuda(), torch.empty(M, N, device="cuda"), torch.empty(M, N, device="cuda")
+    call = lambda: ops.gemm_f32(A, W, out, 1.0, 11, slices)          # noqa: E731
+    call()
+    clean = _fastest(call)
+    want.copy_(out)
+    A[300, 7] = float("nan")
+    call()
+    rows = torch.tensor([m // 16 != 300 // 16 for m in range(M)], device="cuda")
+    assert torch.equal(out[rows], want[rows]) and bool(out[300].isnan().all())
+    _check(out[[m for m in range(288, 304) if m != 300]], a[[m for m in range(288, 304) if m != 300]], w)
+    assert _fastest(call) < 3.0 * clean
