@@ -1,8 +1,8 @@
 // C[M, N] = alpha * A[M, K] * W[N, K]^T in float32 for many rows M, on the bfloat16 matrix cores.
 //
-// A float32 number is the sum of three bfloat16 numbers: its upper 16 bits, those of what is left, and the rest, which has 8 bits at most; every
-// subtraction is exact.  Of the nine products of parts the six of 2^-16 and more are summed in float32, a0 w0 + a0 w1 + a1 w0 + a1 w1 + a0 w2 + a2 w0, the
-// small ones first; the three left out are some 2^-25 of a product, under the rounding of its float32 sum.  Six bfloat16 products take 96 cycles where
+// A float32 number is the sum of three bfloat16 numbers: the nearest, the one nearest to what is left, and the rest, which has 7 bits at most; every
+// subtraction is exact.  Of the nine products of parts the six of 2^-17 and more are summed in float32, a0 w0 + a0 w1 + a1 w0 + a1 w1 + a0 w2 + a2 w0, the
+// small ones first; the three left out are of either sign and 2^-24.2 of a product at most, 2^-27.4 rms, where the rounding of a float32 product is 2^-24 and 2^-25.2.  Six bfloat16 products take 96 cycles where
 // the float32 instruction takes 256.  a0 w0 has a sum of its own, which is rounded once per 32 k; the five others are summed beside it.  Error against 64 bits
 // (relative, 2-norm; normal values, 1,536 / 3,840 / 5,760 k, 33..2,048 rows): 1.3..2.4e-7 / 1.9..3.9e-7 / 2.3..4.8e-7, the library's float32 product 3.5..7.1e-7 / 0.56..1.1e-6 / 0.67..1.4e-6
 // (with all six in one sum 2.9..6.1e-7 / 4.8..9.8e-7).  The 16 rows of a result that is not finite are summed again with the float32
@@ -165,7 +165,7 @@ __global__ void __launch_bounds__(256, 1) gemm_f32_kernel(F32Args a) {
     each<3 * MT>([&](auto i) { a_of(i, Zero{}, 0); });
     each<U>([&](auto u) {
         w_of(u, Zero{}, 0);
-        each<kSplitSteps>([&](auto o) { split_step<decltype(o)::value>(pw[0][decltype(u)::value]); });
+        each<kSplitSteps>([&](auto o) { split_step<decltype(o)::value, true>(pw[0][decltype(u)::value]); });
     });
 
     // One k-step of 32: the operands CUR are multiplied; those of the next step are read from LDS and W's split; the loads of stage s + STAGES go out.
@@ -194,7 +194,7 @@ __global__ void __launch_bounds__(256, 1) gemm_f32_kernel(F32Args a) {
             each<O1 - O0>([&](auto k) {
                 constexpr int o = O0 + decltype(k)::value, u = o / kSplitSteps;
                 if constexpr (o % kSplitSteps == 0 && u + D < U) w_of(std::integral_constant<int, u + D>{}, Next{}, next);
-                split_step<o % kSplitSteps>(pw[CUR ^ 1][u]);
+                split_step<o % kSplitSteps, true>(pw[CUR ^ 1][u]);
             });
             __builtin_amdgcn_sched_barrier(0);
         });

@@ -1,7 +1,7 @@
 """Float32 products on the bfloat16 matrix cores against 64-bit sums.
 
-The bound of an element is (K + 16) 2^-24 sum |a| |w|: K roundings of a float32 sum in any order, and 2^-21 for the three products of parts that are left out
-(a second part is under 2^-7 of its number, a third under 2^-15)."""
+The bound of an element is (K + 16) 2^-24 sum |a| |w|: K roundings of a float32 sum in any order, and room for the three products of parts that are left out, under
+2^-24 of a product (a second part is at most 2^-8 of its number, a third 2^-17)."""
 import ctypes
 
 import pytest
@@ -115,6 +115,34 @@ def test_smaller_error_than_the_library():
         ops.matmul_library(A, W, lib)
         want = A.double() @ W.double().t()
         assert (own.double() - want).norm() <= (lib.double() - want).norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("slices", [1, 2])
+def test_rows_of_one_term(slices):
+    """A result that is one product has that product's error only, and of either sign: 2^-24 for its rounding, 2^-24 for the parts left out (2^-8 2^-17 twice) and the
+    roundings of the five smaller products, under 2^-28 together.  On average nothing is left out: 65,536 errors of 2^-24.2 at most and any sign are under 2^-29."""
+    M, N, K = 256, 256, 256
+    a, w = _inputs(M, N, K)
+    at = torch.arange(M) * 37 % K                                   # (every k once)
+    a = torch.zeros(M, K).scatter_(1, at[:, None], a.gather(1, at[:, None]))
+    out = torch.empty(M, N, device="cuda")
+    ops.gemm_f32(a.cuda(), w.cuda(), out, 1.0, 7, slices)
+    want = a.double() @ w.double().t()
+    off = (out.double().cpu() - want) / want
+    assert float(off.abs().max()) < 2.0 ** -23 + 2.0 ** -28
+    assert abs(float(off.mean())) < 2.0 ** -29
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [32, 64])
+def test_numbers_whose_upper_half_is_small(K):
+    """All operands one number whose lower 16 bits are all ones: its upper half leaves 2^-7 of it, and K products of a sign err alike.  Two float32 roundings per 32 k
+    and one where the two sums meet, 2^-24 each, and 2^-24 for what is left out."""
+    x = torch.tensor(0x3f80ffff, dtype=torch.int32).view(torch.float32).item()
+    a, w, out = torch.full((40, K), x), torch.full((64, K), x), torch.empty(40, 64, device="cuda")
+    ops.gemm_f32(a.cuda(), w.cuda(), out)
+    assert float((out.double().cpu() / (K * float(x) ** 2) - 1.0).abs().max()) < (2 + K / 16) * 2.0 ** -24
 
 
 def _fastest(call, n=7):

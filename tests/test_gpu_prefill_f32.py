@@ -44,3 +44,18 @@ def test_products_of_parts(nh, nkvh, dh, lens):
             wrong += float((out[:, h * dh:(h + 1) * dh].double().cpu() - want).square().sum())
             total += float(want.square().sum())
         assert (wrong / total) ** 0.5 < 2 ** -24 * (dh ** 0.5 + (past + n) ** 0.5)
+
+
+@pytest.mark.parametrize("nh,dh", [(100, 64), (400, 64), (800, 64), (100, 128), (500, 128)])
+def test_products_of_parts_err_to_both_sides(nh, dh):
+    """Values that are all one number whose lower 16 bits are ones: every result is that number, off by the roundings of two sums of at most 16 terms (one chunk of keys, so
+    that no small product meets a large sum), to either side: 2^-24 a rounding.  Parts cut off instead of rounded are off by 2^-23.4 on average, towards zero (rounded: 2^-26.3)."""
+    from infinicore_infer_amd.kernels import ops
+    dev, n, ps = "cuda", 16, 64
+    x = torch.tensor(0x3f80ffff, dtype=torch.int32).view(torch.float32).item()
+    g = torch.Generator().manual_seed(dh + nh)
+    k, q = torch.randn(1, nh, ps, dh, generator=g).to(dev), torch.randn(n, 3 * nh * dh, generator=g).to(dev)
+    tiles, out = torch.tensor([(0, 0, n, 0)], dtype=torch.int32, device=dev), torch.empty(n, nh * dh, device=dev)
+    ops.attention_prefill(q, out, k, torch.full_like(k, x), torch.zeros(1, 1, dtype=torch.int32, device=dev), tiles, 1, nh, nh, dh, ps, dh ** -0.5, 0)
+    off = out.double() / float(x) - 1.0
+    assert abs(float(off.mean())) < 2.0 ** -24 and float(off.abs().max()) < 32 * 2.0 ** -24
