@@ -15,7 +15,7 @@
 // 40 after 700 98 / 41; 36:36, 300 20 / 15; 32:2 of 128, 300 after 130 46 / 37; 2,048 432 / 233; 4,000 1,302 / 869.  Error against 64 bits (relative, 2-norm)
 // 1.4..2.9e-7, with float32 instructions 2.0..4.3e-7.
 //
-// Numbers that are not finite have no parts (inf - inf), and their results are none either: a block that ends with one walks again with the float32
+// A block that ends with a result that is not finite, or under 2^-64 (PartsCheck), walks again with the float32
 // instructions, whose two values of the summed dimension per instruction are free as long as A and B agree: in S^T = K Q^T instruction c takes head
 // dims c and c + DH / 2, in O^T = V^T P^T accumulator r of S^T is the B operand as it stands.
 //
@@ -338,12 +338,13 @@ attn_prefill_f32_kernel(const float* __restrict__ q, int q_stride, float* __rest
     };
     if (tid == 0) odd = 0;
     walk(std::false_type{});
-    float t = 0.f * l;                                        // 0, or not a number
+    PartsCheck check;
+    check.add(l);
 #pragma unroll
     for (int i = 0; i < ND; ++i)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) t = fmaf(oacc[i][r], 0.f, t);
-    if (!(t == 0.f)) odd = 1;
+        for (int r = 0; r < 16; ++r) check.add(oacc[i][r]);
+    if (check.failed()) odd = 1;
     __syncthreads();
     if (odd) walk(std::true_type{});
 

@@ -5,8 +5,8 @@
 // small ones first; the three left out are of either sign and 2^-24.2 of a product at most, 2^-27.4 rms, where the rounding of a float32 product is 2^-24 and 2^-25.2.  Six bfloat16 products take 96 cycles where
 // the float32 instruction takes 256.  a0 w0 has a sum of its own, which is rounded once per 32 k; the five others are summed beside it.  Error against 64 bits
 // (relative, 2-norm; normal values, 1,536 / 3,840 / 5,760 k, 33..2,048 rows): 1.3..2.4e-7 / 1.9..3.9e-7 / 2.3..4.8e-7, the library's float32 product 3.5..7.1e-7 / 0.56..1.1e-6 / 0.67..1.4e-6
-// (with all six in one sum 2.9..6.1e-7 / 4.8..9.8e-7).  The 16 rows of a result that is not finite are summed again with the float32
-// instructions, since inf - inf is no part of infinity.
+// (with all six in one sum 2.9..6.1e-7 / 4.8..9.8e-7).  The 16 rows of a result that is not finite, or under 2^-64, are summed again with
+// the float32 instructions (PartsCheck).
 //
 // A is split once per product by a kernel before (3.7 us and 10 bytes a value), into the order of the matrix cores' operands: 1 KB per 16 rows, 32 k and part, which go to LDS and
 // into registers as they lie.  W stays float32 in memory and in LDS (rows of 128 bytes, the 16-byte chunk c of row r at c ^ (r / 2 % 8)) and is split in registers by the
@@ -223,7 +223,7 @@ __global__ void __launch_bounds__(256, 1) gemm_f32_kernel(F32Args a) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
         const int m = m0 + 16 * mt + r;
-        bool odd = false;
+        PartsCheck odd;
         if (m < a.M) {
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
@@ -231,11 +231,11 @@ __global__ void __launch_bounds__(256, 1) gemm_f32_kernel(F32Args a) {
                 if (n >= a.N) continue;
                 const v4f x = acc[nt][mt] + low[nt][mt];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) odd = odd || !(fabsf(x[e]) <= 3.402823466e38f);
+                for (int e = 0; e < 4; ++e) odd.add(x[e]);
                 store(x, m, n);
             }
         }
-        if (__builtin_amdgcn_ballot_w64(odd)) again |= 1u << mt;
+        if (__builtin_amdgcn_ballot_w64(odd.failed())) again |= 1u << mt;
     }
     for (; again; again &= again - 1) {
         const int m = m0 + 16 * __builtin_ctz(again) + r;

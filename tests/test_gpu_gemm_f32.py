@@ -135,6 +135,31 @@ def test_rows_of_one_term(slices):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("slices", [1, 2])
+@pytest.mark.parametrize("tiny", ["a", "w"])
+def test_tiny_numbers(tiny, slices):
+    """Rows of one term down to 2^-118, whose third part no bfloat16 number holds: a float32 product's error (2^-24; in parts 2^-23 and the five roundings), and other rows as ever."""
+    M, N, K = 60, 132, 128
+    a, w = _inputs(M, N, K)
+    one, many = (a, w) if tiny == "a" else (w, a)
+    n = one.shape[0]
+    at = torch.arange(n) * 37 % K
+    one = torch.zeros(n, K).scatter_(1, at[:, None], one.gather(1, at[:, None]).sign() * (1.0 + torch.rand(n, 1, generator=torch.Generator().manual_seed(3))))
+    one *= torch.exp2(-(torch.arange(n) % 20).double() * 2 - 80).float()[:, None]                 # 2^-80 .. 2^-118
+    many = many.sign() * (1.0 + torch.rand(many.shape, generator=torch.Generator().manual_seed(4)))
+    one[::3] = torch.randn(one[::3].shape, generator=torch.Generator().manual_seed(5))
+    a, w = (one, many) if tiny == "a" else (many, one)
+    out = torch.empty(M, N, device="cuda")
+    ops.gemm_f32(a.cuda(), w.cuda(), out, 1.0, 7, slices)
+    want = a.double() @ w.double().t()
+    _check(out, a, w)
+    off = (out.double().cpu() / want - 1.0).abs()
+    off = off if tiny == "a" else off.t()
+    off[::3] = 0.0
+    assert float(off.max()) < 2.0 ** -23 + 2.0 ** -28
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("K", [32, 64])
 def test_numbers_whose_upper_half_is_small(K):
     """All operands one number whose lower 16 bits are all ones: its upper half leaves 2^-7 of it, and K products of a sign err alike.  Two float32 roundings per 32 k

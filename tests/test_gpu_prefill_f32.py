@@ -59,3 +59,21 @@ def test_products_of_parts_err_to_both_sides(nh, dh):
     ops.attention_prefill(q, out, k, torch.full_like(k, x), torch.zeros(1, 1, dtype=torch.int32, device=dev), tiles, 1, nh, nh, dh, ps, dh ** -0.5, 0)
     off = out.double() / float(x) - 1.0
     assert abs(float(off.mean())) < 2.0 ** -24 and float(off.abs().max()) < 32 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("nh,dh", [(100, 64), (400, 64), (800, 64), (100, 128), (500, 128)])
+def test_tiny_values(nh, dh):
+    """Values under 2^-110, whose third part no bfloat16 number holds: the first token's result is its one value, and the others' keep a float32 sum's error."""
+    from infinicore_infer_amd.kernels import ops
+    dev, n, ps = "cuda", 16, 64
+    g = torch.Generator().manual_seed(dh + nh)
+    k, q = torch.randn(1, nh, ps, dh, generator=g).to(dev), torch.randn(n, 3 * nh * dh, generator=g).to(dev)
+    v = (torch.randn(1, nh, ps, dh, generator=g) * 2.0 ** -113).to(dev)
+    tiles, out = torch.tensor([(0, 0, n, 0)], dtype=torch.int32, device=dev), torch.empty(n, nh * dh, device=dev)
+    ops.attention_prefill(q, out, k, v, torch.zeros(1, 1, dtype=torch.int32, device=dev), tiles, 1, nh, nh, dh, ps, dh ** -0.5, 0)
+    first = v[0, :, 0].reshape(-1).double()
+    whole = first.abs() > 2.0 ** -120
+    assert float((out[0].double() / first - 1.0).abs()[whole].max()) < 2.0 ** -23
+    s = (q[:, :dh].double().cpu() @ k[0, 0, :n].double().cpu().t() * dh ** -0.5).masked_fill(~torch.ones(n, n).tril().bool(), float("-inf"))
+    p, v0 = torch.softmax(s, -1), v[0, 0, :n].double().cpu()
+    assert bool(((out[:, :dh].double().cpu() - p @ v0).abs() <= (64 + 2 * dh ** 0.5) * 2.0 ** -24 * (p @ v0.abs())).all())
