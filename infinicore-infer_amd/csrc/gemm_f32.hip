@@ -411,6 +411,10 @@ int most_slices(int M, int N, int K, long long workspace_bytes) {
 
 IC_EXPORT int ic_gemm_f32_supported(int M, int N, int K, int lda, int ldw, int ldc) { return takes(M, N, K, lda, ldw, ldc); }
 
+IC_EXPORT int ic_gemm_f32_takes(int M, int N, int K, int lda, int ldw, int ldc, const void* workspace, long long workspace_bytes) {
+    return takes(M, N, K, lda, ldw, ldc) && workspace && aligned16(workspace) && rows_at_once(M, K, workspace_bytes) > 0;
+}
+
 IC_EXPORT int ic_gemm_f32_plan_on(int M, int N, int K, int adds_slices, int units, int* slices) {
     if (M <= 0 || N <= 0 || K < 32 || units <= 0) return -1;
     const Plan p = plan_for(M, N, K, adds_slices != 0, kMaxSlices, units);
@@ -438,12 +442,13 @@ IC_EXPORT long long ic_gemm_f32_workspace_bytes(int M, int N, int K) {
     return need < most ? need : most;
 }
 
-// The product by this file's kernels or the library's, by the rule: parts is the caller's own memory for the former, workspace the library's.
+// The product by this file's kernels or the library's, as timed (ic_product_tune) or by the rule: parts is the caller's own memory for the former, workspace the library's.
 IC_EXPORT int ic_product_f32(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, float alpha, void* parts, long long parts_bytes,
                              void* workspace, long long workspace_bytes, hipStream_t stream) {
-    if (A && W && C && parts && aligned16(A) && aligned16(W) && aligned16(C) && aligned16(parts) && takes(M, N, K, lda, ldw, ldc) &&
-        rows_at_once(M, K, parts_bytes) > 0 && ic_gemm_f32_pays(M, N, K))
-        return ic_gemm_f32(A, W, C, M, N, K, lda, ldw, ldc, alpha, parts, parts_bytes, stream);
+    if (M > kFewRows && A && W && C && aligned16(A) && aligned16(W) && aligned16(C) && ic_gemm_f32_takes(M, N, K, lda, ldw, ldc, parts, parts_bytes)) {
+        const int timed = ic_product_f32_timed(M, N, K, lda, ldw, ldc);
+        if (timed >= 0 ? timed : ic_gemm_f32_pays(M, N, K)) return ic_gemm_f32(A, W, C, M, N, K, lda, ldw, ldc, alpha, parts, parts_bytes, stream);
+    }
     return ic_matmul(A, IC_F32, W, C, IC_F32, M, N, K, lda, ldw, ldc, alpha, workspace, workspace_bytes, stream);
 }
 

@@ -598,7 +598,7 @@ IC_EXPORT int ic_gemm_tiles_rope_cfg(const void* A, const void* W, void* C, int 
     return rope_run(A, W, C, M, K, lda, ldw, ldc, positions, slots, cos_t, sin_t, kcache, vcache, nh, nkvh, dh, page_size, tile, stream);
 }
 
-// The product by the kernel that is faster for it, as timed (ic_product_tune) or by the rule: this file's or the library's; in float32, by the rule, gemm_f32.hip's or the library's.
+// The product by the kernel that is faster for it, as timed (ic_product_tune) or by the rule: this file's or the library's, in float32 gemm_f32.hip's or the library's.
 IC_EXPORT int ic_product(const void* A, int a_dtype, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldw, int ldc, float alpha,
                          void* workspace, long long workspace_bytes, hipStream_t stream) {
     if (a_dtype == IC_BF16 && c_dtype == IC_BF16 && alpha == 1.0f && A && W && C && ic_gemm_tiles_supported(M, N, K, lda, ldw, ldc, EPI_BF16) &&

@@ -166,7 +166,7 @@ int ic_gemm_tiles(const void* A, const void* W, void* C, int M, int N, int K, in
 int ic_gemm_tiles_rope_supported(const void* A, const void* W, const void* C, int M, int K, int lda, int ldw, int ldc, const float* cos_t, const float* sin_t, const void* kcache, const void* vcache, int nh, int nkvh, int dh, int page_size);
 int ic_gemm_tiles_rope(const void* A, const void* W, void* C, int M, int K, int lda, int ldw, int ldc, const int* positions, const int* slots, const float* cos_t, const float* sin_t, void* kcache, void* vcache, int nh, int nkvh, int dh, int page_size, hipStream_t stream);
 // C[M, N] = alpha * A[M, K] W[N, K]^T for many rows by the faster of ic_gemm_tiles, ic_gemm_f32 and ic_matmul; arguments and results as ic_matmul.  Which is the
-// faster one ic_gemm_tiles_pays and ic_gemm_f32_pays say, or ic_product_tune found (bfloat16; matmul_library.hip).
+// faster one ic_gemm_tiles_pays and ic_gemm_f32_pays say, or ic_product_tune found (matmul_library.hip).
 int ic_product(const void* A, int a_dtype, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldw, int ldc, float alpha, void* workspace, long long workspace_bytes, hipStream_t stream);
 
 // ---- gemm_f32.hip ---------------------------------------------------------------------------------------
@@ -193,10 +193,11 @@ int ic_matmul(const void* A, int a_dtype, const void* W, void* C, int c_dtype, i
 // Times the algorithms the library has for this shape and keeps the fastest; returns how many were tried.
 // flush (or nullptr): memory larger than the caches, overwritten before every timed launch so that operands come from memory.
 int ic_matmul_tune(const void* A, int a_dtype, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldw, int ldc, void* workspace, long long workspace_bytes, void* flush, long long flush_bytes, int reps, hipStream_t stream);
-// The same, and ic_gemm_tiles timed against the algorithm that is kept, for later calls of ic_product with this shape or a row count within an eighth of it.
+// The same, and ic_gemm_tiles (float32: ic_gemm_f32) timed against the algorithm that is kept, for later calls of ic_product with this shape or a row count within an eighth of it.
 int ic_product_tune(const void* A, int a_dtype, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldw, int ldc, void* workspace, long long workspace_bytes, void* flush, long long flush_bytes, int reps, hipStream_t stream);
-// What that found: 1 the tiles, 0 the library, -1 not timed.
+// What that found, in bfloat16 and in float32: 1 the package's own kernel, 0 the library, -1 not timed.
 int ic_product_timed(int M, int N, int K, int lda, int ldw, int ldc);
+int ic_product_f32_timed(int M, int N, int K, int lda, int ldw, int ldc);
 
 // ---- attn_pooled.hip: a window of tokens plus one mean key/value per block before it, sigmoid weights ---------------
 // Adjacent pairs (2i, 2i+1) of the first rot_dims entries of every q and k head turn by position * f_i (freq: float32

@@ -30,12 +30,15 @@ int ic_gemm_tiles_plan_on(int M, int N, int K, int mode, int units);
 int ic_gemm_tiles_pays_on(int M, int N, int K, int mode, int units);
 // Notes what timing a product found (ic_product_tune does).
 void ic_product_timing(int M, int N, int K, int lda, int ldw, int ldc, int tiles);
+void ic_product_f32_timing(int M, int N, int K, int lda, int ldw, int ldc, int own);
 
 // ic_gemm_f32 with its shape (0..14, the order in gemm_f32.hip) and number of slices of K (1..4) named by the caller; the shape that it chooses by itself on a device of
 // `units` compute units (-1: an argument fault) and the slices (adds_slices: whoever follows adds them up, else a kernel of its own), and ic_gemm_f32_pays for such a device.
 int ic_gemm_f32_cfg(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, float alpha, int shape, int slices, void* workspace, long long workspace_bytes, hipStream_t stream);
 int ic_gemm_f32_plan_on(int M, int N, int K, int adds_slices, int units, int* slices);
 int ic_gemm_f32_pays_on(int M, int N, int K, int units);
+// Whether ic_gemm_f32 takes a product of 16-byte aligned operands with this workspace.
+int ic_gemm_f32_takes(int M, int N, int K, int lda, int ldw, int ldc, const void* workspace, long long workspace_bytes);
 
 // key / page_size as the kernels of single tokens compute it; -1: an argument fault.
 int ic_attn_decode_page_of(int key, int page_size);

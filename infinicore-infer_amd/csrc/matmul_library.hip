@@ -2,7 +2,7 @@
 // C[M, N] = alpha * A[M, K] W[N, K]^T through hipBLASLt.  A product's descriptors and the
 // algorithm chosen for it are kept per shape, so a call costs a table lookup and one
 // hipblasLtMatmul.  ic_matmul_tune times the algorithms the library proposes for a shape on
-// the device and keeps the fastest, ic_product_tune compares it with the tiles of gemm_tiles.hip as well.  Host
+// the device and keeps the fastest, ic_product_tune compares it with gemm_tiles.hip's product (float32: gemm_f32.hip's) as well.  Host
 // code only: there is no kernel in this file.
 //
 // hipBLASLt is column-major.  Row-major C[M, N] = A W^T is column-major C^T[N, M] =
@@ -258,53 +258,64 @@ IC_EXPORT int ic_matmul_tune(const void* A, int a_dtype, const void* W, void* C,
     return tried;
 }
 
-// ---- products whose library algorithms were timed, against the tiles of gemm_tiles.hip ---------------------------------
+// ---- products whose library algorithms were timed, against the package's own kernels: gemm_tiles.hip's, in float32 gemm_f32.hip's ------------------------
 namespace {
 
-struct TimedProduct { int M, N, K, lda, ldw, ldc; bool tiles; };
+struct TimedProduct { int dtype, M, N, K, lda, ldw, ldc; bool own; };
 std::vector<TimedProduct> g_timed;           // one a timed shape, guarded by g_mu
 std::atomic<int> g_n_timed{0};               // (most programs time none and ask without the lock)
 
-}  // namespace
-
-IC_EXPORT void ic_product_timing(int M, int N, int K, int lda, int ldw, int ldc, int tiles) {
+void note_timing(int dtype, int M, int N, int K, int lda, int ldw, int ldc, bool own) {
     std::lock_guard<std::mutex> lock(g_mu);
     for (TimedProduct& t : g_timed)
-        if (t.M == M && t.N == N && t.K == K && t.lda == lda && t.ldw == ldw && t.ldc == ldc) { t.tiles = tiles != 0; return; }
-    g_timed.push_back(TimedProduct{M, N, K, lda, ldw, ldc, tiles != 0});
+        if (t.dtype == dtype && t.M == M && t.N == N && t.K == K && t.lda == lda && t.ldw == ldw && t.ldc == ldc) { t.own = own; return; }
+    g_timed.push_back(TimedProduct{dtype, M, N, K, lda, ldw, ldc, own});
     g_n_timed.store((int)g_timed.size());
 }
 
-IC_EXPORT int ic_product_timed(int M, int N, int K, int lda, int ldw, int ldc) {
+int timing_found(int dtype, int M, int N, int K, int lda, int ldw, int ldc) {
     if (g_n_timed.load() == 0) return -1;
     std::lock_guard<std::mutex> lock(g_mu);
     const TimedProduct* from = nullptr;
     int dist = 0;
     for (const TimedProduct& t : g_timed) {
-        if (t.N != N || t.K != K || t.lda != lda || t.ldw != ldw || t.ldc != ldc) continue;
+        if (t.dtype != dtype || t.N != N || t.K != K || t.lda != lda || t.ldw != ldw || t.ldc != ldc) continue;
         const int d = t.M > M ? t.M - M : M - t.M;
         if (8LL * d <= t.M && (!from || d < dist)) { from = &t; dist = d; }
     }
-    return from ? (from->tiles ? 1 : 0) : -1;
+    return from ? (from->own ? 1 : 0) : -1;
 }
 
-// As ic_matmul_tune, and where the product could run in tiles the two are timed against each other, the rows of A in the caches as the kernel before leaves
-// them (with A out of memory too, 871 x 4,096 x 16,384 seems faster in the library, which takes 150 us where the tiles take 133): ic_product then takes, for
+}  // namespace
+
+IC_EXPORT void ic_product_timing(int M, int N, int K, int lda, int ldw, int ldc, int tiles) { note_timing(IC_BF16, M, N, K, lda, ldw, ldc, tiles != 0); }
+
+IC_EXPORT int ic_product_timed(int M, int N, int K, int lda, int ldw, int ldc) { return timing_found(IC_BF16, M, N, K, lda, ldw, ldc); }
+
+IC_EXPORT void ic_product_f32_timing(int M, int N, int K, int lda, int ldw, int ldc, int own) { note_timing(IC_F32, M, N, K, lda, ldw, ldc, own != 0); }
+
+IC_EXPORT int ic_product_f32_timed(int M, int N, int K, int lda, int ldw, int ldc) { return timing_found(IC_F32, M, N, K, lda, ldw, ldc); }
+
+// As ic_matmul_tune, and where the product could run in the package's own kernel the two are timed against each other, the rows of A in the caches as the kernel before
+// leaves them (with A out of memory too, 871 x 4,096 x 16,384 in bfloat16 seems faster in the library, which takes 150 us where the tiles take 133): ic_product then takes, for
 // this shape and the neighbours that take the timed algorithm, the one that the rule names without timing unless the other was 3 % faster.
 IC_EXPORT int ic_product_tune(const void* A, int a_dtype, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldw, int ldc,
                               void* workspace, long long workspace_bytes, void* flush, long long flush_bytes, int reps, hipStream_t stream) {
     const int tried = ic_matmul_tune(A, a_dtype, W, C, c_dtype, M, N, K, lda, ldw, ldc, workspace, workspace_bytes, flush, flush_bytes, reps, stream);
-    if (tried < 0 || a_dtype != IC_BF16 || c_dtype != IC_BF16 || M <= 32 || !ic_gemm_tiles_supported(M, N, K, lda, ldw, ldc, 0) ||
-        (((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) & 15)) return tried;
+    if (tried < 0 || a_dtype != c_dtype || (a_dtype != IC_BF16 && a_dtype != IC_F32) || M <= 32 || (((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) & 15)) return tried;
+    const bool f32 = a_dtype == IC_F32;
+    if (f32 ? !ic_gemm_f32_takes(M, N, K, lda, ldw, ldc, workspace, workspace_bytes) : !ic_gemm_tiles_supported(M, N, K, lda, ldw, ldc, 0)) return tried;
     const Events ev;
     if (!ev.ok) return tried;
     if (!flush) flush_bytes = 0;
-    const long long rows = 2 * ((long long)(M - 1) * lda + K);
+    const long long rows = (f32 ? 4 : 2) * ((long long)(M - 1) * lda + K);
     auto timed = [&](auto call) { return time_calls(call, reps, flush, flush_bytes, A, rows, ev.e0, ev.e1, stream); };
     const float library = timed([&] { return ic_matmul(A, a_dtype, W, C, c_dtype, M, N, K, lda, ldw, ldc, 1.0f, workspace, workspace_bytes, stream); });
-    const float tiles = timed([&] { return ic_gemm_tiles(A, W, C, M, N, K, lda, ldw, ldc, 0, stream); });
-    if (library < 0.f || tiles < 0.f) return tried;
-    const bool rule = ic_gemm_tiles_pays(M, N, K, 0) != 0;
-    ic_product_timing(M, N, K, lda, ldw, ldc, rule ? library >= 0.97f * tiles : tiles < 0.97f * library);
+    const float own = timed([&] {
+        return f32 ? ic_gemm_f32(A, W, C, M, N, K, lda, ldw, ldc, 1.0f, workspace, workspace_bytes, stream) : ic_gemm_tiles(A, W, C, M, N, K, lda, ldw, ldc, 0, stream);
+    });
+    if (library < 0.f || own < 0.f) return tried;
+    const bool rule = (f32 ? ic_gemm_f32_pays(M, N, K) : ic_gemm_tiles_pays(M, N, K, 0)) != 0;
+    note_timing(a_dtype, M, N, K, lda, ldw, ldc, rule ? library >= 0.97f * own : own < 0.97f * library);
     return tried + 1;
 }

@@ -625,12 +625,12 @@ class Engine:
         """Let the plain matrix products for prompt portions of the given token counts use the fastest
         kernel: one dummy step per count is run in which every product of many rows first times the
         algorithms the library has for its shape on the device, keeps the best, and times the package's
-        own product in tiles against it (unless gemm_impl is "library").  QKV and gate/up that run in
+        own product against it (unless gemm_impl is "library").  QKV and gate/up that run in
         tiles with what follows them in the epilogue are not asked about.  Between
         timed launches 512 MB of scratch memory are overwritten: in a model every product's weights
         come from memory, not from the cache lines a repeated launch would find.  A step whose
         token count is within an eighth of a timed one takes that one's choices; other shapes keep
-        the rule between tiles and the library's first choice and cost nothing.  Optional; results
+        the rule between the package's product and the library's first choice and cost nothing.  Optional; results
         live for this process."""
         from ..parts import linear as _linear
         _linear.TUNE_LIBRARY = True

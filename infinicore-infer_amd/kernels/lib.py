@@ -186,6 +186,8 @@ _SIGNATURES = {
     "ic_matmul": [_P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _P, _LL, _P],
     "ic_product_tune": [_P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _LL, _P, _LL, _I, _P],
     "ic_product_timed": [_I] * 6,
+    "ic_product_f32_timed": [_I] * 6,
+    "ic_product_f32_timing": [_I] * 7,
     "ic_product_timing": [_I] * 7,
     "ic_matmul_tune": [_P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _LL, _P, _LL, _I, _P],
     "ic_gemm_qkv_rope_variant": [_P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _RF, _I, _P],
@@ -239,7 +241,7 @@ _SIGNATURES = {
     "ic_decoder_pack": [_P, _c.POINTER(IcHostBatch), _P, _P, _LL, _c.POINTER(IcStepBatch)],
     "ic_decoder_step": [_P, _c.POINTER(IcHostBatch), _P, _P, _LL, _P, _LL, _P, _LL, _P, _c.POINTER(IcStepBatch), _P],
 }
-_RESTYPES = {"ic_product_timing": None, "ic_decoder_create": _P, "ic_decoder_create_error": _c.c_char_p, "ic_decoder_destroy": None,
+_RESTYPES = {"ic_product_timing": None, "ic_product_f32_timing": None, "ic_decoder_create": _P, "ic_decoder_create_error": _c.c_char_p, "ic_decoder_destroy": None,
              "ic_decoder_last_error": _c.c_char_p, "ic_decoder_workspace_bytes": _LL, "ic_decoder_step_ints": _LL,
              "ic_peak_mfma_bf16": _LL, "ic_attn_prefill_scratch_floats": _LL, "ic_gemm_f32_parts_bytes": _LL, "ic_gemm_f32_workspace_bytes": _LL}
 

@@ -627,8 +627,8 @@ def matmul_library(a, w, out, alpha: float = 1.0):
 
 
 def product(a, w, out, alpha: float = 1.0, parts=None):
-    """matmul_library, or the package's own product where that is the faster one: in tiles (gemm_tiles; by the rule, or as product_tune found), in
-    float32 gemm_f32 (by the rule).  parts (float32): a uint8 tensor of product_parts_bytes(M, N, K) for gemm_f32, in place of the library's scratch memory."""
+    """matmul_library, or the package's own product where that is the faster one: in tiles (gemm_tiles), in float32 gemm_f32, by the rule
+    or as product_tune found.  parts (float32): a uint8 tensor of product_parts_bytes(M, N, K) for gemm_f32, in place of the library's scratch memory."""
     return _matmul(get_lib().ic_product, a, w, out, alpha, "product", parts)
 
 
@@ -716,14 +716,16 @@ def matmul_library_tune(a, w, out, reps: int = 5, flush=None) -> int:
 
 
 def product_tune(a, w, out, reps: int = 5, flush=None) -> int:
-    """matmul_library_tune, and the product in tiles (gemm_tiles) timed against the algorithm that is kept: ``product`` then takes the
-    faster one for this shape."""
+    """matmul_library_tune, and the package's own product (in tiles, gemm_tiles; in float32 gemm_f32) timed against the algorithm that is kept: ``product`` then
+    takes the faster one for this shape."""
     return _tune(get_lib().ic_product_tune, a, w, out, reps, flush, "product_tune")
 
 
-def product_timed(m: int, n: int, k: int, lda=None, ldw=None, ldc=None):
-    """What product_tune found for this shape or the nearest row count within an eighth: True the tiles, False the library, None not timed."""
-    found = get_lib().ic_product_timed(int(m), int(n), int(k), int(lda or k), int(ldw or k), int(ldc or n))
+def product_timed(m: int, n: int, k: int, lda=None, ldw=None, ldc=None, dtype=torch.bfloat16):
+    """What product_tune found for this shape or the nearest row count within an eighth: True the package's own kernel, False the library, None not timed."""
+    lib = get_lib()
+    entry = lib.ic_product_f32_timed if dtype == torch.float32 else lib.ic_product_timed
+    found = entry(int(m), int(n), int(k), int(lda or k), int(ldw or k), int(ldc or n))
     return None if found < 0 else bool(found)
 
 

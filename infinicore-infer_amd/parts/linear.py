@@ -21,7 +21,7 @@ torch.backends.cudnn.allow_tf32 = False
 # Which product runs where (own kernel up to some rows, slices over K for the projections into the residual
 # stream, the library beyond) is the kernel library's rule, asked through ops.rule_*: its native step function
 # asks the same functions, so the two ways of issuing a step choose alike.
-TUNE_LIBRARY = False   # while True, every product of many rows first times the library's algorithms for its shape, and the tiles against them
+TUNE_LIBRARY = False   # while True, every product of many rows first times the library's algorithms for its shape, and the package's own kernel against them
 TUNE_FLUSH = None      # while tuning: a tensor larger than the caches, overwritten before every timed launch
 # Products with a side (N or K) below this keep the library's first choice: timing compares speed alone, and among the
 # algorithms the library lists as taking a product with K = 64 one was met that is fastest and returns NaN.  Products this

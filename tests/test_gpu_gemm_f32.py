@@ -73,6 +73,41 @@ def test_chosen(M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows", [264, 72])
+def test_products_follow_what_timing_found(rows):
+    """After timing, ops.product runs the kernel that was found the faster one, whatever the rule says, here and with the caller's own scratch memory; bfloat16 products of
+    the same shape are not asked about."""
+    M, N, K = rows, 2560, 4032
+    a, w = _inputs(M, N, K)
+    A, W, (out, own, lib) = a.cuda(), w.cuda(), (torch.empty(M, N, device="cuda") for _ in range(3))
+    assert ops.product_timed(M, N, K, dtype=torch.float32) is None
+    flush = torch.empty(64 << 20, dtype=torch.uint8, device="cuda")
+    assert ops.product_tune(A, W, out, reps=3, flush=flush) >= 2
+    found = ops.product_timed(M, N, K, dtype=torch.float32)
+    assert found is not None
+    ops.gemm_f32(A, W, own)
+    ops.matmul_library(A, W, lib)
+    assert not torch.equal(own, lib)
+    parts = torch.empty(ops.product_parts_bytes(M, N, K), dtype=torch.uint8, device="cuda")
+    for want in (found, not found):
+        get_lib().ic_product_f32_timing(M, N, K, K, K, N, int(want))
+        for mine in (None, parts):
+            ops.product(A, W, out.zero_(), parts=mine)
+            _check(out, a, w)
+            assert torch.equal(out, own if want else lib)
+    get_lib().ic_product_f32_timing(M, N, K, K, K, N, int(found))
+
+
+def test_what_timing_found_cpu():
+    """A timed float32 shape says nothing about the bfloat16 one, nor the other way."""
+    lib, n, k = get_lib(), 5128, 1120                  # (no other test times this matrix)
+    lib.ic_product_f32_timing(800, n, k, k, k, n, 1)
+    assert ops.product_timed(700, n, k, dtype=torch.float32) is True and ops.product_timed(800, n, k) is None
+    lib.ic_product_timing(800, n, k, k, k, n, 0)
+    assert ops.product_timed(800, n, k, dtype=torch.float32) is True and ops.product_timed(800, n, k) is False
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,lda,off", [(300, 2560, 1536, 1538, 0), (300, 2560, 1528, 1528, 0), (300, 2560, 1536, 1540, 1), (300, 2557, 1536, 1536, 0)])
 def test_product_of_forms_the_kernel_does_not_take(M, N, K, lda, off):
     """Odd strides, rows that are no whole k-steps, misaligned operands: the product by the rule is right as ever."""
