@@ -407,6 +407,12 @@ int most_slices(int M, int N, int K, long long workspace_bytes) {
     return s;
 }
 
+// What ic_gemm_f32 costs with this workspace, in microseconds: every run of rows has its split and its product, which reads all of W again.
+double cost_with(int M, int N, int K, long long workspace_bytes, int units) {
+    const int rows = rows_at_once(M, K, workspace_bytes), runs = (M + rows - 1) / rows;
+    return runs * (3.73 + 10.0 * rows * K / (14.8e6 * units / 256.0) + plan_for(rows, N, K, false, most_slices(M, N, K, workspace_bytes), units).cost);
+}
+
 }  // namespace
 
 IC_EXPORT int ic_gemm_f32_supported(int M, int N, int K, int lda, int ldw, int ldc) { return takes(M, N, K, lda, ldw, ldc); }
@@ -422,19 +428,6 @@ IC_EXPORT int ic_gemm_f32_plan_on(int M, int N, int K, int adds_slices, int unit
     return p.shape;
 }
 
-// Whether the split, the product and the sum of its slices beat the library's float32 product, whose time is within 17 % (rms) of 12 us or 8.7 us and 127 TFLOP/s; from 33 rows on,
-// since fewer are a matter of the weights' bytes, which it reads as fast (8 x 7,680 x 1,536: 13 us, the split alone 4).  Over the sweep above the choice loses 1.1 % to the
-// better of the two.  130 x 7,680 x 1,536: 35 -> 29, 256 x 2,560 x 1,536: 28 -> 22, on the other side 96 x 2,560 x 1,536: 11 against 18.
-IC_EXPORT int ic_gemm_f32_pays_on(int M, int N, int K, int units) {
-    if (M <= kFewRows || N <= 0 || K < 32 || units <= 0) return 0;
-    const double products = 2.0 * M * N * K / (127e6 * units / 256.0) + 8.7;
-    return 3.73 + 10.0 * M * K / (14.8e6 * units / 256.0) + plan_for(M, N, K, false, kMaxSlices, units).cost < (products > 12.0 ? products : 12.0);
-}
-
-IC_EXPORT int ic_gemm_f32_pays(int M, int N, int K) { return ic_gemm_f32_pays_on(M, N, K, compute_units()); }
-
-IC_EXPORT long long ic_gemm_f32_parts_bytes(int M, int K) { return M > 0 && K >= 32 ? parts_bytes(M, K) : 0; }
-
 // Memory for any plan of the product: A's parts and all slices, up to 64 MB; grows with M.  None where the rule takes the library's product in any case.
 IC_EXPORT long long ic_gemm_f32_workspace_bytes(int M, int N, int K) {
     if (M <= kFewRows || N <= 0 || K < 32) return 0;
@@ -442,12 +435,28 @@ IC_EXPORT long long ic_gemm_f32_workspace_bytes(int M, int N, int K) {
     return need < most ? need : most;
 }
 
+// Whether the split, the product and the sum of its slices beat the library's float32 product, whose time is within 17 % (rms) of 12 us or 8.7 us and 127 TFLOP/s; from 33 rows on,
+// since fewer are a matter of the weights' bytes, which it reads as fast (8 x 7,680 x 1,536: 13 us, the split alone 4).  Over the sweep above the choice loses 1.1 % to the
+// better of the two.  130 x 7,680 x 1,536: 35 -> 29, 256 x 2,560 x 1,536: 28 -> 22, on the other side 96 x 2,560 x 1,536: 11 against 18.  With the workspace there
+// is: 64 MB hold 672 rows of 16,384, and 2,048 x 4,096 x 16,384 is four runs of 512 rows (1,403 us, the library 1,798); 16 rows at a time never pay.
+IC_EXPORT int ic_gemm_f32_pays_with(int M, int N, int K, long long workspace_bytes, int units) {
+    if (M <= kFewRows || N <= 0 || K < 32 || units <= 0 || rows_at_once(M, K, workspace_bytes) <= 0) return 0;
+    const double products = 2.0 * M * N * K / (127e6 * units / 256.0) + 8.7;
+    return cost_with(M, N, K, workspace_bytes, units) < (products > 12.0 ? products : 12.0);
+}
+
+IC_EXPORT int ic_gemm_f32_pays_on(int M, int N, int K, int units) { return ic_gemm_f32_pays_with(M, N, K, ic_gemm_f32_workspace_bytes(M, N, K), units); }
+
+IC_EXPORT int ic_gemm_f32_pays(int M, int N, int K) { return ic_gemm_f32_pays_on(M, N, K, compute_units()); }
+
+IC_EXPORT long long ic_gemm_f32_parts_bytes(int M, int K) { return M > 0 && K >= 32 ? parts_bytes(M, K) : 0; }
+
 // The product by this file's kernels or the library's, as timed (ic_product_tune) or by the rule: parts is the caller's own memory for the former, workspace the library's.
 IC_EXPORT int ic_product_f32(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, float alpha, void* parts, long long parts_bytes,
                              void* workspace, long long workspace_bytes, hipStream_t stream) {
     if (M > kFewRows && A && W && C && aligned16(A) && aligned16(W) && aligned16(C) && ic_gemm_f32_takes(M, N, K, lda, ldw, ldc, parts, parts_bytes)) {
         const int timed = ic_product_f32_timed(M, N, K, lda, ldw, ldc);
-        if (timed >= 0 ? timed : ic_gemm_f32_pays(M, N, K)) return ic_gemm_f32(A, W, C, M, N, K, lda, ldw, ldc, alpha, parts, parts_bytes, stream);
+        if (timed >= 0 ? timed : ic_gemm_f32_pays_with(M, N, K, parts_bytes, compute_units())) return ic_gemm_f32(A, W, C, M, N, K, lda, ldw, ldc, alpha, parts, parts_bytes, stream);
     }
     return ic_matmul(A, IC_F32, W, C, IC_F32, M, N, K, lda, ldw, ldc, alpha, workspace, workspace_bytes, stream);
 }

@@ -37,6 +37,8 @@ void ic_product_f32_timing(int M, int N, int K, int lda, int ldw, int ldc, int o
 int ic_gemm_f32_cfg(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, float alpha, int shape, int slices, void* workspace, long long workspace_bytes, hipStream_t stream);
 int ic_gemm_f32_plan_on(int M, int N, int K, int adds_slices, int units, int* slices);
 int ic_gemm_f32_pays_on(int M, int N, int K, int units);
+// The same with a workspace of that size (ic_gemm_f32_pays: of ic_gemm_f32_workspace_bytes).
+int ic_gemm_f32_pays_with(int M, int N, int K, long long workspace_bytes, int units);
 // Whether ic_gemm_f32 takes a product of 16-byte aligned operands with this workspace.
 int ic_gemm_f32_takes(int M, int N, int K, int lda, int ldw, int ldc, const void* workspace, long long workspace_bytes);
 

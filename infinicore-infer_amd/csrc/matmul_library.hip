@@ -315,7 +315,7 @@ IC_EXPORT int ic_product_tune(const void* A, int a_dtype, const void* W, void* C
         return f32 ? ic_gemm_f32(A, W, C, M, N, K, lda, ldw, ldc, 1.0f, workspace, workspace_bytes, stream) : ic_gemm_tiles(A, W, C, M, N, K, lda, ldw, ldc, 0, stream);
     });
     if (library < 0.f || own < 0.f) return tried;
-    const bool rule = (f32 ? ic_gemm_f32_pays(M, N, K) : ic_gemm_tiles_pays(M, N, K, 0)) != 0;
+    const bool rule = (f32 ? ic_gemm_f32_pays_with(M, N, K, workspace_bytes, compute_units()) : ic_gemm_tiles_pays(M, N, K, 0)) != 0;
     note_timing(a_dtype, M, N, K, lda, ldw, ldc, rule ? library >= 0.97f * own : own < 0.97f * library);
     return tried + 1;
 }

@@ -43,6 +43,29 @@ def test_plans(units):
     assert not sup(100, 64, 64, 64, 60, 64) and not sup(100, 64, 64, 64, 64, 60) and not sup(0, 64, 64, 64, 64, 64)
 
 
+def test_the_rule_prices_the_runs_that_a_workspace_makes():
+    """A workspace for some of the rows means a split and a product per run of rows, each of which reads all weights again: what pays with room for all rows need not
+    with less, never the other way, and none pays with none."""
+    lib = get_lib()
+    for M, N, K in ((130, 7680, 1536), (517, 1536, 3840), (2048, 4096, 16384), (8192, 4096, 16384)):
+        room = [lib.ic_gemm_f32_parts_bytes(rows, K) for rows in (16, 48, 256, M)] + [64 << 20, 1 << 40]
+        pays = [lib.ic_gemm_f32_pays_with(M, N, K, n, 256) for n in sorted(room)]
+        assert pays == sorted(pays) and pays[0] == 0 and pays[-1] == 1
+        assert not lib.ic_gemm_f32_pays_with(M, N, K, 0, 256) and not lib.ic_gemm_f32_pays_with(M, N, K, room[0] - 1, 256)
+        assert lib.ic_gemm_f32_pays_on(M, N, K, 256) == lib.ic_gemm_f32_pays_with(M, N, K, lib.ic_gemm_f32_workspace_bytes(M, N, K), 256)
+
+
+@pytest.mark.gpu
+def test_a_small_workspace_goes_to_the_library():
+    """With scratch memory for 16 rows at a time (129 runs over 32 MB of weights) the product by the rule is the library's."""
+    M, N, K = 2064, 2048, 4096
+    a, w = _inputs(M, N, K)
+    A, W, out, lib = a.cuda(), w.cuda(), torch.empty(M, N, device="cuda"), torch.empty(M, N, device="cuda")
+    parts = torch.empty(int(get_lib().ic_gemm_f32_parts_bytes(16, K)), dtype=torch.uint8, device="cuda")
+    ops.product(A, W, out, parts=parts)
+    assert torch.equal(out, ops.matmul_library(A, W, lib))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("shape", range(len(SHAPES)))
 def test_edges(shape):
