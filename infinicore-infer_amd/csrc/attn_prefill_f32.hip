@@ -11,8 +11,9 @@
 //
 // Six bfloat16 products take 0.375 of the time of v_mfma_f32_32x32x2_f32, the float32 instruction, and with that a step's products no longer bound the kernel: a step of
 // 32 keys a wave takes 3.2 us where it is alone on its SIMD, 0.65 of it products.  With float32 instructions / so, us (one block's keys by themselves in
-// registers, lookups in a chain, the way before): 24:8 heads of 64, 509 tokens after 130 34 / 24; 100 after 900 45 / 29; 2,048 164 / 88; 4,000 559 / 282; 12 portions of
-// 40 after 700 98 / 41; 36:36, 300 20 / 15; 32:2 of 128, 300 after 130 46 / 37; 2,048 432 / 233; 4,000 1,302 / 869.  Error against 64 bits (relative, 2-norm)
+// registers, lookups in a chain, the way before): 24:8 heads of 64, 509 tokens after 130 33 / 26; 100 after 900 45 / 31; 4,000 548 / 298; 12 portions of
+// 40 after 700 99 / 44; 36:36, 300 after 130 30 / 25; 32:2 of 128, 300 after 130 47 / 39; 2,048 424 / 238; 4,000 1,282 / 886, in a window of 300 269 / 229.  Heads of 128 have one
+// block a unit, where 32-bit operands left room for two: 40 portions of two tokens of 32 heads 43 / 41.  Error against 64 bits (relative, 2-norm)
 // 1.4..2.9e-7, with float32 instructions 2.0..4.3e-7.
 //
 // A block that ends with a result that is not finite, or under 2^-64 (PartsCheck), walks again with the float32
@@ -66,9 +67,15 @@ attn_prefill_f32_kernel(const float* __restrict__ q, int q_stride, float* __rest
     uint16_t* const Vp = SHARED ? Kp : Kp + 3 * KEYS * PKS;
 
     // Tile-major, all heads of the longest tile first.  Heads are innermost: blocks go round the XCDs in turn, and where the tiles are low the row groups that
-    // have nothing to do must not all be the same XCDs'.
-    const int h = (int)blockIdx.x % nh, slot = (int)blockIdx.x / nh, sub = slot % KG;
-    const int4 tile = tiles[slot / KG];
+    // have nothing to do must not all be the same XCDs'.  Nor the same shader engines', where a unit holds one block (heads of 128): there the first row groups of as many
+    // tiles as fill the chip come before the second ones.  Portions of two tokens, us: 12 after 2,000 of 16 heads 300 -> 164, 40 after 300 of 8 heads 77 -> 57; elsewhere
+    // -4 to +5 %.  Heads of 64, two blocks a unit, lose by it (2,048 tokens of 8 heads 58 -> 75).
+    constexpr bool ROUNDS = KG > 1 && DH == 128;
+    const int h = (int)blockIdx.x % nh, slot = (int)blockIdx.x / nh;
+    const int round = ROUNDS ? (256 + nh - 1) / nh : 1, first = slot / (KG * round) * round;      // tiles of a round, and its first one
+    const int in_round = n_tiles - first < round ? n_tiles - first : round, at = slot - KG * first;
+    const int sub = ROUNDS ? at / in_round : at;
+    const int4 tile = tiles[ROUNDS ? first + at - sub * in_round : first];
     const int skip = 32 * RW * sub;                           // rows of the tile before this block's
     const int req = tile.x, row0 = tile.y + skip, pos0 = tile.w + skip;
     const int n_rows = tile.z - skip < 32 * RW ? tile.z - skip : 32 * RW;
@@ -206,6 +213,8 @@ attn_prefill_f32_kernel(const float* __restrict__ q, int q_stride, float* __rest
             const int kt = kb + GK * grp;                   // this group's keys
             // is there anything this wave may see?
             const bool seen = wave_ok && kt <= wave_last && !(window > 0 && kt + GK - 1 < wave_first - window + 1);
+            // Where the second tile of 32 keys is beyond the wave's last row it is left out: 40 portions of two tokens of 32 heads of 128 50 -> 42 us.
+            const int nt_seen = NT > 1 && wave_last - kt < 32 ? 1 : NT;
             f32_v16 sacc[NT];
             if (seen) {
                 // ---- S^T = K Q^T : tiles of 32 keys ----------------------------------------------------------
@@ -213,6 +222,7 @@ attn_prefill_f32_kernel(const float* __restrict__ q, int q_stride, float* __rest
                 for (int tt = 0; tt < NT; ++tt) {
 #pragma unroll
                     for (int r = 0; r < 16; ++r) sacc[tt][r] = 0.f;
+                    if (tt >= nt_seen) continue;                // (masked below)
                     if constexpr (EXACT) {
                         const float* kp = &Ks[(GK * grp + 32 * tt + lq) * KS + HALF * half];
 #pragma unroll
@@ -299,6 +309,7 @@ attn_prefill_f32_kernel(const float* __restrict__ q, int q_stride, float* __rest
             // ---- O^T += V^T P^T : the accumulators of S^T are the B operand as they stand -------------------------------
 #pragma unroll
             for (int tt = 0; tt < NT; ++tt) {
+                if (tt >= nt_seen) continue;
                 if constexpr (EXACT) {
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
@@ -391,9 +402,12 @@ attn_prefill_f32_kernel(const float* __restrict__ q, int q_stride, float* __rest
 }
 
 // Key groups a block has, from the number of (tile, head) pairs: several until one group's blocks keep the units busy by themselves.  One / two / four groups, us,
-// heads of 64: 24 pairs (100 tokens after 900) 53 / 38 / 30; 96 (509 after 130) 36 / 27 / 23; 128 (2,048 of 8 heads) 101 / 72 / 56; 144 (509 after 130 of 36 heads) 37 / 28 / 30;
-// 288 (1,000 and 500) 55 / 42 / 48; 432 (12 portions of 40 after 700) 60 / 45 / 62; 576 (2,048) 126 / 131 / 167; 768 (4,000) 282 / 307 / 382.  Of 128: 32 (100 after 900)
-// 108 / 75; 224 (800 after 200) 110 / 99; 384 (1,000 and 500) 110 / 115, (12 portions of 40 after 700) 161 / 117; 512 (2,048) 233 / 317.
+// heads of 64: 24 pairs (100 tokens after 900) 57 / 40 / 31; 96 (509 after 130) 38 / 28 / 26; 128 (2,048 of 8 heads) 108 / 76 / 58; 144 (509 after 130 of 36 heads) 38 / 29 / 34;
+// 288 (1,000 after 500) 88 / 78 / 97; 432 (12 portions of 40 after 700) 64 / 46 / 67; 576 (2,048) 131 / 134 / 172, (the same in a window of 300) 59 / 55 / 81; 768 (4,000) 298 / 317 / 401.
+// Of 128: 32 (100 after 900) 110 / 77; 224 (800 after 200) 111 / 96; 256 (1,000 after 500) 162 / 157, (twice 512 after 512) 114 / 123; 384 (12 portions of 40 after 700) 164 / 120,
+// (1,500 after 1,500) 430 / 505; 512 (2,048) 238 / 309.  Over 440 forms (8..64 heads, 1..40 portions of 2..4,000 tokens after 0..3,000, all and a window of 300) no other
+// lines do better by more than 0.5 % on average.  Against the float32 instructions throughout: 0.71 of the time for heads of 64, 0.79 of 128, and slower only where a
+// walk is one step: 2 tokens after nothing 7.7 -> 8.0 us (64) and 9.6 -> 10.3 (128), 40 such portions of 8 heads 9.4 -> 10.9 and 17.6 -> 19.2.
 IC_EXPORT int ic_attn_prefill_f32_groups(int dh, long long pairs) {
     if (dh == 128) return pairs <= 400 ? 2 : 1;
     return pairs <= 128 ? 4 : pairs <= 700 ? 2 : 1;

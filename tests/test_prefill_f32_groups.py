@@ -29,3 +29,42 @@ def test_key_groups(nh, nkvh, dh, page, groups, window):
     assert _groups(dh, nh) == groups
     got, want = _attention_case(torch.float32, nh, nkvh, dh, page, LENS, window, 61, "prefill")
     _close(got, want, torch.float32, factor=3)
+
+
+@pytest.mark.gpu
+def test_row_groups_without_work_do_not_crowd_the_others():
+    """Heads of 128, one block a unit, two key groups: of portions of two tokens every second block has no rows.  12 portions of 16 heads (192 pairs, 192 blocks with work for 256
+    units) take about as long as of 8; with empty and full blocks in turn they took 2.1 times as long, since the full ones met on half the units."""
+    from infinicore_infer_amd.kernels import ops
+    ps, dh, past, n = 64, 128, 2000, 12
+    pages = -(-(past + 2) // ps)
+    assert _groups(dh, 16, n) == 2
+
+    def fastest(nh):
+        k, v = (torch.randn(n * pages, nh, ps, dh, device="cuda") for _ in range(2))
+        q, out = torch.randn(2 * n, 3 * nh * dh, device="cuda"), torch.empty(2 * n, nh * dh, device="cuda")
+        table = torch.arange(n * pages, dtype=torch.int32, device="cuda").view(n, pages)
+        tiles = torch.tensor([(r, 2 * r, 2, past) for r in range(n)], dtype=torch.int32, device="cuda")
+        times = []
+        for _ in range(8):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(4):
+                ops.attention_prefill(q, out, k, v, table, tiles, n, nh, nh, dh, ps, dh ** -0.5, 0)
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+    assert fastest(16) < 1.6 * fastest(8)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nh,nkvh,dh,lens", [(100, 20, 128, [(0, 2), (0, 33), (31, 34), (62, 2), (63, 130), (0, 65)]), (120, 24, 64, [(0, 2), (0, 33), (31, 34), (62, 2), (63, 130), (0, 65)]),
+                                             (90, 30, 128, [(0, 130)] * 2), (3, 3, 128, [(0, 2)] * 88 + [(40, 20)])])
+@pytest.mark.parametrize("window", [None, 20])
+def test_half_steps_and_rounds(nh, nkvh, dh, lens, window):
+    """One group: the last step's second half of keys beyond, at and before a wave's last row.  Two groups of heads of 128: rounds of 3 and of 86 tiles, and what is left."""
+    from test_gpu_kernels import _attention_case, _close
+    assert _groups(dh, nh, sum(-(-n // 128) for _, n in lens)) == (1 if nh >= 100 else 2)
+    got, want = _attention_case(torch.float32, nh, nkvh, dh, 64, lens, window, 61, "prefill")
+    _close(got, want, torch.float32, factor=3)
