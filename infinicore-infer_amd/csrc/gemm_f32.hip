@@ -328,11 +328,10 @@ double cost_of(const ShapeCost& c, int M, int N, int K, int slices, int units) {
 }
 
 struct Plan { int shape, slices; double cost; };
-// adds_slices: whoever follows adds the slices up (else a kernel of its own does).
-Plan plan_for(int M, int N, int K, bool adds_slices, int max_slices, int units) {
+Plan plan_for(int M, int N, int K, int max_slices, int units) {
     Plan best{-1, 1, 0.0};
     for (int s = 1; s <= max_slices && s <= kMaxSlices && s <= K / 32 && (s == 1 || N % 4 == 0); ++s) {
-        const double bytes = 4.0 * M * N, extra = s == 1 ? 0.0 : adds_slices ? (s - 1) * bytes / 5e6 : 3.5 + (s + 1) * bytes / 6e6;
+        const double bytes = 4.0 * M * N, extra = s == 1 ? 0.0 : 3.5 + (s + 1) * bytes / 6e6;
         for (int i = 0; i < kShapes; ++i) {
             const double c = cost_of(kCosts[i], M, N, K, s, units) + extra;
             if (best.shape < 0 || c < best.cost) best = Plan{i, s, c};
@@ -410,7 +409,7 @@ int most_slices(int M, int N, int K, long long workspace_bytes) {
 // What ic_gemm_f32 costs with this workspace, in microseconds: every run of rows has its split and its product, which reads all of W again.
 double cost_with(int M, int N, int K, long long workspace_bytes, int units) {
     const int rows = rows_at_once(M, K, workspace_bytes), runs = (M + rows - 1) / rows;
-    return runs * (3.73 + 10.0 * rows * K / (14.8e6 * units / 256.0) + plan_for(rows, N, K, false, most_slices(M, N, K, workspace_bytes), units).cost);
+    return runs * (3.73 + 10.0 * rows * K / (14.8e6 * units / 256.0) + plan_for(rows, N, K, most_slices(M, N, K, workspace_bytes), units).cost);
 }
 
 }  // namespace
@@ -421,9 +420,9 @@ IC_EXPORT int ic_gemm_f32_takes(int M, int N, int K, int lda, int ldw, int ldc, 
     return takes(M, N, K, lda, ldw, ldc) && workspace && aligned16(workspace) && rows_at_once(M, K, workspace_bytes) > 0;
 }
 
-IC_EXPORT int ic_gemm_f32_plan_on(int M, int N, int K, int adds_slices, int units, int* slices) {
+IC_EXPORT int ic_gemm_f32_plan_on(int M, int N, int K, int units, int* slices) {
     if (M <= 0 || N <= 0 || K < 32 || units <= 0) return -1;
-    const Plan p = plan_for(M, N, K, adds_slices != 0, kMaxSlices, units);
+    const Plan p = plan_for(M, N, K, kMaxSlices, units);
     if (slices) *slices = p.slices;
     return p.shape;
 }
@@ -466,7 +465,7 @@ IC_EXPORT int ic_gemm_f32(const void* A, const void* W, void* C, int M, int N, i
                           long long workspace_bytes, hipStream_t stream) {
     if (M <= 0) return IC_OK;
     if (!A || !W || !C || !workspace || !takes(M, N, K, lda, ldw, ldc) || !aligned16(A) || !aligned16(W) || !aligned16(C) || !aligned16(workspace)) return IC_ERR_ARG;
-    const Plan p = plan_for(rows_at_once(M, K, workspace_bytes), N, K, false, most_slices(M, N, K, workspace_bytes), compute_units());
+    const Plan p = plan_for(rows_at_once(M, K, workspace_bytes), N, K, most_slices(M, N, K, workspace_bytes), compute_units());
     return product((const float*)A, (const float*)W, (float*)C, M, N, K, lda, ldw, ldc, alpha, p.shape, p.slices, workspace, workspace_bytes, stream);
 }
 

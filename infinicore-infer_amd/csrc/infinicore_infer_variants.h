@@ -33,9 +33,9 @@ void ic_product_timing(int M, int N, int K, int lda, int ldw, int ldc, int tiles
 void ic_product_f32_timing(int M, int N, int K, int lda, int ldw, int ldc, int own);
 
 // ic_gemm_f32 with its shape (0..14, the order in gemm_f32.hip) and number of slices of K (1..4) named by the caller; the shape that it chooses by itself on a device of
-// `units` compute units (-1: an argument fault) and the slices (adds_slices: whoever follows adds them up, else a kernel of its own), and ic_gemm_f32_pays for such a device.
+// `units` compute units (-1: an argument fault) and the slices, and ic_gemm_f32_pays for such a device.
 int ic_gemm_f32_cfg(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, float alpha, int shape, int slices, void* workspace, long long workspace_bytes, hipStream_t stream);
-int ic_gemm_f32_plan_on(int M, int N, int K, int adds_slices, int units, int* slices);
+int ic_gemm_f32_plan_on(int M, int N, int K, int units, int* slices);
 int ic_gemm_f32_pays_on(int M, int N, int K, int units);
 // The same with a workspace of that size (ic_gemm_f32_pays: of ic_gemm_f32_workspace_bytes).
 int ic_gemm_f32_pays_with(int M, int N, int K, long long workspace_bytes, int units);

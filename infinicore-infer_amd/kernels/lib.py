@@ -209,7 +209,7 @@ _SIGNATURES = {
     "ic_gemm_f32_pays": [_I] * 3,
     "ic_gemm_f32_pays_on": [_I] * 4,
     "ic_gemm_f32_pays_with": [_I, _I, _I, _LL, _I],
-    "ic_gemm_f32_plan_on": [_I] * 5 + [_c.POINTER(_I)],
+    "ic_gemm_f32_plan_on": [_I] * 4 + [_c.POINTER(_I)],
     "ic_gemm_f32_parts_bytes": [_I, _I],
     "ic_gemm_f32_workspace_bytes": [_I] * 3,
     "ic_product_f32": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P, _LL, _P, _LL, _P],

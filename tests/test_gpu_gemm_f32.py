@@ -27,17 +27,28 @@ def _check(got, a, w, alpha=1.0):
     assert bool(((got.double().cpu() - alpha * (A @ W.t())).abs() <= bound).all())
 
 
+def _check_norm(got, a, w, alpha=1.0):
+    """Rows and columns scaled to one size, so that each counts alike: over all elements the error is under (4 + (K / 32)^(1/2)) 2^-24 of the result, a rounding per 32 k
+    of a sum that is no larger, of either sign, and a few where the sums meet; a single row's or column's, of few elements, under four times that.  A third part that is
+    missing shows by 2^-18.5, a second part's product by 2^-19.5 (rms)."""
+    A, W = a.double(), w.double()
+    A, W, scale = A / A.norm(dim=1, keepdim=True), W / W.norm(dim=1, keepdim=True), alpha * A.norm(dim=1)[:, None] * W.norm(dim=1)[None] / a.shape[1] ** 0.5
+    off = got.double().cpu() / scale - (A @ W.t()) * a.shape[1] ** 0.5
+    bound = (4 + (a.shape[1] / 32) ** 0.5) * 2.0 ** -24
+    assert float(off.square().mean().sqrt()) < bound
+    assert all(float(off.square().mean(dim).sqrt().max()) < 4 * bound for dim in (0, 1))
+
+
 @pytest.mark.parametrize("units", [256, 64])
 def test_plans(units):
     """Every plan names a shape and slices that the kernel takes; up to 32 rows the library's product stays."""
     lib, n = get_lib(), ctypes.c_int()
     for M in (1, 32, 33, 130, 517, 2048, 30000):
         for N, K in ((4, 32), (65, 64), (1536, 1536), (7680, 1536), (1536, 3840), (73440, 4096)):
-            for adds in (0, 1):
-                assert 0 <= lib.ic_gemm_f32_plan_on(M, N, K, adds, units, n) < len(SHAPES)
-                assert 1 <= n.value <= min(4, K // 32) and (n.value == 1 or N % 4 == 0)
+            assert 0 <= lib.ic_gemm_f32_plan_on(M, N, K, units, n) < len(SHAPES)
+            assert 1 <= n.value <= min(4, K // 32) and (n.value == 1 or N % 4 == 0)
             assert not (M <= 32 and lib.ic_gemm_f32_pays_on(M, N, K, units))
-    assert lib.ic_gemm_f32_plan_on(0, 64, 64, 0, units, n) == -1 and not lib.ic_gemm_f32_pays_on(100, 0, 64, units)
+    assert lib.ic_gemm_f32_plan_on(0, 64, 64, units, n) == -1 and not lib.ic_gemm_f32_pays_on(100, 0, 64, units)
     sup = lib.ic_gemm_f32_supported
     assert sup(100, 64, 64, 64, 64, 64) and not sup(100, 64, 48, 64, 64, 64) and not sup(100, 64, 64, 66, 64, 64)
     assert not sup(100, 64, 64, 64, 60, 64) and not sup(100, 64, 64, 64, 64, 60) and not sup(0, 64, 64, 64, 64, 64)
@@ -80,6 +91,7 @@ def test_edges(shape):
         A[:, :K], W[:, :K] = a.cuda(), w.cuda()
         ops.gemm_f32(A[:, :K], W[:, :K], out[:M, :N], alpha, shape, slices)
         _check(out[:M, :N], a, w, alpha)
+        _check_norm(out[:M, :N], a, w, alpha)
         assert bool((out[M:] == 7.0).all()) and bool((out[:, N:] == 7.0).all())
 
 
@@ -90,9 +102,11 @@ def test_chosen(M, N, K):
     a, w = _inputs(M, N, K)
     A, W, out = a.cuda(), w.cuda(), torch.empty(M, N, device="cuda")
     _check(ops.gemm_f32(A, W, out), a, w)
+    _check_norm(out, a, w)
     _check(ops.product(A, W, out, 0.25), a, w, 0.25)
     small = torch.empty(int(get_lib().ic_gemm_f32_parts_bytes(48, K)) + 16, dtype=torch.uint8, device="cuda")
     _check(ops.gemm_f32(A, W, out.zero_(), workspace=small), a, w)
+    _check_norm(out, a, w)
 
 
 @pytest.mark.gpu
