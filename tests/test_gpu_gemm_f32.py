@@ -66,6 +66,17 @@ def test_the_rule_prices_the_runs_that_a_workspace_makes():
         assert lib.ic_gemm_f32_pays_on(M, N, K, 256) == lib.ic_gemm_f32_pays_with(M, N, K, lib.ic_gemm_f32_workspace_bytes(M, N, K), 256)
 
 
+def test_short_rows_and_narrow_matrices_go_to_the_library():
+    """Of few k the library's product takes 3.6..8.5 us, less than the split of A and the product of parts (5.5..17), and of narrow matrices whose tiles fill the chip once 12..19
+    (17..26); wide and long ones are faster in parts."""
+    pays = get_lib().ic_gemm_f32_pays_on
+    for M, N, K in ((33, 32, 32), (64, 512, 128), (300, 512, 128), (130, 1536, 512), (2048, 256, 512), (1000, 128, 256), (2048, 128, 64), (517, 1536, 128), (300, 1536, 512),
+                    (1500, 512, 768), (1000, 768, 768), (2048, 512, 1024), (1000, 1024, 1024), (700, 1024, 768)):
+        assert not pays(M, N, K, 256)
+    for M, N, K in ((2048, 4096, 512), (1000, 4096, 512), (130, 7680, 1536), (517, 1536, 3840), (517, 1536, 1536), (517, 2560, 1536), (2048, 7680, 1536)):
+        assert pays(M, N, K, 256)
+
+
 @pytest.mark.gpu
 def test_a_small_workspace_goes_to_the_library():
     """With scratch memory for 16 rows at a time (129 runs over 32 MB of weights) the product by the rule is the library's."""
