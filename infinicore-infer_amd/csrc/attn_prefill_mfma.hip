@@ -15,7 +15,7 @@ attn_prefill_mfma_kernel(const uint16_t* __restrict__ q, int q_stride, uint16_t*
                                               page_shift, scale_log2e, window, parts, part_len, scratch, counters, blockIdx.x, stage0, stage1, pages);
 }
 
-// bfloat16: the kernel above.  float32: the true-float32 kernel of attn_prefill_f32.hip (same tiles, one to four key groups a block, walks never cut).
+// bfloat16: the kernel above.  float32: the kernel of attn_prefill_f32.hip, in three bfloat16 parts a number (same tiles, one to four key groups a block, walks never cut).
 IC_EXPORT int ic_attn_prefill_supported(int dtype, int dh, int page_size) {
     return (dtype == IC_BF16 || dtype == IC_F32) && (dh == 64 || dh == 128) && page_size > 0 && (page_size & (page_size - 1)) == 0;
 }

@@ -53,7 +53,7 @@ int ic_attn_decode_waves(int head_dim, int pairs, int nsplit);
 int ic_attn_decode_wants_order(int n_rows, int nkvh, int nsplit, int compute_units);
 int ic_attn_decode_order(const int* positions, int* order, int n_rows, hipStream_t stream);
 int ic_attn_decode(const void* q, int q_stride, void* out, int out_stride, int dtype, const void* kcache, const void* vcache, const int* block_tables, int bt_stride, const int* tok_list, const int* token_req, const int* positions, float* part_acc, float* part_ml, int n_tok, int nh, int nkvh, int dh, int page_size, float scale, int window, int nsplit, hipStream_t stream);
-// Matrix-core kernels for prompt portions (bfloat16; and true float32 with float32 matrix instructions, walks never cut).
+// Matrix-core kernels for prompt portions (bfloat16; and float32, every number as three bfloat16 numbers, walks never cut).
 // tiles: int32 [n_tiles, 4] = (request row, first token row, rows <= tile_rows, first position).
 int ic_attn_prefill_supported(int dtype, int dh, int page_size);
 // Key groups (1, 2 or 4) that share a walk in a block of the float32 kernel, from the number of (tile, head) pairs of a launch.
@@ -170,7 +170,8 @@ int ic_gemm_tiles_rope(const void* A, const void* W, void* C, int M, int K, int 
 int ic_product(const void* A, int a_dtype, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldw, int ldc, float alpha, void* workspace, long long workspace_bytes, hipStream_t stream);
 
 // ---- gemm_f32.hip ---------------------------------------------------------------------------------------
-// C[M, N] = alpha * A[M, K] W[N, K]^T in float32 on the bfloat16 matrix cores, every number as the sum of three bfloat16 numbers (errors as a float32 product's or smaller).  K a multiple
+// C[M, N] = alpha * A[M, K] W[N, K]^T in float32 on the bfloat16 matrix cores, every number as the sum of three bfloat16 numbers: one product alone is off by 2^-23 at most, where
+// a float32 product is by 2^-24 (2^-25.2 rms both); sums of 32 terms and more of either sign have a third to a half of a float32 chain's error.  K a multiple
 // of 32, strides multiples of 4, operands and workspace 16-byte aligned; workspace: ic_gemm_f32_parts_bytes(M, K) bytes, or any smaller number from
 // ic_gemm_f32_parts_bytes(16, K) on (then the rows are taken in several launches).  ic_gemm_f32_pays: whether it beats ic_matmul.
 int ic_gemm_f32_supported(int M, int N, int K, int lda, int ldw, int ldc);

@@ -5,9 +5,9 @@ The matrix product itself is the package's own matrix-core kernel for few rows
 (decoding, the output head) and for most many-row products, and a library
 routine for the rest (the reference calls the library's Gemm for every product,
 inference_context.cpp:59-79).
-float32 operands go to the package's product of bfloat16 parts (``ops.gemm_f32``, errors as a
-float32 product's or smaller) where it is the faster one, else to the library with reduced-precision
-matrix modes switched off.
+float32 operands go to the package's product of bfloat16 parts (``ops.gemm_f32``: a product off by
+2^-23 at most, sums with less error than float32 instructions have) where it is the faster one, else to
+the library with reduced-precision matrix modes switched off.
 """
 import torch
 
