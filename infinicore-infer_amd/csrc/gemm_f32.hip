@@ -436,12 +436,11 @@ IC_EXPORT long long ic_gemm_f32_workspace_bytes(int M, int N, int K) {
 
 namespace {
 
-// What the library's float32 product costs, in microseconds: a start, which few k make shorter, and 128 TFLOP/s; no less than a start that few operations do not fill; and where whole
-// rounds of tiles of 64 x 64 fit, those.  Fitted to 1,134 products (33..2,048 rows, 256..7,680 columns, 256..4,096 k, weights out of memory) and 392 of 32..1,536 k and 32..4,096 columns.
+// What the library's float32 product costs, in microseconds: a start, which few k make shorter, and 127 TFLOP/s; no less than 1.4 such starts; and where whole rounds of tiles of
+// 64 x 64 cost less, those.  Over 1,134 products (33..2,048 rows, 256..7,680 columns, 256..4,096 k, weights out of memory) and 392 of 32..1,536 k and 32..4,096 columns.
 double library_cost(int M, int N, int K, int units) {
-    const double start = 3.3 + 0.0072 * K, least = 8.0 + 0.0015 * K, products = 2.0 * M * N * K / (128e6 * units / 256.0) + (start < 6.2 ? start : 6.2);
-    const double any = start < least ? start : least, whole = products > any ? products : any;
-    const double rounds = 4.4 + 0.014 * K * __builtin_ceil((double)((M + 63) / 64) * ((N + 63) / 64) / units);
+    const double start = K < 750 ? 3.3 + 0.0072 * K : 8.7, least = start * 12.0 / 8.7, products = 2.0 * M * N * K / (127e6 * units / 256.0) + start;
+    const double rounds = 4.4 + 0.014 * K * __builtin_ceil((double)((M + 63) / 64) * ((N + 63) / 64) / units), whole = products > least ? products : least;
     return rounds < whole ? rounds : whole;
 }
 
@@ -449,9 +448,10 @@ double library_cost(int M, int N, int K, int units) {
 
 // Whether the split, the product and the sum of its slices beat the library's float32 product; from 33 rows on, since fewer are a matter of the weights' bytes, which it reads as fast
 // (8 x 7,680 x 1,536: 13 us, the split alone 4).  Over the 1,134 products above the choice takes 0.907 of the library's time and loses 4 % to the better of the two (the library's choice of
-// algorithm is uneven); 11 are 5..35 % slower than the library, most of them of 256..768 columns and many rows.  130 x 7,680 x 1,536: 33 -> 28, 400 x 2,560 x 1,536: 33 -> 28, 2,048 x 4,096 x 512
-// 74 -> 58, on the other side 96 x 2,560 x 1,536: 11 against 16, 1,500 x 512 x 768 13 against 19, 2,048 x 256 x 512 8.5 against 17.  (Without the rounds, and with 8.7 us as the
-// start and 12 as the least for any K, 58 of the 1,134 were over 5 % slower than the library, and 280 products of up to 512 k took 1.24 of its time.)  With the workspace there
+// algorithm is uneven); 28 are 5..35 % slower than the library, most of them of 256..1,024 columns.  130 x 7,680 x 1,536: 33 -> 28, 300 x 2,560 x 1,536: 26 -> 25, 2,048 x 4,096 x 512
+// 74 -> 58, on the other side 96 x 2,560 x 1,536: 11 against 16, 1,500 x 512 x 768 13 against 19, 2,048 x 256 x 512 8.5 against 17.  Where the two are near each other parts run,
+// whose error is the smaller one.  (Without the rounds, and with 8.7 us as the start for any K, 58 of the 1,134 were over 5 % slower than the library, and 280 products of up to
+// 512 k took 1.24 of its time.)  With the workspace there
 // is: 64 MB hold 672 rows of 16,384, and 2,048 x 4,096 x 16,384 is four runs of 512 rows (1,403 us, the library 1,798); 16 rows at a time never pay.
 IC_EXPORT int ic_gemm_f32_pays_with(int M, int N, int K, long long workspace_bytes, int units) {
     if (M <= kFewRows || N <= 0 || K < 32 || units <= 0 || rows_at_once(M, K, workspace_bytes) <= 0) return 0;

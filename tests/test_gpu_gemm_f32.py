@@ -73,7 +73,8 @@ def test_short_rows_and_narrow_matrices_go_to_the_library():
     for M, N, K in ((33, 32, 32), (64, 512, 128), (300, 512, 128), (130, 1536, 512), (2048, 256, 512), (1000, 128, 256), (2048, 128, 64), (517, 1536, 128), (300, 1536, 512),
                     (1500, 512, 768), (1000, 768, 768), (2048, 512, 1024), (1000, 1024, 1024), (700, 1024, 768)):
         assert not pays(M, N, K, 256)
-    for M, N, K in ((2048, 4096, 512), (1000, 4096, 512), (130, 7680, 1536), (517, 1536, 3840), (517, 1536, 1536), (517, 2560, 1536), (2048, 7680, 1536)):
+    for M, N, K in ((2048, 4096, 512), (1000, 4096, 512), (130, 7680, 1536), (517, 1536, 3840), (517, 1536, 1536), (517, 2560, 1536), (2048, 7680, 1536),
+                    (300, 2560, 1536), (388, 1536, 1536), (76, 7680, 1536), (216, 1536, 3840)):
         assert pays(M, N, K, 256)
 
 
@@ -191,7 +192,7 @@ def test_values_that_are_not_finite(slices):
 @pytest.mark.gpu
 def test_smaller_error_than_the_library():
     """Against 64 bits the parts' error is no larger than the library's float32 product has it."""
-    for M, N, K in ((40, 1536, 1536), (256, 2560, 1536), (517, 1536, 3840)):
+    for M, N, K in ((40, 1536, 1536), (256, 2560, 1536), (517, 1536, 3840), (130, 512, 32), (517, 1536, 64), (33, 4096, 128), (300, 256, 256), (1000, 512, 512)):
         a, w = _inputs(M, N, K, seed=9)
         A, W, own, lib = a.cuda(), w.cuda(), torch.empty(M, N, device="cuda"), torch.empty(M, N, device="cuda")
         ops.gemm_f32(A, W, own)
