@@ -1,7 +1,8 @@
 // The step function in native code: every kernel of a step issued by one call (host code only; the
 // kernels are the library's own entry points).  The reference's is src/models/jiuge/jiuge.cpp:114-298.
 //
-// What runs for a layer depends on the step alone, never on the model: up to 16 rows in bfloat16 take the
+// What runs for a layer depends on the step alone, never on the model, but for the decode steps of up to 8 rows that one kernel takes with all their layers
+// (decode_chain.hip, for the sizes that it is built for).  Up to 16 rows in bfloat16 take the
 // few-row products with their epilogues (rotary and cache write after QKV; residual add, the next norm's
 // weight and sums of squares after O and down; SwiGLU after gate/up), the norm between two products being
 // split over them; more rows take the products in tiles (QKV with rotary and cache write, gate/up with SwiGLU in
@@ -9,7 +10,9 @@
 // Single-token rows go to the split-key attention kernel, prompt portions to the tiled one, both of a mixed step to one launch
 // where that is faster, what neither takes to the general one.
 #include "common.h"
+#include "decode_chain.h"
 #include "infinicore_infer_engine.h"
+#include "infinicore_infer_variants.h"
 #include <algorithm>
 #include <cstdio>
 #include <cstring>
@@ -22,6 +25,9 @@ namespace {
 // forward both ask those functions, so a rule is written once.
 constexpr int kFewRows = 16;        // up to here the few-row products beat the library
 constexpr int kMidRows = 64;        // up to here the sliced product beats it for results as wide as the model
+// Layers from which on a decode step runs them in one launch: each layer saves 6 us at one row of the 1B and 2B shapes (1B shape, 600 keys: 93.4 -> 79.8 us with three
+// layers, 223.8 -> 183.8 with eight), starting costs 4.  One and two layers save 3 and 8 us and stay kernel by kernel, as the steps issued from Python are.
+constexpr int kChainMinEntries = 3;
 constexpr int kMaxSumsqParts = 256; // column blocks of sums of squares a product takes as row factors
 
 thread_local std::string g_create_error;
@@ -32,7 +38,7 @@ inline int dtype_size(int dtype) { return dtype == IC_BF16 ? 2 : 4; }
 struct Workspace {
     // byte offsets into the caller's workspace
     size_t residual, normed, qkv, attn_out, mixer_out, ffn_out, mixer_tail, mixer_sumsq, ffn_tail, ffn_sumsq, gate_up, act,
-        part_acc, part_ml, decode_order, head_in, tail_parts, tile_parts, f32_parts, total;
+        part_acc, part_ml, decode_order, head_in, tail_parts, tile_parts, f32_parts, chain, total;
 };
 
 // Rows whose norm is half done: values = x * w, sums of squares per column block; the row factor
@@ -122,6 +128,7 @@ struct IcDecoder {
     std::vector<IcLayer> layers;
     std::vector<IcRunEntry> entries;
     int max_qkv_width = 0, max_attn_width = 0, max_intermediate = 0;
+    bool chained = false;        // the layers are alike and their table lies on the device
     std::string error;
 
     int fail(int status, const char* what, int entry) {
@@ -161,6 +168,48 @@ struct IcDecoder {
     int mixed_parts_for(const IcStepBatch& b, const IcAttention& a, int* part_len) const {
         if (!meta.attention_counters) { if (part_len) *part_len = 0; return 1; }
         return ic_attn_mixed_parts_of_step(meta.dtype, b.n_prefill_tiles, a.n_heads, a.head_dim, tiles_end(b), a.window, meta.compute_units, part_len);
+    }
+
+    ChainShape chain_shape() const {
+        const IcLayer& l = layers[entries[0].layer];
+        return ChainShape{meta.hidden, l.attention.n_heads, l.attention.n_kv_heads, l.attention.head_dim, l.ffn.intermediate, meta.page_size, meta.compute_units};
+    }
+
+    // All layers in one launch: every row a request's single new token, all logits wanted.
+    bool takes_chain(const IcStepBatch& b) const {
+        return chained && b.fixed_decode_splits <= 0 && b.decode_rows_identity && b.want_rows_identity && b.n_want == b.n_tokens && b.n_decode_rows == b.n_tokens &&
+               b.n_prefill_tiles == 0 && b.n_tokens <= kChainMaxRows && chain_supported(chain_shape(), b.n_tokens, meta.n_entries, std::max(b.max_context, b.max_position + 1));
+    }
+
+    // Whether the layers are alike enough for one launch, and if so their table.
+    bool make_table() {
+        if (!meta.layer_table || meta.dtype != IC_BF16 || meta.n_entries < kChainMinEntries) return false;
+        const IcRunEntry& e0 = entries[0];
+        const IcLayer& l0 = layers[e0.layer];
+        const IcAttention& a0 = l0.attention;
+        if (a0.window != 0 || a0.shared_kv || a0.rot_dim != a0.head_dim) return false;
+        std::vector<ChainEntry> table;
+        for (const IcRunEntry& e : entries) {
+            const IcLayer& l = layers[e.layer];
+            const IcAttention& a = l.attention;
+            if (!e.writes_cache || e.group != e0.group || a.n_heads != a0.n_heads || a.n_kv_heads != a0.n_kv_heads || a.head_dim != a0.head_dim || a.window != 0 ||
+                a.shared_kv || a.rot_dim != a0.rot_dim || a.max_positions != a0.max_positions || a.softmax_scale != a0.softmax_scale || a.cos != a0.cos ||
+                a.sin != a0.sin || l.mixer_norm.eps != l0.mixer_norm.eps || l.ffn_norm.eps != l0.ffn_norm.eps || l.ffn.intermediate != l0.ffn.intermediate ||
+                l.residual_scale != l0.residual_scale) return false;
+            if (((uintptr_t)a.w_qkv | (uintptr_t)a.w_o | (uintptr_t)l.ffn.w_gate_up | (uintptr_t)l.ffn.w_down | (uintptr_t)e.k_cache | (uintptr_t)e.v_cache) & 15) return false;
+            for (const ChainEntry& other : table)
+                if (other.k_cache == e.k_cache || other.v_cache == e.v_cache) return false;
+            table.push_back(ChainEntry{a.w_qkv, a.w_o, l.ffn.w_gate_up, l.ffn.w_down, l.mixer_norm.weight, l.ffn_norm.weight, e.k_cache, e.v_cache});
+        }
+        if (!chain_supported(chain_shape(), 1, meta.n_entries, 1)) return false;
+        ChainEntry end{};
+        end.norm_in = meta.final_norm_scaled;
+        table.push_back(end);
+        if (hipMemcpy(meta.layer_table, table.data(), table.size() * sizeof(ChainEntry), hipMemcpyHostToDevice) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        return true;
     }
 
     Workspace layout(const IcStepBatch& b) const {
@@ -217,6 +266,10 @@ struct IcDecoder {
             f32 = std::max(f32, ic_gemm_f32_workspace_bytes(b.n_want, meta.vocab, meta.hidden));
         }
         w.f32_parts = take((size_t)f32);
+        if (chained && b.decode_rows_identity) {      // (what any smaller step needs too: recorded steps share one workspace)
+            const int rows = std::min(b.n_tokens, kChainMaxRows);
+            w.chain = take(chain_scratch_bytes(chain_shape(), rows, meta.n_entries));
+        }
         w.total = o;
         return w;
     }
@@ -247,7 +300,7 @@ struct IcDecoder {
     }
 
     int forward(const IcStepBatch& b, void* workspace, long long workspace_bytes, void* lib_ws, long long lib_ws_bytes,
-                float* logits, hipStream_t stream) {
+                float* logits, hipStream_t stream, int absent = 0) {
         error.clear();
         const int T = b.n_tokens, d = meta.hidden, dt = meta.dtype, ps = meta.page_size;
         if (T <= 0) return IC_OK;
@@ -265,8 +318,11 @@ struct IcDecoder {
         const int parts = ic_gemm_nt_residual_parts(d);
         int st;
 
-        st = ic_embed(b.tokens, meta.embed_table, dt, x, T, d, meta.embed_scale, stream);
-        if (st) return fail(st, "the embedding gather", -1);
+        const bool chain = takes_chain(b);
+        if (!chain) {
+            st = ic_embed(b.tokens, meta.embed_table, dt, x, T, d, meta.embed_scale, stream);
+            if (st) return fail(st, "the embedding gather", -1);
+        }
 
         const int* decode_rows = b.decode_rows_identity ? nullptr : b.decode_rows;
         bool ordered = !b.decode_rows_identity;      // a list of the caller's has the longest rows first
@@ -277,7 +333,21 @@ struct IcDecoder {
         float branch_alpha = 0.f;
         Deferred def;
 
-        const int last = meta.n_entries - 1;
+        if (chain) {
+            const IcRunEntry& e = entries[0];
+            const IcLayer& l = layers[e.layer];
+            const IcAttention& A = l.attention;
+            if (!b.group_tables[e.group] || !b.group_slots[e.group]) return fail(IC_ERR_ARG, "the cache group of the entry", 0);
+            if (b.max_position >= A.max_positions) return fail(IC_ERR_ARG, "a position beyond the rotary tables", 0);
+            ChainStep c{(const ChainEntry*)meta.layer_table, meta.n_entries, T, A.softmax_scale, l.residual_scale, l.mixer_norm.eps, l.ffn_norm.eps, meta.embed_scale,
+                        b.tokens, b.positions, b.group_slots[e.group], b.token_req, b.group_tables[e.group], b.group_table_stride[e.group], A.cos, A.sin,
+                        meta.embed_table, l.mixer_norm.weight, x, base + ws.chain, base + ws.ffn_tail, (float*)(base + ws.ffn_sumsq)};
+            st = chain_launch(chain_shape(), c, absent, stream);
+            if (st) return fail(st, "the layers in one launch", 0);
+            def = Deferred{base + ws.ffn_tail, (const float*)(base + ws.ffn_sumsq), chain_sumsq_parts(chain_shape()), d, meta.final_norm.eps};
+            owed = DEFERRED;
+        }
+        const int last = chain ? -1 : meta.n_entries - 1;
         for (int i = 0; i <= last; ++i) {
             const IcRunEntry& e = entries[i];
             const IcLayer& L = layers[e.layer];
@@ -467,6 +537,8 @@ struct IcDecoder {
     }
 };
 
+IC_EXPORT long long ic_decoder_table_bytes(int n_entries) { return n_entries < 0 ? -1 : (long long)(n_entries + 1) * (long long)sizeof(ChainEntry); }
+
 IC_EXPORT const char* ic_decoder_create_error() { return g_create_error.c_str(); }
 
 IC_EXPORT IcDecoder* ic_decoder_create(const IcDecoderMeta* meta, const IcLayer* layers, const IcRunEntry* entries) {
@@ -503,6 +575,7 @@ IC_EXPORT IcDecoder* ic_decoder_create(const IcDecoderMeta* meta, const IcLayer*
             return bad("a run-order entry names no layer, no group or no cache planes");
         }
     }
+    d->chained = d->make_table();
     return d;
 }
 
@@ -520,6 +593,16 @@ IC_EXPORT int ic_decoder_forward(IcDecoder* decoder, const IcStepBatch* batch, v
     if (!decoder || !batch) return IC_ERR_ARG;
     return decoder->forward(*batch, workspace, workspace_bytes, library_workspace, library_workspace_bytes, logits, stream);
 }
+
+// The same with `absent` of the blocks that a step's layers are dealt to not taking part, as if they found no room.
+IC_EXPORT int ic_decoder_forward_absent(IcDecoder* decoder, const IcStepBatch* batch, void* workspace, long long workspace_bytes, void* library_workspace,
+                                        long long library_workspace_bytes, float* logits, int absent, hipStream_t stream) {
+    if (!decoder || !batch || absent < 0 || absent >= decoder->meta.compute_units) return IC_ERR_ARG;
+    return decoder->forward(*batch, workspace, workspace_bytes, library_workspace, library_workspace_bytes, logits, stream, absent);
+}
+
+// Whether a step runs its layers in one launch.
+IC_EXPORT int ic_decoder_takes_chain(const IcDecoder* decoder, const IcStepBatch* batch) { return decoder && batch ? decoder->takes_chain(*batch) : 0; }
 
 // ---- the key split of single-token rows --------------------------------------------------------------------------
 // One split writes the result itself; more cost a second kernel.  A rule by a model of the two kernels' time, one for each way of walking the

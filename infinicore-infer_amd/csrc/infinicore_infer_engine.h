@@ -88,6 +88,8 @@ typedef struct {
     const float* final_norm_scaled;   // final_norm.weight * logit_scale
     int* attention_counters;          // ic_attn_prefill_counter_ints() ints of the caller's, zero when the decoder is made; every step
                                       // leaves them zero.  Steps that overlap in time (two streams) need decoders with counters of their own
+    void* layer_table;                // ic_decoder_table_bytes(n_entries) bytes of device memory of the caller's, written when the decoder is made; NULL: a decode
+                                      // step's layers are launched kernel by kernel
 } IcDecoderMeta;
 
 // A step's batch where it lies on the device.  Tokens of all requests are concatenated in request order.
@@ -129,6 +131,7 @@ typedef struct {
 
 // Copies the descriptions (not the tensors they point to).  NULL when a field is out of range;
 // ic_decoder_create_error() then says which.
+long long ic_decoder_table_bytes(int n_entries);
 IcDecoder* ic_decoder_create(const IcDecoderMeta* meta, const IcLayer* layers, const IcRunEntry* entries);
 const char* ic_decoder_create_error();
 void ic_decoder_destroy(IcDecoder* decoder);

@@ -2,7 +2,7 @@
 // by themselves.  Not part of the interface a caller of the library needs: ic_gemm_nt and ic_gemm_qkv_rope choose for themselves.
 // A variant holds for the one call that names it and changes nothing for any other call, thread or engine.
 #pragma once
-#include "infinicore_infer_hip.h"
+#include "infinicore_infer_engine.h"
 
 #ifdef __cplusplus
 extern "C" {
@@ -44,6 +44,15 @@ int ic_gemm_f32_takes(int M, int N, int K, int lda, int ldw, int ldc, const void
 
 // key / page_size as the kernels of single tokens compute it; -1: an argument fault.
 int ic_attn_decode_page_of(int key, int page_size);
+
+// The pieces of a decode step's attention as the kernel of whole layers deals them (decode_chain.hip), six ints each: block, row, kv head, first key, key after the
+// last, place; and for every (row, kv head) the blocks from .. to whose pieces are brought together (from > to: a block walks the whole head).  Returns their number.
+int ic_decode_chain_pieces(const int* positions, int rows, int kv_heads, int compute_units, int* pieces, int capacity, int* from_to);
+
+// ic_decoder_forward with `absent` of the blocks that a decode step's layers are dealt to not taking part, as if they found no room on the device; and whether a step
+// runs its layers in one launch (on which it has no effect where it does not).
+int ic_decoder_forward_absent(IcDecoder* decoder, const IcStepBatch* batch, void* workspace, long long workspace_bytes, void* library_workspace, long long library_workspace_bytes, float* logits, int absent, hipStream_t stream);
+int ic_decoder_takes_chain(const IcDecoder* decoder, const IcStepBatch* batch);
 
 // Whether ic_causal_conv runs a thread over a run of tokens (four taps, aligned rows), and whether ic_hc_step's threads send several rounds of a row's
 // loads ahead.

@@ -65,14 +65,15 @@ class NativeDecoder:
             k, v = engine.storage.kv(e.cache)
             entries.append(IcRunEntry(e.layer, int(e.writes_cache), engine._slot_group[e.cache], k.data_ptr(), v.data_ptr()))
         entry_arr = (IcRunEntry * len(entries))(*entries)
+        table = torch.zeros(lib.ic_decoder_table_bytes(len(entries)), dtype=torch.uint8, device=engine.device)
         meta = IcDecoderMeta(ops.dtype_code(rt.dtype), model.spec.hidden_size, model.spec.vocab_size, engine.page_size,
                              len(layers), len(entries), len(engine.groups), engine.cu_count, emb[1], head[1], emb[0],
-                             head[0], fin, scaled_w.data_ptr(), counters.data_ptr())
+                             head[0], fin, scaled_w.data_ptr(), counters.data_ptr(), table.data_ptr())
         handle = lib.ic_decoder_create(ctypes.byref(meta), layer_arr, entry_arr)
         if not handle:
             raise KernelError("the native step function refused the model: %s"
                               % lib.ic_decoder_create_error().decode())
-        return cls(handle, lib, model.spec.vocab_size, (layer_arr, entry_arr, meta, scaled_w, counters))
+        return cls(handle, lib, model.spec.vocab_size, (layer_arr, entry_arr, meta, scaled_w, counters, table))
 
     def workspace_bytes_for_decode(self, n_requests: int) -> int:
         """Workspace bytes that any step of up to ``n_requests`` single tokens needs (with the most key

@@ -68,7 +68,7 @@ class IcDecoderMeta(_c.Structure):
     _fields_ = [("dtype", _I), ("hidden", _I), ("vocab", _I), ("page_size", _I), ("n_layers", _I), ("n_entries", _I),
                 ("n_groups", _I), ("compute_units", _I), ("embed_scale", _F), ("logit_scale", _F),
                 ("embed_table", _P), ("head_weight", _P), ("final_norm", IcNorm), ("final_norm_scaled", _P),
-                ("attention_counters", _P)]
+                ("attention_counters", _P), ("layer_table", _P)]
 
 
 class IcStepBatch(_c.Structure):
@@ -233,6 +233,10 @@ _SIGNATURES = {
     "ic_rule_context_bucket": [_I],
     "ic_attn_decode_on_matrix_cores": [_I, _I, _I],
     "ic_decoder_create": [_c.POINTER(IcDecoderMeta), _c.POINTER(IcLayer), _c.POINTER(IcRunEntry)],
+    "ic_decoder_table_bytes": [_I],
+    "ic_decode_chain_pieces": [_P, _I, _I, _I, _P, _I, _P],
+    "ic_decoder_forward_absent": [_P, _c.POINTER(IcStepBatch), _P, _LL, _P, _LL, _P, _I, _P],
+    "ic_decoder_takes_chain": [_P, _c.POINTER(IcStepBatch)],
     "ic_decoder_create_error": [],
     "ic_decoder_destroy": [_P],
     "ic_decoder_last_error": [_P],
@@ -243,7 +247,7 @@ _SIGNATURES = {
     "ic_decoder_step": [_P, _c.POINTER(IcHostBatch), _P, _P, _LL, _P, _LL, _P, _LL, _P, _c.POINTER(IcStepBatch), _P],
 }
 _RESTYPES = {"ic_product_timing": None, "ic_product_f32_timing": None, "ic_decoder_create": _P, "ic_decoder_create_error": _c.c_char_p, "ic_decoder_destroy": None,
-             "ic_decoder_last_error": _c.c_char_p, "ic_decoder_workspace_bytes": _LL, "ic_decoder_step_ints": _LL,
+             "ic_decoder_last_error": _c.c_char_p, "ic_decoder_workspace_bytes": _LL, "ic_decoder_table_bytes": _LL, "ic_decoder_step_ints": _LL,
              "ic_peak_mfma_bf16": _LL, "ic_attn_prefill_scratch_floats": _LL, "ic_gemm_f32_parts_bytes": _LL, "ic_gemm_f32_workspace_bytes": _LL}
 
 

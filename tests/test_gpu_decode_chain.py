@@ -1,0 +1,207 @@
+"""Decode steps whose layers run in one launch (decode_chain.hip): against the plain implementation and the same steps kernel by kernel, over row counts and lengths at
+the edges of what is dealt to the blocks; recorded and eager steps, steps with fewer blocks than compute units and steps of two streams at once, to the bit."""
+import threading
+
+import pytest
+import torch
+
+import helpers as H
+from test_gpu_large import SHAPE_1B, SHAPE_2B, _engine_and_weights
+
+pytestmark = pytest.mark.gpu
+
+LAYERS = 4
+SHAPES = {"1b": dict(SHAPE_1B, vocab_size=2003, num_hidden_layers=LAYERS, max_position_embeddings=4096),
+          "2b": dict(SHAPE_2B, vocab_size=2003, num_hidden_layers=LAYERS)}
+
+
+# (hidden, heads, kv heads, inner): groups of 1..4 in both of the kernel's sizes, with the least and the most columns of a block, and rows of which waves have unlike shares
+OTHERS = [(1536, 12, 12, 2112), (2048, 32, 16, 4096), (1024, 15, 5, 2752), (1088, 16, 4, 2176), (4096, 40, 40, 4160), (2112, 64, 32, 6144), (3072, 48, 16, 4352), (2304, 64, 16, 6080)]
+for _d, _h, _kv, _di in OTHERS:
+    SHAPES["%d-%d-%d-%d" % (_d, _h, _kv, _di)] = dict(SHAPE_1B, vocab_size=2003, num_hidden_layers=3, hidden_size=_d, num_attention_heads=_h, num_key_value_heads=_kv,
+                                                      head_dim=64, intermediate_size=_di)
+
+
+def _engine(shape, **kw):
+    return _engine_and_weights(SHAPES[shape], 21, 0.02, 16 * 2304, 12, **kw)
+
+
+def _chained(engine):
+    return bool(engine.native._lib.ic_decoder_takes_chain(engine.native._h, engine.native._batch_ref))
+
+
+def _hold(engine, doc, lens):
+    from infinicore_infer_amd.engine import StepEntry
+    engine.step([StepEntry("doc", doc, [])])
+    for i, n in enumerate(lens):
+        engine.fork("doc", "r%d" % i, n)
+    engine.free("doc")
+
+
+def _decode(engine, tokens):
+    from infinicore_infer_amd.engine import StepEntry
+    return engine.step([StepEntry("r%d" % i, [t], [0]) for i, t in enumerate(tokens)]).clone()
+
+
+def _drop(engine, n):
+    for i in range(n):
+        engine.free("r%d" % i)
+
+
+LENS = [[1], [62], [63], [64], [257], [320], [384], [600], [1100], [2063], [1, 300], [64, 63, 65], [900, 20], [400, 300, 200, 100], [2000, 1, 1, 1],
+        [700, 3, 1290, 40, 511], [1500] * 6, [2000, 1000, 500, 250, 125, 60, 30], [1] * 8, [2250, 1, 2, 3, 4, 5, 6, 7]]
+
+
+@pytest.mark.parametrize("page_size", [16, 64])
+@pytest.mark.parametrize("shape", ["1b", "2b"])
+def test_rows_and_lengths(shape, page_size):
+    """Each path rounds to bfloat16 some ten times a layer and is 1e-2 off the plain implementation at most (checked below); two of them differ by twice that."""
+    a, _ = _engine(shape, page_size=page_size, use_graphs=False)
+    b, _ = _engine(shape, page_size=page_size, use_native=False)
+    doc = H.random_tokens(2003, 2260, 4)
+    taken = 0
+    for k, lens in enumerate(LENS):
+        for e in (a, b):
+            _hold(e, doc, lens)
+        for j in range(3):
+            toks = H.random_tokens(2003, len(lens), 100 * k + j)
+            la, lb = _decode(a, toks), _decode(b, toks)
+            taken += _chained(a)
+            err = float((la - lb).norm() / lb.norm())
+            assert err < 2e-2, (shape, lens, j, err)
+        for e in (a, b):
+            _drop(e, len(lens))
+    assert taken == 3 * (len(LENS) - (shape == "2b"))        # (288 heads of up to 2,560 keys: more pieces than a block has room for)
+
+
+@pytest.mark.parametrize("shape", ["%d-%d-%d-%d" % o for o in OTHERS])
+def test_other_sizes(shape):
+    a, _ = _engine(shape, use_graphs=False)
+    b, _ = _engine(shape, use_native=False)
+    doc = H.random_tokens(2003, 1300, 4)
+    for k, lens in enumerate([[1], [257], [600, 40], [1200, 1, 64, 700]]):
+        for e in (a, b):
+            _hold(e, doc, lens)
+        for j in range(2):
+            toks = H.random_tokens(2003, len(lens), 100 * k + j)
+            la, lb = _decode(a, toks), _decode(b, toks)
+            err = float((la - lb).norm() / lb.norm())
+            assert _chained(a) and err < 2e-2, (shape, lens, j, err)
+        for e in (a, b):
+            _drop(e, len(lens))
+
+
+@pytest.mark.parametrize("shape", ["1b", "2b"])
+def test_against_the_plain_implementation(shape):
+    from plain_model import plain_forward, round_bf16
+    engine, sd = _engine(shape, use_graphs=False)
+    doc = H.random_tokens(2003, 700, 8)
+    lens, steps = [650, 63, 257], 3
+    _hold(engine, doc, lens)
+    new = [H.random_tokens(2003, len(lens), 50 + j) for j in range(steps)]
+    got = []
+    for j in range(steps):
+        got.append(_decode(engine, new[j]))
+        assert _chained(engine)
+    for i, n in enumerate(lens):
+        tokens = doc[:n] + [new[j][i] for j in range(steps)]
+        want = plain_forward(SHAPES[shape], sd, tokens, rnd=round_bf16, rows=list(range(n, n + steps))).cpu()
+        have = torch.stack([got[j][i] for j in range(steps)]).double().cpu()
+        err = float((have - want).abs().max() / want.abs().max())
+        assert err < H.BF16_TOL, (shape, n, err)
+
+
+@pytest.mark.parametrize("shape", ["1b", "2b"])
+def test_recorded_and_eager_steps_are_equal(shape):
+    """Several replays with the engine's own eager work between them; lengths cross the border of a unit of keys and of a recorded step's range."""
+    from infinicore_infer_amd.engine import StepEntry
+    a, _ = _engine(shape, graph_after=1)
+    b, _ = _engine(shape, use_graphs=False)
+    doc = H.random_tokens(2003, 700, 9)
+    for e in (a, b):
+        _hold(e, doc, [254, 61, 640])
+    for j in range(8):
+        toks = H.random_tokens(2003, 3, 70 + j)
+        la, lb = _decode(a, toks), _decode(b, toks)
+        assert _chained(b) and torch.equal(la, lb), j
+        if j % 3 == 2:
+            for e in (a, b):
+                e.step([StepEntry("other", H.random_tokens(2003, 40, j), [])])
+                e.free("other")
+            torch.cuda.synchronize()
+    assert a.graph_replays >= 5
+
+
+@pytest.mark.parametrize("absent", [1, 100, 240])
+@pytest.mark.parametrize("lens", [[257], [600, 40], [1500] * 3])
+@pytest.mark.parametrize("shape", ["1b", "2b"])
+def test_blocks_that_find_no_room(shape, lens, absent):
+    """The others do their work, with the same results to the bit."""
+    a, _ = _engine(shape, use_graphs=False)
+    b, _ = _engine(shape, use_graphs=False)
+    forward = a.native._lib.ic_decoder_forward_absent
+    doc = H.random_tokens(2003, 1600, 3)
+    for e in (a, b):
+        _hold(e, doc, lens)
+    a.native._forward = lambda *args: forward(*args[:-1], absent, args[-1])
+    for j in range(2):
+        toks = H.random_tokens(2003, len(lens), 30 + j)
+        la, lb = _decode(a, toks), _decode(b, toks)
+        assert _chained(a) and torch.equal(la, lb), (shape, lens, absent, j)
+
+
+def test_two_streams_at_once():
+    """Two engines decode on streams of their own at the same time: neither keeps the other from ending, and each has the logits that it has alone."""
+    engines = [_engine("1b")[0], _engine("1b", graph_after=1)[0]]
+    doc = H.random_tokens(2003, 700, 5)
+    toks = [H.random_tokens(2003, 2, 10 + j) for j in range(12)]
+
+    def hold():
+        for e in engines:
+            _hold(e, doc, [600, 257])
+        torch.cuda.synchronize()
+
+    def go(i):
+        out = [_decode(engines[i], t) for t in toks]
+        torch.cuda.current_stream().synchronize()
+        _drop(engines[i], 2)
+        return out
+    hold()
+    want = [go(0), go(1)]
+    assert all(torch.equal(x, y) for x, y in zip(*want))
+    for _ in range(3):
+        hold()
+        got, wrong, start = [None, None], [], threading.Barrier(2)
+
+        def run(i):
+            try:
+                with torch.cuda.stream(torch.cuda.Stream()):
+                    start.wait()
+                    got[i] = go(i)
+            except BaseException as e:
+                wrong.append(e)
+        threads = [threading.Thread(target=run, args=(i,)) for i in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not wrong, wrong
+        bad = [(i, j) for i in range(2) for j in range(len(toks)) if not torch.equal(got[i][j], want[i][j])]
+        assert not bad, bad
+
+
+def test_weights_that_are_not_numbers():
+    """A NaN of that pattern in an embedding row makes the logits of its request NaN (and ends: what is handed on is never what stands for "not there yet"), the others' stay."""
+    engine, _ = _engine("1b", use_graphs=False)
+    doc = [t for t in H.random_tokens(2003, 300, 6) if t != 5]
+    _hold(engine, doc, [200, 100])
+    want = _decode(engine, [7, 9])
+    _drop(engine, 2)
+    table = engine.model.embedding.table
+    row = table[5].clone()
+    table[5].view(torch.int16).fill_(-1)                     # all ones: a NaN whose bits stand for "not there yet"
+    _hold(engine, doc, [200, 100])
+    got = _decode(engine, [7, 5])
+    table[5].copy_(row)
+    got[0, 5] = want[0, 5]                                   # (the table is the head's too)
+    assert _chained(engine) and torch.equal(got[0], want[0]) and bool(got[1].isnan().all())
