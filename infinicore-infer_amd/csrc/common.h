@@ -125,6 +125,12 @@ template <int LPK> __device__ __forceinline__ float group_sum(float d) {
     return d;
 }
 
+// A thread's sum of squares, four values at a time (which product of a sum is rounded first is written out, so that kernels that norm the same rows agree in every bit).
+__device__ __forceinline__ void add_squares(float& ss, const float* v, bool first) {
+    ss = first ? fmaf(v[0], v[0], v[1] * v[1]) : fmaf(v[1], v[1], fmaf(v[0], v[0], ss));
+    ss = fmaf(v[3], v[3], fmaf(v[2], v[2], ss));
+}
+
 // Sum over a whole block; every thread gets the result.  `red` is LDS of at
 // least blockDim.x / 64 floats.  Safe to call repeatedly with the same `red`.
 __device__ __forceinline__ float block_sum(float v, float* red) {

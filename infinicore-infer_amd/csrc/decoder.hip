@@ -288,6 +288,13 @@ struct IcDecoder {
         return ic_product(a, meta.dtype, w, out, out_dtype, M, N, K, lda, K, N, alpha, lib_ws, lib_ws_bytes, stream);
     }
 
+    // Float32 products of many rows in parts: slices of K where the product runs in parts of all rows at once, else 0 (then `linear` it is).
+    int whole_f32(const void* a, const void* w, const void* out, int M, int N, int K, const void* parts) const {
+        return meta.dtype == IC_F32 ? ic_gemm_f32_whole(a, w, out, M, N, K, K, K, N, parts, ic_gemm_f32_workspace_bytes(M, N, K)) : 0;
+    }
+    // Into the residual stream, with slices that the norm after it adds up (slices > 1): those lie behind the K columns' parts, and the norm's parts must not reach them.
+    bool leaves_slices(int slices, int K) const { return slices > 1 && meta.hidden <= K && ic_norm_parts_f32_supported(meta.hidden); }
+
     // 17..64 rows (and 13..16 long ones) into the residual stream: x += alpha * (a w^T), out = rmsnorm(x) * weight, through the sliced
     // product and the kernel that sums the slices.
     int tail_in_slices(const void* a, int K, const void* w, float* parts, float* x, float alpha, const float* weight, float eps,
@@ -331,7 +338,23 @@ struct IcDecoder {
         enum { NONE, BRANCH, DEFERRED, NORMED } owed = NONE;      // NORMED: the add and the whole norm are done, `normed` holds the rows
         const void* branch = nullptr;
         float branch_alpha = 0.f;
+        int branch_slices = 1;                       // of the float32 product that left them for the norm to add
         Deferred def;
+        // Float32: x += alpha * (the sum of the slices y), normed = its norm, with normed's parts where the product behind it takes them.
+        bool in_parts = false;                       // f32_parts holds the parts of the rows that the next product reads
+        auto add_norm = [&](const void* y, int slices, float alpha, const IcNorm& norm, int next_slices) {
+            in_parts = next_slices > 0 && ic_norm_parts_f32_supported(d);
+            if (in_parts || slices > 1)
+                return ic_norm_parts_f32(x, (const float*)y, slices, alpha, norm.weight, (float*)normed, in_parts ? f32_parts : nullptr, T, d, norm.eps, stream);
+            return ic_add_rmsnorm(x, y, dt, alpha, norm.weight, normed, dt, T, d, norm.eps, stream);
+        };
+        // a product of these rows, the parts there or not; keep: its slices are left
+        auto product = [&](const void* a, const void* w, void* out, int N, int K, int slices, bool keep) {
+            const bool ready = in_parts;
+            in_parts = false;
+            if (slices > 0) return ic_gemm_f32_between(a, w, out, T, N, K, K, K, N, f32_parts, ic_gemm_f32_workspace_bytes(T, N, K), ready, keep, stream);
+            return linear(a, K, w, out, dt, T, N, K, 1.0f, nullptr, f32_parts, lib_ws, lib_ws_bytes, stream);
+        };
 
         if (chain) {
             const IcRunEntry& e = entries[0];
@@ -359,6 +382,9 @@ struct IcDecoder {
             if (i < last) { succ = &layers[entries[i + 1].layer].mixer_norm; succ_weight = succ->weight; }
             else if (b.want_rows_identity) { succ = &meta.final_norm; succ_weight = meta.final_norm_scaled; }
 
+            const int qkv_width = (A.n_heads + 2 * (A.shared_kv ? 0 : A.n_kv_heads)) * A.head_dim;
+            const int qkv_slices = whole_f32(normed, A.w_qkv, qkv, T, qkv_width, d, f32_parts);
+
             // ---- norm before the mixer -------------------------------------------------------------
             const Deferred* h_def = nullptr;
             if (owed == DEFERRED) h_def = &def;
@@ -367,14 +393,14 @@ struct IcDecoder {
                 st = ic_rmsnorm(x, nullptr, L.mixer_norm.weight, normed, dt, T, d, L.mixer_norm.eps, 1.0f, stream);
                 if (st) return fail(st, "the norm before attention", i);
             } else {
-                st = ic_add_rmsnorm(x, branch, dt, branch_alpha, L.mixer_norm.weight, normed, dt, T, d, L.mixer_norm.eps, stream);
+                st = add_norm(branch, branch_slices, branch_alpha, L.mixer_norm, qkv_slices);
                 if (st) return fail(st, "the residual add and norm before attention", i);
             }
             const void* h = h_def ? h_def->values : normed;
 
             // ---- attention: QKV, rotary, cache write -------------------------------------------------
             const int nkv = (A.shared_kv || !e.writes_cache) ? 0 : A.n_kv_heads;
-            const int width = (A.n_heads + 2 * (A.shared_kv ? 0 : A.n_kv_heads)) * A.head_dim;
+            const int width = qkv_width;
             const int* slots = b.group_slots[e.group];
             if (A.rot_dim > 0 && b.max_position >= A.max_positions) return fail(IC_ERR_ARG, "a position beyond the rotary tables", i);
             if (nkv > 0 && !slots) return fail(IC_ERR_ARG, "the cache slots of the entry's group", i);
@@ -391,7 +417,8 @@ struct IcDecoder {
                                         A.head_dim, ps, stream);
                 if (st) return fail(st, "the QKV product with rotary and cache write, in tiles", i);
             } else {
-                st = linear(h, d, A.w_qkv, qkv, dt, T, width, d, 1.0f, h_def, f32_parts, lib_ws, lib_ws_bytes, stream);
+                st = h_def ? linear(h, d, A.w_qkv, qkv, dt, T, width, d, 1.0f, h_def, f32_parts, lib_ws, lib_ws_bytes, stream)
+                           : product(h, A.w_qkv, qkv, width, d, qkv_slices, false);
                 if (st) return fail(st, "the QKV product", i);
                 if (A.rot_dim > 0 || nkv > 0) {
                     st = ic_rope_kv_write(qkv, dt, b.positions, A.rot_dim > 0 ? A.cos : nullptr, A.rot_dim > 0 ? A.sin : nullptr,
@@ -450,6 +477,10 @@ struct IcDecoder {
             }
 
             // ---- O projection, residual add, norm before the feed-forward --------------------------------
+            const int di = L.ffn.intermediate;
+            void* act = base + ws.act;
+            const int down_slices = whole_f32(act, L.ffn.w_down, base + ws.ffn_out, T, d, di, f32_parts);
+            const int gate_up_slices = whole_f32(normed, L.ffn.w_gate_up, base + ws.gate_up, T, 2 * di, d, f32_parts);
             Deferred mid;
             const Deferred* g_def = nullptr;
             const int o_tail = ic_rule_tail(dt, T, d, ow, ow, ow);
@@ -465,16 +496,16 @@ struct IcDecoder {
                 mid = Deferred{base + ws.mixer_tail, (const float*)(base + ws.mixer_sumsq), parts, d, L.ffn_norm.eps};
                 g_def = &mid;
             } else {
-                st = linear(attn_out, ow, A.w_o, base + ws.mixer_out, dt, T, d, ow, 1.0f, nullptr, f32_parts, lib_ws, lib_ws_bytes, stream);
+                const int o_slices = whole_f32(attn_out, A.w_o, base + ws.mixer_out, T, d, ow, f32_parts);
+                const bool keep = leaves_slices(o_slices, ow);
+                st = product(attn_out, A.w_o, base + ws.mixer_out, d, ow, o_slices, keep);
                 if (st) return fail(st, "the O product", i);
-                st = ic_add_rmsnorm(x, base + ws.mixer_out, dt, L.residual_scale, L.ffn_norm.weight, normed, dt, T, d, L.ffn_norm.eps, stream);
+                st = add_norm(keep ? (char*)f32_parts + ic_gemm_f32_parts_bytes(T, ow) : base + ws.mixer_out, keep ? o_slices : 1, L.residual_scale, L.ffn_norm, gate_up_slices);
                 if (st) return fail(st, "the residual add and norm before the feed-forward", i);
             }
             const void* g = g_def ? g_def->values : normed;
 
             // ---- feed-forward ----------------------------------------------------------------------------------
-            const int di = L.ffn.intermediate;
-            void* act = base + ws.act;
             if (ic_rule_gate_up_fused(dt, T, d, d, d, g_def != nullptr)) {
                 IcRowFactor gf{};
                 if (g_def) gf = IcRowFactor{g_def->sumsq, g_def->parts, g_def->width, g_def->eps};
@@ -485,9 +516,11 @@ struct IcDecoder {
                 st = ic_gemm_tiles(g, L.ffn.w_gate_up, act, T, 2 * di, d, d, d, di, 1, stream);
                 if (st) return fail(st, "the gate/up product with SwiGLU, in tiles", i);
             } else {
-                st = linear(g, d, L.ffn.w_gate_up, base + ws.gate_up, dt, T, 2 * di, d, 1.0f, nullptr, f32_parts, lib_ws, lib_ws_bytes, stream);
+                st = product(g, L.ffn.w_gate_up, base + ws.gate_up, 2 * di, d, gate_up_slices, false);
                 if (st) return fail(st, "the gate/up product", i);
-                st = ic_swiglu(base + ws.gate_up, act, dt, T, di, stream);
+                in_parts = down_slices > 0;
+                st = in_parts ? ic_swiglu_parts_f32((const float*)(base + ws.gate_up), (float*)act, f32_parts, T, di, stream)
+                              : ic_swiglu(base + ws.gate_up, act, dt, T, di, stream);
                 if (st) return fail(st, "SwiGLU", i);
             }
             const int down_tail = succ ? ic_rule_tail(dt, T, d, di, di, di) : IC_TAIL_PLAIN;
@@ -504,9 +537,11 @@ struct IcDecoder {
                 def = Deferred{base + ws.ffn_tail, (const float*)(base + ws.ffn_sumsq), parts, d, succ->eps};
                 owed = DEFERRED;
             } else {
-                st = linear(act, di, L.ffn.w_down, base + ws.ffn_out, dt, T, d, di, 1.0f, nullptr, f32_parts, lib_ws, lib_ws_bytes, stream);
+                const bool keep = i < last && leaves_slices(down_slices, di);      // (the last one's are added up: the final norm takes the wanted rows only)
+                st = product(act, L.ffn.w_down, base + ws.ffn_out, d, di, down_slices, keep);
                 if (st) return fail(st, "the down product", i);
-                branch = base + ws.ffn_out;
+                branch = keep ? (const char*)f32_parts + ic_gemm_f32_parts_bytes(T, di) : base + ws.ffn_out;
+                branch_slices = keep ? down_slices : 1;
                 branch_alpha = L.residual_scale;
                 owed = BRANCH;
             }

@@ -73,8 +73,7 @@ __global__ void norm_row_kernel(float* __restrict__ x, const int* __restrict__ r
                 for (int e = 0; e < 4; ++e) v[i][e] += alpha * yv[e];
                 store4(xr + c, v[i]);
             }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) ss += v[i][e] * v[i][e];
+            add_squares(ss, v[i], i == 0);
         }
     }
     ss = block_sum(ss, red);

@@ -8,7 +8,7 @@
 // (with all six in one sum 2.9..6.1e-7 / 4.8..9.8e-7).  The 16 rows of a result that is not finite, or under 2^-64, are summed again with
 // the float32 instructions (PartsCheck).
 //
-// A is split once per product by a kernel before (3.7 us and 10 bytes a value), into the order of the matrix cores' operands: 1 KB per 16 rows, 32 k and part, which go to LDS and
+// A is split once per product, by the norm or the gated unit that computes it or by a kernel before (3.7 us and 10 bytes a value), into the order of the matrix cores' operands: 1 KB per 16 rows, 32 k and part, which go to LDS and
 // into registers as they lie.  W stays float32 in memory and in LDS (rows of 128 bytes, the 16-byte chunk c of row r at c ^ (r / 2 % 8)) and is split in registers by the
 // one wave that multiplies it: 22 vector instructions per 4 values and 6 MT products, where MT row tiles of 16 share the split.  The matrix cores hide two
 // vector instructions per product of 16 cycles (measured: 8.3 ns a product with none to two, 10.3 with three, 12.1 with four), hence no split of A in the loop
@@ -18,7 +18,7 @@
 // What bounds it: the products' rate, 8.9 ns each (a lone wave a SIMD, power), some 5 us for launch, first loads and way out; the fill of the last round of blocks.  Few rows:
 // the weights' bytes.  517 x 7,680 x 1,536: 61.6 us and 4.2 for the split, 1.19 PFLOP/s of parts (library 99); 517 x 1,536 x 3,840 in 4 slices 33.9 (library 61); 2,048 x 7,680 x 1,536 233 (391).
 //
-// Few tiles: K in slices, blocks of their own, whose sums a second kernel adds up.
+// Few tiles: K in slices, blocks of their own, whose sums a second kernel adds up, or the norm that reads them.
 #include "common.h"
 #include "float_parts.h"
 #include "infinicore_infer_variants.h"
@@ -272,6 +272,88 @@ __global__ void __launch_bounds__(256) split_rows_kernel(const float* A, int lda
     for (int p = 0; p < 3; ++p) out[(size_t)w * 192 + p * 64 + lane] = uint4{s[0].p[p][0], s[0].p[p][1], s[1].p[p][0], s[1].p[p][1]};
 }
 
+// SwiGLU of gate_up [M, 2 di] (gate, then up), as float32 rows and in three parts as above.  One pass where the unit's kernel and the split of its result were two: 517 x 3,840
+// 6.6 + 5.5 -> 8.5 us.  (Rows of 16 and 32 k a wave, as the split, so that the parts leave in whole lines.)
+__global__ void __launch_bounds__(256) swiglu_parts_kernel(const float* gate_up, float* act, int M, int di, uint4* out) {
+    const int lane = threadIdx.x & 63, r = lane & 15, kq = lane >> 4, KG = di / 32;
+    const int w = blockIdx.x * 4 + (threadIdx.x >> 6), rt = w / KG, kg = w - rt * KG;
+    if (rt >= (M + 15) / 16) return;
+    const int row = min(16 * rt + r, M - 1), k = 32 * kg + 4 * kq;
+    const float* const from = gate_up + (size_t)row * 2 * di + k;
+    Split4 s[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const v4f g = *reinterpret_cast<const v4f*>(from + 16 * h), u = *reinterpret_cast<const v4f*>(from + di + 16 * h);
+        v4f o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float x = g[e] / (1.0f + expf(-g[e]));
+            s[h].y[e] = o[e] = u[e] * x;
+        }
+        if (16 * rt + r < M) *reinterpret_cast<v4f*>(act + (size_t)row * di + k + 16 * h) = o;
+        each<kSplitSteps>([&](auto o) { split_step<decltype(o)::value>(s[h]); });
+    }
+#pragma unroll
+    for (int p = 0; p < 3; ++p) out[(size_t)w * 192 + p * 64 + lane] = uint4{s[0].p[p][0], s[0].p[p][1], s[1].p[p][0], s[1].p[p][1]};
+}
+
+// x += alpha * the sum of the slices y [S][M][d]; out = rmsnorm(x) * w, as rows and (parts given) in three parts for the product that follows: one kernel where the sum of the
+// slices, the norm and the split were three.  Values, and the order of every sum, are those of the three (norm_row_kernel of elementwise.hip: a row to threads * VPT vectors of 4).
+// R rows a block: a row's pieces of the parts are 16 bytes, R neighbours' make R times as many in a line.  Bound by latency: one trip to memory for x and y, the sum across the
+// row, the way out.  517 x 1,536, every second one with the down product's slices: 5.4 + 5.5 (and 5.2)
+// -> 7.9 us on average; one row a block 8.0.
+constexpr int kNormRows = 2;
+template <int VPT, int R>
+__global__ void __launch_bounds__(1024) norm_parts_kernel(float* x, const float* y, int S, long long stride, float alpha, const float* w, float* out, unsigned char* parts, int M,
+                                                          int d, float eps) {
+    __shared__ float red[16];
+    const int per_row = blockDim.x / R, waves = per_row >> 6, in_block = R == 1 ? 0 : (int)threadIdx.x / per_row;
+    const int t = (int)threadIdx.x - in_block * per_row, row = blockIdx.x * R + in_block;
+    const bool mine = row < M;
+    const size_t at = (size_t)min(row, M - 1) * d;
+    v4f v[VPT], wv[VPT];
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+        const int c = 4 * (t + i * per_row);
+        v[i] = wv[i] = v4f{0.f, 0.f, 0.f, 0.f};
+        if (mine && c < d) {
+            wv[i] = *reinterpret_cast<const v4f*>(w + c);
+            const v4f xv = *reinterpret_cast<const v4f*>(x + at + c);
+            v4f sum = *reinterpret_cast<const v4f*>(y + at + c);
+            for (int s = 1; s < S; ++s) sum += *reinterpret_cast<const v4f*>(y + s * stride + at + c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[i][e] = fmaf(alpha, sum[e], xv[e]);
+            *reinterpret_cast<v4f*>(x + at + c) = v[i];
+            const float q[4] = {v[i][0], v[i][1], v[i][2], v[i][3]};
+            add_squares(ss, q, i == 0);
+        }
+    }
+    ss = wave_sum(ss);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    float sum = 0.f;
+    for (int i = 0; i < waves; ++i) sum += red[in_block * waves + i];
+    const float inv = 1.0f / sqrtf(sum / (float)d + eps);
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+        const int c = 4 * (t + i * per_row);
+        if (c >= d) continue;
+        Split4 s;
+        v4f o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s.y[e] = o[e] = mine ? v[i][e] * inv * wv[i][e] : 0.f;
+        if (mine) *reinterpret_cast<v4f*>(out + at + c) = o;
+        if (parts) {                                               // (rows beyond M up to a whole tile of 16: zeros)
+            each<kSplitSteps>([&](auto o) { split_step<decltype(o)::value>(s); });
+            const int kq = (c >> 2) & 3, h = (c >> 4) & 1;
+            unsigned char* const to = parts + ((size_t)(row >> 4) * (d >> 5) + (c >> 5)) * 3072 + ((row & 15) + 16 * kq) * 16 + 8 * h;
+#pragma unroll
+            for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2*>(to + 1024 * p) = uint2{s.p[p][0], s.p[p][1]};
+        }
+    }
+}
+
 // C = alpha * the sum of the slices P [S][M][N]; N a multiple of 4.
 __global__ void __launch_bounds__(256) sum_slices_kernel(const v4f* P, int S, int M, int N4, float* C, int ldc, float alpha) {
     const long long i = (long long)blockIdx.x * 256 + threadIdx.x, n = (long long)M * N4;
@@ -374,23 +456,25 @@ int rows_at_once(int M, int K, long long workspace_bytes) {
     return (int)(((M + runs - 1) / runs + 15) / 16 * 16);
 }
 
+// ready: A's parts lie in the workspace; keep: slices are left there behind them, not added up.
 int product(const float* A, const float* W, float* C, int M, int N, int K, int lda, int ldw, int ldc, float alpha, int shape, int slices, void* workspace,
-            long long workspace_bytes, hipStream_t stream) {
+            long long workspace_bytes, hipStream_t stream, bool ready = false, bool keep = false) {
     const int at_once = rows_at_once(M, K, workspace_bytes);
     if (at_once <= 0) return IC_ERR_ARG;
     if (slices > 1 && (at_once < M || parts_bytes(M, K) + 4LL * slices * M * N > workspace_bytes)) return IC_ERR_ARG;
+    if ((ready || keep) && at_once < M) return IC_ERR_ARG;
     std::lock_guard<std::mutex> lock(workspace_lock());
     for (int m = 0; m < M; m += at_once) {
         const int rows = M - m < at_once ? M - m : at_once;
         const float* const a0 = A + (size_t)m * lda;
         float* const sums = slices > 1 ? (float*)((char*)workspace + parts_bytes(M, K)) : C + (size_t)m * ldc;
-        int st = split_rows(a0, lda, rows, K, workspace, stream);
+        int st = ready ? IC_OK : split_rows(a0, lda, rows, K, workspace, stream);
         if (st) return st;
         st = run(F32Args{a0, W, sums, (const unsigned char*)workspace, rows, N, K, lda, ldw, slices > 1 ? N : ldc, 0, 0, slices, (long long)rows * N,
                          slices > 1 ? 1.0f : alpha}, shape, stream);
         if (st) return st;
     }
-    if (slices > 1) {
+    if (slices > 1 && !keep) {
         const long long n = (long long)M * (N / 4);
         if (n > (1LL << 38)) return IC_ERR_ARG;
         hipLaunchKernelGGL(sum_slices_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream,
@@ -464,13 +548,20 @@ IC_EXPORT int ic_gemm_f32_pays(int M, int N, int K) { return ic_gemm_f32_pays_on
 
 IC_EXPORT long long ic_gemm_f32_parts_bytes(int M, int K) { return M > 0 && K >= 32 ? parts_bytes(M, K) : 0; }
 
+namespace {
+
+bool own_product(const void* A, const void* W, const void* C, int M, int N, int K, int lda, int ldw, int ldc, const void* parts, long long parts_bytes) {
+    if (!(M > kFewRows && A && W && C && aligned16(A) && aligned16(W) && aligned16(C) && ic_gemm_f32_takes(M, N, K, lda, ldw, ldc, parts, parts_bytes))) return false;
+    const int timed = ic_product_f32_timed(M, N, K, lda, ldw, ldc);
+    return (timed >= 0 ? timed : ic_gemm_f32_pays_with(M, N, K, parts_bytes, compute_units())) != 0;
+}
+
+}  // namespace
+
 // The product by this file's kernels or the library's, as timed (ic_product_tune) or by the rule: parts is the caller's own memory for the former, workspace the library's.
 IC_EXPORT int ic_product_f32(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, float alpha, void* parts, long long parts_bytes,
                              void* workspace, long long workspace_bytes, hipStream_t stream) {
-    if (M > kFewRows && A && W && C && aligned16(A) && aligned16(W) && aligned16(C) && ic_gemm_f32_takes(M, N, K, lda, ldw, ldc, parts, parts_bytes)) {
-        const int timed = ic_product_f32_timed(M, N, K, lda, ldw, ldc);
-        if (timed >= 0 ? timed : ic_gemm_f32_pays_with(M, N, K, parts_bytes, compute_units())) return ic_gemm_f32(A, W, C, M, N, K, lda, ldw, ldc, alpha, parts, parts_bytes, stream);
-    }
+    if (own_product(A, W, C, M, N, K, lda, ldw, ldc, parts, parts_bytes)) return ic_gemm_f32(A, W, C, M, N, K, lda, ldw, ldc, alpha, parts, parts_bytes, stream);
     return ic_matmul(A, IC_F32, W, C, IC_F32, M, N, K, lda, ldw, ldc, alpha, workspace, workspace_bytes, stream);
 }
 
@@ -489,4 +580,55 @@ IC_EXPORT int ic_gemm_f32_cfg(const void* A, const void* W, void* C, int M, int 
     if (!A || !W || !C || !workspace || !takes(M, N, K, lda, ldw, ldc) || !aligned16(A) || !aligned16(W) || !aligned16(C) || !aligned16(workspace) || shape < 0 ||
         shape >= kShapes || slices < 1 || slices > kMaxSlices || slices > K / 32 || (slices > 1 && N % 4)) return IC_ERR_ARG;
     return product((const float*)A, (const float*)W, (float*)C, M, N, K, lda, ldw, ldc, alpha, shape, slices, workspace, workspace_bytes, stream);
+}
+
+// Slices of K that ic_product_f32 would use with these arguments where it runs ic_gemm_f32 on all rows at once, else 0.  Then A's parts may be made by what computes A, and the
+// slices be added by what reads C.
+IC_EXPORT int ic_gemm_f32_whole(const void* A, const void* W, const void* C, int M, int N, int K, int lda, int ldw, int ldc, const void* parts, long long parts_bytes) {
+    if (!own_product(A, W, C, M, N, K, lda, ldw, ldc, parts, parts_bytes) || rows_at_once(M, K, parts_bytes) < M) return 0;
+    return plan_for(M, N, K, most_slices(M, N, K, parts_bytes), compute_units()).slices;
+}
+
+// ic_gemm_f32 of all rows at once.  ready: A's parts lie in the workspace already; keep: more than one slice are left [slice][M][N] at ic_gemm_f32_parts_bytes(M, K) of the
+// workspace, and C is not written.
+IC_EXPORT int ic_gemm_f32_between(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, void* workspace, long long workspace_bytes, int ready,
+                                  int keep, hipStream_t stream) {
+    if (M <= 0) return IC_OK;
+    if (!A || !W || !C || !workspace || !takes(M, N, K, lda, ldw, ldc) || !aligned16(A) || !aligned16(W) || !aligned16(C) || !aligned16(workspace)) return IC_ERR_ARG;
+    if (rows_at_once(M, K, workspace_bytes) < M) return IC_ERR_ARG;
+    const Plan p = plan_for(M, N, K, most_slices(M, N, K, workspace_bytes), compute_units());
+    return product((const float*)A, (const float*)W, (float*)C, M, N, K, lda, ldw, ldc, 1.0f, p.shape, p.slices, workspace, workspace_bytes, stream, ready != 0, keep != 0);
+}
+
+// Rows of whole k-steps that one block holds.
+IC_EXPORT int ic_norm_parts_f32_supported(int d) { return d >= 32 && d % 32 == 0 && d <= 16384; }
+
+// x (float32 [M, d]) += alpha * (the sum of n_slices slices y [M, d], one behind the other); out = rmsnorm(x) * w, in three parts at `parts` too (null: not); all 16-byte aligned.
+// y and parts must not overlap.
+IC_EXPORT int ic_norm_parts_f32(float* x, const float* y, int n_slices, float alpha, const float* w, float* out, void* parts, int M, int d, float eps, hipStream_t stream) {
+    if (M <= 0) return IC_OK;
+    if (!x || !y || !w || !out || n_slices < 1 || n_slices > kMaxSlices || M > (1 << 26) || !ic_norm_parts_f32_supported(d)) return IC_ERR_ARG;
+    if (!aligned16(x) || !aligned16(y) || !aligned16(w) || !aligned16(out) || !aligned16(parts)) return IC_ERR_ARG;
+    const int vecs = d / 4, t = (vecs + 63) / 64 * 64, per_row = t < 1024 ? t : 1024, vpt = (vecs + per_row - 1) / per_row;
+    const int whole = parts ? (M + 15) / 16 * 16 : M, rows = per_row * kNormRows <= 1024 ? kNormRows : 1;
+    const dim3 grid((whole + rows - 1) / rows), block(per_row * rows);
+    const long long stride = (long long)M * d;
+#define IC_NORM_PARTS(V, R) hipLaunchKernelGGL((norm_parts_kernel<V, R>), grid, block, 0, stream, x, y, n_slices, stride, alpha, w, out, (unsigned char*)parts, M, d, eps)
+    if (rows > 1) IC_NORM_PARTS(1, kNormRows);
+    else if (vpt == 1) IC_NORM_PARTS(1, 1);
+    else if (vpt == 2) IC_NORM_PARTS(2, 1);
+    else if (vpt == 3) IC_NORM_PARTS(3, 1);
+    else IC_NORM_PARTS(4, 1);
+#undef IC_NORM_PARTS
+    return ic_launch_status();
+}
+
+// act (float32 [M, di]) = up * silu(gate) of gate_up [M, 2 di] (gate, then up), in three parts at `parts` too; di a multiple of 32, all 16-byte aligned.
+IC_EXPORT int ic_swiglu_parts_f32(const float* gate_up, float* act, void* parts, int M, int di, hipStream_t stream) {
+    if (M <= 0) return IC_OK;
+    if (!gate_up || !act || !parts || di < 32 || di % 32 || M > (1 << 26) || !aligned16(gate_up) || !aligned16(act) || !aligned16(parts)) return IC_ERR_ARG;
+    const long long waves = (long long)((M + 15) / 16) * (di / 32);
+    if (waves >= (1LL << 30)) return IC_ERR_ARG;
+    hipLaunchKernelGGL(swiglu_parts_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream, gate_up, act, M, di, (uint4*)parts);
+    return ic_launch_status();
 }

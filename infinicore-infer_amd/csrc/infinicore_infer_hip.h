@@ -181,6 +181,14 @@ long long ic_gemm_f32_parts_bytes(int M, int K);
 long long ic_gemm_f32_workspace_bytes(int M, int N, int K);
 int ic_gemm_f32(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, float alpha, void* workspace, long long workspace_bytes, hipStream_t stream);
 
+// What a product in parts shares with its neighbours (float32, all rows at once).  ic_gemm_f32_whole: the slices of K that ic_product_f32 would use, 0 where it runs otherwise.
+// ic_gemm_f32_between: that product, A's parts in the workspace already (ready), its slices left [slice][M][N] at ic_gemm_f32_parts_bytes(M, K) of it (keep).
+// ic_norm_parts_f32: x += alpha * (the sum of the slices y), out = rmsnorm(x) * w as rows and, parts given, as parts (d: ic_norm_parts_f32_supported).  ic_swiglu_parts_f32: SwiGLU likewise.
+int ic_gemm_f32_whole(const void* A, const void* W, const void* C, int M, int N, int K, int lda, int ldw, int ldc, const void* parts, long long parts_bytes);
+int ic_gemm_f32_between(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, void* workspace, long long workspace_bytes, int ready, int keep, hipStream_t stream);
+int ic_norm_parts_f32_supported(int d);
+int ic_norm_parts_f32(float* x, const float* y, int n_slices, float alpha, const float* w, float* out, void* parts, int M, int d, float eps, hipStream_t stream);
+int ic_swiglu_parts_f32(const float* gate_up, float* act, void* parts, int M, int di, hipStream_t stream);
 // ic_product in float32 with memory of the caller's own for ic_gemm_f32 (parts, 16-byte aligned) beside ic_matmul's workspace.
 int ic_product_f32(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, float alpha, void* parts, long long parts_bytes, void* workspace, long long workspace_bytes, hipStream_t stream);
 

@@ -212,6 +212,11 @@ _SIGNATURES = {
     "ic_gemm_f32_plan_on": [_I] * 4 + [_c.POINTER(_I)],
     "ic_gemm_f32_parts_bytes": [_I, _I],
     "ic_gemm_f32_workspace_bytes": [_I] * 3,
+    "ic_gemm_f32_whole": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _LL],
+    "ic_gemm_f32_between": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _LL, _I, _I, _P],
+    "ic_norm_parts_f32_supported": [_I],
+    "ic_norm_parts_f32": [_P, _P, _I, _F, _P, _P, _P, _I, _I, _F, _P],
+    "ic_swiglu_parts_f32": [_P, _P, _P, _I, _I, _P],
     "ic_product_f32": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P, _LL, _P, _LL, _P],
     "ic_gemm_f32": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P, _LL, _P],
     "ic_gemm_f32_cfg": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _I, _P, _LL, _P],
