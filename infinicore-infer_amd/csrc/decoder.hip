@@ -128,7 +128,8 @@ struct IcDecoder {
     std::vector<IcLayer> layers;
     std::vector<IcRunEntry> entries;
     int max_qkv_width = 0, max_attn_width = 0, max_intermediate = 0;
-    bool chained = false;        // the layers are alike and their table lies on the device
+    std::vector<ChainEntry> table;       // of layers that are alike enough for one launch, else empty
+    const ChainEntry* device_table = nullptr;      // the same on the device: steps may run the layers in one launch
     std::string error;
 
     int fail(int status, const char* what, int entry) {
@@ -177,39 +178,35 @@ struct IcDecoder {
 
     // All layers in one launch: every row a request's single new token, all logits wanted.
     bool takes_chain(const IcStepBatch& b) const {
-        return chained && b.fixed_decode_splits <= 0 && b.decode_rows_identity && b.want_rows_identity && b.n_want == b.n_tokens && b.n_decode_rows == b.n_tokens &&
+        return device_table && b.fixed_decode_splits <= 0 && b.decode_rows_identity && b.want_rows_identity && b.n_want == b.n_tokens && b.n_decode_rows == b.n_tokens &&
                b.n_prefill_tiles == 0 && b.n_tokens <= kChainMaxRows && chain_supported(chain_shape(), b.n_tokens, meta.n_entries, std::max(b.max_context, b.max_position + 1));
     }
 
-    // Whether the layers are alike enough for one launch, and if so their table.
-    bool make_table() {
-        if (!meta.layer_table || meta.dtype != IC_BF16 || meta.n_entries < kChainMinEntries) return false;
+    // The layers' table, if they are alike enough for one launch.  Only what the description says: nothing is asked of the device, which other threads may be recording on.
+    void make_table() {
+        if (meta.dtype != IC_BF16 || meta.n_entries < kChainMinEntries) return;
         const IcRunEntry& e0 = entries[0];
         const IcLayer& l0 = layers[e0.layer];
         const IcAttention& a0 = l0.attention;
-        if (a0.window != 0 || a0.shared_kv || a0.rot_dim != a0.head_dim) return false;
-        std::vector<ChainEntry> table;
+        if (a0.window != 0 || a0.shared_kv || a0.rot_dim != a0.head_dim) return;
+        std::vector<ChainEntry> made;
         for (const IcRunEntry& e : entries) {
             const IcLayer& l = layers[e.layer];
             const IcAttention& a = l.attention;
             if (!e.writes_cache || e.group != e0.group || a.n_heads != a0.n_heads || a.n_kv_heads != a0.n_kv_heads || a.head_dim != a0.head_dim || a.window != 0 ||
                 a.shared_kv || a.rot_dim != a0.rot_dim || a.max_positions != a0.max_positions || a.softmax_scale != a0.softmax_scale || a.cos != a0.cos ||
                 a.sin != a0.sin || l.mixer_norm.eps != l0.mixer_norm.eps || l.ffn_norm.eps != l0.ffn_norm.eps || l.ffn.intermediate != l0.ffn.intermediate ||
-                l.residual_scale != l0.residual_scale) return false;
-            if (((uintptr_t)a.w_qkv | (uintptr_t)a.w_o | (uintptr_t)l.ffn.w_gate_up | (uintptr_t)l.ffn.w_down | (uintptr_t)e.k_cache | (uintptr_t)e.v_cache) & 15) return false;
-            for (const ChainEntry& other : table)
-                if (other.k_cache == e.k_cache || other.v_cache == e.v_cache) return false;
-            table.push_back(ChainEntry{a.w_qkv, a.w_o, l.ffn.w_gate_up, l.ffn.w_down, l.mixer_norm.weight, l.ffn_norm.weight, e.k_cache, e.v_cache});
+                l.residual_scale != l0.residual_scale) return;
+            if (((uintptr_t)a.w_qkv | (uintptr_t)a.w_o | (uintptr_t)l.ffn.w_gate_up | (uintptr_t)l.ffn.w_down | (uintptr_t)e.k_cache | (uintptr_t)e.v_cache) & 15) return;
+            for (const ChainEntry& other : made)
+                if (other.k_cache == e.k_cache || other.v_cache == e.v_cache) return;
+            made.push_back(ChainEntry{a.w_qkv, a.w_o, l.ffn.w_gate_up, l.ffn.w_down, l.mixer_norm.weight, l.ffn_norm.weight, e.k_cache, e.v_cache});
         }
-        if (!chain_supported(chain_shape(), 1, meta.n_entries, 1)) return false;
+        if (!chain_supported(chain_shape(), 1, meta.n_entries, 1)) return;
         ChainEntry end{};
         end.norm_in = meta.final_norm_scaled;
-        table.push_back(end);
-        if (hipMemcpy(meta.layer_table, table.data(), table.size() * sizeof(ChainEntry), hipMemcpyHostToDevice) != hipSuccess) {
-            (void)hipGetLastError();
-            return false;
-        }
-        return true;
+        made.push_back(end);
+        table = std::move(made);
     }
 
     Workspace layout(const IcStepBatch& b) const {
@@ -266,7 +263,7 @@ struct IcDecoder {
             f32 = std::max(f32, ic_gemm_f32_workspace_bytes(b.n_want, meta.vocab, meta.hidden));
         }
         w.f32_parts = take((size_t)f32);
-        if (chained && b.decode_rows_identity) {      // (what any smaller step needs too: recorded steps share one workspace)
+        if (device_table && b.decode_rows_identity) {      // (what any smaller step needs too: recorded steps share one workspace)
             const int rows = std::min(b.n_tokens, kChainMaxRows);
             w.chain = take(chain_scratch_bytes(chain_shape(), rows, meta.n_entries));
         }
@@ -362,7 +359,7 @@ struct IcDecoder {
             const IcAttention& A = l.attention;
             if (!b.group_tables[e.group] || !b.group_slots[e.group]) return fail(IC_ERR_ARG, "the cache group of the entry", 0);
             if (b.max_position >= A.max_positions) return fail(IC_ERR_ARG, "a position beyond the rotary tables", 0);
-            ChainStep c{(const ChainEntry*)meta.layer_table, meta.n_entries, T, A.softmax_scale, l.residual_scale, l.mixer_norm.eps, l.ffn_norm.eps, meta.embed_scale,
+            ChainStep c{device_table, meta.n_entries, T, A.softmax_scale, l.residual_scale, l.mixer_norm.eps, l.ffn_norm.eps, meta.embed_scale,
                         b.tokens, b.positions, b.group_slots[e.group], b.token_req, b.group_tables[e.group], b.group_table_stride[e.group], A.cos, A.sin,
                         meta.embed_table, l.mixer_norm.weight, x, base + ws.chain, base + ws.ffn_tail, (float*)(base + ws.ffn_sumsq)};
             st = chain_launch(chain_shape(), c, absent, stream);
@@ -574,6 +571,19 @@ struct IcDecoder {
 
 IC_EXPORT long long ic_decoder_table_bytes(int n_entries) { return n_entries < 0 ? -1 : (long long)(n_entries + 1) * (long long)sizeof(ChainEntry); }
 
+IC_EXPORT int ic_decoder_layer_table(const IcDecoder* decoder, void* host) {
+    if (!decoder || !host) return IC_ERR_ARG;
+    if (decoder->table.empty()) return 0;
+    memcpy(host, decoder->table.data(), decoder->table.size() * sizeof(ChainEntry));
+    return 1;
+}
+
+IC_EXPORT int ic_decoder_use_layer_table(IcDecoder* decoder, const void* table) {
+    if (!decoder || ((uintptr_t)table & 7) || (table && decoder->table.empty())) return IC_ERR_ARG;
+    decoder->device_table = (const ChainEntry*)table;
+    return IC_OK;
+}
+
 IC_EXPORT const char* ic_decoder_create_error() { return g_create_error.c_str(); }
 
 IC_EXPORT IcDecoder* ic_decoder_create(const IcDecoderMeta* meta, const IcLayer* layers, const IcRunEntry* entries) {
@@ -610,7 +620,7 @@ IC_EXPORT IcDecoder* ic_decoder_create(const IcDecoderMeta* meta, const IcLayer*
             return bad("a run-order entry names no layer, no group or no cache planes");
         }
     }
-    d->chained = d->make_table();
+    d->make_table();
     return d;
 }
 

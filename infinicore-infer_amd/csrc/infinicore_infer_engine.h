@@ -88,8 +88,6 @@ typedef struct {
     const float* final_norm_scaled;   // final_norm.weight * logit_scale
     int* attention_counters;          // ic_attn_prefill_counter_ints() ints of the caller's, zero when the decoder is made; every step
                                       // leaves them zero.  Steps that overlap in time (two streams) need decoders with counters of their own
-    void* layer_table;                // ic_decoder_table_bytes(n_entries) bytes of device memory of the caller's, written when the decoder is made; NULL: a decode
-                                      // step's layers are launched kernel by kernel
 } IcDecoderMeta;
 
 // A step's batch where it lies on the device.  Tokens of all requests are concatenated in request order.
@@ -131,11 +129,17 @@ typedef struct {
 
 // Copies the descriptions (not the tensors they point to).  NULL when a field is out of range;
 // ic_decoder_create_error() then says which.
-long long ic_decoder_table_bytes(int n_entries);
 IcDecoder* ic_decoder_create(const IcDecoderMeta* meta, const IcLayer* layers, const IcRunEntry* entries);
 const char* ic_decoder_create_error();
 void ic_decoder_destroy(IcDecoder* decoder);
 const char* ic_decoder_last_error(const IcDecoder* decoder);
+
+// Decode steps of few rows whose layers are alike can run them all in one launch.  ic_decoder_layer_table writes the table that this takes (ic_decoder_table_bytes) to
+// host memory: 1, or 0 and nothing where the layers do not allow it.  The caller takes those bytes to device memory of its own, ordered before the steps that
+// follow, and hands that over (ic_decoder_use_layer_table; NULL takes it back): without it a step's layers are launched kernel by kernel.
+long long ic_decoder_table_bytes(int n_entries);
+int ic_decoder_layer_table(const IcDecoder* decoder, void* host);
+int ic_decoder_use_layer_table(IcDecoder* decoder, const void* table);
 
 // Bytes of device workspace ic_decoder_forward needs for this batch (activations and partial results).
 long long ic_decoder_workspace_bytes(const IcDecoder* decoder, const IcStepBatch* batch);

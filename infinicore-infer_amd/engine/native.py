@@ -65,15 +65,24 @@ class NativeDecoder:
             k, v = engine.storage.kv(e.cache)
             entries.append(IcRunEntry(e.layer, int(e.writes_cache), engine._slot_group[e.cache], k.data_ptr(), v.data_ptr()))
         entry_arr = (IcRunEntry * len(entries))(*entries)
-        table = torch.zeros(lib.ic_decoder_table_bytes(len(entries)), dtype=torch.uint8, device=engine.device)
         meta = IcDecoderMeta(ops.dtype_code(rt.dtype), model.spec.hidden_size, model.spec.vocab_size, engine.page_size,
                              len(layers), len(entries), len(engine.groups), engine.cu_count, emb[1], head[1], emb[0],
-                             head[0], fin, scaled_w.data_ptr(), counters.data_ptr(), table.data_ptr())
+                             head[0], fin, scaled_w.data_ptr(), counters.data_ptr())
         handle = lib.ic_decoder_create(ctypes.byref(meta), layer_arr, entry_arr)
         if not handle:
             raise KernelError("the native step function refused the model: %s"
                               % lib.ic_decoder_create_error().decode())
-        return cls(handle, lib, model.spec.vocab_size, (layer_arr, entry_arr, meta, scaled_w, counters, table))
+        decoder = cls(handle, lib, model.spec.vocab_size, (layer_arr, entry_arr, meta, scaled_w, counters))
+        decoder._hand_over_table(len(entries), engine.device)
+        return decoder
+
+    def _hand_over_table(self, n_entries: int, device) -> None:
+        """Where the layers are alike: their table, by which a decode step of few rows runs them in one launch."""
+        host = torch.empty(self._lib.ic_decoder_table_bytes(n_entries), dtype=torch.uint8)
+        if self._lib.ic_decoder_layer_table(self._h, host.data_ptr()) == 1:
+            self._layer_table = host.to(device)          # a copy on the current stream, which has ended when this returns: any stream may read it
+            if self._lib.ic_decoder_use_layer_table(self._h, self._layer_table.data_ptr()):
+                raise KernelError("native step: the layers' table was refused")
 
     def workspace_bytes_for_decode(self, n_requests: int) -> int:
         """Workspace bytes that any step of up to ``n_requests`` single tokens needs (with the most key

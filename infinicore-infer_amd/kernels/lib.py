@@ -68,7 +68,7 @@ class IcDecoderMeta(_c.Structure):
     _fields_ = [("dtype", _I), ("hidden", _I), ("vocab", _I), ("page_size", _I), ("n_layers", _I), ("n_entries", _I),
                 ("n_groups", _I), ("compute_units", _I), ("embed_scale", _F), ("logit_scale", _F),
                 ("embed_table", _P), ("head_weight", _P), ("final_norm", IcNorm), ("final_norm_scaled", _P),
-                ("attention_counters", _P), ("layer_table", _P)]
+                ("attention_counters", _P)]
 
 
 class IcStepBatch(_c.Structure):
@@ -239,6 +239,8 @@ _SIGNATURES = {
     "ic_attn_decode_on_matrix_cores": [_I, _I, _I],
     "ic_decoder_create": [_c.POINTER(IcDecoderMeta), _c.POINTER(IcLayer), _c.POINTER(IcRunEntry)],
     "ic_decoder_table_bytes": [_I],
+    "ic_decoder_layer_table": [_P, _P],
+    "ic_decoder_use_layer_table": [_P, _P],
     "ic_decode_chain_pieces": [_P, _I, _I, _I, _P, _I, _P],
     "ic_decoder_forward_absent": [_P, _c.POINTER(IcStepBatch), _P, _LL, _P, _LL, _P, _I, _P],
     "ic_decoder_takes_chain": [_P, _c.POINTER(IcStepBatch)],

@@ -205,3 +205,24 @@ def test_weights_that_are_not_numbers():
     table[5].copy_(row)
     got[0, 5] = want[0, 5]                                   # (the table is the head's too)
     assert _chained(engine) and torch.equal(got[0], want[0]) and bool(got[1].isnan().all())
+
+
+def test_the_table_of_an_engine_made_on_a_stream_of_its_own():
+    """Work is queued on that stream when the table is handed over: it holds the layers' addresses all the same (looked at, not run)."""
+    from infinicore_infer_amd.engine.native import NativeDecoder
+    engine, _ = _engine("1b")
+    lib = engine.native._lib
+    host = torch.empty(lib.ic_decoder_table_bytes(LAYERS), dtype=torch.uint8)
+    assert lib.ic_decoder_layer_table(engine.native._h, host.data_ptr()) == 1
+    a = torch.randn(4096, 4096, device="cuda")
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        for _ in range(40):
+            a = a @ a
+            a /= a.norm()
+        made = NativeDecoder.try_build(engine)
+    stream.synchronize()
+    own = torch.empty_like(host)                             # (the scaled final norm is this decoder's own)
+    assert lib.ic_decoder_layer_table(made._h, own.data_ptr()) == 1
+    assert torch.equal(own[:-64], host[:-64]) and torch.equal(made._layer_table.cpu(), own)
