@@ -416,7 +416,8 @@ __device__ __forceinline__ void walk_piece(Args a, const Shared& sh, const Piece
                 w[u] = kb + stage * H::STEP + u * H::KPB < hi ? d : -INFINITY;
                 mx = fmaxf(mx, w[u]);
             }
-            const float base = mx == -INFINITY ? 0.f : mx, corr = __builtin_amdgcn_exp2f(m - base);      // (no key yet: every weight is 0)
+            if (mx == -INFINITY) return;                     // this lane group has seen no key yet
+            const float corr = __builtin_amdgcn_exp2f(m - mx);
             l *= corr;
 #pragma unroll
             for (int i = 0; i < 8; ++i) acc[i] *= corr;
@@ -424,7 +425,7 @@ __device__ __forceinline__ void walk_piece(Args a, const Shared& sh, const Piece
             for (int u = 0; u < H::U; ++u) {
                 float v[8];
                 Vec16<bf16>::unpack(at[H::U + u], v);
-                w[u] = __builtin_amdgcn_exp2f(w[u] - base);
+                w[u] = __builtin_amdgcn_exp2f(w[u] - mx);
                 l += w[u];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) acc[i] = fmaf(w[u], v[i], acc[i]);
@@ -497,15 +498,16 @@ __device__ __forceinline__ void walk_piece(Args a, const Shared& sh, const Piece
             }
             mx = swap_max<16>(swap_max<32>(mx));
             if (__builtin_amdgcn_ballot_w64(mx > m)) {
-                const float now = fmaxf(m, mx), corr = __builtin_amdgcn_exp2f(m - now);
+                const float now = fmaxf(m, mx), corr = __builtin_amdgcn_exp2f(m - (now == -INFINITY ? 0.f : now));
                 l *= corr;
                 m = now;
 #pragma unroll
                 for (int c = 0; c < ND; ++c) acc[c] *= corr;
             }
             ch_v8f pf;
+            const float base = m == -INFINITY ? 0.f : m;     // (no key of this head yet whose score is not -inf: weights 0)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) { pf[e] = __builtin_amdgcn_exp2f(w[e] - m); l += pf[e]; }
+            for (int e = 0; e < 8; ++e) { pf[e] = __builtin_amdgcn_exp2f(w[e] - base); l += pf[e]; }
             const ch_v8b pb = __builtin_convertvector(pf, ch_v8b);
             const uint16_t* const vrow = mine + (4 * lg + (lr >> 2)) * VS + 4 * (lr & 3);
 #pragma unroll
@@ -854,14 +856,15 @@ decode_chain_kernel(const ChainArgs) {
                         float m = own ? sh.own[i][j] : -INFINITY, acc = 0.f, l = 0.f;
 #pragma unroll
                         for (int v = 0; v < kStream; ++v) m = fmaxf(m, st[v * H::STATE + GQ * DH + 2 * j]);
+                        const float base = m == -INFINITY ? 0.f : m;         // (every score is: all weights are 0, not exp2(-inf + inf))
 #pragma unroll
                         for (int v = 0; v < kStream; ++v) {
-                            const float k = __builtin_amdgcn_exp2f(st[v * H::STATE + GQ * DH + 2 * j] - m);
+                            const float k = __builtin_amdgcn_exp2f(st[v * H::STATE + GQ * DH + 2 * j] - base);
                             acc = fmaf(st[v * H::STATE + j * DH + c], k, acc);
                             l = fmaf(st[v * H::STATE + GQ * DH + 2 * j + 1], k, l);
                         }
-                        if (own) {
-                            const float k = __builtin_amdgcn_exp2f(sh.own[i][j] - m);
+                        if (own && sh.own[i][j] != -INFINITY) {
+                            const float k = __builtin_amdgcn_exp2f(sh.own[i][j] - base);
                             acc = fmaf(bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(rows + 1024 * i)[(GQ + 1) * DH + c]), k, acc);
                             l += k;
                         }

@@ -226,3 +226,35 @@ def test_the_table_of_an_engine_made_on_a_stream_of_its_own():
     own = torch.empty_like(host)                             # (the scaled final norm is this decoder's own)
     assert lib.ic_decoder_layer_table(made._h, own.data_ptr()) == 1
     assert torch.equal(own[:-64], host[:-64]) and torch.equal(made._layer_table.cpu(), own)
+
+
+@pytest.mark.parametrize("lens", [[1024], [64], [1024, 320, 640]])
+@pytest.mark.parametrize("shape", ["1b", "2b"])
+def test_pieces_whose_scores_are_all_minus_infinity(shape, lens):
+    """Keys of weight 0 beside others, in pieces of their own among others: whether their scores are -inf or finite and far below is one to the bit.  The step's own key (a
+    unit of its own: the lengths are multiples of 64) and the last unit's cached ones, in the first layer: its keys are minus its queries, times 4e37 and 1e10."""
+    engine, _ = _engine(shape, use_graphs=False)
+    doc, toks = H.random_tokens(2003, 1100, 4), H.random_tokens(2003, len(lens), 9)
+    mixer = engine.model.layers[0].mixer
+    w, nh, nkv = mixer.w_qkv, mixer.nh, mixer.nkvh
+    keep = w.clone()
+    out = []
+    for size in (4e37, 1e10):
+        w.copy_(keep)
+        _hold(engine, doc, lens)
+        q = w[:nh * 64].view(nkv, nh // nkv, 64, -1)
+        q.copy_(q[:, :1].clone().expand_as(q))               # a group's heads alike
+        w[nh * 64:(nh + nkv) * 64].view(nkv, 64, -1).copy_(q[:, 0].float() * -size)
+        _decode(engine, toks)
+        keys = engine.storage.kv(0)[0]                       # [page, kv head, place, 64]
+        for i, n in enumerate(lens):
+            page = lambda p: engine.cache.block_table("r%d" % i, 0)[p // 64]
+            own = keys[page(n), :, n % 64].clone()
+            assert n % 64 == 0 and bool(own.isfinite().all())
+            if n > 64:
+                keys[page(n - 64)] = own[:, None]
+            engine.cache.truncate("r%d" % i, n)
+        out.append(_decode(engine, toks))
+        assert _chained(engine)
+        _drop(engine, len(lens))
+    assert bool(out[1].isfinite().all()) and torch.equal(*out)
