@@ -3,6 +3,7 @@
 #include "common.h"
 
 constexpr int kChainMaxRows = 8;
+constexpr int kChainTries = 1 << 22;
 
 // One run-order entry where it lies on the device; the table has one more than there are entries, whose norm_in is the final norm's weight.
 struct ChainEntry {
@@ -34,6 +35,8 @@ struct ChainStep {
     void* scratch;             // chain_scratch_bytes
     void* y_out;               // bfloat16 [rows, hidden]: x times the final norm's weight
     float* sumsq_out;          // [parts, 16] sums of squares of x per column block
+    int* gave_up;              // set to 1 (null: not) where a wait of a block was given up after `tries` questions
+    int tries;
 };
 
 // 1: the kernel takes these sizes.  max_keys: an upper bound of the keys that a row sees.

@@ -51,12 +51,13 @@ constexpr int kMaxPieces = 40;              // of a block's attention work
 constexpr int kMaxGroup = 4;               // query heads of a kv head
 constexpr int kMaxPageIds = 2048;
 constexpr int kUnit = 64;                  // keys of a unit of attention work
-constexpr int kSyncWords = 2 * kCounters * kLineWords;
+constexpr int kGaveUp = 2 * kCounters * kLineWords;     // not 0: a block has given up a wait
+constexpr int kSyncWords = kGaveUp + kLineWords;
 constexpr unsigned long long kJoinTicks = 100000;      // 1 ms of the 100 MHz clock
 constexpr int kFarLoad = 16;                // sc1: past this die's caches
 constexpr int kPace = 10;                   // loads of a streaming wave in flight while it sends ahead (3: 1,532 us a step of the 2B shape, 6: 1,489, 10: 1,460, 16: 1,458)
-// A wait ends when blocks that run have written; should it not end after some seconds all the same, the block gives up and its results, with them the step's, are NaN.
-constexpr int kPollLimit = 1 << 22;
+// A wait ends when blocks that run have written.  Should it not end after some seconds (kChainTries questions) all the same, the block gives up: its results, with them the
+// step's logits, are NaN, no keys and values are cached of what came from it, and the caller is told (gave_up).
 
 struct Layout {                            // byte offsets within one entry's scratch
     long long y_in, ss_in, q, kv, attn, acc, ml, y_mid, ss_mid, act, stride;
@@ -74,6 +75,8 @@ struct ChainArgs {
     unsigned char* scratch;
     Layout at;
     unsigned* sync;
+    int* gave_up;
+    int tries;
     bf16* y_out;
     float* ss_out;
     int G, cols, t_qkv, t_res, t_gu;
@@ -110,7 +113,7 @@ struct Piece { int row, kvh, lo, hi, slot, page_lo, page_off, pos; };
 // What a block knows about the step, in LDS.
 struct Shared {
     int n, rank;                           // blocks that take part, this one's number
-    int dead;                              // a wait was given up
+    int tries;                             // questions of a wait; -1: one was given up, no other lasts
     int n_pieces, n_ids;
     int direct, workers;                   // 1: a block walks whole heads; blocks that walk
     int tiles[kChainMaxRows], before[kChainMaxRows + 1];      // units of attention work: of a row's head, of the rows before
@@ -581,7 +584,7 @@ decode_chain_kernel(const ChainArgs) {
         }
         if (lane == 0) {
             sh.n = n; sh.rank = rank;
-            sh.dead = 0;
+            sh.tries = a->tries;
         }
     } else if (wave == kStream + 1) {
         // the units of attention work, and how they are dealt
@@ -671,7 +674,15 @@ decode_chain_kernel(const ChainArgs) {
     const int oi = lane & 7, om = lane >> 3;
     // Chunks of 1 KB, dealt over the control waves, to `rows` in order, again and again until no element in them is empty: what others write arrives so without a
     // further signal.  where(c): the lane's 16 bytes of chunk c.  Chunks from `halves` on hold `sums` float32 (some of the last 16 bytes may be nobody's).
-    auto dead = [&]() { return *const_cast<const volatile int*>(&sh.dead) != 0; };
+    auto tries_left = [&]() { return *const_cast<const volatile int*>(&sh.tries); };
+    auto give_up = [&]() {                                   // (known to the other blocks before anything that is computed from here on)
+        if (tries_left() < 0) return;
+        const Args b = again(a);
+        st_far(b->sync + kGaveUp, 1u);
+        if (b->gave_up) __hip_atomic_store(b->gave_up, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __threadfence_system();
+        sh.tries = -1;
+    };
     auto fetch = [&](int chunks, int halves, int sums, auto where) {
         ch_u64 open = cw < chunks ? ~0ull >> (64 - (chunks - cw + kControl - 1) / kControl) : 0ull;
         int tries = 0;
@@ -692,7 +703,7 @@ decode_chain_kernel(const ChainArgs) {
                 }
                 if (!__any(lacks)) open &= ~(1ull << k);
             }
-            if (dead() || ++tries > kPollLimit) { sh.dead = 1; break; }
+            if (++tries > tries_left()) { give_up(); break; }
         }
     };
     // The rows [row][K] of a product, with ss the sums of squares [row][task] behind them.
@@ -715,7 +726,7 @@ decode_chain_kernel(const ChainArgs) {
             float s = 0.f;
             for (int i = lane; i < parts; i += 64) s += ss[t * parts + i];
             s = wave_sum(s);
-            if (lane == 0) sh.factor[t] = sh.dead ? __uint_as_float(0x7fc00000u) : rsqrtf(s / (float)K + eps);
+            if (lane == 0) sh.factor[t] = sh.tries < 0 ? __uint_as_float(0x7fc00000u) : rsqrtf(s / (float)K + eps);
         }
     };
     auto sum_of = [&](int out, int at) {
@@ -745,7 +756,7 @@ decode_chain_kernel(const ChainArgs) {
             meet();
             if (cw == 0) {
                 float sq = 0.f;
-                const float poison = sh.dead ? __uint_as_float(0x7fc00000u) : 0.f;
+                const float poison = sh.tries < 0 ? __uint_as_float(0x7fc00000u) : 0.f;
 #pragma unroll
                 for (int r = 0; r < RR; ++r) {
                     if (!mine[r]) continue;
@@ -805,7 +816,8 @@ decode_chain_kernel(const ChainArgs) {
                                                  : (bf16*)(s + b->at.kv) + ((size_t)om * 2 * nkv + (head - nh)) * DH;
                     put(near + i0, v0);
                     put(near + i1, v1);
-                    if (head >= nh && slot >= 0) {           // for later steps
+                    // For later steps; not of rows that are NaN because a wait was given up.
+                    if (head >= nh && slot >= 0 && !(f != f && ld_far(b->sync + kGaveUp) != 0u)) {
                         const int page = slot / b->page_size, off = slot - page * b->page_size;
                         bf16 __attribute__((address_space(1)))* const plane = (bf16 __attribute__((address_space(1)))*)uniform(value ? E->v_cache : E->k_cache) + (((size_t)page * nkv + (head - nh - (value ? nkv : 0))) * b->page_size + off) * DH;
                         ((uint16_t __attribute__((address_space(1)))*)plane)[i0] = f32_to_bf16_bits(v0);
@@ -909,7 +921,7 @@ decode_chain_kernel(const ChainArgs) {
                             ml[k][0] = __uint_as_float((unsigned)z); ml[k][1] = __uint_as_float((unsigned)(z >> 32));
                         }
                         if (!__any(lacks)) break;
-                        if (dead() || ++tries > kPollLimit) { sh.dead = 1; break; }
+                        if (++tries > tries_left()) { give_up(); break; }
                     }
                     float mx = m;
 #pragma unroll
@@ -1117,6 +1129,7 @@ int chain_launch(const ChainShape& s, const ChainStep& st, int absent, hipStream
     a.at = chain_layout(s, p, st.rows);
     a.sync = (unsigned*)st.scratch;
     a.scratch = (unsigned char*)st.scratch + kSyncWords * 4;
+    a.gave_up = st.gave_up; a.tries = st.tries;
     a.y_out = (bf16*)st.y_out; a.ss_out = st.sumsq_out;
     a.G = s.compute_units; a.cols = p.cols; a.t_qkv = p.t_qkv; a.t_res = p.t_res; a.t_gu = p.t_gu;
     const size_t lds = lds_bytes(s, p, st.rows, st.n_entries, &a.rows_bytes, &a.red_floats);

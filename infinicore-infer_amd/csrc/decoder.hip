@@ -130,6 +130,7 @@ struct IcDecoder {
     int max_qkv_width = 0, max_attn_width = 0, max_intermediate = 0;
     std::vector<ChainEntry> table;       // of layers that are alike enough for one launch, else empty
     const ChainEntry* device_table = nullptr;      // the same on the device: steps may run the layers in one launch
+    int* gave_up = nullptr;              // the caller's, see ic_decoder_use_layer_table
     std::string error;
 
     int fail(int status, const char* what, int entry) {
@@ -304,7 +305,7 @@ struct IcDecoder {
     }
 
     int forward(const IcStepBatch& b, void* workspace, long long workspace_bytes, void* lib_ws, long long lib_ws_bytes,
-                float* logits, hipStream_t stream, int absent = 0) {
+                float* logits, hipStream_t stream, int absent = 0, int tries = kChainTries) {
         error.clear();
         const int T = b.n_tokens, d = meta.hidden, dt = meta.dtype, ps = meta.page_size;
         if (T <= 0) return IC_OK;
@@ -361,7 +362,7 @@ struct IcDecoder {
             if (b.max_position >= A.max_positions) return fail(IC_ERR_ARG, "a position beyond the rotary tables", 0);
             ChainStep c{device_table, meta.n_entries, T, A.softmax_scale, l.residual_scale, l.mixer_norm.eps, l.ffn_norm.eps, meta.embed_scale,
                         b.tokens, b.positions, b.group_slots[e.group], b.token_req, b.group_tables[e.group], b.group_table_stride[e.group], A.cos, A.sin,
-                        meta.embed_table, l.mixer_norm.weight, x, base + ws.chain, base + ws.ffn_tail, (float*)(base + ws.ffn_sumsq)};
+                        meta.embed_table, l.mixer_norm.weight, x, base + ws.chain, base + ws.ffn_tail, (float*)(base + ws.ffn_sumsq), gave_up, tries};
             st = chain_launch(chain_shape(), c, absent, stream);
             if (st) return fail(st, "the layers in one launch", 0);
             def = Deferred{base + ws.ffn_tail, (const float*)(base + ws.ffn_sumsq), chain_sumsq_parts(chain_shape()), d, meta.final_norm.eps};
@@ -578,9 +579,10 @@ IC_EXPORT int ic_decoder_layer_table(const IcDecoder* decoder, void* host) {
     return 1;
 }
 
-IC_EXPORT int ic_decoder_use_layer_table(IcDecoder* decoder, const void* table) {
-    if (!decoder || ((uintptr_t)table & 7) || (table && decoder->table.empty())) return IC_ERR_ARG;
+IC_EXPORT int ic_decoder_use_layer_table(IcDecoder* decoder, const void* table, int* gave_up) {
+    if (!decoder || ((uintptr_t)table & 7) || ((uintptr_t)gave_up & 3) || (table && decoder->table.empty())) return IC_ERR_ARG;
     decoder->device_table = (const ChainEntry*)table;
+    decoder->gave_up = table ? gave_up : nullptr;
     return IC_OK;
 }
 
@@ -644,6 +646,13 @@ IC_EXPORT int ic_decoder_forward_absent(IcDecoder* decoder, const IcStepBatch* b
                                         long long library_workspace_bytes, float* logits, int absent, hipStream_t stream) {
     if (!decoder || !batch || absent < 0 || absent >= decoder->meta.compute_units) return IC_ERR_ARG;
     return decoder->forward(*batch, workspace, workspace_bytes, library_workspace, library_workspace_bytes, logits, stream, absent);
+}
+
+// The same where a block gives up a wait after `tries` questions.
+IC_EXPORT int ic_decoder_forward_tries(IcDecoder* decoder, const IcStepBatch* batch, void* workspace, long long workspace_bytes, void* library_workspace,
+                                       long long library_workspace_bytes, float* logits, int tries, hipStream_t stream) {
+    if (!decoder || !batch || tries < 0) return IC_ERR_ARG;
+    return decoder->forward(*batch, workspace, workspace_bytes, library_workspace, library_workspace_bytes, logits, stream, 0, tries);
 }
 
 // Whether a step runs its layers in one launch.

@@ -137,9 +137,11 @@ const char* ic_decoder_last_error(const IcDecoder* decoder);
 // Decode steps of few rows whose layers are alike can run them all in one launch.  ic_decoder_layer_table writes the table that this takes (ic_decoder_table_bytes) to
 // host memory: 1, or 0 and nothing where the layers do not allow it.  The caller takes those bytes to device memory of its own, ordered before the steps that
 // follow, and hands that over (ic_decoder_use_layer_table; NULL takes it back): without it a step's layers are launched kernel by kernel.
+// gave_up: NULL, or an int that host and device reach (pinned host memory), 0.  The blocks of such a step wait for each other; should a wait not end within seconds, the
+// step ends all the same, its logits are NaN, and it sets the int to 1: to be looked at where the step has been waited for.
 long long ic_decoder_table_bytes(int n_entries);
 int ic_decoder_layer_table(const IcDecoder* decoder, void* host);
-int ic_decoder_use_layer_table(IcDecoder* decoder, const void* table);
+int ic_decoder_use_layer_table(IcDecoder* decoder, const void* table, int* gave_up);
 
 // Bytes of device workspace ic_decoder_forward needs for this batch (activations and partial results).
 long long ic_decoder_workspace_bytes(const IcDecoder* decoder, const IcStepBatch* batch);

@@ -223,9 +223,12 @@ class Engine:
         """Run the entries' tokens as one batch.  Returns float32 logits
         [number of wanted places, vocab] on the device, in the order of the entries and
         of each entry's ``want`` (None when nothing is wanted).  The tensor is a
-        workspace view: it is valid until the next step."""
+        workspace view: it is valid until the next step.  Should the device not get a step done (its
+        layers' blocks gave up waiting for each other), its logits are NaN; the sampling of its tokens raises,
+        or the next step."""
         if not entries:
             return None
+        self._check_native()
         if self.use_graphs and len(entries) <= self.graph_max_batch:
             starts = self._append_single_tokens(entries)
             if starts is not None:                   # a pure decode step: the lean way through the same checks
@@ -678,7 +681,12 @@ class Engine:
             host = self._sampled_host = torch.empty(max(R, self.graph_max_batch, 1), dtype=torch.int32, pin_memory=True)
         host[:R].copy_(out, non_blocking=True)
         torch.cuda.current_stream().synchronize()
+        self._check_native()
         return host[:R].tolist()
+
+    def _check_native(self):
+        if self.native is not None:
+            self.native.check()
 
     def sample_ahead(self, logits, temperature=None, top_k=None, top_p=None, uniform=None):
         """As ``sample``, without waiting for the device: returns (the tokens on the device, int32 [rows], and a
@@ -716,6 +724,7 @@ class Engine:
 
         def wait() -> List[int]:
             done.synchronize()
+            self._check_native()
             return host[:R].tolist()
         return out, wait
 

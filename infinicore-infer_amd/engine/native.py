@@ -27,6 +27,7 @@ class NativeDecoder:
         self._h = ctypes.c_void_p(handle)
         self._lib = lib
         self.vocab = vocab
+        self._gave_up = None              # set by the device where a step's blocks gave up waiting for each other
         self._keep = keep                 # the description arrays and derived tensors the C side points into
         self._batch = IcStepBatch()
         self._batch_ref = ctypes.byref(self._batch)
@@ -81,8 +82,16 @@ class NativeDecoder:
         host = torch.empty(self._lib.ic_decoder_table_bytes(n_entries), dtype=torch.uint8)
         if self._lib.ic_decoder_layer_table(self._h, host.data_ptr()) == 1:
             self._layer_table = host.to(device)          # a copy on the current stream, which has ended when this returns: any stream may read it
-            if self._lib.ic_decoder_use_layer_table(self._h, self._layer_table.data_ptr()):
+            self._gave_up = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+            if self._lib.ic_decoder_use_layer_table(self._h, self._layer_table.data_ptr(), self._gave_up.data_ptr()):
                 raise KernelError("native step: the layers' table was refused")
+
+    def check(self) -> None:
+        """Of the steps that have been waited for: raises when one has ended without its results (its logits are NaN, and so are those of
+        steps that went on from its tokens).  The requests that took part are to be freed: their last tokens are not in the cache."""
+        if self._gave_up is not None and self._gave_up[0]:
+            self._gave_up[0] = 0
+            raise KernelError("native step: the layers of a decode step gave up waiting for each other; its logits are not valid")
 
     def workspace_bytes_for_decode(self, n_requests: int) -> int:
         """Workspace bytes that any step of up to ``n_requests`` single tokens needs (with the most key

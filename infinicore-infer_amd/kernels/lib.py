@@ -240,9 +240,10 @@ _SIGNATURES = {
     "ic_decoder_create": [_c.POINTER(IcDecoderMeta), _c.POINTER(IcLayer), _c.POINTER(IcRunEntry)],
     "ic_decoder_table_bytes": [_I],
     "ic_decoder_layer_table": [_P, _P],
-    "ic_decoder_use_layer_table": [_P, _P],
+    "ic_decoder_use_layer_table": [_P, _P, _P],
     "ic_decode_chain_pieces": [_P, _I, _I, _I, _P, _I, _P],
     "ic_decoder_forward_absent": [_P, _c.POINTER(IcStepBatch), _P, _LL, _P, _LL, _P, _I, _P],
+    "ic_decoder_forward_tries": [_P, _c.POINTER(IcStepBatch), _P, _LL, _P, _LL, _P, _I, _P],
     "ic_decoder_takes_chain": [_P, _c.POINTER(IcStepBatch)],
     "ic_decoder_create_error": [],
     "ic_decoder_destroy": [_P],

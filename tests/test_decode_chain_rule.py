@@ -43,7 +43,7 @@ class Decoder:
         return host.reshape(-1, 8).tolist() if self.lib.ic_decoder_layer_table(self.h, host.ctypes.data) == 1 else None
 
     def use(self):
-        return self.lib.ic_decoder_use_layer_table(self.h, 1 << 16)
+        return self.lib.ic_decoder_use_layer_table(self.h, 1 << 16, None)
 
     def step(self, rows=1, keys=258):
         b = IcStepBatch()
@@ -66,10 +66,10 @@ def test_the_table_is_made_without_the_device():
         assert d.table() == d.want
         assert not d.takes()
         before = d.lib.ic_decoder_workspace_bytes(d.h, ctypes.byref(d.step()))
-        assert d.lib.ic_decoder_use_layer_table(d.h, (1 << 16) + 4) != 0 and not d.takes()
+        assert d.lib.ic_decoder_use_layer_table(d.h, (1 << 16) + 4, None) != 0 and not d.takes()
         assert d.use() == 0 and d.takes()
         assert d.lib.ic_decoder_workspace_bytes(d.h, ctypes.byref(d.step())) > before
-        assert d.lib.ic_decoder_use_layer_table(d.h, None) == 0 and not d.takes()
+        assert d.lib.ic_decoder_use_layer_table(d.h, None, None) == 0 and not d.takes()
 
 
 def _set(path, value, at=1):

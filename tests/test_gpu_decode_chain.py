@@ -258,3 +258,31 @@ def test_pieces_whose_scores_are_all_minus_infinity(shape, lens):
         assert _chained(engine)
         _drop(engine, len(lens))
     assert bool(out[1].isfinite().all()) and torch.equal(*out)
+
+
+@pytest.mark.parametrize("lens", [[1100], [700, 3, 1290]])
+@pytest.mark.parametrize("shape", ["1b", "2b"])
+def test_waits_that_are_given_up(shape, lens):
+    """No question is asked twice, so that most blocks give up at their first wait: the step ends, sampling its tokens raises, the cache holds nothing that came of it (what
+    the first layers wrote is right), and later steps are as ever."""
+    from infinicore_infer_amd.kernels.lib import KernelError
+    engine, _ = _engine(shape, use_graphs=False)
+    toks, doc = H.random_tokens(2003, len(lens), 7), H.random_tokens(2003, 1400, 3)
+    planes = [plane.zero_() for s in range(LAYERS) for plane in engine.storage.kv(s)]        # (pages that nobody holds have what the memory held)
+    _hold(engine, doc, lens)
+    want = _decode(engine, toks)
+    back = lambda: [engine.cache.truncate("r%d" % i, n) for i, n in enumerate(lens)]
+    back()
+    forward, usual = engine.native._lib.ic_decoder_forward_tries, engine.native._forward
+    for sample in (engine.sample, lambda logits: engine.sample_ahead(logits)[1](), lambda logits: (torch.cuda.synchronize(), _decode(engine, toks))):
+        engine.native._forward = lambda *args: forward(*args[:-1], 0, args[-1])
+        got = _decode(engine, toks)
+        engine.native._forward = usual
+        assert _chained(engine) and bool(got.isnan().all())
+        with pytest.raises(KernelError, match="gave up"):
+            sample(got)
+        assert all(bool(plane.isfinite().all()) for plane in planes)
+        back()
+        assert torch.equal(_decode(engine, toks), want)
+        engine.sample(got)                                   # (told once)
+        back()
