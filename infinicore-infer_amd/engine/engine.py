@@ -584,7 +584,8 @@ class Engine:
         g.meta.copy_(g.host, non_blocking=True)
         g.copied.record()
         if device_tokens is not None:               # (only with a recording at hand: step_ahead has looked)
-            g.ctx.tokens.copy_(device_tokens)
+            # (a row of NaN samples no token of the vocabulary; no kernel may look such a one up; a step whose tokens come from the host refuses it)
+            torch.clamp(device_tokens.reshape(-1), 0, self.model.spec.vocab_size - 1, out=g.ctx.tokens)
         g.ctx.max_position = max(starts)
         g.ctx.req_pos = list(starts)
         g.ctx.req_ids = [e.req_id for e in entries]

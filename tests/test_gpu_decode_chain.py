@@ -286,3 +286,21 @@ def test_waits_that_are_given_up(shape, lens):
         assert torch.equal(_decode(engine, toks), want)
         engine.sample(got)                                   # (told once)
         back()
+
+
+@pytest.mark.parametrize("native", [True, False])
+def test_steps_ahead_of_rows_that_sampled_no_token(native):
+    """Logits of NaN sample what is no token of the vocabulary.  A step that takes it from the device looks up the last one (whose logits nobody wants) and nothing beyond."""
+    from infinicore_infer_amd.engine import StepEntry
+    engine, _ = _engine("1b", graph_after=1, use_native=native)
+    doc, V = H.random_tokens(2003, 90, 3), 2003
+    _hold(engine, doc, [70, 50])
+    nan = torch.full((2, V), float("nan"), device="cuda")
+    sampled, wait = engine.sample_ahead(nan)
+    assert all(not 0 <= t < V for t in wait())
+    ents = [StepEntry("r%d" % i, [0], [0]) for i in range(2)]
+    want = engine.step([StepEntry("r%d" % i, [V - 1], [0]) for i in range(2)]).clone()      # recorded here
+    for i, n in enumerate([70, 50]):
+        engine.cache.truncate("r%d" % i, n)
+    got = engine.step_ahead(ents, sampled)
+    assert got is not None and torch.equal(got, want)
