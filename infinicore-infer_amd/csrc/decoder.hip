@@ -226,7 +226,7 @@ struct IcDecoder {
         w.mixer_tail = take(few * d * 2);
         w.mixer_sumsq = take((size_t)parts * 16 * 4);
         w.ffn_tail = take(few * d * 2);
-        w.ffn_sumsq = take((size_t)parts * 16 * 4);
+        w.ffn_sumsq = take((size_t)(device_table ? std::max(parts, chain_sumsq_parts(chain_shape())) : parts) * 16 * 4);
         w.gate_up = take(T * 2 * (size_t)max_intermediate * ds);
         w.act = take(T * (size_t)max_intermediate * ds);
         size_t acc = 0, ml = 0;      // partial results of the key splits: [row, head, split, head size] and [row, head, split, 2]

@@ -95,3 +95,13 @@ def test_steps_that_run_kernel_by_kernel():
         assert d.use() == 0 and d.takes(4)
         assert not d.takes(9) and not d.takes(4, fixed_decode_splits=2) and not d.takes(4, n_want=3) and not d.takes(4, want_rows_identity=0)
         assert not d.takes(4, decode_rows_identity=0) and not d.takes(4, n_decode_rows=3, n_prefill_tiles=1)
+
+
+@pytest.mark.parametrize("hidden,heads,kv,inner,units,taken", [(2496, 64, 16, 6144, 304, False), (2496, 64, 16, 6144, 256, True), (1216, 24, 8, 3840, 304, False), (1216, 24, 8, 3840, 256, True),
+                                                                  (1536, 24, 8, 3840, 304, True)])
+def test_more_sums_of_squares_than_the_head_product_takes(hidden, heads, kv, inner, units, taken):
+    """A row has a sum for every block's columns of the stream; the product behind the chain takes 256 of them."""
+    blocks = -(-hidden // -(-hidden // units))
+    with Decoder(hidden=hidden, heads=heads, kv=kv, inner=inner, units=units) as d:
+        assert taken == (blocks <= d.lib.ic_rule_sumsq_parts_max())
+        assert (d.use() == 0) == taken and d.takes() == taken
