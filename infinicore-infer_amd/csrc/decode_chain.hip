@@ -1105,6 +1105,7 @@ int chain_supported(const ChainShape& s, int rows, int n_entries, int max_keys) 
     if (rows < 1 || rows > kChainMaxRows || s.compute_units < 64 || s.n_kv_heads < 1 || s.n_heads % s.n_kv_heads) return 0;
     if (s.hidden % 64 || s.intermediate % 64 || s.n_heads * s.head_dim % 64 || s.page_size < 16 || s.hidden > 16 * s.compute_units) return 0;
     if (2LL * 2 * s.intermediate * s.hidden > 0x7fffffffLL || 2LL * (s.n_heads + 2 * s.n_kv_heads) * s.head_dim * s.hidden > 0x7fffffffLL) return 0;
+    if (2LL * s.n_kv_heads * s.page_size * s.head_dim > 0xffffffffLL) return 0;      // (a page's bytes are multiplied in 32 bits)
     const Plan p = chain_plan(s);
     if (!instance(s, p) || p.t_res > ic_rule_sumsq_parts_max()) return 0;      // (the head product takes the row factors)
     const long long heads = (long long)rows * s.n_kv_heads, units = heads * ((max_keys + kUnit - 1) / kUnit);

@@ -105,3 +105,10 @@ def test_more_sums_of_squares_than_the_head_product_takes(hidden, heads, kv, inn
     with Decoder(hidden=hidden, heads=heads, kv=kv, inner=inner, units=units) as d:
         assert taken == (blocks <= d.lib.ic_rule_sumsq_parts_max())
         assert (d.use() == 0) == taken and d.takes() == taken
+
+
+@pytest.mark.parametrize("page,taken", [(1 << 20, True), ((1 << 22) - 1, True), (1 << 22, False), (1 << 24, False)])
+def test_pages_beyond_32_bits(page, taken):
+    """8 kv heads of 64 in bfloat16: a page of 2^22 keys has 2^32 bytes."""
+    with Decoder(page=page) as d:
+        assert (d.use() == 0) == taken and d.takes() == taken
