@@ -177,9 +177,9 @@ struct IcDecoder {
         return ChainShape{meta.hidden, l.attention.n_heads, l.attention.n_kv_heads, l.attention.head_dim, l.ffn.intermediate, meta.page_size, meta.compute_units};
     }
 
-    // All layers in one launch: every row a request's single new token, all logits wanted.
-    bool takes_chain(const IcStepBatch& b) const {
-        return device_table && b.fixed_decode_splits <= 0 && b.decode_rows_identity && b.want_rows_identity && b.n_want == b.n_tokens && b.n_decode_rows == b.n_tokens &&
+    // All layers in one launch: every row a request's single new token, all logits wanted, memory in which its 16-byte accesses are aligned.
+    bool takes_chain(const IcStepBatch& b, const void* workspace) const {
+        return device_table && !((uintptr_t)workspace & 15) && b.fixed_decode_splits <= 0 && b.decode_rows_identity && b.want_rows_identity && b.n_want == b.n_tokens && b.n_decode_rows == b.n_tokens &&
                b.n_prefill_tiles == 0 && b.n_tokens <= kChainMaxRows && chain_supported(chain_shape(), b.n_tokens, meta.n_entries, std::max(b.max_context, b.max_position + 1));
     }
 
@@ -323,7 +323,7 @@ struct IcDecoder {
         const int parts = ic_gemm_nt_residual_parts(d);
         int st;
 
-        const bool chain = takes_chain(b);
+        const bool chain = takes_chain(b, workspace);
         if (!chain) {
             st = ic_embed(b.tokens, meta.embed_table, dt, x, T, d, meta.embed_scale, stream);
             if (st) return fail(st, "the embedding gather", -1);
@@ -656,7 +656,8 @@ IC_EXPORT int ic_decoder_forward_tries(IcDecoder* decoder, const IcStepBatch* ba
 }
 
 // Whether a step runs its layers in one launch.
-IC_EXPORT int ic_decoder_takes_chain(const IcDecoder* decoder, const IcStepBatch* batch) { return decoder && batch ? decoder->takes_chain(*batch) : 0; }
+IC_EXPORT int ic_decoder_takes_chain_at(const IcDecoder* decoder, const IcStepBatch* batch, const void* workspace) { return decoder && batch ? decoder->takes_chain(*batch, workspace) : 0; }
+IC_EXPORT int ic_decoder_takes_chain(const IcDecoder* decoder, const IcStepBatch* batch) { return ic_decoder_takes_chain_at(decoder, batch, nullptr); }
 
 // ---- the key split of single-token rows --------------------------------------------------------------------------
 // One split writes the result itself; more cost a second kernel.  A rule by a model of the two kernels' time, one for each way of walking the

@@ -50,10 +50,12 @@ int ic_attn_decode_page_of(int key, int page_size);
 int ic_decode_chain_pieces(const int* positions, int rows, int kv_heads, int compute_units, int* pieces, int capacity, int* from_to);
 
 // ic_decoder_forward with `absent` of the blocks that a decode step's layers are dealt to not taking part, as if they found no room on the device; with waits for other
-// blocks that are given up after `tries` questions; and whether a step runs its layers in one launch (on which the two have no effect where it does not).
+// blocks that are given up after `tries` questions; and whether a step runs its layers in one launch (on which the two have no effect where it does not), with that
+// workspace or an aligned one.
 int ic_decoder_forward_absent(IcDecoder* decoder, const IcStepBatch* batch, void* workspace, long long workspace_bytes, void* library_workspace, long long library_workspace_bytes, float* logits, int absent, hipStream_t stream);
 int ic_decoder_forward_tries(IcDecoder* decoder, const IcStepBatch* batch, void* workspace, long long workspace_bytes, void* library_workspace, long long library_workspace_bytes, float* logits, int tries, hipStream_t stream);
 int ic_decoder_takes_chain(const IcDecoder* decoder, const IcStepBatch* batch);
+int ic_decoder_takes_chain_at(const IcDecoder* decoder, const IcStepBatch* batch, const void* workspace);
 
 // Whether ic_causal_conv runs a thread over a run of tokens (four taps, aligned rows), and whether ic_hc_step's threads send several rounds of a row's
 // loads ahead.

@@ -244,6 +244,7 @@ _SIGNATURES = {
     "ic_decode_chain_pieces": [_P, _I, _I, _I, _P, _I, _P],
     "ic_decoder_forward_absent": [_P, _c.POINTER(IcStepBatch), _P, _LL, _P, _LL, _P, _I, _P],
     "ic_decoder_forward_tries": [_P, _c.POINTER(IcStepBatch), _P, _LL, _P, _LL, _P, _I, _P],
+    "ic_decoder_takes_chain_at": [_P, _c.POINTER(IcStepBatch), _P],
     "ic_decoder_takes_chain": [_P, _c.POINTER(IcStepBatch)],
     "ic_decoder_create_error": [],
     "ic_decoder_destroy": [_P],

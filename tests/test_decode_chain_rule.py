@@ -112,3 +112,11 @@ def test_pages_beyond_32_bits(page, taken):
     """8 kv heads of 64 in bfloat16: a page of 2^22 keys has 2^32 bytes."""
     with Decoder(page=page) as d:
         assert (d.use() == 0) == taken and d.takes() == taken
+
+
+def test_workspaces_that_are_not_aligned():
+    """The other kernels take any; the one launch hands values on in pieces of 8 and 16 bytes."""
+    with Decoder() as d:
+        at = lambda p: bool(d.lib.ic_decoder_takes_chain_at(d.h, ctypes.byref(d.step()), p))
+        assert not at(1 << 20) and d.use() == 0
+        assert at(1 << 20) and at((1 << 20) + 16) and not at((1 << 20) + 4) and not at((1 << 20) + 8)
