@@ -189,7 +189,7 @@ struct IcDecoder {
         const IcRunEntry& e0 = entries[0];
         const IcLayer& l0 = layers[e0.layer];
         const IcAttention& a0 = l0.attention;
-        if (a0.window != 0 || a0.shared_kv || a0.rot_dim != a0.head_dim) return;
+        if (a0.window != 0 || a0.shared_kv || a0.rot_dim != a0.head_dim || (((uintptr_t)a0.cos | (uintptr_t)a0.sin) & 15)) return;      // (such tables ic_gemm_qkv_rope refuses)
         std::vector<ChainEntry> made;
         for (const IcRunEntry& e : entries) {
             const IcLayer& l = layers[e.layer];

@@ -107,6 +107,15 @@ def test_more_sums_of_squares_than_the_head_product_takes(hidden, heads, kv, inn
         assert (d.use() == 0) == taken and d.takes() == taken
 
 
+def test_rotary_tables_that_are_not_aligned():
+    """The QKV product refuses them in a step of few rows, so the one launch does not take them."""
+    def change(meta, layers, runs):
+        for l in layers:
+            l.attention.sin += 8
+    with Decoder(change=change) as d:
+        assert d.table() is None and d.use() != 0 and not d.takes()
+
+
 @pytest.mark.parametrize("page,taken", [(1 << 20, True), ((1 << 22) - 1, True), (1 << 22, False), (1 << 24, False)])
 def test_pages_beyond_32_bits(page, taken):
     """8 kv heads of 64 in bfloat16: a page of 2^22 keys has 2^32 bytes."""
@@ -115,7 +124,7 @@ def test_pages_beyond_32_bits(page, taken):
 
 
 def test_workspaces_that_are_not_aligned():
-    """The other kernels take any; the one launch hands values on in pieces of 8 and 16 bytes."""
+    """The one launch hands values on in pieces of 8 and 16 bytes; kernel by kernel the attention refuses such a step."""
     with Decoder() as d:
         at = lambda p: bool(d.lib.ic_decoder_takes_chain_at(d.h, ctypes.byref(d.step()), p))
         assert not at(1 << 20) and d.use() == 0
