@@ -290,8 +290,10 @@ struct IcDecoder {
     int whole_f32(const void* a, const void* w, const void* out, int M, int N, int K, const void* parts) const {
         return meta.dtype == IC_F32 ? ic_gemm_f32_whole(a, w, out, M, N, K, K, K, N, parts, ic_gemm_f32_workspace_bytes(M, N, K)) : 0;
     }
+    // Whether ic_norm_parts_f32 takes a norm (ic_add_rmsnorm takes any weight).
+    bool norm_in_parts(const IcNorm& norm) const { return ic_norm_parts_f32_supported(meta.hidden) && !((uintptr_t)norm.weight & 15); }
     // Into the residual stream, with slices that the norm after it adds up (slices > 1): those lie behind the K columns' parts, and the norm's parts must not reach them.
-    bool leaves_slices(int slices, int K) const { return slices > 1 && meta.hidden <= K && ic_norm_parts_f32_supported(meta.hidden); }
+    bool leaves_slices(int slices, int K, const IcNorm& norm) const { return slices > 1 && meta.hidden <= K && norm_in_parts(norm); }
 
     // 17..64 rows (and 13..16 long ones) into the residual stream: x += alpha * (a w^T), out = rmsnorm(x) * weight, through the sliced
     // product and the kernel that sums the slices.
@@ -341,7 +343,7 @@ struct IcDecoder {
         // Float32: x += alpha * (the sum of the slices y), normed = its norm, with normed's parts where the product behind it takes them.
         bool in_parts = false;                       // f32_parts holds the parts of the rows that the next product reads
         auto add_norm = [&](const void* y, int slices, float alpha, const IcNorm& norm, int next_slices) {
-            in_parts = next_slices > 0 && ic_norm_parts_f32_supported(d);
+            in_parts = next_slices > 0 && norm_in_parts(norm);
             if (in_parts || slices > 1)
                 return ic_norm_parts_f32(x, (const float*)y, slices, alpha, norm.weight, (float*)normed, in_parts ? f32_parts : nullptr, T, d, norm.eps, stream);
             return ic_add_rmsnorm(x, y, dt, alpha, norm.weight, normed, dt, T, d, norm.eps, stream);
@@ -495,7 +497,7 @@ struct IcDecoder {
                 g_def = &mid;
             } else {
                 const int o_slices = whole_f32(attn_out, A.w_o, base + ws.mixer_out, T, d, ow, f32_parts);
-                const bool keep = leaves_slices(o_slices, ow);
+                const bool keep = leaves_slices(o_slices, ow, L.ffn_norm);
                 st = product(attn_out, A.w_o, base + ws.mixer_out, d, ow, o_slices, keep);
                 if (st) return fail(st, "the O product", i);
                 st = add_norm(keep ? (char*)f32_parts + ic_gemm_f32_parts_bytes(T, ow) : base + ws.mixer_out, keep ? o_slices : 1, L.residual_scale, L.ffn_norm, gate_up_slices);
@@ -535,7 +537,7 @@ struct IcDecoder {
                 def = Deferred{base + ws.ffn_tail, (const float*)(base + ws.ffn_sumsq), parts, d, succ->eps};
                 owed = DEFERRED;
             } else {
-                const bool keep = i < last && leaves_slices(down_slices, di);      // (the last one's are added up: the final norm takes the wanted rows only)
+                const bool keep = i < last && leaves_slices(down_slices, di, layers[entries[i + 1].layer].mixer_norm);      // (the last one's are added up: the final norm takes the wanted rows only)
                 st = product(act, L.ffn.w_down, base + ws.ffn_out, d, di, down_slices, keep);
                 if (st) return fail(st, "the down product", i);
                 branch = keep ? (const char*)f32_parts + ic_gemm_f32_parts_bytes(T, di) : base + ws.ffn_out;

@@ -102,3 +102,25 @@ def test_steps_in_parts_equal_steps_product_by_product(tmp_path_factory):
     for j, n in enumerate((517, 33, 130, 300)):
         ents = [StepEntry("p%d" % j, H.random_tokens(5003, n, j), [0, n - 1])] + [StepEntry("p%d" % i, [9 + i], [0]) for i in range(j)]
         assert torch.equal(a.step(ents), b.step(ents))
+
+
+def test_norm_weights_that_are_not_aligned():
+    """The norms without parts take any weight, and a step with such weights runs as it did: bit for bit the one issued kernel by kernel."""
+    import helpers as H
+    from infinicore_infer_amd.engine import StepEntry
+    from test_gpu_large import SHAPE_1B, _engine_and_weights
+    cfg = dict(SHAPE_1B, vocab_size=2003, num_hidden_layers=4)
+    engines = [_engine_and_weights(cfg, 21, 0.02, 4096, 8, dtype=torch.float32, use_native=False)[0] for _ in range(2)]
+    from infinicore_infer_amd.engine.native import NativeDecoder
+    for e in engines:
+        for i, norm in enumerate(n for l in e.model.layers for n in (l.mixer_norm, l.feed_forward_norm)):
+            if i % 3 != 2:                                   # (aligned ones beside them: a product's slices and parts, or none)
+                off = torch.empty(norm.weight.numel() + 1, device="cuda")
+                off[1:].copy_(norm.weight)
+                norm.weight = off[1:]
+    engines[0].native = NativeDecoder.try_build(engines[0])
+    assert engines[0].native is not None
+    for n in (517, 130):
+        got, want = [e.step([StepEntry("p%d" % n, H.random_tokens(2003, n, 3), [0, n - 1])]).clone() for e in engines]
+        assert torch.equal(got, want)
+    assert engines[0].native_steps == 2
