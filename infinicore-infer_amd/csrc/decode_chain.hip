@@ -15,8 +15,15 @@
 // counters cost a wait for the writes, an atomic, a question and then the read (1B shape, one row: 28.4 -> 23.6 us a layer).  What is sent ahead waits until a block's
 // results are written (a second meeting of the waves): with loads in front of them results come late (1,060 -> 1,280 us a step of the 1B shape).
 //
-// Who takes part.  A block waits only for blocks that run: those that have come join at the start, and after a millisecond nobody else does (other work fills the device, or
-// another such kernel does); tasks are dealt to those n, what they compute does not depend on n.
+// Who takes part.  A block waits only for blocks that run: those that have come join at the start, and after a while nobody else does (other work fills the device, or
+// another such kernel does); tasks are dealt to those n, what they compute does not depend on n.  The while: what the missing ones cost, which is a step's time for every
+// round beyond the first in which n blocks do the tasks of G, so that such a step takes about twice its best at most; a millisecond at least.  (Closing after a millisecond whatever n is, with
+// the layers in launches of 4, 13 and 26, steps beside another engine's decoding: the slowest of 150 took 13.9, 37 and 72 ms, and 3.6, 4.8 and 6.1 so; of whole steps the
+// slowest is 3.3 either way.)
+// Beside other streams' work (1B shape, one row of 258 keys; kernel by kernel / so, us a step): another engine's prompts of 2,048 (2B shape) 3,700 / 1,200, its steps of 7 rows 2,450 /
+// 2,950, products of 4,096^3 13,800 / 1,450, of 16,384^3 706,000 / 18,000; two engines of 4, 12 and 24 layers 426 / 294, 923 / 750, 1,680 / 1,430.  The blocks fill the units'
+// registers, so other work runs between steps: those prompts take 181 ms instead of 15 meanwhile, the products of 4,096^3 360 us each instead of 110.  In launches
+// of 20 layers 97 ms and 250 us, for 0.3 % of a step alone and 1.1..1.8 times a step beside others; left so.
 //
 // One row, us a step, kernel by kernel / so: 1B shape at 100, 600, 2,000 keys 1,380 / 995, 1,535 / 1,142, 1,553 / 1,229; 2B shape 1,621 / 1,333, 1,722 / 1,453,
 // 1,839 / 1,507.  Four rows: 1,514 / 1,162, 1,628 / 1,344, 1,725 / 1,423; 1,632 / 1,446, 1,730 / 1,567, 2,027 / 1,859.  What bounds it: each phase is about 1 us of products and
@@ -53,7 +60,8 @@ constexpr int kMaxPageIds = 2048;
 constexpr int kUnit = 64;                  // keys of a unit of attention work
 constexpr int kGaveUp = 2 * kCounters * kLineWords;     // not 0: a block has given up a wait
 constexpr int kSyncWords = kGaveUp + kLineWords;
-constexpr unsigned long long kJoinTicks = 100000;      // 1 ms of the 100 MHz clock
+constexpr unsigned kJoinTicks = 100000;                 // 1 ms of the 100 MHz clock
+constexpr unsigned kLayerTicks = 2500;                  // a layer with a block on every unit, about
 constexpr int kFarLoad = 16;                // sc1: past this die's caches
 constexpr int kPace = 10;                   // loads of a streaming wave in flight while it sends ahead (3: 1,532 us a step of the 2B shape, 6: 1,489, 10: 1,460, 16: 1,458)
 // A wait ends when blocks that run have written.  Should it not end after some seconds (kChainTries questions) all the same, the block gives up: its results, with them the
@@ -566,7 +574,12 @@ decode_chain_kernel(const ChainArgs) {
                 if (__all(v == cap)) { count = cap; break; }
                 const unsigned f = lane < kCounters ? ld_far(frozen + lane * kLineWords) : 1u;
                 if (__all(f != 0u)) { count = f - 1u; break; }
-                if (!closing && wall_clock64() - t0 > kJoinTicks) {
+                const unsigned long long waited = wall_clock64() - t0;
+                if (!closing && waited > kJoinTicks) {
+                    unsigned here = lane < kCounters ? v & (kClosed - 1u) : 0u;
+                    for (int o = 1; o < kCounters; o <<= 1) here += __shfl_xor(here, o);
+                    const unsigned rounds = (unsigned)(a->G - 1) / max((unsigned)__builtin_amdgcn_readfirstlane((int)here), 1u);     // beyond the one that all together need
+                    if (waited < (unsigned long long)rounds * max(kJoinTicks, kLayerTicks * (unsigned)a->n_entries)) continue;
                     closing = true;
                     if (lane < kCounters) {
                         const unsigned old = __hip_atomic_fetch_or(joined + lane * kLineWords, kClosed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

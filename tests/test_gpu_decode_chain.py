@@ -304,3 +304,24 @@ def test_steps_ahead_of_rows_that_sampled_no_token(native):
         engine.cache.truncate("r%d" % i, n)
     got = engine.step_ahead(ents, sampled)
     assert got is not None and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("absent,rounds", [(1, 1), (100, 1), (192, 3), (240, 15)])
+def test_how_long_blocks_wait_for_others(absent, rounds):
+    """A round of the tasks beyond the first costs a step's time; blocks wait that long (a millisecond at least) for those that would spare it, before they begin without."""
+    engine, _ = _engine("1b", use_graphs=False)
+    _hold(engine, H.random_tokens(2003, 300, 3), [257])
+    forward = engine.native._lib.ic_decoder_forward_absent
+    engine.native._forward = lambda *args: forward(*args[:-1], absent, args[-1])
+    if engine.cu_count != 256:
+        pytest.skip("rounds are counted for 256 units")
+    took = []
+    for j in range(4):
+        events = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        torch.cuda.synchronize()
+        events[0].record()
+        _decode(engine, [5])
+        events[1].record()
+        torch.cuda.synchronize()
+        took.append(events[0].elapsed_time(events[1]))
+    assert _chained(engine) and rounds * 0.999 < min(took[1:]) < rounds * 1.0 + 5.0, took       # (ms; the clock is 100 MHz, the step itself under 3 ms with 16 blocks)
