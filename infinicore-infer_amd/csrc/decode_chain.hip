@@ -28,7 +28,7 @@
 // One row, us a step, kernel by kernel / so: 1B shape at 100, 600, 2,000 keys 1,380 / 995, 1,535 / 1,142, 1,553 / 1,229; 2B shape 1,621 / 1,333, 1,722 / 1,453,
 // 1,839 / 1,507.  Four rows: 1,514 / 1,162, 1,628 / 1,344, 1,725 / 1,423; 1,632 / 1,446, 1,730 / 1,567, 2,027 / 1,859.  What bounds it: each phase is about 1 us of products and
 // results and 1.5..2.5 for the slowest block's results to be seen, in which memory idles or brings the next weights; rows are read by every block, so it grows with them
-// (8 rows: 1.02..1.09 of the kernels' speed at the 1B shape, 0.98..1.03 at the 2B shape).
+// (`most_rows`).
 // Tried and no faster: two questions under way at a time (1,062 -> 1,124 us), pauses between them (1,080 at 4 x 64 cycles), up to 8 copies of what all blocks read
 // (1,063, 16: 1,097), loads for the next phase before a block's results are written (2B shape 1,458 -> 1,465), gate/up's first lines already while attention ends (1,448: what
 // it saves there the merging of the pieces loses), keys and values with QKV's weights (1,522).
@@ -1098,6 +1098,14 @@ bool instance(const ChainShape& s, const Plan& p) {
     return s.head_dim == 64 && group >= 1 && group <= kMaxGroup && ((p.pq == 1 && p.pg == 2 && p.rr == 1) || (p.pq == 2 && p.pg == 3 && p.rr == 2));
 }
 
+// Up to here one launch is faster than the kernels one by one.  Rows are read by every block, so its advantage falls with them.  Speed of the kernels over its own at 40, 600,
+// 2,000 keys and 2,000 beside 40: up to 2,048 wide (six shapes) 1.34..1.41, 1.26..1.32, 1.19..1.29 with one row, 1.04..1.12, 0.98..1.08, 1.02..1.11, 0.98..1.09 with eight (1.05 on average).
+// Wider, groups of 1 and 2 (2,304 36:36, 4,096 40:40, 2,112 64:32): 1.24..1.25, 1.18..1.21, 1.20..1.22 with one row, 1.03..1.08, 1.04..1.08, 1.02..1.07, 1.01..1.05 with seven, 1.00..1.05, 0.99..1.03,
+// 1.00..1.02, 0.98..1.00 with eight (0.96..0.98 with four to six of unlike lengths at one of them).  Groups of 3 and 4 (3,072 48:16, 2,304 64:16): 1.15..1.24, 1.11..1.17, 1.12..1.17; with five 1.08, 1.00..1.03, 1.04..1.07, 1.05..1.07, with six 1.03..1.06, 0.95..0.97, 1.01..1.03, 1.02..1.04,
+// with seven 1.00..1.04, 0.92..0.94, 0.99..1.01, 0.99..1.00.
+int most_rows(const ChainShape& s, const Plan& p) { return p.rr == 1 ? 8 : s.n_heads / s.n_kv_heads <= 2 ? 7 : 5; }
+static_assert(kChainMaxRows >= 8, "rows of the narrow sizes");
+
 template <int DH, int GQ, int PQ, int PG, int RR>
 int go(const ChainArgs& a, int blocks, size_t lds, hipStream_t stream) {
     static bool raised[64] = {};
@@ -1120,7 +1128,7 @@ int chain_supported(const ChainShape& s, int rows, int n_entries, int max_keys) 
     if (2LL * 2 * s.intermediate * s.hidden > 0x7fffffffLL || 2LL * (s.n_heads + 2 * s.n_kv_heads) * s.head_dim * s.hidden > 0x7fffffffLL) return 0;
     if (2LL * s.n_kv_heads * s.page_size * s.head_dim > 0xffffffffLL) return 0;      // (a page's bytes are multiplied in 32 bits)
     const Plan p = chain_plan(s);
-    if (!instance(s, p) || p.t_res > ic_rule_sumsq_parts_max()) return 0;      // (the head product takes the row factors)
+    if (!instance(s, p) || rows > most_rows(s, p) || p.t_res > ic_rule_sumsq_parts_max()) return 0;      // (the head product takes the row factors)
     const long long heads = (long long)rows * s.n_kv_heads, units = heads * ((max_keys + kUnit - 1) / kUnit);
     const long long keys = ((units + s.compute_units - 1) / s.compute_units + 6) * kUnit;
     const long long pieces = most_pieces(heads, units, s.compute_units);

@@ -129,3 +129,11 @@ def test_workspaces_that_are_not_aligned():
         at = lambda p: bool(d.lib.ic_decoder_takes_chain_at(d.h, ctypes.byref(d.step()), p))
         assert not at(1 << 20) and d.use() == 0
         assert at(1 << 20) and at((1 << 20) + 16) and not at((1 << 20) + 4) and not at((1 << 20) + 8)
+
+
+@pytest.mark.parametrize("hidden,heads,kv,inner,most", [(1536, 24, 8, 3840, 8), (2048, 32, 16, 4096, 8), (1088, 16, 4, 2176, 8), (2304, 36, 36, 5760, 7), (2112, 64, 32, 6144, 7),
+                                                        (3072, 48, 16, 4352, 5), (2304, 64, 16, 6080, 5)])
+def test_rows_up_to_which_one_launch_is_faster(hidden, heads, kv, inner, most):
+    with Decoder(hidden=hidden, heads=heads, kv=kv, inner=inner) as d:
+        assert d.use() == 0
+        assert [d.takes(rows, 600) for rows in range(1, 10)] == [rows <= most for rows in range(1, 10)]

@@ -71,7 +71,7 @@ def test_rows_and_lengths(shape, page_size):
             assert err < 2e-2, (shape, lens, j, err)
         for e in (a, b):
             _drop(e, len(lens))
-    assert taken == 3 * (len(LENS) - (shape == "2b"))        # (288 heads of up to 2,560 keys: more pieces than a block has room for)
+    assert taken == 3 * sum(len(lens) <= (7 if shape == "2b" else 8) for lens in LENS)      # (more rows of the wide shape are faster kernel by kernel)
 
 
 @pytest.mark.parametrize("shape", ["%d-%d-%d-%d" % o for o in OTHERS])
