@@ -55,6 +55,7 @@ constexpr int kCounters = 32;              // of the blocks that have come, a ca
 constexpr int kLineWords = 32;
 constexpr unsigned kClosed = 0x10000u;
 constexpr int kMaxPieces = 40;              // of a block's attention work
+constexpr int DH = 64;                     // elements of a head
 constexpr int kMaxGroup = 4;               // query heads of a kv head
 constexpr int kMaxPageIds = 2048;
 constexpr int kUnit = 64;                  // keys of a unit of attention work
@@ -130,6 +131,7 @@ struct Shared {
     float own[kMaxPieces][kMaxGroup];      // scores of the step's own keys, units of log 2
     int ids[kMaxPageIds];
 };
+static_assert(sizeof(Shared) % alignof(ChainEntry) == 0, "the layers' table lies behind it");
 
 // ---- streaming waves: products --------------------------------------------------------------------------------------------
 // The four products of a layer.  RG: groups of 8 weight rows of a task; EPI as in gemm_rows.hip.
@@ -154,7 +156,7 @@ template <int KIND> __device__ __forceinline__ Far weights_of(const ChainEntry* 
 
 // Byte offsets of this lane's rows of task t.
 template <int KIND, int RG>
-__device__ __forceinline__ void row_offsets(Args a, int t, int K, int lane, int dh, unsigned (&off)[RG]) {
+__device__ __forceinline__ void row_offsets(Args a, int t, int K, int lane, unsigned (&off)[RG]) {
     const int r8 = lane & 7, hi = (lane >> 3) & 1, kq = lane >> 4, col8 = 8 * (kq + 4 * hi);
 #pragma unroll
     for (int g = 0; g < RG; ++g) {
@@ -164,10 +166,10 @@ __device__ __forceinline__ void row_offsets(Args a, int t, int K, int lane, int 
             row = t * (4 * RG) + 8 * (g % (RG / 2)) + r8 + up;
             last = a->di - 1 + up;
         } else if constexpr (KIND == QKV) {
-            const int pair = t * (RG / 2) + (g >> 1), per_head = dh >> 4;
+            const int pair = t * (RG / 2) + (g >> 1), per_head = DH >> 4;
             const int head = pair / per_head, j = 8 * (pair - head * per_head);
-            row = head * dh + r8 + (head < a->nh + a->nkv ? j + (g & 1) * (dh >> 1) : 2 * j + 8 * (g & 1));
-            last = (a->nh + 2 * a->nkv) * dh - 1;
+            row = head * DH + r8 + (head < a->nh + a->nkv ? j + (g & 1) * (DH >> 1) : 2 * j + 8 * (g & 1));
+            last = (a->nh + 2 * a->nkv) * DH - 1;
         } else {
             row = t * a->cols + 8 * g + r8;
             last = min((t + 1) * a->cols, a->d) - 1;
@@ -200,7 +202,7 @@ __device__ __forceinline__ void send_line(Far w, int line, const unsigned (&off)
 template <int RG> constexpr int kLines = kRing / RG < kLinesAhead ? kRing / RG : kLinesAhead;      // of a product that the ring holds
 
 // A task's first lines into the ring.
-template <int KIND, int RG, int DH>
+template <int KIND, int RG>
 __device__ __forceinline__ void send_ahead(Args a, const ChainEntry* E, int t, int lane, int wave, uint4* ring) {
     a = again(a);
     lane = again_v(lane);
@@ -208,7 +210,7 @@ __device__ __forceinline__ void send_ahead(Args a, const ChainEntry* E, int t, i
     const int K = depth_of<KIND>(a), nl = ((K >> 6) - wave + kStream - 1) / kStream;
     const Far w = weights_of<KIND>(E);
     unsigned off[RG];
-    row_offsets<KIND, RG>(a, t, K, lane, DH, off);
+    row_offsets<KIND, RG>(a, t, K, lane, off);
 #pragma unroll
     for (int s = 0; s < kLines<RG>; ++s)
         if (s < nl) {
@@ -216,7 +218,7 @@ __device__ __forceinline__ void send_ahead(Args a, const ChainEntry* E, int t, i
         } else clear(ring + s * RG, RG);
 }
 
-template <int KIND, int RG, int DH>
+template <int KIND, int RG>
 __device__ __forceinline__ void multiply(Args a, const ChainEntry* E, int t, int lane, int wave, uint4* ring, const unsigned char* rows, float* red) {
     constexpr int S = kLines<RG>, OUT = RG * 64;
     a = again(a);
@@ -238,7 +240,7 @@ __device__ __forceinline__ void multiply(Args a, const ChainEntry* E, int t, int
     if (left > S) {
         const Far w = weights_of<KIND>(E);
         unsigned off[RG];
-        row_offsets<KIND, RG>(a, t, K, lane, DH, off);
+        row_offsets<KIND, RG>(a, t, K, lane, off);
         while (left >= 2 * S) {
 #pragma unroll
             for (int s = 0; s < S; ++s) {
@@ -318,7 +320,7 @@ __device__ void plan_pieces(Args a, Shared& sh, int w) {
     sh.n_ids = ids;
 }
 
-template <int DH, int GQ> struct Heads {
+template <int GQ> struct Heads {
     static constexpr int LPK = DH / 8;                       // lanes that share a key's row
     static_assert((GQ + 2) * LPK <= 64, "a piece's queries, its new key and value are one chunk");
     // One query head a kv head: a lane group of LPK walks every KPW-th key.  Several: tiles of 32 keys on the matrix cores.
@@ -341,9 +343,9 @@ __device__ __forceinline__ Piece piece_of(const Shared& sh, int i) {
 }
 
 // Stage `stage` of a piece's cached keys and values; keys beyond them read the last one.
-template <int DH, int GQ>
+template <int GQ>
 __device__ __forceinline__ void send_keys(Args a, const Shared& sh, const Piece& p, Far kc, Far vc, int stage, int lane, int wave, uint4* dst) {
-    using H = Heads<DH, GQ>;
+    using H = Heads<GQ>;
     a = again(a);
     lane = again_v(lane);
     const int sub = lane % H::LPK, grp = lane / H::LPK;
@@ -374,10 +376,10 @@ __device__ __forceinline__ float dot2(unsigned a, unsigned b, float c) {
 }
 
 // A piece's cached keys, first stages sent ahead: the waves' softmax states (maximum in units of log 2, sum, weighted values) to `state`.
-template <int DH, int GQ>
+template <int GQ>
 __device__ __forceinline__ void walk_piece(Args a, const Shared& sh, const Piece& p, Far kc, Far vc, int lane, int wave, uint4 (&ring)[kRing],
                                            const uint16_t* queries, uint16_t* tile, float* state) {
-    using H = Heads<DH, GQ>;
+    using H = Heads<GQ>;
     a = again(a);
     lane = again_v(lane);
     const int hi = min(p.hi, p.pos), ns = (max(hi - p.lo, 0) + H::STEP - 1) / H::STEP;
@@ -389,7 +391,7 @@ __device__ __forceinline__ void walk_piece(Args a, const Shared& sh, const Piece
             for (int s = 0; s < H::S; ++s) {
                 take(st + s, ring + s * H::SLOTS);
                 __builtin_amdgcn_sched_barrier(0);
-                send_keys<DH, GQ>(a, sh, p, kc, vc, st + s + H::S, lane, wave, ring + s * H::SLOTS);
+                send_keys<GQ>(a, sh, p, kc, vc, st + s + H::S, lane, wave, ring + s * H::SLOTS);
             }
             left -= H::S;
             st += H::S;
@@ -400,7 +402,7 @@ __device__ __forceinline__ void walk_piece(Args a, const Shared& sh, const Piece
             for (int s = 0; s < H::S; ++s) {
                 take(st + s, ring + s * H::SLOTS);
                 __builtin_amdgcn_sched_barrier(0);
-                if (s < more) send_keys<DH, GQ>(a, sh, p, kc, vc, st + s + H::S, lane, wave, ring + s * H::SLOTS);
+                if (s < more) send_keys<GQ>(a, sh, p, kc, vc, st + s + H::S, lane, wave, ring + s * H::SLOTS);
             }
             left -= H::S;
             st += H::S;
@@ -450,10 +452,7 @@ __device__ __forceinline__ void walk_piece(Args a, const Shared& sh, const Piece
 #pragma unroll
         for (int o = H::LPK; o < 64; o <<= 1) mw = fmaxf(mw, lane_xor(mw, o));
         const float c = __builtin_amdgcn_exp2f(m - (mw == -INFINITY ? 0.f : mw));
-        auto sum = [&](float v) {
-            if (H::LPK <= 8) v = dpp_add<0x128>(v);
-            return swap_add<32>(swap_add<16>(v));
-        };
+        auto sum = [&](float v) { return swap_add<32>(swap_add<16>(dpp_add<0x128>(v))); };
         l = sum(l * c);
 #pragma unroll
         for (int i = 0; i < 8; ++i) acc[i] = sum(acc[i] * c);
@@ -541,11 +540,11 @@ __device__ __forceinline__ void walk_piece(Args a, const Shared& sh, const Piece
 }
 
 // ---- the kernel -------------------------------------------------------------------------------------------------------------------
-template <int DH, int GQ, int PQ, int PG, int RR>
+template <int GQ, int PQ, int PG, int RR>
 __global__ void __launch_bounds__(kThreads)
 decode_chain_kernel(const ChainArgs) {
     Args a = (Args)__builtin_amdgcn_kernarg_segment_ptr();
-    using H = Heads<DH, GQ>;
+    using H = Heads<GQ>;
     extern __shared__ __align__(16) unsigned char ch_smem[];
     unsigned char* const rows = ch_smem;                                    // token rows [line of 64][row][128 bytes]; staged queries
     float* const red = reinterpret_cast<float*>(ch_smem + a->rows_bytes);    // partial results of the waves; their softmax states
@@ -644,9 +643,9 @@ decode_chain_kernel(const ChainArgs) {
             constexpr int KIND = kind, RG = groups;
             for (int t = rank; t < tasks_of<KIND>(a); t += n) {
                 uint4 ring[kRing];
-                send_ahead<KIND, RG, DH>(a, E, t, lane, wave, ring);
+                send_ahead<KIND, RG>(a, E, t, lane, wave, ring);
                 meet();
-                multiply<KIND, RG, DH>(a, E, t, lane, wave, ring, rows, red);
+                multiply<KIND, RG>(a, E, t, lane, wave, ring, rows, red);
                 meet();
                 meet();                                      // the results are on their way
             }
@@ -666,10 +665,10 @@ decode_chain_kernel(const ChainArgs) {
                     uint4 ring[kRing];
 #pragma unroll
                     for (int s = 0; s < H::S; ++s)
-                        if (hi > p.lo + s * H::STEP) send_keys<DH, GQ>(a, sh, p, kc, vc, s, lane, wave, ring + s * H::SLOTS);
+                        if (hi > p.lo + s * H::STEP) send_keys<GQ>(a, sh, p, kc, vc, s, lane, wave, ring + s * H::SLOTS);
                         else clear(ring + s * H::SLOTS, H::SLOTS);
                     if (i == 0) meet();                      // the queries
-                    walk_piece<DH, GQ>(a, sh, p, kc, vc, lane, wave, ring, reinterpret_cast<const uint16_t*>(rows + 1024 * i), tile, red + (i & 1) * kStream * H::STATE);
+                    walk_piece<GQ>(a, sh, p, kc, vc, lane, wave, ring, reinterpret_cast<const uint16_t*>(rows + 1024 * i), tile, red + (i & 1) * kStream * H::STATE);
                     meet();
                 }
                 meet();                                      // the plan has been used, the results are on their way
@@ -864,9 +863,7 @@ decode_chain_kernel(const ChainArgs) {
                 for (int i = 0; i < np; ++i) {               // the score of the step's own key, while the others are walked
                     const uint16_t* const at = reinterpret_cast<const uint16_t*>(rows + 1024 * i);
                     for (int j = cw; j < GQ; j += kControl) {
-                        float d = 0.f;
-#pragma unroll
-                        for (int c = 0; c < DH; c += 64) d = fmaf(bf16_bits_to_f32(at[j * DH + c + lane]), bf16_bits_to_f32(at[GQ * DH + c + lane]), d);
+                        float d = bf16_bits_to_f32(at[j * DH + lane]) * bf16_bits_to_f32(at[GQ * DH + lane]);
                         d = wave_sum(d) * b->scale * 1.4426950408889634f;
                         if (lane == 0) sh.own[i][j] = d;
                     }
@@ -1095,7 +1092,7 @@ size_t lds_bytes(const ChainShape& s, const Plan& p, int T, int n_entries, int* 
 // columns of the residual stream (up to 2,048 wide on 256 units), or two, three and 16 (up to 4,096 wide).
 bool instance(const ChainShape& s, const Plan& p) {
     const int group = s.n_heads / s.n_kv_heads;
-    return s.head_dim == 64 && group >= 1 && group <= kMaxGroup && ((p.pq == 1 && p.pg == 2 && p.rr == 1) || (p.pq == 2 && p.pg == 3 && p.rr == 2));
+    return s.head_dim == DH && group >= 1 && group <= kMaxGroup && ((p.pq == 1 && p.pg == 2 && p.rr == 1) || (p.pq == 2 && p.pg == 3 && p.rr == 2));
 }
 
 // Up to here one launch is faster than the kernels one by one.  Rows are read by every block, so its advantage falls with them.  Speed of the kernels over its own at 40, 600,
@@ -1106,17 +1103,17 @@ bool instance(const ChainShape& s, const Plan& p) {
 int most_rows(const ChainShape& s, const Plan& p) { return p.rr == 1 ? 8 : s.n_heads / s.n_kv_heads <= 2 ? 7 : 5; }
 static_assert(kChainMaxRows >= 8, "rows of the narrow sizes");
 
-template <int DH, int GQ, int PQ, int PG, int RR>
+template <int GQ, int PQ, int PG, int RR>
 int go(const ChainArgs& a, int blocks, size_t lds, hipStream_t stream) {
     static bool raised[64] = {};
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return IC_ERR_UNSUPPORTED;
     if (!raised[dev]) {
-        const hipError_t st = hipFuncSetAttribute((const void*)decode_chain_kernel<DH, GQ, PQ, PG, RR>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        const hipError_t st = hipFuncSetAttribute((const void*)decode_chain_kernel<GQ, PQ, PG, RR>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (st != hipSuccess) { (void)hipGetLastError(); return (int)st; }
         raised[dev] = true;
     }
-    hipLaunchKernelGGL((decode_chain_kernel<DH, GQ, PQ, PG, RR>), dim3(blocks), dim3(kThreads), lds, stream, a);
+    hipLaunchKernelGGL((decode_chain_kernel<GQ, PQ, PG, RR>), dim3(blocks), dim3(kThreads), lds, stream, a);
     return ic_launch_status();
 }
 
@@ -1160,16 +1157,16 @@ int chain_launch(const ChainShape& s, const ChainStep& st, int absent, hipStream
     const int e = ic_launch_status();
     if (e) return e;
     const int group = s.n_heads / s.n_kv_heads;
-#define CH_GO(DH, GQ, PQ, PG, RR)                                                                            \
-    if (s.head_dim == DH && group == GQ && p.pq == PQ && p.pg == PG && p.rr == RR) return go<DH, GQ, PQ, PG, RR>(a, s.compute_units - absent, lds, stream)
-    CH_GO(64, 1, 1, 2, 1);
-    CH_GO(64, 2, 1, 2, 1);
-    CH_GO(64, 3, 1, 2, 1);
-    CH_GO(64, 4, 1, 2, 1);
-    CH_GO(64, 1, 2, 3, 2);
-    CH_GO(64, 2, 2, 3, 2);
-    CH_GO(64, 3, 2, 3, 2);
-    CH_GO(64, 4, 2, 3, 2);
+#define CH_GO(GQ, PQ, PG, RR)                                                                                \
+    if (group == GQ && p.pq == PQ && p.pg == PG && p.rr == RR) return go<GQ, PQ, PG, RR>(a, s.compute_units - absent, lds, stream)
+    CH_GO(1, 1, 2, 1);
+    CH_GO(2, 1, 2, 1);
+    CH_GO(3, 1, 2, 1);
+    CH_GO(4, 1, 2, 1);
+    CH_GO(1, 2, 3, 2);
+    CH_GO(2, 2, 3, 2);
+    CH_GO(3, 2, 3, 2);
+    CH_GO(4, 2, 3, 2);
 #undef CH_GO
     return IC_ERR_UNSUPPORTED;
 }
