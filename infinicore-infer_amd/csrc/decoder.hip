@@ -25,8 +25,9 @@ namespace {
 // forward both ask those functions, so a rule is written once.
 constexpr int kFewRows = 16;        // up to here the few-row products beat the library
 constexpr int kMidRows = 64;        // up to here the sliced product beats it for results as wide as the model
-// Layers from which on a decode step runs them in one launch: each layer saves 6 us at one row of the 1B and 2B shapes (1B shape, 600 keys: 93.4 -> 79.8 us with three
-// layers, 223.8 -> 183.8 with eight), starting costs 4.  One and two layers save 3 and 8 us and stay kernel by kernel, as the steps issued from Python are.
+// Layers from which on a decode step runs them in one launch.  Not a line of speed: each layer saves 6 us at one row of the 1B and 2B shapes (1B shape, 600 keys: 93.4 -> 79.8
+// us with three layers, 223.8 -> 183.8 with eight), starting costs 4, so one and two layers would save 3 and 8 us too.  They stay kernel by kernel for the sake of
+// comparison: such steps equal those issued from Python bit for bit, on the layer sizes that deeper models have.
 constexpr int kChainMinEntries = 3;
 constexpr int kMaxSumsqParts = 256; // column blocks of sums of squares a product takes as row factors
 

@@ -6,7 +6,9 @@ kernel from the parts' Python ``forward``.  The reference's step function is nat
 It is a capability, not a requirement: a model takes this path when every part of it has a
 native description (``Part.native_desc``); any other model is stepped by its parts' ``forward``
 as before.  Both paths launch the same kernels with the same arguments, so their logits are
-bit-equal (tested).
+bit-equal (tested), but for the decode steps whose layers run in one launch (csrc/decode_chain.hip: up to 8 rows in
+bfloat16 of three layers and more, of the sizes that it takes): there sums run in another order, and the two paths are
+each as far from 64 bits and differ from one another by up to 2e-2 of the logits' norm (tested).
 """
 import ctypes
 from itertools import chain

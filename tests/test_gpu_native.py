@@ -1,7 +1,9 @@
 """The step issued by one native call against the same step issued kernel by kernel from the parts'
 Python forward: the logits must be bit-equal, since both launch the same kernels with the same
 arguments.  (Each path is compared with the plain implementation elsewhere; the engine's default is
-the native one.)"""
+the native one.)  Not so the decode steps whose layers run in one launch: the models here that have three layers
+and more have sizes that it does not take, those of its sizes two layers, and the last test has the steps
+of four layers on either side of its line."""
 import pytest
 import torch
 
@@ -170,3 +172,19 @@ def test_the_c_step_function_through_ctypes(tmp_path_factory):
     # a batch that does not add up is refused before anything is launched
     bad = IcHostBatch(5, 1, 0, 0, 0, 0, 0, 0, 0, 128, 0)
     assert lib.ic_decoder_step_ints(dec, ctypes.byref(bad)) == -1
+
+
+@pytest.mark.parametrize("rows", [1, 8, 9, 16, 20])
+def test_native_steps_of_more_layers(rows):
+    """Four layers of the 1B shape: up to 8 rows run in one launch and are near the Python-issued steps (the bound of test_gpu_decode_chain.py), more rows equal them bit for bit."""
+    from infinicore_infer_amd.engine import StepEntry
+    from test_gpu_large import SHAPE_1B, _engine_and_weights
+    out, took = [], []
+    for native in (True, False):
+        engine = _engine_and_weights(dict(SHAPE_1B, vocab_size=2003, num_hidden_layers=4), 21, 0.02, 24 * 320, 24, use_native=native, use_graphs=False)[0]
+        engine.step([StepEntry("r%d" % i, H.random_tokens(2003, 20 + 13 * i, i), []) for i in range(rows)])
+        out.append(engine.step([StepEntry("r%d" % i, [5 + i], [0]) for i in range(rows)]).clone())
+        if native:
+            took = bool(engine.native._lib.ic_decoder_takes_chain(engine.native._h, engine.native._batch_ref))
+    assert took == (rows <= 8)
+    assert float((out[0] - out[1]).norm() / out[1].norm()) < 2e-2 if took else torch.equal(*out)
