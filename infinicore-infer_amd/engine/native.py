@@ -84,8 +84,9 @@ class NativeDecoder:
         host = torch.empty(self._lib.ic_decoder_table_bytes(n_entries), dtype=torch.uint8)
         if self._lib.ic_decoder_layer_table(self._h, host.data_ptr()) == 1:
             self._layer_table = host.to(device)          # a copy on the current stream, which has ended when this returns: any stream may read it
-            self._gave_up = torch.zeros(1, dtype=torch.int32, pin_memory=True)
-            if self._lib.ic_decoder_use_layer_table(self._h, self._layer_table.data_ptr(), self._gave_up.data_ptr()):
+            flag = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+            self._gave_up = flag.numpy()                 # (which keeps the tensor's memory)
+            if self._lib.ic_decoder_use_layer_table(self._h, self._layer_table.data_ptr(), flag.data_ptr()):
                 raise KernelError("native step: the layers' table was refused")
 
     def check(self) -> None:
