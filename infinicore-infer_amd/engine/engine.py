@@ -161,6 +161,7 @@ class Engine:
         from .native import NativeDecoder
         self.native = NativeDecoder.try_build(self) if use_native else None
         self.native_steps = 0
+        self._in_doubt = -1          # steps up to this one were issued before one of them was found to have no results
 
     # ---- construction -----------------------------------------------------------------
     @classmethod
@@ -228,7 +229,7 @@ class Engine:
         or the next step."""
         if not entries:
             return None
-        self._check_native()
+        self._check_results(None)
         if self.use_graphs and len(entries) <= self.graph_max_batch:
             starts = self._append_single_tokens(entries)
             if starts is not None:                   # a pure decode step: the lean way through the same checks
@@ -319,6 +320,7 @@ class Engine:
         if (not self.use_graphs or R == 0 or R > self.graph_max_batch or self._has_window
                 or device_tokens is None or device_tokens.numel() != R or device_tokens.dtype != torch.int32):
             return None
+        self._check_results(self.steps_run)          # (the tokens are the last step's)
         reqs = self.cache.requests
         longest = 0
         for e in entries:
@@ -682,12 +684,20 @@ class Engine:
             host = self._sampled_host = torch.empty(max(R, self.graph_max_batch, 1), dtype=torch.int32, pin_memory=True)
         host[:R].copy_(out, non_blocking=True)
         torch.cuda.current_stream().synchronize()
-        self._check_native()
+        self._check_results(self.steps_run)
         return host[:R].tolist()
 
-    def _check_native(self):
-        if self.native is not None:
-            self.native.check()
+    def _check_results(self, step: Optional[int]):
+        """Raises when a step that has been waited for has no results, and for every step issued before that was found:
+        their tokens may stem from it."""
+        try:
+            if self.native is not None:
+                self.native.check()
+        except ops.KernelError:
+            self._in_doubt = self.steps_run
+            raise
+        if step is not None and step <= self._in_doubt:
+            raise ops.KernelError("a step before this one ended without results; the requests that took part are to be freed")
 
     def sample_ahead(self, logits, temperature=None, top_k=None, top_p=None, uniform=None):
         """As ``sample``, without waiting for the device: returns (the tokens on the device, int32 [rows], and a
@@ -709,7 +719,7 @@ class Engine:
         self._ahead_turn ^= 1
         b = self._ahead_out[self._ahead_turn]
         b["done"].synchronize()                     # what this set of buffers held two calls ago has been copied out
-        out, host, done = b["tokens"][:R], b["host"], b["done"]
+        out, host, done, issued = b["tokens"][:R], b["host"], b["done"], self.steps_run
         if temperature is None:
             ops.argmax(logits, out, self.ws.buffer("argmax_val", (64 * R,), torch.float32),
                        self.ws.buffer("argmax_idx", (64 * R,), torch.int32))
@@ -725,7 +735,7 @@ class Engine:
 
         def wait() -> List[int]:
             done.synchronize()
-            self._check_native()
+            self._check_results(issued)
             return host[:R].tolist()
         return out, wait
 

@@ -325,3 +325,26 @@ def test_how_long_blocks_wait_for_others(absent, rounds):
         torch.cuda.synchronize()
         took.append(events[0].elapsed_time(events[1]))
     assert _chained(engine) and rounds * 0.999 < min(took[1:]) < rounds * 1.0 + 5.0, took       # (ms; the clock is 100 MHz, the step itself under 3 ms with 16 blocks)
+
+
+def test_steps_issued_before_one_was_found_without_results():
+    """While the host has not seen a step's tokens, the step after it is under way from them: it is refused too, and so is one that would go on from it; then the flag (set here by the
+    host, as the device does) is forgotten."""
+    from infinicore_infer_amd.engine import StepEntry
+    from infinicore_infer_amd.kernels.lib import KernelError
+    engine, _ = _engine("1b", graph_after=1)
+    _hold(engine, H.random_tokens(2003, 90, 3), [70, 50])
+    ents = [StepEntry("r%d" % i, [0], [0]) for i in range(2)]
+    engine.sample(_decode(engine, [5, 6]))                   # recorded
+    first, wait_first = engine.sample_ahead(_decode(engine, [7, 8]))
+    second, wait_second = engine.sample_ahead(engine.step_ahead(ents, first))
+    assert _chained(engine)
+    torch.cuda.synchronize()
+    engine.native._gave_up[0] = 1
+    held = engine.length("r0")
+    for refused in (wait_first, wait_second, lambda: engine.step_ahead(ents, second)):
+        with pytest.raises(KernelError, match="gave up|without results"):
+            refused()
+    assert engine.length("r0") == held and engine.native._gave_up[0] == 0
+    logits = engine.step([StepEntry("r0", [3], [0])])
+    assert len(engine.sample(logits)) == 1
