@@ -1,4 +1,4 @@
-// All layers of a decode step in one launch, for up to 8 rows in bfloat16 (sizes: `instance` below).
+// All layers of a decode step in one launch, for up to 8 rows in bfloat16 (sizes: `instance` below, rows: `most_rows`).
 //
 // Why: with few rows a layer is five or six kernels of 5..12 us each, of which 2..5 go by before the first weights are there and after the last block has ended; the
 // 1B shape's layer brings 48 MB, 6.8 us at 7.1 TB/s, and took 28.  Here one block a compute unit stays for the whole step.  Its 12 waves have two trades:
